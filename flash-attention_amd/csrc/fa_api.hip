@@ -120,6 +120,35 @@ SplitPlan split_plan(int batch, int nheads, int head_dim, int total_q, int max_s
   return sp;
 }
 
+// Forward of at most kDecodeMaxQ query rows per sequence without mask, dropout or bias: fa_decode_kernel, while the
+// (batch, head) pairs are at most 1024.  Measured (one new token, us, fa_fwd_kernel with its own key split / fa_decode_kernel):
+// 128 pairs d = 128 up to 4096 keys 95 / 41, 16 pairs d = 128 12000 keys 31 / 27, 208 pairs d = 64 1866 keys 31 / 29, 512 pairs
+// d = 128 up to 300 keys 16 / 13.5, 1024 pairs d = 64 70 keys 11 / 8; with 1600 and 3200 pairs the forward kernel's smaller LDS keeps
+// more workgroups on a compute unit and the two are equal for long caches (46 / 46 at 512 keys) or it wins (9.7 / 12.3 at 64 keys).
+bool decode_launch(int batch, int nheads, int max_sq, bool causal, bool sparse, bool dropout, bool bias) {
+  return max_sq <= fa::kDecodeMaxQ && (int64_t)batch * nheads <= 1024 && !causal && !sparse && !dropout && !bias;
+}
+// Its key splits: as many as give every compute unit two workgroups (what its LDS holds; with four or eight per compute unit the
+// same launches take 2 to 20 % longer, a workgroup's start and the merging cost more than the evener load saves), each at least
+// two rounds of its waves' 32-key tiles (8 pairs with 300 keys at d = 64: 8 us split into single rounds, 6 us not split).
+SplitPlan decode_plan(int batch, int nheads, int head_dim, int total_q, int max_sk, int sq_r, int* split_keys) {
+  SplitPlan sp{1, 0, 0};
+  const int round = 32 * fa::kDecodeWaves(head_dim);
+  const int64_t rounds = ((int64_t)max_sk + round - 1) / round, pairs = (int64_t)batch * nheads;
+  int64_t n = (512 + pairs - 1) / pairs;
+  if (n > rounds / 2) n = rounds / 2;
+  if (n > 64) n = 64;
+  if (n < 1) n = 1;
+  const int64_t per = (rounds + n - 1) / n;
+  *split_keys = (int)(per * round);
+  n = (rounds + per - 1) / per;
+  if (n < 2) return sp;
+  sp.n_splits = (int)n;
+  sp.o_bytes = align16((size_t)n * total_q * nheads * head_dim * 4);
+  sp.bytes = sp.o_bytes + align16((size_t)n * batch * nheads * sq_r * 4);
+  return sp;
+}
+
 int build_maps(const int32_t* blockmask, const int32_t* row_order, unsigned char* ws, const SparseLayout& sl,
                fa::SparseMaps* out, hipStream_t stream) {
   FA_LAUNCH(fa::launch_fill_f32(reinterpret_cast<float*>(ws), sl.bytes / 4, 0.f, stream));
@@ -274,15 +303,20 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
     p.kw_kb = (int)fa::keep_words_key_blocks(a->max_seqlen_k);
   }
   // short query side, long key side: split the keys over several workgroups if the caller brought the scratch for it
-  const SplitPlan sp = split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
-                                  a->is_causal != 0, sparse);
+  const bool decode = decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->is_causal != 0, sparse, dropout,
+                                    a->alibi_slopes || a->attn_bias);
+  const SplitPlan sp = decode ? decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &p.split_keys)
+                              : split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
+                                           a->is_causal != 0, sparse);
   const bool split = sp.n_splits > 1 && a->workspace && a->workspace_bytes >= sp.bytes && aligned16(a->workspace);
+  if (decode && !split) p.split_keys = a->max_seqlen_k;
   if (split) {
     p.n_splits = sp.n_splits;
     p.o_part = reinterpret_cast<float*>(a->workspace);
     p.lse_part = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(a->workspace) + sp.o_bytes);
   }
-  FA_LAUNCH(fa::launch_fwd(p, a->dtype, a->head_dim, a->is_causal != 0, dropout, sparse, stream));
+  if (decode) FA_LAUNCH(fa::launch_decode(p, a->dtype, a->head_dim, stream));
+  else FA_LAUNCH(fa::launch_fwd(p, a->dtype, a->head_dim, a->is_causal != 0, dropout, sparse, stream));
   if (split) FA_LAUNCH(fa::launch_fwd_combine(p, a->dtype, a->head_dim, stream));
 
   if (a->s_dmask) {
@@ -525,6 +559,11 @@ size_t fa_fwd_workspace_bytes(const fa_fwd_args* a) {
   if (!a) return 0;
   if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes;
   const Rounded r = round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, false);
+  if (decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->is_causal != 0, false, a->p_dropout > 0.f,
+                    a->alibi_slopes || a->attn_bias)) {
+    int split_keys;
+    return decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &split_keys).bytes;
+  }
   return split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
                     a->is_causal != 0, false).bytes;
 }

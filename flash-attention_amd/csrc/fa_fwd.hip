@@ -37,6 +37,13 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(const FwdParams p, int
   const int b = (int)(t / cpr / p.max_sq / p.H);
   int q_begin, Lq;
   if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq) || row >= Lq) return;
+  // fa_decode_kernel's splits are a number of keys each: a short sequence has fewer of them
+  int n_splits = p.n_splits;
+  if (p.split_keys > 0) {
+    int k_begin, Lk;
+    if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;
+    n_splits = (Lk + p.split_keys - 1) / p.split_keys;
+  }
   // The splits are read eight at a time, all loads of a group in flight together: with few query rows (decoding) the
   // kernel has a handful of workgroups and its time is the latency of this loop, not bandwidth.
   constexpr int U = 8;
@@ -44,35 +51,33 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(const FwdParams p, int
   const int64_t lstep = (int64_t)p.B * p.H * p.sq_r;
   const float* opart = p.o_part + ((int64_t)(q_begin + row) * p.H + h) * D + ch * 4;
   const int64_t ostep = (int64_t)p.total_q * p.H * D;
-  float m = -INFINITY;
-  for (int s0 = 0; s0 < p.n_splits; s0 += U) {
-    float l[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) l[u] = s0 + u < p.n_splits ? lp[(s0 + u) * lstep] : -INFINITY;
-#pragma unroll
-    for (int u = 0; u < U; u++) m = fmaxf(m, l[u]);
-  }
-  float sum = 0.f;
+  float m = -INFINITY, sum = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (m > -INFINITY) {
-    for (int s0 = 0; s0 < p.n_splits; s0 += U) {
-      float l[U];
-      f32x4 o[U];
+  for (int s0 = 0; s0 < n_splits; s0 += U) {
+    float l[U];
+    f32x4 o[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const bool in = s0 + u < p.n_splits;
-        l[u] = in ? lp[(s0 + u) * lstep] : -INFINITY;
-        o[u] = in ? *reinterpret_cast<const f32x4*>(opart + (s0 + u) * ostep) : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const float w = __expf(l[u] - m);  // 0 for a split past the end or without keys
-        sum += w;
-        acc = acc + o[u] * w;
-      }
+    for (int u = 0; u < U; u++) {
+      const bool in = s0 + u < n_splits;
+      l[u] = in ? lp[(s0 + u) * lstep] : -INFINITY;
+      o[u] = in ? *reinterpret_cast<const f32x4*>(opart + (s0 + u) * ostep) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    acc = acc * (1.f / sum);
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < U; u++) mn = fmaxf(mn, l[u]);
+    if (mn == -INFINITY) continue;
+    const float alpha = __expf(m - mn);  // 0 while nothing has been summed
+    m = mn;
+    sum *= alpha;
+    acc = acc * alpha;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float w = __expf(l[u] - m);  // 0 for a split past the end or without keys
+      sum += w;
+      acc = acc + o[u] * w;
+    }
   }
+  if (m > -INFINITY) acc = acc * (1.f / sum);
   if (ch == 0) p.lse[((int64_t)b * p.H + h) * p.sq_r + row] = m > -INFINITY ? m + __logf(sum) : -INFINITY;
   T* op = reinterpret_cast<T*>(p.o) + (int64_t)(q_begin + row) * p.o_rs + (int64_t)h * p.o_hs + ch * 4;
   *reinterpret_cast<typename Elem<T>::vec4*>(op) = cvt4<T>(acc);

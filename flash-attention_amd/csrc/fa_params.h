@@ -74,6 +74,7 @@ struct FwdParams {
   // and writes its normalised fp32 output and its lse to o_part [n_splits, total_q, H, d] / lse_part
   // [n_splits, B, H, sq_r]; fwd_combine_kernel merges them into o / lse.  n_splits <= 1: single pass.
   int n_splits;
+  int split_keys;  // fa_decode_kernel: keys per split (a multiple of its waves' 32-key tiles); 0: shares of fa_fwd_kernel's tiles
   float* o_part;
   float* lse_part;
   const float* alibi;  // null, or one slope per head: the score of (query i, key j) gets -slope * |i - j| added
@@ -299,6 +300,8 @@ inline bool merged_backward_launch(int head_dim, int BH, int max_sq, bool causal
 // p.alibi != null selects the ALiBi variants (not available together with sparse)
 hipError_t launch_fwd(const FwdParams& p, int dtype, int head_dim, bool causal, bool dropout, bool sparse,
                       hipStream_t stream);
+// A few query rows (at most kDecodeMaxQ) against many keys: fa_decode_kernel (fa_decode.hip)
+hipError_t launch_decode(const FwdParams& p, int dtype, int head_dim, hipStream_t stream);
 hipError_t launch_fwd_combine(const FwdParams& p, int dtype, int head_dim, hipStream_t stream);
 hipError_t launch_dq_combine(const BwdParams& p, int dtype, int head_dim, hipStream_t stream);
 // The whole backward in one kernel (fa_bwd_fused_kernel.h; head_dim 64, dense, no mask, no dropout, no bias): softmax_d pass, then
@@ -343,6 +346,8 @@ hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride,
 // Tile shapes, needed by the front end for grid sizes and workspace layout.
 constexpr int kFwdBM = 128;   // query rows per forward workgroup
 constexpr int kBwdBN = 128;   // keys per dK/dV workgroup
+constexpr int kDecodeMaxQ = 32;  // query rows of fa_decode_kernel
+constexpr int kDecodeWaves(int head_dim) { return head_dim == 128 ? 2 : 4; }  // its waves: 64 KB of tiles a workgroup at most
 constexpr int kFusedBM = 32;  // query rows per step of the one-kernel backward
 
 }  // namespace fa

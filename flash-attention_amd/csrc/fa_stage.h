@@ -60,6 +60,19 @@ FA_DEVICE int tr_off(int r0, int cp, int lane) {
   return r * D + ((chunk ^ tile_swz<D, KIND>(r)) * 8) + 4 * (j16 & 1);
 }
 
+// One direct-to-LDS wave instruction: lane l's 16 bytes at (uniform base + per-lane offset) go to lds_dst + 16 * l.
+// Written as inline assembly on purpose: the compiler makes every ds_read_b64_tr_b16 that follows a direct-to-LDS
+// load it knows about wait for vmcnt(0) (it cannot tell that they touch different buffers), which would serialise the
+// prefetch of the next tile with the use of the current one.  The kernels order these loads against their LDS
+// reads themselves (wait_vmem() + workgroup barrier).  M0 carries the LDS address, as the instruction requires.
+FA_DEVICE void dma16(const char* base, uint32_t lane_off, unsigned char* lds_dst) {
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(FA_LDS void*)lds_dst;
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(lane_off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+
 // Stages a pair of ROWS x D tiles per step: tile 0 (swizzle KIND0) by waves 0 and 1, tile 1 (KIND1) by waves 2 and 3,
 // into [lds, lds + kTileBytes) and [lds + kTileBytes, lds + 2 * kTileBytes).  A workgroup has 4 waves.
 template <int D, int ROWS, int KIND0, int KIND1>
@@ -72,9 +85,6 @@ struct TilePairStager {
   static constexpr int kTileBytes = ROWS * D * 2;
   static constexpr int kPairBytes = 2 * kTileBytes;
   static_assert(TI % 4 == 0 && NI % NOFF == 0 && (ROWS / 2) % 16 == 0, "tile does not split evenly over 4 waves");
-
-  typedef __attribute__((address_space(1))) const void* gptr_t;
-  typedef __attribute__((address_space(3))) void* lptr_t;
 
   const char* base;          // wave-uniform: first row of this wave's tensor
   int64_t rsb;               // wave-uniform: row stride in bytes
@@ -98,19 +108,6 @@ struct TilePairStager {
     for (int j = 0; j < NOFF; j++) src_off[j] = (uint32_t)(rl * rsb) + 16u * (uint32_t)(pch ^ swz(j * RPI + rl));
   }
   FA_DEVICE int swz(int r) const { return second ? tile_swz<D, KIND1>(r) : tile_swz<D, KIND0>(r); }
-
-  // One direct-to-LDS wave instruction: lane l's 16 bytes at (uniform base + per-lane offset) go to lds_dst + 16 * l.
-  // Written as inline assembly on purpose: the compiler makes every ds_read_b64_tr_b16 that follows a direct-to-LDS
-  // load it knows about wait for vmcnt(0) (it cannot tell that they touch different buffers), which would serialise the
-  // prefetch of the next tile with the use of the current one.  The kernels order these loads against their LDS
-  // reads themselves (wait_vmem() + workgroup barrier).  M0 carries the LDS address, as the instruction requires.
-  static FA_DEVICE void dma16(const char* base, uint32_t lane_off, unsigned char* lds_dst) {
-    const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds_dst;
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(lane_off), "s"(base), "s"(lds_addr)
-                 : "memory", "m0");
-  }
 
   // Issues the loads of tile rows [first_row, first_row + ROWS) of both tensors; rows >= n_rows (the tensors' valid
   // extent, > first_row) re-read the last valid row so that LDS never holds anything but real tensor data.

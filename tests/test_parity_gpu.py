@@ -2013,6 +2013,21 @@ def test_rotary_2d_kernel_path_matches_oracle(dtype, D):
 # ------------------------------------------------------------------------------------------------
 # key-split forward (short query side, long key side: decode / cross-attention shapes)
 # ------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("lens_q,lens_k,H,D,dtype", [
+    ([1, 1, 1], [1, 31, 32], 2, 64, torch.float16),             # around one 32-key tile
+    ([1, 2, 32], [33, 127, 129], 3, 128, torch.bfloat16),       # around a round of the waves' tiles; all 32 columns
+    ([5, 31], [1025, 700], 2, 128, torch.float16),              # several splits, the last one short or absent
+    ([32, 1, 7], [2049, 64, 511], 1, 64, torch.bfloat16),
+    ([3, 17], [300, 1111], 2, 32, torch.float16),
+    ([1, 9], [257, 640], 2, 16, torch.float16),
+    ([1] * 64, [40 + b for b in range(64)], 16, 64, torch.float16),   # 1024 (batch, head) pairs: the last launch of the rule
+    ([1] * 65, [40 + b for b in range(65)], 16, 64, torch.float16),   # ... and the first past it
+])
+def test_decode_forward_edges(lens_q, lens_k, H, D, dtype):
+    """A few query rows per sequence: fa_decode_kernel around its tiles, its waves' rounds and its key splits."""
+    _parity_case(lens_q, lens_k, H, D, dtype, False, packing="kv", seed=sum(lens_k))
+
+
 @pytest.mark.parametrize("lens_q,lens_k,D,p", [
     ([1, 1], [2048, 1500], 64, 0.0),        # one query per sequence
     ([16, 5, 128], [1024, 4000, 513], 64, 0.0),
