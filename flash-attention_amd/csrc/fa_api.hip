@@ -122,21 +122,24 @@ SplitPlan split_plan(int batch, int nheads, int head_dim, int total_q, int max_s
 
 // Forward of at most kDecodeMaxQ query rows per sequence without mask, dropout or bias: fa_decode_kernel, while the
 // (batch, head) pairs are at most 1024.  Measured (one new token, us, fa_fwd_kernel with its own key split / fa_decode_kernel):
-// 128 pairs d = 128 up to 4096 keys 95 / 41, 16 pairs d = 128 12000 keys 31 / 27, 208 pairs d = 64 1866 keys 31 / 29, 512 pairs
-// d = 128 up to 300 keys 16 / 13.5, 1024 pairs d = 64 70 keys 11 / 8; with 1600 and 3200 pairs the forward kernel's smaller LDS keeps
+// 128 pairs d = 128 up to 4096 keys 95 / 41, 16 pairs d = 128 12000 keys 31 / 27, 208 pairs d = 64 1866 keys 30 / 27, 512 pairs
+// d = 128 up to 300 keys 16 / 13.5, 1024 pairs d = 64 70 keys 11 / 6; with 1600 and 3200 pairs the forward kernel's smaller LDS keeps
 // more workgroups on a compute unit and the two are equal for long caches (46 / 46 at 512 keys) or it wins (9.7 / 12.3 at 64 keys).
 bool decode_launch(int batch, int nheads, int max_sq, bool causal, bool sparse, bool dropout, bool bias) {
   return max_sq <= fa::kDecodeMaxQ && (int64_t)batch * nheads <= 1024 && !causal && !sparse && !dropout && !bias;
 }
-// Its key splits: as many as give every compute unit two workgroups (what its LDS holds; with four or eight per compute unit the
-// same launches take 2 to 20 % longer, a workgroup's start and the merging cost more than the evener load saves), each at least
-// two rounds of its waves' 32-key tiles (8 pairs with 300 keys at d = 64: 8 us split into single rounds, 6 us not split).
+// Its key splits: as many as give every compute unit two workgroups, three where there are fewer than 128 pairs and the head
+// dimension is at most 64 (two workgroups of 32 KB or less do not keep enough of a short stream in flight: 96 pairs d = 64 2048
+// keys 17.0 / 16.3 us; 320 pairs of up to 8000 keys 96 / 103 us, 16 pairs d = 128 12000 keys 27 / 33 us the other way round), each of
+// at least 256 keys at d = 64, two rounds of the waves' 32-key tiles elsewhere (8 pairs, 300 keys: 6 us in one piece, 8 us in three).
 SplitPlan decode_plan(int batch, int nheads, int head_dim, int total_q, int max_sk, int sq_r, int* split_keys) {
   SplitPlan sp{1, 0, 0};
   const int round = 32 * fa::kDecodeWaves(head_dim);
   const int64_t rounds = ((int64_t)max_sk + round - 1) / round, pairs = (int64_t)batch * nheads;
-  int64_t n = (512 + pairs - 1) / pairs;
-  if (n > rounds / 2) n = rounds / 2;
+  const int target = head_dim < 128 && pairs < 128 ? 768 : 512;
+  int64_t n = (target + pairs - 1) / pairs;
+  const int64_t least = head_dim == 64 ? 4 : 2;
+  if (n > rounds / least) n = rounds / least;
   if (n > 64) n = 64;
   if (n < 1) n = 1;
   const int64_t per = (rounds + n - 1) / n;

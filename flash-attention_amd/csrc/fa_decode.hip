@@ -8,8 +8,9 @@
 // the one before it is used) and never meets another wave before the end, when the NW partial (maximum, sum, output)
 // triples are merged through LDS.  All products are MFMAs in the forward kernel's orientation (S^T = K Q^T, O^T = V^T P^T):
 // the up to 32 query rows are the 32 columns, so one row costs what 32 do and the matrix work stays far below the stream.
-// Two waves at d = 128, four below: two stages of a (K, V) tile pair per wave are then 64 KB a workgroup, and two workgroups
-// a compute unit keep up to 128 KB in flight.  Measured with the merge (bf16, one new token): 8 sequences of 1024 to 4096 keys,
+// Two waves (four at d <= 32): two stages of a (K, V) tile pair per wave are then 64 KB a workgroup at d = 128, and two
+// workgroups a compute unit keep up to 128 KB in flight; at d = 64 (32 KB) four waves took 8.3 us where two take 6.1 (1024
+// pairs with 70 keys) and 73.5 against 76.5 where every stream is long (2000 keys).  Measured with the merge (bf16, one new token): 8 sequences of 1024 to 4096 keys,
 // 16 heads, d = 128 (168 MB) 95 us before, 41 us now (4.0 TB/s); all of 4096 keys 98 -> 54 us (5.0 TB/s, what a large copy
 // reaches); 16 sequences of 3600 to 6000 keys 151 -> 121 us (5.2 TB/s).
 #include "fa_params.h"
@@ -179,9 +180,11 @@ __global__ void __launch_bounds__(64 * DecodeCfg<D>::NW) fa_decode_kernel(const 
     for (int tt = 0; tt < 2; tt++) {
       f32x8 pf;
 #pragma unroll
-      for (int i = 0; i < 8; i++) pf[i] = fast_exp2(__builtin_fmaf(s[8 * tt + i], cs, -mc));
+      for (int i = 0; i < 8; i++) {
+        pf[i] = fast_exp2(__builtin_fmaf(s[8 * tt + i], cs, -mc));
+        l_i += pf[i];
+      }
       pb[tt] = cvt8<T>(pf);
-      l_i = sum8_acc(pb[tt], l_i);
     }
     if (next) wait_vmcnt<2 * NI>();
     else wait_vmcnt<0>();

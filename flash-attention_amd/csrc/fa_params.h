@@ -347,7 +347,7 @@ hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride,
 constexpr int kFwdBM = 128;   // query rows per forward workgroup
 constexpr int kBwdBN = 128;   // keys per dK/dV workgroup
 constexpr int kDecodeMaxQ = 32;  // query rows of fa_decode_kernel
-constexpr int kDecodeWaves(int head_dim) { return head_dim == 128 ? 2 : 4; }  // its waves: 64 KB of tiles a workgroup at most
+constexpr int kDecodeWaves(int head_dim) { return head_dim >= 64 ? 2 : 4; }  // its waves (64 KB of tiles a workgroup at d = 128)
 constexpr int kFusedBM = 32;  // query rows per step of the one-kernel backward
 
 }  // namespace fa
