@@ -72,30 +72,6 @@ FA_DEVICE typename Elem<T>::vec4 cvt4(f32x4 x) {
   return __builtin_convertvector(x, typename Elem<T>::vec4);
 }
 
-// acc + sum of 8 half-precision values, accumulated in fp32 (v_dot2c_f32_{f16,bf16} against (1, 1)): the forward
-// kernel's row sum costs half the VALU instructions of fp32 adds and sums exactly the rounded probabilities that
-// multiply V.
-FA_DEVICE float sum8_acc(f16x8 v, float acc) {
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  const h2 one = {(_Float16)1.f, (_Float16)1.f};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const h2 x = {v[2 * i], v[2 * i + 1]};
-    acc = __builtin_amdgcn_fdot2(x, one, acc, false);
-  }
-  return acc;
-}
-FA_DEVICE float sum8_acc(bf16x8 v, float acc) {
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  const b2 one = {(__bf16)1.f, (__bf16)1.f};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const b2 x = {v[2 * i], v[2 * i + 1]};
-    acc = __builtin_amdgcn_fdot2_f32_bf16(x, one, acc, false);
-  }
-  return acc;
-}
-
 // Threshold (log2 units) of the forward kernel's lazy accumulator rescale.
 constexpr float kRescaleLog2 = 8.f;
 constexpr float kRescaleLimit = 256.f;  // 2^kRescaleLog2

@@ -59,7 +59,7 @@ struct FwdCfg {
 // kWords (dropout, dense): the keep decisions are also left in p.keep_words for the backward (fa_common.h)
 template <typename T, int D, int BN, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
           bool kWords = false>
-__global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && D <= 64) ? 4 : ((!kDropout && kBias == kBiasTensor && D <= 64) ? 3 : 2)) fa_fwd_kernel(const FwdParams p) {
+__global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && D <= 64) ? 4 : ((!kDropout && (kBias == 0 || (D <= 64 && !(kSparse && kBias == kBiasAlibi)))) ? 3 : 2)) fa_fwd_kernel(const FwdParams p) {
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
   static_assert(!kWords || (kDropout && !kSparse), "keep words: dense dropout variants only");
   using Cfg = FwdCfg<T, D, BN, KS>;
@@ -355,23 +355,42 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
         }
       };
       // ---- P = exp2(scores - reference point m_i), rounded to the tensor dtype (what the P V product consumes); lt = this
-      // lane's share of the tile's row sums: of the rounded values, or with dropout of P before the mask, in fp32 as the
-      // reference has it (fmha_fprop_kernel_1xN.h:454 vs :471)
+      // lane's share of the tile's row sums: of P before rounding (and before the dropout mask), in fp32, as the reference has
+      // it (fmha_fprop_kernel_1xN.h:454 vs :471).  Plain additions on purpose: v_dot2c_f32_f16 of the rounded pairs against (1, 1)
+      // is half the instructions, but the dot products run on the matrix core - beside a saturated stream of MFMAs a wave gets
+      // 0.04 of them per 32 cycles where it gets 5.7 additions - so the row sums stood in line with every other wave's MFMAs.
+      // With additions (and, at d = 128, the registers that the shorter live ranges give back: three waves per SIMD for two):
+      // 16 x 12 heads x 2048 d = 128 bf16 436 -> 395 us, causal 262 -> 235; 8 x 12 x 2048 d = 64 fp16 124 -> 119.5, causal 4096 245 -> 230.
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {
         float mc = ((m_i == -INFINITY) ? 0.f : m_i) * cse;
         if (kSparse && !row_on) mc = INFINITY;  // this lane's row block does not attend the tile: P = exp2(x - inf) = 0
-        lt = 0.f;
+        float lp[KBW];  // (two chains of additions where a tile has two 32-key blocks, one register where it has one)
 #pragma unroll
-        for (int kb = 0; kb < KBW; kb++)
+        for (int kb = 0; kb < KBW; kb++) {
+          lp[kb] = 0.f;
 #pragma unroll
-          for (int r = 0; r < 16; r++) {
-            const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
-            const float pe = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
-            s[kb][r] = pe;
-            if (kDropout) lt += pe;
+          for (int t = 0; t < 2; t++) {
+            f32x8 pf;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+              const int r = 8 * t + i;
+              const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
+              pf[i] = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
+              if constexpr ((FA_ABLATE_FWD & 32) == 0) lp[kb] += pf[i];
+              if (kDropout) s[kb][r] = pf[i];
+            }
+            if (!kDropout) {
+              pb[kb][t] = cvt8<T>(pf);
+              // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it
+              asm volatile("" : "+v"(pb[kb][t]));
+            }
           }
+        }
+        lt = lp[0];
+#pragma unroll
+        for (int kb = 1; kb < KBW; kb++) lt += lp[kb];
         if (kDropout) {
 #pragma unroll
           for (int kb = 0; kb < KBW; kb++) {
@@ -399,16 +418,17 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
             }
           }
         }
+        if (kDropout) {
 #pragma unroll
-        for (int kb = 0; kb < KBW; kb++)
+          for (int kb = 0; kb < KBW; kb++)
 #pragma unroll
-          for (int t = 0; t < 2; t++) {
-            f32x8 pf;
+            for (int t = 0; t < 2; t++) {
+              f32x8 pf;
 #pragma unroll
-            for (int i = 0; i < 8; i++) pf[i] = s[kb][8 * t + i];
-            pb[kb][t] = cvt8<T>(pf);
-            if (!kDropout && (FA_ABLATE_FWD & 32) == 0) lt = sum8_acc(pb[kb][t], lt);
-          }
+              for (int i = 0; i < 8; i++) pf[i] = s[kb][8 * t + i];
+              pb[kb][t] = cvt8<T>(pf);
+            }
+        }
       };
       // ---- online softmax (fmha_fprop_kernel_1xN.h:408-454,560-611 restated for a register-resident row).
       // The reference point m_i of the exponentials only moves when it has to: P may exceed 1 by a factor of up to
