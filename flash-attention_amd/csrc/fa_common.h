@@ -232,29 +232,45 @@ FA_DEVICE void philox_micro_block(const PhiloxKey& pk, uint32_t bh, uint32_t Q4,
   for (int i = 0; i < 4; i++) { a[i] = r0[i]; a[4 + i] = r1[i]; }  // row rho of the micro-block: a[2 rho], a[2 rho + 1]
 }
 
+// Row layout: lane t of the quad needs row t of the four micro-blocks, i.e. half of the words of output (t / 2) of each.  Lanes
+// 2 u and 2 u + 1 share the outputs numbered u: the even one draws those of micro-blocks 0 and 1, the odd one of 2 and 3, and
+// one exchange between the two gives each its half of the words - a select whose unselected side comes from the
+// neighbour, one v_cndmask with a DPP operand per word.  (Drawing both outputs of one micro-block per lane took a transpose over the
+// whole quad: two stages of moves and selects, 32 instructions for these 8.)
 FA_DEVICE KeepFields keep_fields_row_layout(const PhiloxKey& pk, uint32_t bh, int qrow, int key0, int hf) {
-  const int t = qrow & 3;
-  uint32_t a[8];
-  philox_micro_block(pk, bh, (uint32_t)qrow >> 2, ((uint32_t)key0 >> 2) + 2 * t + hf, a);
-  // 4 x 4 transpose over (lane, row): swap bit 0 of both, then bit 1
-  const bool t0 = (t & 1) != 0, t1 = (t & 2) != 0;
-  uint32_t c[8];
+  const uint32_t t = (uint32_t)qrow & 3u;
+  const uint32_t c0 = ((((uint32_t)key0 >> 2) + hf + 4 * (t & 1)) << 1) | (t >> 1);
+  const u32x4 a = philox4x32_7(c0, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);       // micro-block 0 (odd lanes: 2)
+  const u32x4 b = philox4x32_7(c0 + 4, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);   // micro-block 1 (odd lanes: 3)
   KeepFields e;
-#pragma unroll
-  for (int rho = 0; rho < 4; rho++)
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t nb = quad_perm<kQuadXor1>(a[2 * (rho ^ 1) + h]);
-      c[2 * rho + h] = (((rho & 1) != 0) == t0) ? a[2 * rho + h] : nb;
-    }
-#pragma unroll
-  for (int rho = 0; rho < 4; rho++)
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t nb = quad_perm<kQuadXor2>(c[2 * (rho ^ 2) + h]);
-      e.w[2 * rho + h] = (((rho & 2) != 0) == t1) ? c[2 * rho + h] : nb;
-    }
+  // (s_nop: a DPP operand may not be read within two wait states of the vector instruction that wrote it)
+  asm("s_mov_b32 vcc_lo, 0x55555555\n\t"
+      "s_mov_b32 vcc_hi, 0x55555555\n\t"
+      "s_nop 1\n\t"
+      "v_cndmask_b32_dpp %0, %10, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %11, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %2, %14, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %15, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %4, %8, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %9, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %12, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %13, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "=&v"(e.w[0]), "=&v"(e.w[1]), "=&v"(e.w[2]), "=&v"(e.w[3]), "=&v"(e.w[4]), "=&v"(e.w[5]), "=&v"(e.w[6]), "=&v"(e.w[7])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3])
+      : "vcc", "scc");
   return e;
+}
+// The keep decisions of a word of two fields as 1 (keep) or 0 in each half: 1 - min(1, field - threshold), both saturating at 0.
+FA_DEVICE uint32_t keep_pair(uint32_t fields, uint32_t thr) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const u16x2 above = __builtin_elementwise_sub_sat(bitcast<u16x2>(fields), u16x2{(uint16_t)thr, (uint16_t)thr});
+  return bitcast<uint32_t>(__builtin_elementwise_sub_sat(u16x2{1, 1}, above));
+}
+// Two 16-bit values, each times its 0 or 1
+FA_DEVICE uint32_t mul_pair(uint32_t x, uint32_t keep) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  return bitcast<uint32_t>(bitcast<u16x2>(x) * bitcast<u16x2>(keep));
 }
 
 // Q4: the micro-block row (query row / 4) this lane draws - micro-block 2 (key % 4) + hf of the eight that cover the
@@ -305,18 +321,15 @@ FA_DEVICE float keep_word_select(uint32_t w, int pos, float a, float b) {
   const uint32_t m = (uint32_t)((int32_t)(w << (31 - pos)) >> 31);
   return __uint_as_float((m & __float_as_uint(a)) | (~m & __float_as_uint(b)));
 }
-// w <- 2 w + (this lane's bit of `mask`): one v_addc with the mask as carry-in
-FA_DEVICE uint32_t shift_in_lane_bit(uint32_t w, uint64_t mask) {
-  asm("v_addc_co_u32_e64 %0, vcc, %1, %1, %2" : "=v"(w) : "v"(w), "s"(mask) : "vcc");
-  return w;
-}
 // this lane's bit of a wave-uniform mask, as a condition the compiler selects on with the mask register as it is
 FA_DEVICE bool lane_bit(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
-// The 16 keep bits of a lane in the row layout (register r <-> key 8 (r / 4) + 4 hf + r % 4 of a 32-key block), shifted in
-// register by register with shift_in_lane_bit and a 4-bit gap after every fourth: turned into the lane's share of the
-// 32-bit keep word of its query row, then joined with the share of the lane that holds the row's other 16 keys.
-FA_DEVICE uint32_t keep_word_from_shares(uint32_t w, int hf) {
-  w = __builtin_bitreverse32(w) >> (hf ? 0 : 4);  // register r of half hf now sits at bit 8 (r / 4) + 4 hf + r % 4
+// The keep word of a query row from what its two lanes hold: keep[i] are the decisions (keep_pair) of a lane's registers 2 i and
+// 2 i + 1 in the row layout (register r <-> key 8 (r / 4) + 4 hf + r % 4 of a 32-key block).
+FA_DEVICE uint32_t keep_word_of_row(const uint32_t (&keep)[8], int hf) {
+  const uint32_t x = keep[0] | (keep[1] << 2) | (keep[2] << 8) | (keep[3] << 10);  // even registers 0 .. 6 in the low half, odd ones above
+  const uint32_t y = keep[4] | (keep[5] << 2) | (keep[6] << 8) | (keep[7] << 10);  // ... 8 .. 14
+  const uint32_t even = __builtin_amdgcn_perm(y, x, 0x05040100u), odd = __builtin_amdgcn_perm(y, x, 0x07060302u);
+  const uint32_t w = (even | (odd << 1)) << (4 * hf);
   auto r = __builtin_amdgcn_permlane32_swap(w, w, false, false);
   return r[0] | r[1];
 }

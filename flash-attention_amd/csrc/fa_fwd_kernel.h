@@ -379,13 +379,10 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
               const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
               pf[i] = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
               if constexpr ((FA_ABLATE_FWD & 32) == 0) lp[kb] += pf[i];
-              if (kDropout) s[kb][r] = pf[i];
             }
-            if (!kDropout) {
-              pb[kb][t] = cvt8<T>(pf);
-              // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it
-              asm volatile("" : "+v"(pb[kb][t]));
-            }
+            pb[kb][t] = cvt8<T>(pf);
+            // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it
+            asm volatile("" : "+v"(pb[kb][t]));
           }
         }
         lt = lp[0];
@@ -395,39 +392,27 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
 #pragma unroll
           for (int kb = 0; kb < KBW; kb++) {
             const KeepFields keep = keep_fields_row_layout(p.pk, (uint32_t)bh, qrow, n0 + (kb0 + kb) * 32, hf);
-            if (kWords) {
-              // the lane's 16 keep bits are gathered into its share of the row's keep word (fa_common.h) for the backward
-              // (dead scores keep whatever bit they drew: their P is 0)
-              uint32_t kw = 0;
+            // Dropped probabilities become 0 after the rounding, two a time: the keep decisions of a word of fields are 1 or 0 in each
+            // half (two packed saturating subtractions), a packed 16-bit integer product applies them, and shifted together they are the
+            // row's keep word.  With the exchange of keep_fields_row_layout a 64-key tile takes 331 vector instructions; with a compare, a
+            // select and a shift per score and the drawn words transposed over the quad it took 417 (Philox, the exponentials and the
+            // additions are 195 of them, and the kernel is bound by their issue): 64 x 16 heads x 1004 .. 1023, d = 64, p = 0.1, fp16:
+            // forward and backward together 1861 -> 1805 us.
+            uint32_t kept[8];
 #pragma unroll
-              for (int r = 0; r < 16; r++) {
-                const bool kept = keep.keep_row(r, p.keep_thr);
-                if (!kept) s[kb][r] = 0.f;
-                kw = shift_in_lane_bit(kw, __builtin_amdgcn_ballot_w64(kept));
-                if ((r & 3) == 3 && r != 15) kw <<= 4;
-                // (a compare's 64-bit result is to be used up before the next is made: all sixteen held at once would
-                // overflow the scalar registers into vector ones)
-                if ((r & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-              }
-              kwout[kb] = keep_word_from_shares(kw, hf);
-              kw_pending = (n0 >> 5) + kb0;
-            } else {
-#pragma unroll
-              for (int r = 0; r < 16; r++)
-                if (!keep.keep_row(r, p.keep_thr)) s[kb][r] = 0.f;
-            }
-          }
-        }
-        if (kDropout) {
-#pragma unroll
-          for (int kb = 0; kb < KBW; kb++)
+            for (int i = 0; i < 8; i++) kept[i] = keep_pair(keep.w[i], p.keep_thr);
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-              f32x8 pf;
+              u32x4 pw = bitcast<u32x4>(pb[kb][t]);
 #pragma unroll
-              for (int i = 0; i < 8; i++) pf[i] = s[kb][8 * t + i];
-              pb[kb][t] = cvt8<T>(pf);
+              for (int i = 0; i < 4; i++) pw[i] = mul_pair(pw[i], kept[4 * t + i]);
+              pb[kb][t] = bitcast<vec8>(pw);
             }
+            if (kWords) {  // (dead scores keep whatever bit they drew: their P is 0)
+              kwout[kb] = keep_word_of_row(kept, hf);
+              kw_pending = (n0 >> 5) + kb0;
+            }
+          }
         }
       };
       // ---- online softmax (fmha_fprop_kernel_1xN.h:408-454,560-611 restated for a register-resident row).

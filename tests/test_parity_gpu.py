@@ -404,6 +404,35 @@ def test_dropout_mask_is_the_defined_one_and_is_applied(D, dtype, causal, tile_s
     check_against_oracle(ours, ref, half, dtype, what="dropout D%d" % D)
 
 
+@pytest.mark.parametrize("p", [2e-5, 0.5, 0.9999])  # (thresholds of the 16-bit fields: 65533, 32767, 6)
+@pytest.mark.parametrize("lens,D,dtype", [([129, 3, 64], 64, torch.float16), ([70, 33], 128, torch.bfloat16)])
+def test_dropout_rates_at_the_ends_of_the_range(lens, D, dtype, p, tile_shape, monkeypatch):
+    """The forward decides two 16-bit fields at a time with saturating arithmetic: at rates whose thresholds lie at the ends and in the
+    middle of the fields' range the keep words are the defined mask, and an output row is 0 exactly where all its keys are dropped."""
+    from flash_attn import flash_attn_gfx950 as be
+    monkeypatch.setattr(be, "KEEP_WORDS_MAX_INPUT_RATIO", None)
+    H, mx = 2, max(lens)
+    q, k, v, _ = (x.cuda() for x in _inputs(lens, lens, H, D, dtype, 11))
+    cu = _cu(lens)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9)
+    seed, offset = g.initial_seed(), g.get_offset()
+    kw = be.new_keep_words(q, cu, mx, mx, p)
+    out, _ = be.fwd(q, k, v, cu, cu, mx, mx, p, D ** -0.5, False, False, False, g, keep_words=kw)
+    ext = (mx + 127) // 128 * 128
+    words = kw.view(torch.int32).view(len(lens) * H, ext // 32, ext).cpu().numpy().astype(np.uint32)
+    start = 0
+    for b, L in enumerate(lens):
+        for h in range(H):
+            want = orc.dropout_keep_mask(seed, offset, b * H + h, L, L, p)
+            qs, keys = np.arange(L), np.arange(L)
+            slot = (qs & ~31) | (qs & 24) | ((qs & 3) << 1) | ((qs >> 2) & 1)
+            got = (words[b * H + h][keys[None, :] // 32, slot[:, None]] >> (keys[None, :] % 32).astype(np.uint32)) & 1
+            assert np.array_equal(got.astype(bool), want)
+            assert np.array_equal(out[start:start + L, h].cpu().float().abs().sum(-1).numpy() > 0, want.any(-1))
+        start += L
+
+
 def test_dropout_random_shapes_sweep(tile_shape, dropout_path):
     """Eight seeded random dropout cases (rates, head dims, ragged self- and cross-attention lengths, packings): the
     returned mask equals its definition bit for bit and out / gradients equal the closed form with that mask."""
