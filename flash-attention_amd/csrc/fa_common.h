@@ -316,10 +316,11 @@ FA_DEVICE int keep_word_slot(int q) { return (q & ~31) | (q & 24) | ((q & 3) << 
 inline size_t keep_words_q_extent(int max_sq) { return (size_t)((max_sq + 127) & ~127); }
 inline size_t keep_words_key_blocks(int max_sk) { return (size_t)(((max_sk + 127) & ~127) / 32); }
 
-// bit `pos` (a constant) of w ? a : b, as a sign-extended one-bit field and a bitwise select: two instructions
+// bit `pos` (a constant) of w ? a : b, as a sign-extended one-bit field and a bitwise select: two instructions (bitop3 as the
+// select: written with & and | the compiler makes a mask, a compare and a v_cndmask of it, and waits for the compare)
 FA_DEVICE float keep_word_select(uint32_t w, int pos, float a, float b) {
   const uint32_t m = (uint32_t)((int32_t)(w << (31 - pos)) >> 31);
-  return __uint_as_float((m & __float_as_uint(a)) | (~m & __float_as_uint(b)));
+  return __uint_as_float(__builtin_amdgcn_bitop3_b32(m, __float_as_uint(a), __float_as_uint(b), 0xCA));
 }
 // this lane's bit of a wave-uniform mask, as a condition the compiler selects on with the mask register as it is
 FA_DEVICE bool lane_bit(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
