@@ -65,7 +65,11 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(const FwdParams p, int
     float mn = m;
 #pragma unroll
     for (int u = 0; u < U; u++) mn = fmaxf(mn, l[u]);
-    if (mn == -INFINITY) continue;
+    if (mn == -INFINITY) {  // no keys so far, or scores that are not numbers: the output of such a split is 0 or NaN, and stays
+#pragma unroll
+      for (int u = 0; u < U; u++) acc = acc + o[u];
+      continue;
+    }
     const float alpha = __expf(m - mn);  // 0 while nothing has been summed
     m = mn;
     sum *= alpha;

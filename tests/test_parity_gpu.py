@@ -2057,6 +2057,21 @@ def test_decode_forward_edges(lens_q, lens_k, H, D, dtype):
     _parity_case(lens_q, lens_k, H, D, dtype, False, packing="kv", seed=sum(lens_k))
 
 
+@pytest.mark.parametrize("lens_k", [[64, 40], [4000, 900]])  # in one piece, in several splits
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_forward_keeps_nan(lens_k, D):
+    """A query row that is not a number gives an output row that is not one, merged from key splits or not; the others are untouched."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_func
+    q, k, v, _ = (x.cuda() for x in _inputs([2, 2], lens_k, 2, D, torch.float16, seed=D))
+    args = (k, v, _cu([2, 2], "cuda"), _cu(lens_k, "cuda"), 2, max(lens_k), 0.0)
+    want = flash_attn_unpadded_func(q, *args)
+    q[1] = float("nan")
+    out = flash_attn_unpadded_func(q, *args)
+    assert bool(torch.isnan(out[1]).all())
+    keep = [0, 2, 3]
+    assert torch.equal(out[keep], want[keep]) and bool(torch.isfinite(want).all())
+
+
 @pytest.mark.parametrize("lens_q,lens_k,D,p", [
     ([1, 1], [2048, 1500], 64, 0.0),        # one query per sequence
     ([16, 5, 128], [1024, 4000, 513], 64, 0.0),
