@@ -14,6 +14,8 @@
 //                 accumulator registers hold them; the V^T fragment is fetched in the same order.
 #pragma once
 
+#include <type_traits>
+
 #include "fa_common.h"
 #include "fa_params.h"
 #include "fa_stage.h"
@@ -292,7 +294,9 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       const int kb0 = kh * KBW;
       f32x16 s[KBW];
       // ---- S^T = K Q^T, dead scores set to -inf, bias added
-      auto scores = [&]() {
+      // (again: the rare second time for a tile.  The fragments are then read one at a time: with the dropout decisions around them four at
+      // once did not fit the half-size kernel's 128 registers, and went through scratch.)
+      auto scores = [&](auto again) {
         // kTensorBias: the lane's 4 x 4 consecutive bias values per 32-key block (registers 4 j .. 4 j + 3 <-> keys
         // 8 j + 4 hf ..) of its row
         typename E::vec4 bv[kTensorBias ? KBW : 1][4];
@@ -312,6 +316,7 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
             vec8 a = (FA_ABLATE_FWD & 16) ? qreg[(ks + 1) % (D / 16)] : *reinterpret_cast<const vec8*>(Ks + (kb0 + kb) * 32 * D + koff[ks]);
             if constexpr ((FA_ABLATE_FWD & 8) == 0) s[kb] = E::mfma32(a, qreg[ks], s[kb]);
             else s[kb][ks] = (float)a[ks] * (float)qreg[ks][0];
+            if constexpr (decltype(again)::value && kDropout && KS == 2) __builtin_amdgcn_sched_barrier(0);
           }
         }
         // mask: only tiles that straddle the key length or the diagonal.  (An inactive row block inside an active tile is
@@ -422,12 +427,12 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       // share is at most 2^kRescaleLog2, so is every P behind it - so the common tile takes no row maximum at all.  A tile
       // that fails the test (the first of a row always does: no reference point yet) is redone the long way: scores again,
       // row maxima, rescaled accumulators, probabilities against the new reference point.
-      scores();
+      scores(std::false_type{});
       bool redo = __any(m_i == -INFINITY && (!kSparse || row_on));
       if (!redo) {
         probabilities();
         if constexpr ((FA_ABLATE_FWD & 32) == 0) redo = __any(!(lt <= kRescaleLimit));  // also catches inf and NaN
-        if (__builtin_expect(redo, 0)) scores();
+        if (__builtin_expect(redo, 0)) scores(std::true_type{});
       }
       if (__builtin_expect(redo, 0)) {
         float mt = s[0][0];
