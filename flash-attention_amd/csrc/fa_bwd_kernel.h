@@ -1244,8 +1244,9 @@ FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char
   }
 }
 
+// (with the dropout decisions drawn here the compiler takes 170 registers if it may, and 168 - a third wave per SIMD - without a spill if it has to)
 template <typename T, int D, int BN, bool kCausal, int kDrop, bool kSparse, int kBias = 0, int KS = 1>
-__global__ void __launch_bounds__(256, (D <= 64 && kDrop == 0 && kBias != kBiasTensor) ? 3 : 2) fa_bwd_dq_kernel(const BwdParams p) {
+__global__ void __launch_bounds__(256, (D <= 64 && ((kDrop == 0 && kBias != kBiasTensor) || (kDrop == 1 && kBias == 0 && !kSparse))) ? 3 : 2) fa_bwd_dq_kernel(const BwdParams p) {
   using Cfg = DqCfg<T, D, BN, KS>;
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kBias == kBiasTensor ? 4 * Cfg::kBiasWaveBytes : 0)];
   fa_bwd_dq_body<T, D, BN, kCausal, kDrop, kSparse, kBias, KS>(p, blockIdx.x, lds_raw);
