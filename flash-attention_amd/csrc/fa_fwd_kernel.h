@@ -366,6 +366,8 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       // 0.04 of them per 32 cycles where it gets 5.7 additions - so the row sums stood in line with every other wave's MFMAs.
       // With additions (and, at d = 128, the registers that the shorter live ranges give back: three waves per SIMD for two):
       // 16 x 12 heads x 2048 d = 128 bf16 436 -> 395 us, causal 262 -> 235; 8 x 12 x 2048 d = 64 fp16 124 -> 119.5, causal 4096 245 -> 230.
+      // Against float64 (61 .. 2048 tokens, normal inputs) the error of o is 2.3e-4 .. 2.9e-4 of its norm in fp16, 1.8e-3 .. 2.3e-3 in
+      // bf16: 0.2 .. 2.9 % above that of the sum of rounded values, which shared P's rounding with the product; lse is exact for it.
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {
