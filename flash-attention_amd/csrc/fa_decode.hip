@@ -180,11 +180,9 @@ __global__ void __launch_bounds__(64 * DecodeCfg<D>::NW) fa_decode_kernel(const 
     for (int tt = 0; tt < 2; tt++) {
       f32x8 pf;
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        pf[i] = fast_exp2(__builtin_fmaf(s[8 * tt + i], cs, -mc));
-        l_i += pf[i];
-      }
+      for (int i = 0; i < 8; i++) pf[i] = fast_exp2(__builtin_fmaf(s[8 * tt + i], cs, -mc));
       pb[tt] = cvt8<T>(pf);
+      l_i = sum8_acc(pb[tt], l_i);
     }
     if (next) wait_vmcnt<2 * NI>();
     else wait_vmcnt<0>();

@@ -360,38 +360,40 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
         }
       };
       // ---- P = exp2(scores - reference point m_i), rounded to the tensor dtype (what the P V product consumes); lt = this
-      // lane's share of the tile's row sums: of P before rounding (and before the dropout mask), in fp32, as the reference has
-      // it (fmha_fprop_kernel_1xN.h:454 vs :471).  Plain additions on purpose: v_dot2c_f32_f16 of the rounded pairs against (1, 1)
-      // is half the instructions, but the dot products run on the matrix core - beside a saturated stream of MFMAs a wave gets
-      // 0.04 of them per 32 cycles where it gets 5.7 additions - so the row sums stood in line with every other wave's MFMAs.
-      // With additions (and, at d = 128, the registers that the shorter live ranges give back: three waves per SIMD for two):
-      // 16 x 12 heads x 2048 d = 128 bf16 436 -> 395 us, causal 262 -> 235; 8 x 12 x 2048 d = 64 fp16 124 -> 119.5, causal 4096 245 -> 230.
-      // Against float64 (61 .. 2048 tokens, normal inputs) the error of o is 2.3e-4 .. 2.9e-4 of its norm in fp16, 1.8e-3 .. 2.3e-3 in
-      // bf16: 0.2 .. 2.9 % above that of the sum of rounded values, which shared P's rounding with the product; lse is exact for it.
+      // lane's share of the tile's row sums: of the rounded values (sum8_acc), so that numerator and denominator of o share that
+      // rounding, or with dropout of P before the rounding and the mask, in fp32 as the reference has it
+      // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 2 to 3 % of the kernel
+      // (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 391 for 402) and put o up to 15 % further from float64
+      // (8 x 12 x 1024, normal inputs x 2.5: 1.75e-3 of its norm with the rounded values, 2.01e-3 without; x 1: 2.359e-3 / 2.364e-3).
+      // At d = 128 three waves per SIMD run: 427 us with two.
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {
         float mc = ((m_i == -INFINITY) ? 0.f : m_i) * cse;
         if (kSparse && !row_on) mc = INFINITY;  // this lane's row block does not attend the tile: P = exp2(x - inf) = 0
-        float lp[KBW];  // (two chains of additions where a tile has two 32-key blocks, one register where it has one)
+        float lp[KBW];  // (dropout: two chains of additions where a tile has two 32-key blocks; else lp[0] is the only one)
 #pragma unroll
         for (int kb = 0; kb < KBW; kb++) {
           lp[kb] = 0.f;
 #pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
+            s[kb][r] = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
+            if constexpr (kDropout && (FA_ABLATE_FWD & 32) == 0) lp[kb] += s[kb][r];
+          }
+        }
+#pragma unroll
+        for (int kb = 0; kb < KBW; kb++)
+#pragma unroll
           for (int t = 0; t < 2; t++) {
             f32x8 pf;
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-              const int r = 8 * t + i;
-              const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
-              pf[i] = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
-              if constexpr ((FA_ABLATE_FWD & 32) == 0) lp[kb] += pf[i];
-            }
+            for (int i = 0; i < 8; i++) pf[i] = s[kb][8 * t + i];
             pb[kb][t] = cvt8<T>(pf);
+            if constexpr (!kDropout && (FA_ABLATE_FWD & 32) == 0) lp[0] = sum8_acc(pb[kb][t], lp[0]);
             // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it
             asm volatile("" : "+v"(pb[kb][t]));
           }
-        }
         lt = lp[0];
 #pragma unroll
         for (int kb = 1; kb < KBW; kb++) lt += lp[kb];

@@ -2057,6 +2057,32 @@ def test_decode_forward_edges(lens_q, lens_k, H, D, dtype):
     _parity_case(lens_q, lens_k, H, D, dtype, False, packing="kv", seed=sum(lens_k))
 
 
+@pytest.mark.parametrize("n_q", [100, 1])  # the forward kernel's tiles; the decode kernel
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_output_shares_the_rounding_of_the_probabilities(dtype, D, n_q, tile_shape):
+    """The row sum is the sum of the probabilities as they are rounded for the P V product.  One key in 32 has the top score and a
+    value row of zeros, the other 31 the probability x = 0.25 (1 + 0.9 u) before normalisation, which rounds to 0.25 (u: half
+    an ulp, relative), and value rows c: o = 31 x c / (1 + 31 x).  The rounding then moves o by at most 0.9 u / (1 + 31 x) of
+    itself, to which the output's own rounding adds up to u; against the sum of the unrounded x it would be 0.9 u + u."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_func
+    u, H, n_k = HALF_ULP[dtype], 4, 192
+    x = 0.25 * (1.0 + 0.9 * u)
+    q = torch.zeros(n_q, H, D, dtype=dtype)
+    q[..., 0] = 1.0
+    k = torch.zeros(n_k, H, D, dtype=dtype)
+    k[::32, :, 0] = 1.0
+    g = torch.Generator().manual_seed(D)
+    c = torch.randn(H, D, generator=g).to(dtype)
+    v = c.expand(n_k, H, D).clone()
+    v[::32] = 0
+    out = flash_attn_unpadded_func(q.cuda(), k.cuda(), v.cuda(), _cu([n_q], "cuda"), _cu([n_k], "cuda"), n_q, n_k, 0.0,
+                                   softmax_scale=-math.log(x))
+    want = c.double() * (31 * x / (1 + 31 * x))
+    err = ((out.cpu().double() - want).abs() / want.abs()).max().item()
+    assert err <= u * (1 + 0.9 / (1 + 31 * x)) + 2e-6, (err / u, u)  # (2e-6: fp32 sums, exponential and reciprocal)
+
+
 @pytest.mark.parametrize("lens_k", [[64, 40], [4000, 900]])  # in one piece, in several splits
 @pytest.mark.parametrize("D", [64, 128])
 def test_decode_forward_keeps_nan(lens_k, D):
