@@ -107,6 +107,7 @@ SplitPlan split_plan(int batch, int nheads, int head_dim, int total_q, int max_s
                      bool sparse) {
   SplitPlan sp{1, 0, 0};
   if (causal || sparse || max_sq <= 0 || max_sq > fa::kFwdBM) return sp;  // one query tile per (batch, head) only
+  if (batch <= 0 || nheads <= 0) return sp;  // (the size queries come before any check of the arguments)
   const int64_t blocks = (int64_t)batch * nheads * ((max_sq + fa::kFwdBM - 1) / fa::kFwdBM);
   const int key_tiles = (max_sk + 63) / 64;
   if (blocks >= 128 || key_tiles < 8) return sp;
@@ -125,7 +126,9 @@ SplitPlan split_plan(int batch, int nheads, int head_dim, int total_q, int max_s
 // 128 pairs d = 128 up to 4096 keys 95 / 41, 16 pairs d = 128 12000 keys 31 / 27, 208 pairs d = 64 1866 keys 30 / 27, 512 pairs
 // d = 128 up to 300 keys 16 / 13.5, 1024 pairs d = 64 70 keys 11 / 6; with 1600 and 3200 pairs the forward kernel's smaller LDS keeps
 // more workgroups on a compute unit and the two are equal for long caches (46 / 46 at 512 keys) or it wins (9.7 / 12.3 at 64 keys).
-bool decode_launch(int batch, int nheads, int max_sq, bool causal, bool sparse, bool dropout, bool bias) {
+// (The size query comes before any check of the arguments: what fa_fwd refuses is not a decode launch.)
+bool decode_launch(int batch, int nheads, int max_sq, int max_sk, bool causal, bool sparse, bool dropout, bool bias) {
+  if (batch <= 0 || nheads <= 0 || max_sq <= 0 || max_sk <= 0) return false;
   return max_sq <= fa::kDecodeMaxQ && (int64_t)batch * nheads <= 1024 && !causal && !sparse && !dropout && !bias;
 }
 // Its key splits: as many as give every compute unit two workgroups, three where there are fewer than 128 pairs and the head
@@ -306,7 +309,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
     p.kw_kb = (int)fa::keep_words_key_blocks(a->max_seqlen_k);
   }
   // short query side, long key side: split the keys over several workgroups if the caller brought the scratch for it
-  const bool decode = decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->is_causal != 0, sparse, dropout,
+  const bool decode = decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, sparse, dropout,
                                     a->alibi_slopes || a->attn_bias);
   const SplitPlan sp = decode ? decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &p.split_keys)
                               : split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
@@ -562,7 +565,7 @@ size_t fa_fwd_workspace_bytes(const fa_fwd_args* a) {
   if (!a) return 0;
   if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes;
   const Rounded r = round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, false);
-  if (decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->is_causal != 0, false, a->p_dropout > 0.f,
+  if (decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, false, a->p_dropout > 0.f,
                     a->alibi_slopes || a->attn_bias)) {
     int split_keys;
     return decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &split_keys).bytes;

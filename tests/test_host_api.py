@@ -94,6 +94,28 @@ def test_null_pointers_and_alignment_are_errors_not_crashes(lib):
     assert lib.fa_fwd(None) == -1
 
 
+@pytest.mark.parametrize("max_q", [1, 100])  # decode kernel, forward kernel
+@pytest.mark.parametrize("keys", [100, 4096])
+@pytest.mark.parametrize("field,value", [("batch", 0), ("nheads", 0), ("max_seqlen_q", 0), ("max_seqlen_k", 0), ("max_seqlen_k", -1),
+                                         ("batch", -1), ("nheads", -1)])
+def test_size_queries_of_calls_that_are_refused(lib, field, value, keys, max_q):
+    """The callers ask for the scratch before the call checks its arguments (an empty cache, an empty batch): the queries answer
+    0 and the call returns its error."""
+    from flash_attn import flash_attn_gfx950 as be
+    a = _valid_fwd_args(be)
+    a.max_seqlen_q, a.max_seqlen_k = max_q, keys
+    setattr(a, field, value)
+    assert lib.fa_fwd_workspace_bytes(ctypes.byref(a)) == 0
+    assert lib.fa_fwd(ctypes.byref(a)) == -1 and b"must be positive" in lib.fa_last_error()
+    g = be.BwdArgs()
+    g.struct_bytes = ctypes.sizeof(g)
+    g.batch, g.nheads, g.head_dim, g.total_q, g.total_k, g.max_seqlen_q, g.max_seqlen_k = 1, 2, 64, 100, 5000, max_q, keys
+    g.softmax_scale = 0.125
+    setattr(g, field, value)
+    assert lib.fa_bwd_workspace_bytes(ctypes.byref(g)) == 0
+    assert lib.fa_bwd(ctypes.byref(g)) == -1 and b"must be positive" in lib.fa_last_error()
+
+
 def test_block_sparse_needs_workspace_also_when_causal(lib):
     from flash_attn import flash_attn_gfx950 as be
     a = _valid_fwd_args(be)

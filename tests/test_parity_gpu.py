@@ -2083,6 +2083,14 @@ def test_output_shares_the_rounding_of_the_probabilities(dtype, D, n_q, tile_sha
     assert err <= u * (1 + 0.9 / (1 + 31 * x)) + 2e-6, (err / u, u)  # (2e-6: fp32 sums, exponential and reciprocal)
 
 
+def test_decode_over_an_empty_cache_is_an_error():
+    """A decode step whose caches are all empty (max_seqlen_k = 0) raises like every other refused call."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_kvpacked_func
+    q, kv = torch.zeros(2, 2, 64, dtype=torch.float16, device="cuda"), torch.zeros(0, 2, 2, 64, dtype=torch.float16, device="cuda")
+    with pytest.raises(RuntimeError, match="max_seqlen must be positive"):
+        flash_attn_unpadded_kvpacked_func(q, kv, _cu([1, 1]), _cu([0, 0]), 1, 0, 0.0)
+
+
 @pytest.mark.parametrize("lens_k", [[64, 40], [4000, 900]])  # in one piece, in several splits
 @pytest.mark.parametrize("D", [64, 128])
 def test_decode_forward_keeps_nan(lens_k, D):
