@@ -294,8 +294,9 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       const int kb0 = kh * KBW;
       f32x16 s[KBW];
       // ---- S^T = K Q^T, dead scores set to -inf, bias added
-      // (again: the rare second time for a tile.  The fragments are then read one at a time: with the dropout decisions around them four at
-      // once did not fit the half-size kernel's 128 registers, and went through scratch.)
+      // (again: the rare second time for a tile.  The fragments are then read one at a time where four at once do not fit the registers
+      // and went through scratch, whose loads wait for the next tile's prefetch: eight registers at d = 128, and the half-size kernel's
+      // dropout variants.)
       auto scores = [&](auto again) {
         // kTensorBias: the lane's 4 x 4 consecutive bias values per 32-key block (registers 4 j .. 4 j + 3 <-> keys
         // 8 j + 4 hf ..) of its row
@@ -316,7 +317,7 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
             vec8 a = (FA_ABLATE_FWD & 16) ? qreg[(ks + 1) % (D / 16)] : *reinterpret_cast<const vec8*>(Ks + (kb0 + kb) * 32 * D + koff[ks]);
             if constexpr ((FA_ABLATE_FWD & 8) == 0) s[kb] = E::mfma32(a, qreg[ks], s[kb]);
             else s[kb][ks] = (float)a[ks] * (float)qreg[ks][0];
-            if constexpr (decltype(again)::value && kDropout && KS == 2) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(again)::value && (D == 128 || (kDropout && KS == 2))) __builtin_amdgcn_sched_barrier(0);
           }
         }
         // mask: only tiles that straddle the key length or the diagonal.  (An inactive row block inside an active tile is
@@ -365,7 +366,8 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 2 to 3 % of the kernel
       // (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 391 for 402) and put o up to 15 % further from float64
       // (8 x 12 x 1024, normal inputs x 2.5: 1.75e-3 of its norm with the rounded values, 2.01e-3 without; x 1: 2.359e-3 / 2.364e-3).
-      // At d = 128 three waves per SIMD run: 427 us with two.
+      // At d = 128 three waves per SIMD run: 427 us with two.  (Over a block layout without a causal mask two registers are in scratch for it: 4 x
+      // 16 heads x 4096, a quarter of the blocks, 305 us; 351 with two waves.)
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {

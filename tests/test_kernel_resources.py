@@ -8,6 +8,7 @@ import os
 import re
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -125,3 +126,29 @@ def test_d128_backward_keeps_two_waves_per_simd():
         for flags in ("Lb0ELb0E", "Lb1ELb0E", "Lb0ELb1E", "Lb1ELb1E"):
             k = _pick(bwd, "fa_bwd_dkdv_pair_kernel%s" % dt, flags + "EEv")
             assert k["Occupancy"] >= 3 and k["VGPRs Spill"] <= 2 and k["LDS Size"] <= 160 * 1024 // 3, (dt, flags, k)
+
+
+@pytest.mark.timeout(600)
+def test_forward_and_decode_variants_keep_their_waves_per_simd():
+    """The forward at the other head dimensions, over block layouts and with ALiBi, and the decode kernel: (waves per SIMD at least,
+    spilled registers at most) of each."""
+    with ThreadPoolExecutor(4) as ex:
+        d16, d64, d128, dec = ex.map(_resources, ("fa_fwd_d16.hip", "fa_fwd_d64.hip", "fa_fwd_d128.hip", "fa_decode.hip"))
+    T, F = "Lb1E", "Lb0E"
+
+    def flags(causal, dropout, sparse, bias, ks=1, words=F):
+        return causal + dropout + sparse + "Li%dELi%dE" % (bias, ks) + words + "EEv"
+
+    for dt in ("IDF16_", "IDF16b"):
+        for causal in (F, T):
+            for what, res, d, variant, waves, spills in (
+                    ("plain", d128, 128, flags(causal, F, F, 0), 3, 0),
+                    ("block layout", d128, 128, flags(causal, F, T, 0), 3, 2 if causal == F else 0),
+                    ("block layout", d64, 64, flags(causal, F, T, 0), 4, 8 if causal == F else 5),
+                    ("block layout", d16, 16, flags(causal, F, T, 0), 5, 0),
+                    ("ALiBi", d16, 16, flags(F, F, F, 1), 4, 0)):
+                k = _pick(res, "fa_fwd_kernel%sLi%dE" % (dt, d), variant)
+                assert k["Occupancy"] >= waves and k["VGPRs Spill"] <= spills, (what, d, dt, causal, k)
+        for d in (16, 32, 64, 128):  # two workgroups of two waves (64 KB of tiles at d = 128) on a compute unit need one per SIMD
+            k = _pick(dec, "fa_decode_kernel%sLi%dE" % (dt, d))
+            assert k["Occupancy"] >= 1 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 64 * 1024 + 64, ("decode", dt, d, k)
