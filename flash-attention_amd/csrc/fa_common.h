@@ -259,33 +259,43 @@ FA_DEVICE void philox_micro_block(const PhiloxKey& pk, uint32_t bh, uint32_t Q4,
   for (int i = 0; i < 4; i++) { a[i] = r0[i]; a[4 + i] = r1[i]; }  // row rho of the micro-block: a[2 rho], a[2 rho + 1]
 }
 
-// Row layout: lane t of the quad needs row t of the four micro-blocks, i.e. half of the words of output (t / 2) of each.  Lanes
-// 2 u and 2 u + 1 share the outputs numbered u: the even one draws those of micro-blocks 0 and 1, the odd one of 2 and 3, and
-// one exchange between the two gives each its half of the words - a select whose unselected side comes from the
-// neighbour, one v_cndmask with a DPP operand per word.  (Drawing both outputs of one micro-block per lane took a transpose over the
-// whole quad: two stages of moves and selects, 32 instructions for these 8.)
-FA_DEVICE KeepFields keep_fields_row_layout(const PhiloxKey& pk, uint32_t bh, int qrow, int key0, int hf) {
-  const uint32_t t = (uint32_t)qrow & 3u;
-  const uint32_t c0 = ((((uint32_t)key0 >> 2) + hf + 4 * (t & 1)) << 1) | (t >> 1);
-  const u32x4 a = philox4x32_7(c0, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);       // micro-block 0 (odd lanes: 2)
-  const u32x4 b = philox4x32_7(c0 + 4, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);   // micro-block 1 (odd lanes: 3)
-  KeepFields e;
-  // (s_nop: a DPP operand may not be read within two wait states of the vector instruction that wrote it)
+// Between the lanes 2 u and 2 u + 1: the even one keeps lo and gets the other's lo as hi, the odd one keeps hi and gets the other's hi as lo.
+// A select whose unselected side comes from the neighbour: one v_cndmask with a DPP operand per word.  (s_nop: a DPP operand may
+// not be read within two wait states of the vector instruction that wrote it.  hi is replaced in place, two words at a time: with eight new registers
+// at once several drawing variants lost a wave per SIMD.)
+FA_DEVICE void exchange_in_lane_pair(uint32_t (&lo)[2], uint32_t (&hi)[2]) {
+  uint32_t n0, n1;
   asm("s_mov_b32 vcc_lo, 0x55555555\n\t"
       "s_mov_b32 vcc_hi, 0x55555555\n\t"
       "s_nop 1\n\t"
-      "v_cndmask_b32_dpp %0, %10, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %1, %11, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %2, %14, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %3, %15, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %0, %2, %4, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %3, %5, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "s_not_b64 vcc, vcc\n\t"
-      "v_cndmask_b32_dpp %4, %8, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %5, %9, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %6, %12, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %7, %13, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-      : "=&v"(e.w[0]), "=&v"(e.w[1]), "=&v"(e.w[2]), "=&v"(e.w[3]), "=&v"(e.w[4]), "=&v"(e.w[5]), "=&v"(e.w[6]), "=&v"(e.w[7])
-      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3])
+      "v_cndmask_b32_dpp %2, %4, %2, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %5, %3, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "=&v"(n0), "=&v"(n1), "+&v"(hi[0]), "+&v"(hi[1])
+      : "v"(lo[0]), "v"(lo[1])
       : "vcc", "scc");
+  lo[0] = n0;
+  lo[1] = n1;
+}
+
+// Row layout: lane t of the quad needs row t of the four micro-blocks, i.e. half of the words of output (t / 2) of each.  Lanes
+// 2 u and 2 u + 1 share the outputs numbered u: the even one draws those of micro-blocks 0 and 1, the odd one of 2 and 3, and
+// one exchange between the two gives each its half of the words.  (Drawing both outputs of one micro-block per lane took a transpose
+// over the whole quad: two stages of moves and selects, 32 instructions for these 8.)
+FA_DEVICE KeepFields keep_fields_row_layout(const PhiloxKey& pk, uint32_t bh, int qrow, int key0, int hf) {
+  const uint32_t t = (uint32_t)qrow & 3u;
+  const uint32_t c0 = ((((uint32_t)key0 >> 2) + hf + 4 * (t & 1)) << 1) | (t >> 1);
+  KeepFields e;
+#pragma unroll
+  for (int m = 0; m < 2; m++) {  // micro-blocks m (odd lanes: 2 + m)
+    const u32x4 a = philox4x32_7(c0 + 4 * m, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);
+    uint32_t lo[2] = {a[0], a[1]}, hi[2] = {a[2], a[3]};
+    exchange_in_lane_pair(lo, hi);
+    e.w[2 * m] = lo[0]; e.w[2 * m + 1] = lo[1];
+    e.w[4 + 2 * m] = hi[0]; e.w[5 + 2 * m] = hi[1];
+  }
   return e;
 }
 // The keep decisions of a word of two fields as 1 (keep) or 0 in each half: 1 - min(1, field - threshold), both saturating at 0.

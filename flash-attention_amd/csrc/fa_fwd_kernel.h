@@ -58,10 +58,19 @@ struct FwdCfg {
 // kBias (fa_params.h): 1 = ALiBi, the score of (query i, key j) gets -slope[head] * |i - j| added after scaling; 2 = it gets
 // bias[b, h, i, j] of a tensor added.  The scores are then moved to the softmax's own units (base-2 exponent) before the row
 // maximum is taken, and the running maximum is kept in those units.
+// Waves per SIMD that the variants are bounded to: what their registers allow without a spill in the main loop, or with the few
+// that tests/test_kernel_resources.py pins where the wave is worth more (d = 128 over a block layout, 4 x 16 heads x 4096, a quarter of
+// the blocks, bf16: two registers in scratch, 305 us; two waves per SIMD 351).
+constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool words) {
+  if (dropout && ks == 2 && bias == 0 && d == 16 && !words) return 6;
+  if ((!dropout || ks == 2) && bias == 0 && d <= 64) return 4;
+  if (!dropout && (bias == 0 || (d <= 64 && !(sparse && bias == kBiasAlibi)))) return 3;
+  return 2;
+}
 // kWords (dropout, dense): the keep decisions are also left in p.keep_words for the backward (fa_common.h)
 template <typename T, int D, int BN, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
           bool kWords = false>
-__global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && D <= 64) ? 4 : ((!kDropout && (kBias == 0 || (D <= 64 && !(kSparse && kBias == kBiasAlibi)))) ? 3 : 2)) fa_fwd_kernel(const FwdParams p) {
+__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
   static_assert(!kWords || (kDropout && !kSparse), "keep words: dense dropout variants only");
   using Cfg = FwdCfg<T, D, BN, KS>;
@@ -366,8 +375,7 @@ __global__ void __launch_bounds__(256, ((!kDropout || KS == 2) && kBias == 0 && 
       // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 2 to 3 % of the kernel
       // (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 391 for 402) and put o up to 15 % further from float64
       // (8 x 12 x 1024, normal inputs x 2.5: 1.75e-3 of its norm with the rounded values, 2.01e-3 without; x 1: 2.359e-3 / 2.364e-3).
-      // At d = 128 three waves per SIMD run: 427 us with two.  (Over a block layout without a causal mask two registers are in scratch for it: 4 x
-      // 16 heads x 4096, a quarter of the blocks, 305 us; 351 with two waves.)
+      // At d = 128 three waves per SIMD run: 427 us with two.
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {

@@ -130,10 +130,11 @@ def test_d128_backward_keeps_two_waves_per_simd():
 
 @pytest.mark.timeout(600)
 def test_forward_and_decode_variants_keep_their_waves_per_simd():
-    """The forward at the other head dimensions, over block layouts and with ALiBi, and the decode kernel: (waves per SIMD at least,
-    spilled registers at most) of each."""
-    with ThreadPoolExecutor(4) as ex:
-        d16, d64, d128, dec = ex.map(_resources, ("fa_fwd_d16.hip", "fa_fwd_d64.hip", "fa_fwd_d128.hip", "fa_decode.hip"))
+    """The forward at every head dimension but the headline's, over block layouts, with ALiBi and with dropout, the dQ variants that
+    draw dropout decisions, and the decode kernel: (waves per SIMD at least, spilled registers at most) of each."""
+    with ThreadPoolExecutor(6) as ex:
+        d16, d32, d64, d128, dec, bwd = ex.map(_resources, ("fa_fwd_d16.hip", "fa_fwd_d32.hip", "fa_fwd_d64.hip", "fa_fwd_d128.hip",
+                                                            "fa_decode.hip", "fa_bwd_d64.hip"))
     T, F = "Lb1E", "Lb0E"
 
     def flags(causal, dropout, sparse, bias, ks=1, words=F):
@@ -146,9 +147,15 @@ def test_forward_and_decode_variants_keep_their_waves_per_simd():
                     ("block layout", d128, 128, flags(causal, F, T, 0), 3, 2 if causal == F else 0),
                     ("block layout", d64, 64, flags(causal, F, T, 0), 4, 8 if causal == F else 5),
                     ("block layout", d16, 16, flags(causal, F, T, 0), 5, 0),
-                    ("ALiBi", d16, 16, flags(F, F, F, 1), 4, 0)):
+                    ("ALiBi", d16, 16, flags(F, F, F, 1), 4, 0),
+                    ("dropout, half-size", d16, 16, flags(causal, T, F, 0, 2), 6, 0),
+                    ("dropout, block layout", d32, 32, flags(causal, T, T, 0), 4, 0),
+                    ("dropout, block layout, ALiBi", d32, 32, flags(causal, T, T, 1), 3, 0)):
                 k = _pick(res, "fa_fwd_kernel%sLi%dE" % (dt, d), variant)
                 assert k["Occupancy"] >= waves and k["VGPRs Spill"] <= spills, (what, d, dt, causal, k)
+            for sparse, alibi, spills in ((F, 0, 0), (F, 1, 0), (T, 0, 1), (T, 1, 3)):
+                k = _pick(bwd, "fa_bwd_dq_kernel%sLi64E" % dt, causal + "Li1E" + sparse + "Li%dELi1EEEv" % alibi)
+                assert k["Occupancy"] >= 3 and k["VGPRs Spill"] <= spills, ("dq, drawn dropout", dt, causal, sparse, alibi, k)
         for d in (16, 32, 64, 128):  # two workgroups of two waves (64 KB of tiles at d = 128) on a compute unit need one per SIMD
             k = _pick(dec, "fa_decode_kernel%sLi%dE" % (dt, d))
             assert k["Occupancy"] >= 1 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 64 * 1024 + 64, ("decode", dt, d, k)
