@@ -122,37 +122,52 @@ SplitPlan split_plan(int batch, int nheads, int head_dim, int total_q, int max_s
 }
 
 // Forward of at most kDecodeMaxQ query rows per sequence without mask, dropout or bias: fa_decode_kernel, while the
-// (batch, head) pairs are at most 1024.  Measured (one new token, us, fa_fwd_kernel with its own key split / fa_decode_kernel):
-// 128 pairs d = 128 up to 4096 keys 95 / 41, 16 pairs d = 128 12000 keys 31 / 27, 208 pairs d = 64 1866 keys 30 / 27, 512 pairs
-// d = 128 up to 300 keys 16 / 13.5, 1024 pairs d = 64 70 keys 11 / 6; with 1600 and 3200 pairs the forward kernel's smaller LDS keeps
-// more workgroups on a compute unit and the two are equal for long caches (46 / 46 at 512 keys) or it wins (9.7 / 12.3 at 64 keys).
+// (batch, head) pairs are at most 1024.  The figures here and at the split plan are us of fa_fwd_kernel with its own key split /
+// fa_decode_kernel (one new token, bf16, K and V from HBM, profiles/decode_split_sweep.md).  128 pairs d = 128 12000 keys 289 / 142,
+// 1024 pairs d = 128 200 keys 32.5 / 27.3, 32 pairs d = 32 600 keys 10.2 / 7.4.
+// - At 1600 pairs the forward kernel's smaller LDS keeps more workgroups on a compute unit: equal at 512 keys, 9.7 / 12.3 at 64.
+// - At d = 128 two workgroups' LDS fits a compute unit: pairs whose second round of 512 workgroups would be less than three quarters full
+//   take as long as two full rounds (640 pairs of 400 keys 29.8 / 35.7), unless short sequences leave them fewer keys than that.
 // (The size query comes before any check of the arguments: what fa_fwd refuses is not a decode launch.)
-bool decode_launch(int batch, int nheads, int max_sq, int max_sk, bool causal, bool sparse, bool dropout, bool bias) {
+bool decode_launch(int batch, int nheads, int head_dim, int total_k, int max_sq, int max_sk, bool causal, bool sparse, bool dropout,
+                   bool bias) {
   if (batch <= 0 || nheads <= 0 || max_sq <= 0 || max_sk <= 0) return false;
-  return max_sq <= fa::kDecodeMaxQ && (int64_t)batch * nheads <= 1024 && !causal && !sparse && !dropout && !bias;
+  if (max_sq > fa::kDecodeMaxQ || causal || sparse || dropout || bias) return false;
+  const int64_t pairs = (int64_t)batch * nheads;
+  const int64_t live = (int64_t)nheads * total_k / max_sk;  // pairs, if every sequence were as long as the longest
+  return pairs <= 1024 && !(head_dim == 128 && pairs < 896 && live > 512);
 }
-// Its key splits: as many as give every compute unit two workgroups, three where there are fewer than 128 pairs and the head
-// dimension is at most 64 (two workgroups of 32 KB or less do not keep enough of a short stream in flight: 96 pairs d = 64 2048
-// keys 17.0 / 16.3 us; 320 pairs of up to 8000 keys 96 / 103 us, 16 pairs d = 128 12000 keys 27 / 33 us the other way round), each of
-// at least 256 keys at d = 64, two rounds of the waves' 32-key tiles elsewhere (8 pairs, 300 keys: 6 us in one piece, 8 us in three).
-SplitPlan decode_plan(int batch, int nheads, int head_dim, int total_q, int max_sk, int sq_r, int* split_keys) {
+// Its key splits.  A merge costs about 3 us, the time in which a workgroup streams 200 keys (400 at d <= 32), so keys are shared from nine
+// rounds of the waves' 32-key tiles on (8 pairs d = 64 400 keys 8.3 in one piece, 8.9 in two; 600 keys 10.9 / 7.9 in eight), and where more than 160
+// pairs fill the chip already from sixteen on (208 pairs d = 128 600 keys 19.9 in one piece, 21.6 in two, 3000 keys 72.4 / 67.6).  As many
+// workgroups as fit a compute unit at a time: two at d = 128, in whole numbers (96 pairs 12000 keys: five splits 113, six, sixteen workgroups too
+// many for the chip, 138), counted by what the sequences' lengths leave of them where the pairs are many; three elsewhere (96 pairs d = 64 8000 keys of uneven length:
+// eight splits 33.9, five 40.1).  At least two rounds each, at most 32 splits (8 pairs 12000 keys d = 128: 22.6 with 32, 24.8 with 64).
+SplitPlan decode_plan(int batch, int nheads, int head_dim, int total_q, int total_k, int max_sk, int sq_r, int* split_keys) {
   SplitPlan sp{1, 0, 0};
   const int round = 32 * fa::kDecodeWaves(head_dim);
   const int64_t rounds = ((int64_t)max_sk + round - 1) / round, pairs = (int64_t)batch * nheads;
-  const int target = head_dim < 128 && pairs < 128 ? 768 : 512;
-  int64_t n = (target + pairs - 1) / pairs;
-  const int64_t least = head_dim == 64 ? 4 : 2;
-  if (n > rounds / least) n = rounds / least;
-  if (n > 64) n = 64;
-  if (n < 1) n = 1;
+  if (rounds < (pairs <= 160 ? 9 : 16)) return sp;
+  int64_t live = pairs;
+  if (head_dim == 128 && pairs > 160) live = (int64_t)nheads * total_k / max_sk;
+  if (live > pairs || live < 1) live = pairs;
+  int64_t n = (head_dim == 128 ? 512 : 768) / live;
+  if (n > rounds / 2) n = rounds / 2;
+  if (n > 32) n = 32;
+  if (n < 2) return sp;
   const int64_t per = (rounds + n - 1) / n;
   *split_keys = (int)(per * round);
   n = (rounds + per - 1) / per;
-  if (n < 2) return sp;
   sp.n_splits = (int)n;
   sp.o_bytes = align16((size_t)n * total_q * nheads * head_dim * 4);
   sp.bytes = sp.o_bytes + align16((size_t)n * batch * nheads * sq_r * 4);
   return sp;
+}
+// In one piece (too few keys to share, or no scratch) the two waves of d = 64 are slower than the four of fa_fwd_kernel once a
+// stream is long, as long as the pairs do not fill the chip: 256 pairs 900 keys 19.1 / 21.8, 128 pairs 12000
+// keys 151 / 206; 512 pairs 900 keys 29.6 / 28.2.
+bool decode_needs_splits(int batch, int nheads, int head_dim, int max_sk) {
+  return head_dim == 64 && (int64_t)batch * nheads < 448 && max_sk > 512;
 }
 
 int build_maps(const int32_t* blockmask, const int32_t* row_order, unsigned char* ws, const SparseLayout& sl,
@@ -309,13 +324,21 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
     p.kw_kb = (int)fa::keep_words_key_blocks(a->max_seqlen_k);
   }
   // short query side, long key side: split the keys over several workgroups if the caller brought the scratch for it
-  const bool decode = decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, sparse, dropout,
-                                    a->alibi_slopes || a->attn_bias);
-  const SplitPlan sp = decode ? decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &p.split_keys)
-                              : split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
-                                           a->is_causal != 0, sparse);
-  const bool split = sp.n_splits > 1 && a->workspace && a->workspace_bytes >= sp.bytes && aligned16(a->workspace);
-  if (decode && !split) p.split_keys = a->max_seqlen_k;
+  auto fits = [&](const SplitPlan& sp) { return sp.n_splits > 1 && a->workspace && a->workspace_bytes >= sp.bytes && aligned16(a->workspace); };
+  bool decode = decode_launch(a->batch, a->nheads, a->head_dim, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, sparse, dropout,
+                              a->alibi_slopes || a->attn_bias);
+  SplitPlan sp{1, 0, 0};
+  if (decode) {
+    sp = decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->total_k, a->max_seqlen_k, r.sq_r, &p.split_keys);
+    if (!fits(sp)) {
+      decode = !decode_needs_splits(a->batch, a->nheads, a->head_dim, a->max_seqlen_k);
+      p.split_keys = decode ? a->max_seqlen_k : 0;
+      sp.n_splits = 1;
+    }
+  } else {
+    sp = split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r, a->is_causal != 0, sparse);
+  }
+  const bool split = fits(sp);
   if (split) {
     p.n_splits = sp.n_splits;
     p.o_part = reinterpret_cast<float*>(a->workspace);
@@ -565,10 +588,10 @@ size_t fa_fwd_workspace_bytes(const fa_fwd_args* a) {
   if (!a) return 0;
   if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes;
   const Rounded r = round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, false);
-  if (decode_launch(a->batch, a->nheads, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, false, a->p_dropout > 0.f,
-                    a->alibi_slopes || a->attn_bias)) {
+  if (decode_launch(a->batch, a->nheads, a->head_dim, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, false,
+                    a->p_dropout > 0.f, a->alibi_slopes || a->attn_bias)) {
     int split_keys;
-    return decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_k, r.sq_r, &split_keys).bytes;
+    return decode_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->total_k, a->max_seqlen_k, r.sq_r, &split_keys).bytes;
   }
   return split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r,
                     a->is_causal != 0, false).bytes;

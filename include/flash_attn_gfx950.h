@@ -211,10 +211,10 @@ int fa_fwd_block_noalloc(const fa_fwd_args* args);
 
 /* Scratch the caller provides.  The dense forward and backward need none to be correct
  * (there is no o_tmp / dq_tmp, fmha_api.cpp:247,403-404).  The block-sparse paths need room for their block activity
- * maps (an error without it).  For a dense, non-causal forward with few query rows and many keys (max_seqlen_q <= 32 and
- * batch * nheads <= 1024, or max_seqlen_q <= 128, batch * nheads < 128 and max_seqlen_k >= 512: decoding and cross-attention
- * shapes) fa_fwd_workspace_bytes() returns the size of the partial results of a key-split pass: if `workspace` holds that much, fa_fwd shares the keys of each query tile
- * among several workgroups and merges their results; if not, it runs the single pass.  fa_bwd_workspace_bytes() does the
+ * maps (an error without it).  For a dense, non-causal forward with few query rows (max_seqlen_q <= 128: decoding and cross-attention
+ * shapes) and more keys than its (batch, head) pairs alone would spread over the GPU, fa_fwd_workspace_bytes() returns the size of
+ * the partial results of a key-split pass: if `workspace` holds that much, fa_fwd shares the keys of each query tile
+ * among several workgroups and merges their results; if not, it runs the single pass.  Arguments that fa_fwd refuses need none.  fa_bwd_workspace_bytes() does the
  * same for the dQ kernel of such shapes (fp32 partial dQ per key split), and, under launch policy 0x20, returns the
  * scratch of the one-kernel backward (fp32 running sums of dQ and their hand-over counters: about twice the bytes of dq).
  * Only shapes, is_causal, p_dropout, the bias pointers and blockmask != NULL are read. */

@@ -461,8 +461,8 @@ def test_launch_policy_values_and_one_kernel_backward_scratch(lib):
 
 
 def test_key_split_workspace_plan(lib):
-    """fa_fwd_workspace_bytes asks for scratch only for dense, non-causal forwards with one query tile, few
-    (batch, head) pairs and many keys; the size is n_splits * (fp32 partial outputs + partial lse)."""
+    """fa_fwd_workspace_bytes asks for scratch only for dense, non-causal forwards with one query tile and more keys than the
+    (batch, head) pairs alone spread over the chip; the size is n_splits * (fp32 partial outputs + partial lse)."""
     from flash_attn import flash_attn_gfx950 as be
     a = _valid_fwd_args(be)
     a.batch, a.nheads, a.head_dim = 8, 12, 64
@@ -490,6 +490,24 @@ def test_key_split_workspace_plan(lib):
     assert lib.fa_bwd_workspace_bytes(ctypes.byref(g)) == 0
     g.is_causal, g.max_seqlen_q, g.total_q = 0, 2048, 8 * 2048
     assert lib.fa_bwd_workspace_bytes(ctypes.byref(g)) == 0
+
+
+@pytest.mark.parametrize("head_dim,batch,nheads,keys,mean,splits", [
+    (128, 20, 16, 200, 1.0, 1), (128, 13, 16, 600, 1.0, 1), (16, 13, 16, 600, 1.0, 1),   # a merge would cost more than it saves
+    (64, 1, 8, 512, 1.0, 1), (64, 1, 8, 513, 1.0, 3), (32, 1, 8, 1024, 1.0, 1), (32, 1, 8, 1025, 1.0, 3),  # eight rounds, nine
+    (64, 16, 10, 600, 1.0, 4), (64, 16, 11, 600, 1.0, 1), (64, 16, 11, 1024, 1.0, 4),    # 160 pairs and more
+    (128, 8, 12, 12000, 1.0, 5), (128, 8, 16, 12000, 1.0, 4), (128, 1, 8, 12000, 1.0, 32),  # whole workgroups per compute unit
+    (128, 20, 16, 3000, 1.0, 1), (128, 20, 16, 3000, 0.6, 2), (64, 20, 16, 3000, 1.0, 2),   # uneven lengths leave room
+    (128, 40, 16, 3000, 1.0, 1), (128, 64, 16, 3000, 1.0, 1), (64, 100, 16, 3000, 1.0, 1),  # the chip is full
+])
+def test_decode_split_plan(lib, head_dim, batch, nheads, keys, mean, splits):
+    """The key splits of a decode step (one new token) by head dimension, pairs and keys, read off the scratch asked for."""
+    from flash_attn import flash_attn_gfx950 as be
+    a = _valid_fwd_args(be)
+    a.batch, a.nheads, a.head_dim = batch, nheads, head_dim
+    a.total_q, a.total_k, a.max_seqlen_q, a.max_seqlen_k = batch, int(batch * keys * mean), 1, keys
+    per_split = batch * nheads * (head_dim + 16) * 4  # partial o, and partial lse with 16 rows
+    assert lib.fa_fwd_workspace_bytes(ctypes.byref(a)) == (splits * per_split if splits > 1 else 0)
 
 
 def test_rows_and_rotary_argument_checks(lib):
