@@ -2083,6 +2083,92 @@ def test_output_shares_the_rounding_of_the_probabilities(dtype, D, n_q, tile_sha
     assert err <= u * (1 + 0.9 / (1 + 31 * x)) + 2e-6, (err / u, u)  # (2e-6: fp32 sums, exponential and reciprocal)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout", ["head-major", "padded rows", "k and v apart"])
+def test_decode_forward_strides(layout, D):
+    """K and V of a decode step as a cache may hold them: whole heads one after the other, rows with room behind them, different
+    strides for the two; in one piece (40 keys) and in several splits.  The values are those of the packed tensors, bit for bit."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_func
+    H, dtype, lens_q = 2, torch.bfloat16, [2, 1]
+    for lens_k in ([40, 33], [1500, 3001]):
+        q, k, v, _ = (x.cuda() for x in _inputs(lens_q, lens_k, H, D, dtype, sum(lens_k)))
+        args = (_cu(lens_q), _cu(lens_k), 2, max(lens_k), 0.0)
+        want = flash_attn_unpadded_func(q, k, v, *args)
+
+        def head_major(x):
+            return x.transpose(0, 1).contiguous().transpose(0, 1)
+
+        def padded(x):
+            y = torch.full((x.shape[0], H + 1, D + 24), float("nan"), dtype=dtype, device="cuda")
+            y[:, :H, :D] = x
+            return y[:, :H, :D]
+
+        k2, v2 = {"head-major": (head_major(k), head_major(v)), "padded rows": (padded(k), padded(v)),
+                  "k and v apart": (padded(k), head_major(v))}[layout]
+        assert torch.equal(flash_attn_unpadded_func(padded(q), k2, v2, *args), want)
+
+
+@pytest.mark.parametrize("lens_k", [[96, 40], [4000, 900]])  # in one piece, in several splits
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_forward_with_a_value_that_is_not_finite(lens_k, D):
+    """A NaN in one key's row makes that sequence and head NaN, an infinity in one key's value its column infinite, wherever the
+    split that holds the key; everything else is untouched."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_func
+    for key in (0, lens_k[0] // 2, lens_k[0] - 33):
+        q, k, v, _ = (x.cuda() for x in _inputs([2, 2], lens_k, 2, D, torch.float16, seed=D + key))
+        args = (_cu([2, 2]), _cu(lens_k), 2, max(lens_k), 0.0)
+        want = flash_attn_unpadded_func(q, k, v, *args)
+        k2, v2 = k.clone(), v.clone()
+        k2[key, 1, 5] = float("nan")
+        out = flash_attn_unpadded_func(q, k2, v, *args)
+        assert bool(torch.isnan(out[:2, 1]).all())
+        out[:2, 1] = want[:2, 1]
+        assert torch.equal(out, want)
+        v2[key, 1, 5] = float("inf")
+        out = flash_attn_unpadded_func(q, k, v2, *args)
+        assert bool((out[:2, 1, 5] == float("inf")).all())
+        out[:2, 1, 5] = want[:2, 1, 5]
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_forward_empty_sequences_in_a_split_launch(D):
+    """Sequences without keys (o = 0, lse = -inf, written by the merge alone) and without queries among ones that are split."""
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_func
+    lens_q, lens_k, H, dtype = [3, 1, 0, 2], [2049, 0, 700, 64], 2, torch.float16
+    q, k, v, _ = _inputs(lens_q, lens_k, H, D, dtype, seed=D)
+    cu_q, cu_k = _cu(lens_q, "cpu"), _cu(lens_k, "cpu")
+    out, lse, _ = flash_attn_unpadded_func(q.cuda(), k.cuda(), v.cuda(), cu_q.cuda(), cu_k.cuda(), 3, 2049, 0.0,
+                                           return_attn_probs=True)
+    ref = orc.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, False)
+    half = half_attention(q.cuda(), k.cuda(), v.cuda(), cu_q.tolist(), cu_k.tolist(), D ** -0.5, False)
+    check_against_oracle({"out": out}, ref, half, dtype, names=("out",), what="decode, empty sequences D%d" % D)
+    for b, L in enumerate(lens_q):
+        check_lse(lse[b, :, :L].cpu(), ref["lse"][b], half["lse"][b], dtype, "decode, empty sequences D%d" % D)
+    assert bool((out[3] == 0).all()) and bool((lse[1, :, 0] == float("-inf")).all())
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16), (32, torch.bfloat16)])
+def test_decode_forward_with_rotary_matches_oracle(D, dtype):
+    """The decode kernel turns the queries it loads: output and the rotated queries it leaves, in one piece and in several splits."""
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.rotary import RotaryEmbedding
+    H, lens_q = 2, [5, 32, 1]
+    cos_h, sin_h = RotaryEmbedding(D).half_tables(torch.empty(1, 64, 3, H, D, device="cuda", dtype=dtype))
+    pos = np.concatenate([np.arange(L) for L in lens_q])
+    for lens_k in ([40, 33, 64], [2500, 1100, 70]):
+        q, k, v, _ = _inputs(lens_q, lens_k, H, D, dtype, seed=sum(lens_k))
+        cu_q, cu_k = _cu(lens_q, "cpu"), _cu(lens_k, "cpu")
+        q_rot = torch.zeros_like(q).cuda()
+        out, _ = be.fwd(q.cuda(), k.cuda(), v.cuda(), cu_q.cuda(), cu_k.cuda(), 32, max(lens_k), 0.0, D ** -0.5, False, False, False,
+                        rotary=(cos_h, sin_h), q_rot=q_rot)
+        turned = torch.tensor(orc.rotary_ref(q.double().numpy(), cos_h.double().cpu().numpy(), sin_h.double().cpu().numpy(), pos))
+        assert _maxerr(q_rot, turned) <= HALF_ULP[dtype] * turned.abs().max().item() + 1e-6  # one rounding of an fp32 sum
+        ref = orc.varlen_attention(turned.to(dtype), k, v, cu_q, cu_k, D ** -0.5, False)
+        half = half_attention(turned.to(dtype).cuda(), k.cuda(), v.cuda(), cu_q.tolist(), cu_k.tolist(), D ** -0.5, False)
+        check_against_oracle({"out": out}, ref, half, dtype, names=("out",), what="decode, rotary D%d" % D)
+
+
 def test_decode_over_an_empty_cache_is_an_error():
     """A decode step whose caches are all empty (max_seqlen_k = 0) raises like every other refused call."""
     from flash_attn.flash_attn_interface import flash_attn_unpadded_kvpacked_func
