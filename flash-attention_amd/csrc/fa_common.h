@@ -238,10 +238,11 @@ constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;  // lane ^ 1, lane ^ 2
 // The 16 random 16-bit fields that decide the 16 score elements one lane owns in a 32x32 MFMA accumulator tile.
 // "Row layout" (S^T = K Q^T tiles: lane -> query row `qrow`, register r -> key key0 + 8*(r/4) + 4*hf + r%4) and
 // "column layout" (S = Q K^T tiles: lane -> key `key`, register r -> query row q0 + 8*(r/4) + 4*hf + r%4).
-// The four lanes of a quad own the four rows (columns) of the same four micro-blocks.  Lane t of the quad draws the
-// two Philox outputs of micro-block t (8 words = 4 rows of 2 words) and the quad then transposes - every lane needs
-// row (column) lane%4 of all four micro-blocks - in two DPP butterfly stages.  The raw fields travel: nothing is
-// compared, packed into bit masks and unpacked again on the way; the consumer compares a half-word with the threshold.
+// The four lanes of a quad own the four rows (columns) of the same four micro-blocks.  The quad shares the drawing and then
+// exchanges words, so that every lane has row (column) lane % 4 of all four: for the row layout in one exchange between the two lanes of a
+// pair (keep_fields_row_layout), for the column layout lane t draws both Philox outputs of micro-block t (8 words = 4 rows of 2 words)
+// and the quad transposes in two DPP butterfly stages.  The raw fields travel: nothing is compared, packed into bit masks and unpacked
+// again on the way; the consumer compares a half-word with the threshold.
 struct KeepFields {
   uint32_t w[8];
   // row layout: w[2 tt + h] holds row lane%4 of micro-block tt = r / 4, columns 2h (low half) and 2h + 1 (high half)

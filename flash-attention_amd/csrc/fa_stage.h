@@ -64,7 +64,9 @@ FA_DEVICE int tr_off(int r0, int cp, int lane) {
 // Written as inline assembly on purpose: the compiler makes every ds_read_b64_tr_b16 that follows a direct-to-LDS
 // load it knows about wait for vmcnt(0) (it cannot tell that they touch different buffers), which would serialise the
 // prefetch of the next tile with the use of the current one.  The kernels order these loads against their LDS
-// reads themselves (wait_vmem() + workgroup barrier).  M0 carries the LDS address, as the instruction requires.
+// reads themselves, in one of two ways: tiles that several waves fetch by wait_vmem() + workgroup barrier; the tiles of fa_decode_kernel, which
+// belong to one wave each, by counting that wave's outstanding loads (wait_vmcnt: loads complete in order, so every load between
+// a tile's and the wait is in the count) and lgkmcnt(0) before a stage is refilled, without a barrier.  M0 carries the LDS address, as the instruction requires.
 FA_DEVICE void dma16(const char* base, uint32_t lane_off, unsigned char* lds_dst) {
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(FA_LDS void*)lds_dst;
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
