@@ -60,19 +60,25 @@ struct FwdCfg {
 // maximum is taken, and the running maximum is kept in those units.
 // Waves per SIMD that the variants are bounded to: what their registers allow without a spill in the main loop, or with the few
 // that tests/test_kernel_resources.py pins where the wave is worth more (d = 128 over a block layout, 4 x 16 heads x 4096, a quarter of
-// the blocks, bf16: two registers in scratch, 305 us; two waves per SIMD 351).
+// the blocks, bf16: two registers in scratch, 305 us; two waves per SIMD 351).  The dense d = 128 forward takes 168 registers, three
+// waves, by itself and is scheduled better than when it is told to (4 x 16 x 600 .. 3001 causal bf16 86.6 us, bounded 89.4).
 constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool words) {
   if (dropout && ks == 2 && bias == 0 && d == 16 && !words) return 6;
   if ((!dropout || ks == 2) && bias == 0 && d <= 64) return 4;
-  if (!dropout && (bias == 0 || (d <= 64 && !(sparse && bias == kBiasAlibi)))) return 3;
+  if (!dropout && ((bias == 0 && sparse) || (d <= 64 && !(sparse && bias == kBiasAlibi)))) return 3;
   return 2;
 }
+// kRoomy (dense, d = 128, no dropout, no bias): launches of at most two workgroups per compute unit, which a third wave per SIMD does not help, keep
+// all K fragments of a tile in flight also where its scores are redone, at two waves per SIMD: us of that build / the other,
+// bf16, 64 workgroups (8 heads x 1000) 24.8 / 27.0, causal 26.5 / 27.8; 192 (16 x 1500) 34.8 / 38.1; 384 (16 x 3000) 92.5 / 95.3, causal 68.6 / 72.3;
+// 576 (64 x 1100) 61.5 / 54.5; 1536 (64 x 3000) 303 / 286.
 // kWords (dropout, dense): the keep decisions are also left in p.keep_words for the backward (fa_common.h)
-template <typename T, int D, int BN, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
+template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
           bool kWords = false>
 __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
   static_assert(!kWords || (kDropout && !kSparse), "keep words: dense dropout variants only");
+  static_assert(!kRoomy || (D == 128 && !kDropout && !kSparse && kBias == 0), "built where a launch may be short of workgroups");
   using Cfg = FwdCfg<T, D, BN, KS>;
   using E = Elem<T>;
   using vec8 = typename E::vec8;
@@ -326,7 +332,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
             vec8 a = (FA_ABLATE_FWD & 16) ? qreg[(ks + 1) % (D / 16)] : *reinterpret_cast<const vec8*>(Ks + (kb0 + kb) * 32 * D + koff[ks]);
             if constexpr ((FA_ABLATE_FWD & 8) == 0) s[kb] = E::mfma32(a, qreg[ks], s[kb]);
             else s[kb][ks] = (float)a[ks] * (float)qreg[ks][0];
-            if constexpr (decltype(again)::value && (D == 128 || (kDropout && KS == 2))) __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(again)::value && ((D == 128 && !kRoomy) || (kDropout && KS == 2))) __builtin_amdgcn_sched_barrier(0);
           }
         }
         // mask: only tiles that straddle the key length or the diagonal.  (An inactive row block inside an active tile is
@@ -375,7 +381,6 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
       // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 2 to 3 % of the kernel
       // (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 391 for 402) and put o up to 15 % further from float64
       // (8 x 12 x 1024, normal inputs x 2.5: 1.75e-3 of its norm with the rounded values, 2.01e-3 without; x 1: 2.359e-3 / 2.364e-3).
-      // At d = 128 three waves per SIMD run: 427 us with two.
       vec8 pb[KBW][2];
       float lt;
       auto probabilities = [&]() {
@@ -401,8 +406,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
             for (int i = 0; i < 8; i++) pf[i] = s[kb][8 * t + i];
             pb[kb][t] = cvt8<T>(pf);
             if constexpr (!kDropout && (FA_ABLATE_FWD & 32) == 0) lp[0] = sum8_acc(pb[kb][t], lp[0]);
-            // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it
-            asm volatile("" : "+v"(pb[kb][t]));
+            // pinned here: sunk below the test of the row sums, the conversions would keep all fp32 values live across it (the dense d = 128
+            // variant has the registers for that)
+            if constexpr (D <= 64 || kDropout || kSparse) asm volatile("" : "+v"(pb[kb][t]));
           }
         lt = lp[0];
 #pragma unroll

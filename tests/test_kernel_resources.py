@@ -151,8 +151,10 @@ def test_forward_and_decode_variants_keep_their_waves_per_simd():
                     ("dropout, half-size", d16, 16, flags(causal, T, F, 0, 2), 6, 0),
                     ("dropout, block layout", d32, 32, flags(causal, T, T, 0), 4, 0),
                     ("dropout, block layout, ALiBi", d32, 32, flags(causal, T, T, 1), 3, 0)):
-                k = _pick(res, "fa_fwd_kernel%sLi%dE" % (dt, d), variant)
+                k = _pick(res, "fa_fwd_kernel%sLi%dELi%dELb0E" % (dt, d, 32 if d == 128 else 64), variant)
                 assert k["Occupancy"] >= waves and k["VGPRs Spill"] <= spills, (what, d, dt, causal, k)
+            k = _pick(d128, "fa_fwd_kernel%sLi128ELi32ELb1E" % dt, flags(causal, F, F, 0))  # launches short of workgroups
+            assert k["Occupancy"] >= 2 and k["VGPRs Spill"] == 0, ("roomy", dt, causal, k)
             for sparse, alibi, spills in ((F, 0, 0), (F, 1, 0), (T, 0, 1), (T, 1, 3)):
                 k = _pick(bwd, "fa_bwd_dq_kernel%sLi64E" % dt, causal + "Li1E" + sparse + "Li%dELi1EEEv" % alibi)
                 assert k["Occupancy"] >= 3 and k["VGPRs Spill"] <= spills, ("dq, drawn dropout", dt, causal, sparse, alibi, k)
