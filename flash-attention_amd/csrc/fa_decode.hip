@@ -10,9 +10,10 @@
 // the up to 32 query rows are the 32 columns, so one row costs what 32 do and the matrix work stays far below the stream.
 // Two waves (four at d <= 32): two stages of a (K, V) tile pair per wave are then 64 KB a workgroup at d = 128, and two
 // workgroups a compute unit keep up to 128 KB in flight; at d = 64 (32 KB) four waves took 8.3 us where two take 6.1 (1024
-// pairs with 70 keys) and 73.5 against 76.5 where every stream is long (2000 keys).  Measured with the merge (bf16, one new token): 8 sequences of 1024 to 4096 keys,
-// 16 heads, d = 128 (168 MB) 95 us before, 41 us now (4.0 TB/s); all of 4096 keys 98 -> 54 us (5.0 TB/s, what a large copy
-// reaches); 16 sequences of 3600 to 6000 keys 151 -> 121 us (5.2 TB/s).
+// pairs with 70 keys) and 73.5 against 76.5 where every stream is long (2000 keys).  Measured with the merge, inputs that change from
+// call to call, bf16, one new token, us of fa_fwd_kernel with its own split / here: 8 sequences of 1024 to 4096 keys, 16 heads, d = 128 (168 MB) 96.6 /
+// 42.8 (the kernel alone 38.8: FETCH_SIZE gives K and V once, 4.3 TB/s); all of 5000 keys 122.8 / 66.2 (5.0 TB/s, what a large copy reaches), of 12000
+// 288 / 144 (5.5 TB/s).
 #include "fa_params.h"
 #include "fa_stage.h"
 

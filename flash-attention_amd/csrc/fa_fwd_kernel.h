@@ -378,8 +378,8 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
       // ---- P = exp2(scores - reference point m_i), rounded to the tensor dtype (what the P V product consumes); lt = this
       // lane's share of the tile's row sums: of the rounded values (sum8_acc), so that numerator and denominator of o share that
       // rounding, or with dropout of P before the rounding and the mask, in fp32 as the reference has it
-      // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 2 to 3 % of the kernel
-      // (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 391 for 402) and put o up to 15 % further from float64
+      // (fmha_fprop_kernel_1xN.h:454 vs :471).  Sums of the unrounded P, one addition per value, save bf16 1.5 to 2.5 % of the
+      // kernel (8 x 12 heads x 2048 d = 64 112.2 us for 114.8, 16 x 12 x 2048 d = 128 388 for 394) and put o up to 15 % further from float64
       // (8 x 12 x 1024, normal inputs x 2.5: 1.75e-3 of its norm with the rounded values, 2.01e-3 without; x 1: 2.359e-3 / 2.364e-3).
       vec8 pb[KBW][2];
       float lt;
@@ -419,10 +419,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
             const KeepFields keep = keep_fields_row_layout(p.pk, (uint32_t)bh, qrow, n0 + (kb0 + kb) * 32, hf);
             // Dropped probabilities become 0 after the rounding, two a time: the keep decisions of a word of fields are 1 or 0 in each
             // half (two packed saturating subtractions), a packed 16-bit integer product applies them, and shifted together they are the
-            // row's keep word.  With the exchange of keep_fields_row_layout a 64-key tile takes 331 vector instructions; with a compare, a
-            // select and a shift per score and the drawn words transposed over the quad it took 417 (Philox, the exponentials and the
-            // additions are 195 of them, and the kernel is bound by their issue): 64 x 16 heads x 1004 .. 1023, d = 64, p = 0.1, fp16:
-            // forward and backward together 1795 -> 1739 us.
+            // row's keep word.  Counted with SQ_INSTS_VALU over 64 x 16 heads x 1004 .. 1023, d = 64, p = 0.1, fp16, the forward issues 25.3 other
+            // vector instructions per MFMA with this and the exchange of keep_fields_row_layout, 31.3 with a compare, a select and a shift per
+            // score and the drawn words transposed over the quad: forward and backward together 1800 -> 1733 us.
             uint32_t kept[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) kept[i] = keep_pair(keep.w[i], p.keep_thr);
