@@ -2051,6 +2051,10 @@ def test_rotary_2d_kernel_path_matches_oracle(dtype, D):
     ([1, 9], [257, 640], 2, 16, torch.float16),
     ([1] * 64, [40 + b for b in range(64)], 16, 64, torch.float16),   # 1024 (batch, head) pairs: the last launch of the rule
     ([1] * 65, [40 + b for b in range(65)], 16, 64, torch.float16),   # ... and the first past it
+    ([1] * 32, [9 + b for b in range(32)], 16, 128, torch.bfloat16),  # d = 128: the last pairs of one round of workgroups
+    ([2] * 33, [40] * 33, 16, 128, torch.bfloat16),                   # ... pairs that go to the forward kernel
+    ([1] * 33, [8 + 32 * (b == 0) for b in range(33)], 16, 128, torch.bfloat16),  # ... unless most sequences are short
+    ([1] * 11, [513 + b for b in range(11)], 16, 64, torch.float16),  # d = 64 in one piece, too long for two waves
 ])
 def test_decode_forward_edges(lens_q, lens_k, H, D, dtype):
     """A few query rows per sequence: fa_decode_kernel around its tiles, its waves' rounds and its key splits."""
