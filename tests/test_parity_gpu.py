@@ -2061,11 +2061,12 @@ def test_decode_forward_edges(lens_q, lens_k, H, D, dtype):
     _parity_case(lens_q, lens_k, H, D, dtype, False, packing="kv", seed=sum(lens_k))
 
 
-@pytest.mark.parametrize("B", [16, 17])  # 512 workgroups, two per compute unit; 544
+@pytest.mark.parametrize("B", [16, 17, 27, 33])  # 512 workgroups, two per compute unit, 544; causal: about 470 and 570 with query rows
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_d128_forward_either_side_of_two_workgroups_per_compute_unit(dtype, causal, B):
-    """The dense d = 128 forward has one build for launches of at most two workgroups per compute unit and one for larger ones."""
+    """The dense d = 128 forward has one build for launches of at most two workgroups per compute unit (causal: with query rows) and one for
+    larger ones."""
     lens = [[129, 33, 1, 128, 64, 97][b % 6] for b in range(B)]
     _parity_case(lens, lens, 16, 128, dtype, causal, packing="qkv", seed=B)
 
