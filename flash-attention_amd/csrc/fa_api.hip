@@ -224,14 +224,15 @@ int check_common(uint32_t struct_bytes, size_t expect, int dtype, int batch, int
   return FA_OK;
 }
 
-int fwd_impl(const fa_fwd_args* a, bool want_block) {
+// row_of, row_info: null, or the rows of a padded batch (fa_fwd_padded)
+int fwd_impl(const fa_fwd_args* a, bool want_block, const int32_t* row_of = nullptr, const int32_t* row_info = nullptr) {
   if (!a) return fail(FA_ERR_INVALID_ARGUMENT, "args is NULL");
   int rc = check_common(a->struct_bytes, sizeof(fa_fwd_args), a->dtype, a->batch, a->nheads, a->head_dim, a->total_q,
                         a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->p_dropout, a->softmax_scale);
   if (rc) return rc;
   const bool sparse = a->blockmask != nullptr;
   FA_REQUIRE(sparse == want_block, want_block ? "fa_fwd_block needs a blockmask" : "fa_fwd takes no blockmask; call fa_fwd_block");
-  FA_REQUIRE(a->q && a->k && a->v && a->o && a->softmax_lse && a->cu_seqlens_q && a->cu_seqlens_k, "NULL tensor pointer");
+  FA_REQUIRE(a->q && a->k && a->v && a->o && a->softmax_lse && (row_of || (a->cu_seqlens_q && a->cu_seqlens_k)), "NULL tensor pointer");
   FA_REQUIRE(aligned16(a->q) && aligned16(a->k) && aligned16(a->v) && aligned16(a->o),
              "q, k, v, o must be 16-byte aligned");
   FA_REQUIRE(stride_ok(a->q_row_stride) && stride_ok(a->q_head_stride) && stride_ok(a->k_row_stride) &&
@@ -274,6 +275,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
 
   p.q = a->q; p.k = a->k; p.v = a->v; p.o = a->o; p.lse = a->softmax_lse;
   p.cu_q = a->cu_seqlens_q; p.cu_k = a->cu_seqlens_k;
+  p.row_of = row_of; p.row_info = row_info;
   p.q_rs = a->q_row_stride; p.q_hs = a->q_head_stride;
   p.k_rs = a->k_row_stride; p.k_hs = a->k_head_stride;
   p.v_rs = a->v_row_stride; p.v_hs = a->v_head_stride;
@@ -325,7 +327,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
   }
   // short query side, long key side: split the keys over several workgroups if the caller brought the scratch for it
   auto fits = [&](const SplitPlan& sp) { return sp.n_splits > 1 && a->workspace && a->workspace_bytes >= sp.bytes && aligned16(a->workspace); };
-  bool decode = decode_launch(a->batch, a->nheads, a->head_dim, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, sparse, dropout,
+  bool decode = !row_of && decode_launch(a->batch, a->nheads, a->head_dim, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, sparse, dropout,
                               a->alibi_slopes || a->attn_bias);
   SplitPlan sp{1, 0, 0};
   if (decode) {
@@ -335,7 +337,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block) {
       p.split_keys = decode ? a->max_seqlen_k : 0;
       sp.n_splits = 1;
     }
-  } else {
+  } else if (!row_of) {
     sp = split_plan(a->batch, a->nheads, a->head_dim, a->total_q, a->max_seqlen_q, a->max_seqlen_k, r.sq_r, a->is_causal != 0, sparse);
   }
   const bool split = fits(sp);
@@ -578,6 +580,37 @@ int fa_fwd_block_noalloc(const fa_fwd_args* args) {
 
 int fa_fwd(const fa_fwd_args* args) { return fwd_impl(args, false); }
 int fa_fwd_block(const fa_fwd_args* args) { return fwd_impl(args, true); }
+
+int fa_padding_rows(const void* mask, int64_t mask_row_stride, int32_t batch, int32_t seqlen, int32_t* row_of, int32_t* row_info, int32_t* lens,
+                    void* stream) {
+  FA_REQUIRE(batch > 0 && seqlen > 0 && (int64_t)batch * seqlen < ((int64_t)1 << 31), "fa_padding_rows: sizes must be positive and below 2^31 rows");
+  FA_REQUIRE(mask && row_of && row_info, "fa_padding_rows: null pointer");
+  FA_REQUIRE(mask_row_stride >= 0, "fa_padding_rows: negative mask stride");
+  FA_REQUIRE(((reinterpret_cast<uintptr_t>(row_of) | reinterpret_cast<uintptr_t>(row_info) | reinterpret_cast<uintptr_t>(lens)) & 3) == 0,
+             "fa_padding_rows: row_of, row_info and lens must be 4-byte aligned");
+  FA_LAUNCH(fa::launch_padding_rows(reinterpret_cast<const unsigned char*>(mask), mask_row_stride, batch, seqlen, row_of, row_info, lens,
+                                    reinterpret_cast<hipStream_t>(stream)));
+  return FA_OK;
+}
+
+int fa_fwd_padded(const fa_fwd_args* a, const int32_t* row_of, const int32_t* row_info) {
+  FA_REQUIRE(a && row_of && row_info, "fa_fwd_padded: null pointer");
+  FA_REQUIRE(a->struct_bytes == sizeof(fa_fwd_args), "struct_bytes is %u, this library expects %zu (ABI mismatch)", a->struct_bytes,
+             sizeof(fa_fwd_args));
+  FA_REQUIRE(((reinterpret_cast<uintptr_t>(row_of) | reinterpret_cast<uintptr_t>(row_info)) & 3) == 0,
+             "fa_fwd_padded: row_of and row_info must be 4-byte aligned");
+  FA_REQUIRE(a->max_seqlen_q == a->max_seqlen_k && a->batch > 0 && a->max_seqlen_q > 0 &&
+                 (int64_t)a->batch * a->max_seqlen_q < ((int64_t)1 << 31) && a->total_q == a->total_k &&
+                 (int64_t)a->total_q == (int64_t)a->batch * a->max_seqlen_q,
+             "fa_fwd_padded: q, k and v have batch * max_seqlen rows each, fewer than 2^31");
+  // (the kernel's lanes address an entry's keys with 32-bit byte offsets)
+  FA_REQUIRE((uint64_t)a->max_seqlen_k * (uint64_t)a->k_row_stride * 2 < ((uint64_t)1 << 32) && a->k_row_stride >= 0 && a->v_row_stride >= 0 &&
+                 (uint64_t)a->max_seqlen_k * (uint64_t)a->v_row_stride * 2 < ((uint64_t)1 << 32),
+             "fa_fwd_padded: the keys of a batch entry may span at most 2^32 bytes");
+  if (a->p_dropout > 0.f || a->alibi_slopes || a->attn_bias || a->rotary_cos || a->rotary_sin || a->s_dmask || a->keep_words)
+    return fail(FA_ERR_UNSUPPORTED, "fa_fwd_padded takes no dropout, bias, rotary tables or s_dmask: gather the rows and call fa_fwd");
+  return fwd_impl(a, false, row_of, row_info);
+}
 int fa_bwd(const fa_bwd_args* args) { return bwd_impl(args, false); }
 int fa_bwd_profiled(const fa_bwd_args* args, void* ev_main_start, void* ev_main_stop) {
   return bwd_impl(args, false, ev_main_start, ev_main_stop);

@@ -73,12 +73,19 @@ constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool
 // bf16, 64 workgroups (8 heads x 1000) 24.8 / 27.0, causal 26.5 / 27.8; 192 (16 x 1500) 34.8 / 38.1; 384 (16 x 3000) 92.5 / 95.3, causal 68.6 / 72.3;
 // 576 (64 x 1100) 61.5 / 54.5; 1536 (64 x 3000) 303 / 286.
 // kWords (dropout, dense): the keep decisions are also left in p.keep_words for the backward (fa_common.h)
+// kBias = kPaddedRows (dense, no dropout): q, k, v and o are a padded batch, (batch, max_sq) rows of which p.row_of and p.row_info name the
+// tokens; these attend each other, counted in their own order, and the padding rows of o are written as zeros.  32 x 512 rows, 256 .. 512 of
+// them tokens, 16 heads, d = 64: one launch of 47 us in place of gather 29, forward 40 and scatter 15,
+// and tokens anywhere in their row instead of in one run cost it 6 % (the module call 49 and 52 us, 175 gathered).
 template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
           bool kWords = false>
-__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
+__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % kPaddedRows, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
+  constexpr bool kRows = kBias == kPaddedRows;
+  constexpr bool kBiased = kBias != 0 && !kRows;
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
   static_assert(!kWords || (kDropout && !kSparse), "keep words: dense dropout variants only");
-  static_assert(!kRoomy || (D == 128 && !kDropout && !kSparse && kBias == 0), "built where a launch may be short of workgroups");
+  static_assert(!kRows || (!kDropout && !kSparse), "padded batches: dense, no dropout");
+  static_assert(!kRoomy || (D == 128 && !kDropout && !kSparse && !kBiased), "built where a launch may be short of workgroups");
   using Cfg = FwdCfg<T, D, BN, KS>;
   using E = Elem<T>;
   using vec8 = typename E::vec8;
@@ -87,7 +94,8 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
 
   // kTensorBias: behind the tiles, per wave 32 rows x BN keys of bias, rows padded by 8 bytes (see load_bias below)
   constexpr int kBiasRowBytes = BN * 2 + 8, kBiasWaveBytes = 32 * kBiasRowBytes;
-  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : 0)];
+  constexpr int kRowSlotBytes = 2 * 64 * 4;  // kRows: behind the tiles, per wave (see fetch_rows below)
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : kRows ? 4 * kRowSlotBytes : 0)];
 
   // Workgroup -> (batch, head, query tile), XCD-aware (see map_tile): the query tiles of one (batch, head) share
   // one XCD's L2 copy of K and V.
@@ -99,12 +107,21 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
   const int qt = kCausal ? p.nq_tiles - 1 - rank : rank;  // under a causal mask the last query tiles cost most
   const int h = bh % p.H;
   // (dense, no mask: the batch entries are taken longest keys first, see longest_first)
-  const int b = (!kCausal && !kSparse && p.tile_group < 0) ? longest_first(p.cu_k, p.B, bh / p.H) : bh / p.H;
+  const int b = (!kCausal && !kSparse && p.tile_group < 0) ? longest_first(p.cu_k, p.B, bh / p.H, kRows ? p.row_info : nullptr) : bh / p.H;
   bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
 
   int q_begin, Lq, k_begin = 0, Lk = 0;
-  if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
-  if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: o = 0, lse = -inf
+  // kRows: this entry's slice of row_of; its tokens lie one after the other (from row q_begin on) or, `listed`, anywhere in it
+  const int32_t* const row_of = kRows ? p.row_of + (int64_t)b * p.max_sq : nullptr;
+  bool listed = false;
+  if constexpr (kRows) {
+    Lq = Lk = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b]);
+    listed = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 2]) == 0;
+    q_begin = k_begin = b * p.max_sq + (listed ? 0 : __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 1]));
+  } else {
+    if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
+    if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: o = 0, lse = -inf
+  }
   const int m0 = qt * BM;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -130,13 +147,24 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
       return;
     }
   } else if (m0 >= Lq) {
+    if constexpr (kRows) {  // padding rows only: zeros
+      for (int i = tid; i < BM * CH; i += 256) {
+        const int j = m0 + i / CH;
+        if (j < p.max_sq)
+          st_global16(reinterpret_cast<T*>(p.o) + ((int64_t)b * p.max_sq + row_of[j]) * p.o_rs + (int64_t)h * p.o_hs + (i % CH) * 8,
+                      u32x4{0, 0, 0, 0});
+      }
+    }
     return;
   }
 
   // ---- Q fragment (B operand of S^T = K Q^T), held in registers for the whole kernel
   vec8 qreg[D / 16];
   {
-    const int qr = qrow < Lq ? qrow : Lq - 1;
+    int qr = qrow < Lq ? qrow : Lq - 1;
+    if constexpr (kRows) {
+      if (listed) qr = row_of[qr];
+    }
     const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)(q_begin + qr) * p.q_rs + (int64_t)h * p.q_hs + hf * 8;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ks++) qreg[ks] = bitcast<vec8>(ld_global16(qp + ks * 16));
@@ -154,7 +182,26 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
   typename Cfg::Stager stager;
   stager.init(wave, lane, reinterpret_cast<const T*>(p.k) + (int64_t)k_begin * p.k_rs + (int64_t)h * p.k_hs, p.k_rs,
               reinterpret_cast<const T*>(p.v) + (int64_t)k_begin * p.v_rs + (int64_t)h * p.v_hs, p.v_rs);
-  auto stage = [&](int it, int buf) { stager.issue(lds_raw + buf * kBufBytes, it * BN, Lk); };
+  // kRows, listed: the rows of a tile are read off row_of, which a wave brings into two LDS slots of its own, a tile ahead of the tile's own
+  // loads (keys past the end: the last key's row)
+  int32_t* const row_slots = reinterpret_cast<int32_t*>(lds_raw + Cfg::kLdsBytes + wave * kRowSlotBytes);
+  auto fetch_rows = [&](int it) {
+    const int j = it * BN + lane;
+    dma4(reinterpret_cast<const char*>(row_of), 4u * (uint32_t)(j < Lk ? j : Lk - 1), reinterpret_cast<unsigned char*>(row_slots + (it & 1) * 64));
+  };
+  auto stage = [&](int it, int buf) {
+    if constexpr (kRows) {
+      if (listed) {
+        stager.issue_listed(lds_raw + buf * kBufBytes, row_slots + (it & 1) * 64);
+        if (it + 1 < ntiles) {
+          __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the list has been read (and the slot of it + 1 was before it)
+          fetch_rows(it + 1);
+        }
+        return;
+      }
+    }
+    stager.issue(lds_raw + buf * kBufBytes, it * BN, Lk);
+  };
 
   // Sparse: tile `it` is computed iff its 256-key block is active for any 16-row block of this query tile.  The tile's
   // and this lane's row block's activity bits of 64 consecutive key blocks (16384 keys) sit in registers.
@@ -194,7 +241,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
   float l_i = 0.f;        // this lane's share of the running row sum (other share in lane^32)
 
   const float cs = p.scale_log2;
-  const float cse = kBias != 0 ? 1.f : cs;                       // units of the scores the softmax works on
+  const float cse = kBiased ? 1.f : cs;                       // units of the scores the softmax works on
   const float sl2 = kAlibi ? p.alibi[h] * kLog2e : 0.f;          // slope in base-2 exponent units
   // kTensorBias: the wave's 32 rows x BN keys of the bias come in as whole rows - BN / 8 lanes fetch the BN * 2 contiguous
   // bytes of one row, 16 bytes each, so that an instruction touches 8 (16) rows and not 32: read lane by lane in the MFMA
@@ -252,6 +299,12 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
   int it = next_active(tile0);
   bool row_on_cur = row_on_next;
   if (it < ntiles) {
+    if constexpr (kRows) {
+      if (listed) {
+        fetch_rows(it);
+        wait_vmem();
+      }
+    }
     stage(it, 0);
     if (kTensorBias) load_bias(it);
   }
@@ -392,7 +445,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
           lp[kb] = 0.f;
 #pragma unroll
           for (int r = 0; r < 16; r++) {
-            const float pe_arg = kBias != 0 ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
+            const float pe_arg = kBiased ? s[kb][r] - mc : __builtin_fmaf(s[kb][r], cs, -mc);
             s[kb][r] = (FA_ABLATE_FWD & 2) ? pe_arg * 1e-3f : fast_exp2(pe_arg);
             if constexpr (kDropout && (FA_ABLATE_FWD & 32) == 0) lp[kb] += s[kb][r];
           }
@@ -576,6 +629,14 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias, KS
   for (int i = 0; i < (32 * CH + 63) / 64; i++) {
     const int ch = lane + i * 64;
     const int row = ch / CH, col = (ch % CH) * 8;
+    if constexpr (kRows) {  // rows past the last token are the entry's padding: zeros
+      if ((32 * CH % 64 == 0 || ch < 32 * CH) && mw + row < p.max_sq) {
+        u32x4 val = *reinterpret_cast<const u32x4*>(Os + row * OS + col);
+        if (mw + row >= Lq) val = u32x4{0, 0, 0, 0};
+        st_global16(reinterpret_cast<T*>(p.o) + ((int64_t)b * p.max_sq + row_of[mw + row]) * p.o_rs + (int64_t)h * p.o_hs + col, val);
+      }
+      continue;
+    }
     int orow = mw + row;  // (sparse: the wave's rows are those of its two row blocks)
     if (kSparse) orow = (row < 16 ? rb_a : rb_b) < 0 ? 0x3fffffff : (row < 16 ? rb_a : rb_b) * 16 + (row & 15);
     if ((32 * CH % 64 == 0 || ch < 32 * CH) && orow < Lq) {

@@ -48,6 +48,7 @@ FA_DEVICE void slab_row_blocks(const SparseMaps& sp, bool ordered, int qt, int s
 constexpr int kBiasNone = 0;    // nothing
 constexpr int kBiasAlibi = 1;   // -slope[head] * |query - key| (alibi)
 constexpr int kBiasTensor = 2;  // bias[b, h, query, key] (bias, strides in elements; batch and head stride may be 0)
+constexpr int kPaddedRows = 3;  // nothing, and the rows are those of a padded batch (row_of; the forward kernel only)
 
 struct FwdParams {
   const void* q;
@@ -93,7 +94,14 @@ struct FwdParams {
   uint32_t* keep_words;
   int kw_q;   // query extent of the buffer (max_seqlen_q rounded up to 128)
   int kw_kb;  // 32-key blocks (max_seqlen_k rounded up to 128, / 32)
+  // Padded batch (the forward's kPaddedRows variants; null: packed sequences), as launch_padding_rows() leaves them: entry b's tokens are the rows
+  // b * max_sq + row_of[b * max_sq + i], i < row_info[4 b]; the rest of row_of's slice lists its padding rows
+  const int32_t* row_of;
+  const int32_t* row_info;
 };
+
+// What launch_padding_rows() leaves per batch entry in row_info: number of tokens, first token's position, 1 if they are consecutive
+constexpr int kRowInfo = 4;
 
 struct DumpParams {  // return_softmax path
   const void* q;
@@ -194,11 +202,12 @@ FA_DEVICE bool seq_extent(const int32_t* cu, int b, int total, int max_len, int*
 // more than 64 entries keep their order.  The search costs every workgroup's prologue a few instructions per batch entry,
 // so the launchers ask for it (tile_group < 0 in a launch without a mask) only for grids that are resident all at once
 // (longest_first_launch), where the spreading is what it buys.
-FA_DEVICE int longest_first(const int32_t* cu, int B, int slot) {
+// (info: the lengths stand in row_info instead, see FwdParams)
+FA_DEVICE int longest_first(const int32_t* cu, int B, int slot, const int32_t* info = nullptr) {
   if (B > 64 || B < 2) return slot;
   const int lane = threadIdx.x & 63;
   const int i = lane < B ? lane : B - 1;
-  const int len = cu[i + 1] - cu[i];
+  const int len = info ? info[kRowInfo * i] : cu[i + 1] - cu[i];
   int before = 0;
   for (int j = 0; j < B; j++) {
     const int lj = __builtin_amdgcn_readlane(len, j);
@@ -326,6 +335,9 @@ hipError_t launch_gather_rows(const void* src, void* dst, const int64_t* idx, in
 hipError_t launch_scatter_rows(const void* src, void* dst, const int64_t* idx, int64_t n_idx, int64_t n_dst,
                                int64_t row_bytes, int64_t src_stride, int64_t dst_stride, int vec, int32_t* inv,
                                hipStream_t stream);
+// From a (batch, seqlen) mask of bytes (nonzero: a token): row_of, row_info (FwdParams) and, if lens is not null, the lengths
+hipError_t launch_padding_rows(const unsigned char* mask, int64_t mask_stride, int batch, int seqlen, int32_t* row_of, int32_t* row_info,
+                               int32_t* lens, hipStream_t stream);
 hipError_t launch_bias_grad_reduce(const void* in, void* out, int dtype, int nb, int nh, int rows, int cols, int64_t in_bs,
                                    int64_t in_hs, int64_t in_rs, int sum_batch, int sum_heads, int64_t out_bs, int64_t out_hs,
                                    int64_t out_rs, bool vec_store, hipStream_t stream);

@@ -88,6 +88,57 @@ __global__ void __launch_bounds__(512) scatter_rows_kernel(const unsigned char* 
     if (i < nrows) *reinterpret_cast<C*>(dst + (row0 + i) * dst_stride + (int64_t)ch * V) = v[i];
 }
 
+// A padding mask read off on the device: one workgroup per batch entry; a thread counts the tokens of its share of consecutive positions, a
+// scan over the workgroup gives everyone's place, and the share is walked again: tokens go to row_of in their order, padding
+// positions behind the last of them.  (Latency: two walks over seqlen / 512 bytes a thread around one scan, 4 us for 32 x 512.)
+constexpr int kMaskThreads = 512;
+__global__ void __launch_bounds__(kMaskThreads) padding_rows_kernel(const unsigned char* __restrict__ mask, int64_t mask_stride, int seqlen,
+                                                                    int32_t* __restrict__ row_of, int32_t* __restrict__ row_info,
+                                                                    int32_t* __restrict__ lens) {
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NW = kMaskThreads / 64;
+  __shared__ int wave_sum[NW], first_l, last_l;
+  mask += b * mask_stride;
+  row_of += (int64_t)b * seqlen;
+  const int per = (seqlen + kMaskThreads - 1) / kMaskThreads;
+  const int s0 = tid * per < seqlen ? tid * per : seqlen, s1 = s0 + per < seqlen ? s0 + per : seqlen;
+  int n = 0;
+  for (int s = s0; s < s1; s++) n += mask[s] != 0;
+  int incl = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  if (tid == 0) first_l = last_l = 0;
+  __syncthreads();
+  int before = incl - n, total = 0;
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    if (w < wave) before += wave_sum[w];
+    total += wave_sum[w];
+  }
+  int kept = before, pad = total + s0 - before;
+  for (int s = s0; s < s1; s++) {
+    if (mask[s] != 0) {
+      if (kept == 0) first_l = s;
+      if (kept == total - 1) last_l = s;
+      row_of[kept++] = s;
+    } else {
+      row_of[pad++] = s;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    row_info[kRowInfo * b] = total;
+    row_info[kRowInfo * b + 1] = first_l;
+    row_info[kRowInfo * b + 2] = total == 0 || last_l - first_l == total - 1 ? 1 : 0;
+    row_info[kRowInfo * b + 3] = 0;
+    if (lens) lens[b] = total;
+  }
+}
+
 // Launch shape: a row's chunks go to one workgroup of whole waves if at most 512, else to 256-thread workgroups; grid.y
 // holds the groups of rows (at most 65535 per launch: longer tensors take several launches, see the launchers).
 struct RowGrid {
@@ -128,6 +179,12 @@ hipError_t launch_gather_rows(const void* src, void* dst, const int64_t* idx, in
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+hipError_t launch_padding_rows(const unsigned char* mask, int64_t mask_stride, int batch, int seqlen, int32_t* row_of, int32_t* row_info,
+                               int32_t* lens, hipStream_t stream) {
+  hipLaunchKernelGGL(padding_rows_kernel, dim3((unsigned)batch), dim3(kMaskThreads), 0, stream, mask, mask_stride, seqlen, row_of, row_info, lens);
+  return hipGetLastError();
 }
 
 hipError_t launch_scatter_rows(const void* src, void* dst, const int64_t* idx, int64_t n_idx, int64_t n_dst,

@@ -75,6 +75,15 @@ FA_DEVICE void dma16(const char* base, uint32_t lane_off, unsigned char* lds_dst
                : "memory", "m0");
 }
 
+// The same with 4 bytes a lane: lane l's go to lds_dst + 4 * l.
+FA_DEVICE void dma4(const char* base, uint32_t lane_off, unsigned char* lds_dst) {
+  const uint32_t lds_addr = (uint32_t)(uintptr_t)(FA_LDS void*)lds_dst;
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+               :
+               : "v"(lane_off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+
 // Stages a pair of ROWS x D tiles per step: tile 0 (swizzle KIND0) by waves 0 and 1, tile 1 (KIND1) by waves 2 and 3,
 // into [lds, lds + kTileBytes) and [lds + kTileBytes, lds + 2 * kTileBytes).  A workgroup has 4 waves.
 template <int D, int ROWS, int KIND0, int KIND1>
@@ -130,6 +139,15 @@ struct TilePairStager {
         const int rc = first_row + r < n_rows ? r : n_rows - 1 - first_row;
         dma16(tb, (uint32_t)(rc * rsb) + 16u * (uint32_t)(pchv ^ swz(r)), lds + dst0 + i * 1024);
       }
+    }
+  }
+
+  // The same for a tile whose row r is tensor row list[r] (list: LDS, one entry per tile row, all of them valid rows).
+  FA_DEVICE void issue_listed(unsigned char* lds, const int32_t* list) const {
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int r = row0 + i * RPI + rl;
+      dma16(base, (uint32_t)list[r] * (uint32_t)rsb + 16u * (uint32_t)(pch ^ swz(r)), lds + dst0 + i * 1024);
     }
   }
 

@@ -3,8 +3,17 @@ flash_attn/flash_attention.py (:12-118)."""
 import torch
 import torch.nn as nn
 
+from . import flash_attn_gfx950 as _backend
 from .bert_padding import pad_input, unpad_input
 from .flash_attn_interface import flash_attn_unpadded_qkvpacked_func, flash_attn_unpadded_qkvpacked_rotary_func
+
+
+class _PaddedAttention(torch.autograd.Function):
+    """Attention of a padded batch that no gradient is asked of: the kernels take the padded rows as they are."""
+
+    @staticmethod
+    def forward(ctx, qkv, mask, softmax_scale, causal):
+        return _backend.fwd_padded(qkv, mask, softmax_scale, causal)
 
 
 class FlashAttention(nn.Module):
@@ -66,6 +75,13 @@ class FlashAttention(nn.Module):
             return out.reshape(batch, seqlen, *out.shape[1:]), None
 
         nheads, headdim = qkv.shape[-2], qkv.shape[-1]
+        mask = key_padding_mask.bool_matrix
+        if (p == 0.0 and alibi_slopes is None and attn_bias is None and not (qkv.requires_grad and torch.is_grad_enabled())
+                and _backend.padded_layout_ok(qkv, mask)):
+            scale = headdim ** (-0.5) if self.softmax_scale is None else self.softmax_scale
+            out = _PaddedAttention.apply(qkv, mask, scale, causal)
+            if out is not None:  # (a batch without a token is refused below)
+                return out, None
         x = qkv.reshape(batch, seqlen, 3 * nheads * headdim)
         x_unpad, indices, cu, max_len = unpad_input(x, key_padding_mask.bool_matrix)
         out_unpad = flash_attn_unpadded_qkvpacked_func(x_unpad.reshape(-1, 3, nheads, headdim), cu, max_len, p,

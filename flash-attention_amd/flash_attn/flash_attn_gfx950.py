@@ -120,7 +120,7 @@ EXPORTED_SYMBOLS = (
     "fa_fwd", "fa_bwd", "fa_fwd_block", "fa_bwd_block", "fa_fwd_block_noalloc", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes",
     "fa_round_seqlens", "fa_philox_offset_increment", "fa_last_error", "fa_abi_version",
     "fa_gather_rows", "fa_scatter_rows", "fa_scatter_rows_workspace_bytes", "fa_rotary", "fa_set_launch_policy",
-    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce",
+    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_padding_rows", "fa_fwd_padded",
 )
 # declared in include/flash_attn_gfx950_bench.h: instrumentation for bench.py, not part of the drop-in boundary
 BENCH_SYMBOLS = ("fa_bwd_profiled",)
@@ -174,6 +174,10 @@ def load_library():
         lib.fa_bias_grad_reduce.argtypes = ([ctypes.c_void_p] * 2 + [ctypes.c_int32] * 5 + [ctypes.c_int64] * 3 +
                                             [ctypes.c_int32] * 2 + [ctypes.c_int64] * 3 + [ctypes.c_void_p])
         lib.fa_bias_grad_reduce.restype = ctypes.c_int
+        lib.fa_padding_rows.argtypes = ([ctypes.c_void_p, ctypes.c_int64] + [ctypes.c_int32] * 2 + [ctypes.c_void_p] * 4)
+        lib.fa_padding_rows.restype = ctypes.c_int
+        lib.fa_fwd_padded.argtypes = [ctypes.POINTER(FwdArgs), ctypes.c_void_p, ctypes.c_void_p]
+        lib.fa_fwd_padded.restype = ctypes.c_int
         lib.fa_scatter_rows_workspace_bytes.argtypes = [ctypes.c_int64]
         lib.fa_scatter_rows_workspace_bytes.restype = ctypes.c_size_t
         lib.fa_rotary.argtypes = [ctypes.POINTER(RotaryArgs)]
@@ -716,6 +720,64 @@ def scatter_rows(values, indices, first_axis_dim):
     if rc != 0:
         _raise(rc, lib)
     return out
+
+
+def padded_layout_ok(qkv, mask):
+    """Whether fwd_padded() takes this (batch, seqlen, 3, nheads, headdim) tensor and mask as they are: a bool mask of one byte a position,
+    rows of qkv one after the other, 16-byte aligned.  (Others are gathered and scattered, bert_padding.py.)"""
+    if not (qkv.is_cuda and qkv.dim() == 5 and qkv.shape[2] == 3 and mask.dtype == torch.bool and mask.device == qkv.device):
+        return False
+    B, S, _, H, D = qkv.shape
+    st = qkv.stride()
+    return (tuple(mask.shape) == (B, S) and mask.stride(1) == 1 and D in (16, 32, 64, 128) and B > 0 and S > 0 and H > 0 and
+            st[4] == 1 and st[0] == S * st[1] and all(x % 8 == 0 and 0 <= x < 1 << 24 for x in st[1:4]) and
+            qkv.data_ptr() % 16 == 0 and S * st[1] < 1 << 31 and B * S < 1 << 31)
+
+
+def fwd_padded(qkv, mask, softmax_scale, is_causal):
+    """Attention of a padded batch without gathering it first (fa_padding_rows, fa_fwd_padded): qkv (batch, seqlen, 3, nheads, headdim) and
+    a (batch, seqlen) bool mask, True = token, for which padded_layout_ok() holds.  Returns (batch, seqlen, nheads, headdim) with zeros in
+    the padding, or None if the mask holds no token at all.  The lengths are read back for that while the attention kernel runs."""
+    lib = load_library()
+    B, S, _, H, D = qkv.shape
+    st = qkv.stride()
+    dev = qkv.device
+    sq_r, _ = round_seqlens(D, S, S, False)
+    with _OnDevice(dev):
+        out = torch.empty((B, S, H, D), dtype=qkv.dtype, device=dev)
+        lse = torch.empty((B, H, sq_r), dtype=torch.float32, device=dev)
+        rows = torch.empty((B * (S + 4),), dtype=torch.int32, device=dev)
+        lens = torch.empty((B,), dtype=torch.int32, pin_memory=True)
+        row_of, stream = rows.data_ptr(), _stream_handle(dev)
+        row_info = row_of + 4 * B * S
+        rc = lib.fa_padding_rows(mask.data_ptr(), mask.stride(0), B, S, row_of, row_info, lens.data_ptr(), stream)
+        if rc != 0:
+            _raise(rc, lib)
+        written = torch.cuda.Event()
+        written.record()
+
+        def fill(a):
+            a.dtype = _dtype_code(qkv)
+            a.q_row_stride = a.k_row_stride = a.v_row_stride = st[1]
+            a.q_head_stride = a.k_head_stride = a.v_head_stride = st[3]
+            a.o_row_stride, a.o_head_stride = H * D, D
+            a.batch, a.nheads, a.head_dim = B, H, D
+            a.total_q = a.total_k = B * S
+            a.max_seqlen_q = a.max_seqlen_k = S
+            a.is_causal = int(bool(is_causal))
+            return 0
+
+        a, _ = _cached_args(("padded", qkv.dtype, qkv.shape, st, bool(is_causal)), FwdArgs, fill)
+        a.q = qkv.data_ptr()
+        a.k, a.v = a.q + 2 * st[2], a.q + 4 * st[2]
+        a.o, a.softmax_lse = out.data_ptr(), lse.data_ptr()
+        a.softmax_scale = float(softmax_scale)
+        a.stream = stream
+        rc = lib.fa_fwd_padded(ctypes.byref(a), row_of, row_info)
+        if rc != 0:
+            _raise(rc, lib)
+        written.synchronize()
+    return out if lens.any() else None
 
 
 def rotary(src, dst, cos, sin, n_rotated, conjugate=False, positions=None):

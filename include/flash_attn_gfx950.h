@@ -251,6 +251,22 @@ int fa_scatter_rows(const void* src, void* dst, const int64_t* indices, int64_t 
                     size_t workspace_bytes, void* stream);
 size_t fa_scatter_rows_workspace_bytes(int64_t n_dst_rows);
 
+/* Attention over a padded batch as it is (the reference's FlashAttention module gathers the tokens, calls the packed forward and
+ * scatters its output: flash_attention.py:53-66, bert_padding.py:60-95; these two do the same without moving q, k, v or o).
+ *
+ * fa_padding_rows reads a (batch, seqlen) mask of bytes (nonzero: a token; mask_row_stride bytes apart) and writes, per batch entry, the
+ * positions of its tokens followed by those of its padding (row_of: batch * seqlen int32) and four int32 for the kernels (row_info:
+ * batch * 4).  lens: NULL, or batch int32 that receive the numbers of tokens (device memory, or host memory the GPU can write).
+ *
+ * fa_fwd_padded is fa_fwd on q, k, v and o of batch * max_seqlen rows (total_q = total_k = batch * max_seqlen, max_seqlen_q =
+ * max_seqlen_k): an entry's tokens attend each other, counted in their own order (is_causal), the rows of o that are padding become
+ * zero, and softmax_lse holds the tokens' values, in their order, at the front of each row of its own.  cu_seqlens_q / k are not read.  No
+ * dropout, bias, rotary tables or s_dmask; max_seqlen * row stride of k and v below 2^32 bytes.  row_of and row_info: as fa_padding_rows
+ * leaves them for the same batch and seqlen (they are trusted: entries that are no positions make the kernel read and write elsewhere). */
+int fa_padding_rows(const void* mask, int64_t mask_row_stride, int32_t batch, int32_t seqlen, int32_t* row_of, int32_t* row_info,
+                    int32_t* lens, void* stream);
+int fa_fwd_padded(const fa_fwd_args* args, const int32_t* row_of, const int32_t* row_info);
+
 /* Sum of the bias gradient over the batch entries and / or heads that shared one bias (no counterpart in the
  * reference, which takes no bias).  fa_bwd writes `dbias` per (batch, head); a bias of batch or head extent 1 that
  * was broadcast wants the sum.  dbias: [batch, heads, rows, >= cols rounded up to 8] in `dtype` (strides in elements,

@@ -1307,6 +1307,52 @@ def test_blocksparse_causal_sweep():
 # ------------------------------------------------------------------------------------------------
 # modules
 # ------------------------------------------------------------------------------------------------
+def _padding_masks(B, S, seed):
+    """(B, S) bool masks: right padding, left padding, holes, one run in the middle; entry 0 full, entry 1 (if there is one) without tokens."""
+    g = torch.Generator().manual_seed(seed)
+    pos = torch.arange(S)
+    lens = torch.randint(1, S + 1, (B, 1), generator=g)
+    first = (torch.rand(B, 1, generator=g) * (S - lens + 1)).long()
+    for m in (pos < lens, pos >= S - lens, torch.rand(B, S, generator=g) < 0.6, (pos >= first) & (pos < first + lens)):
+        m = m.expand(B, S).clone()
+        m[0] = True
+        if B > 1:
+            m[1] = False
+        yield m
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape):
+    """Evaluation of a padded batch reads q, k, v where they lie and writes the padded output at once (fa_padding_rows, fa_fwd_padded).
+    With one entry full both ways run the same tiles over the same tokens in the same order (beyond the decode kernel's 32 rows): equal bit
+    for bit to unpad, packed attention, pad.  Lengths around the 64- and 128-row tiles, tokens in one run or anywhere, entries without any."""
+    from flash_attn.bert_padding import pad_input, unpad_input
+    from flash_attn.flash_attention import FlashAttention
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_qkvpacked_func
+    m = FlashAttention(attention_dropout=0.3).eval()
+    for S, B, H in ((1, 1, 2), (33, 3, 2), (64, 2, 3), (127, 4, 1), (129, 5, 2), (200, 9, 3), (513, 3, 4)):
+        g = torch.Generator(device="cuda").manual_seed(S)
+        wide = torch.randn(B, S, 4, H, D, generator=g, device="cuda").half()
+        for i, mask in enumerate(_padding_masks(B, S, S)):
+            qkv = wide[:, :, :3] if i % 2 else wide[:, :, :3].contiguous()  # rows apart by more than their width, or packed
+            kpm = type("Mask", (), {"bool_matrix": mask.cuda()})
+            with torch.no_grad():
+                got = m(qkv, key_padding_mask=kpm, causal=causal)[0]
+                rows, idx, cu, mx = unpad_input(qkv.reshape(B, S, -1), kpm.bool_matrix)
+                out = flash_attn_unpadded_qkvpacked_func(rows.view(-1, 3, H, D), cu, mx, 0.0, causal=causal)
+                want = pad_input(out.view(-1, H * D), idx, B, S).view(B, S, H, D)
+            what = (S, B, H, i)
+            assert got.shape == want.shape and (got[~kpm.bool_matrix] == 0).all(), what
+            if S > 32:
+                assert torch.equal(got, want), what
+            else:  # the packed call takes the decode kernel, which sums in another order: two roundings of the result
+                assert (got.float() - want.float()).abs().max() <= 2 * HALF_ULP[torch.float16] * want.abs().max().clamp(min=1), what
+    with pytest.raises(RuntimeError):  # a batch without a token is refused
+        with torch.no_grad():
+            m(qkv, key_padding_mask=type("Mask", (), {"bool_matrix": torch.zeros(B, S, dtype=torch.bool, device="cuda")}), causal=causal)
+
+
 def test_flash_attention_module_three_input_modes():
     from flash_attn.flash_attention import FlashAttention
     B, S, H, D = 3, 96, 2, 64
