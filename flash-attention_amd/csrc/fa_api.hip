@@ -172,11 +172,10 @@ bool decode_needs_splits(int batch, int nheads, int head_dim, int max_sk) {
 
 int build_maps(const int32_t* blockmask, const int32_t* row_order, unsigned char* ws, const SparseLayout& sl,
                fa::SparseMaps* out, hipStream_t stream) {
-  FA_LAUNCH(fa::launch_fill_f32(reinterpret_cast<float*>(ws), sl.bytes / 4, 0.f, stream));
   FA_LAUNCH(fa::launch_build_sparse_maps(blockmask, reinterpret_cast<uint64_t*>(ws + sl.offr),
                                          reinterpret_cast<uint64_t*>(ws + sl.offq),
                                          reinterpret_cast<uint64_t*>(ws + sl.offc), sl.nrb, sl.ncb, fa::kFwdBM, sl.nqt,
-                                         sl.ncw, sl.nrw, row_order, reinterpret_cast<int32_t*>(ws + sl.offi), stream));
+                                         sl.ncw, sl.nrw, row_order, reinterpret_cast<int32_t*>(ws + sl.offi), ws, sl.bytes, stream));
   out->order = row_order;
   out->rbits = reinterpret_cast<const uint64_t*>(ws + sl.offr);
   out->qbits = reinterpret_cast<const uint64_t*>(ws + sl.offq);

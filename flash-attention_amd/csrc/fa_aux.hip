@@ -54,6 +54,44 @@ __global__ void sparse_maps_kernel(const int32_t* blockmask, uint32_t* rbits, ui
   atomicOr(cbits + ((int64_t)cb * nrw * 2 + (rb >> 5)), 1u << (rb & 31));
 }
 
+// The same maps in one launch without clears, an inverse order or atomics in memory, for layouts of at most kMapsRows row blocks: a
+// workgroup owns 64 key blocks, i.e. word blockIdx.x of rbits and qbits and 64 rows of cbits, builds the bits in LDS and writes every word it
+// owns once; a query tile's bits are the OR of its row blocks', read off the order as it is.  Latency-bound; with many entries one workgroup
+// per 64 key blocks is too few, see launch_build_sparse_maps.  (A training step builds them twice: 4 x 16 heads x 4096, a quarter of the
+// blocks, 508 -> 501 us.)
+constexpr int kMapsRows = 2048, kMapsThreads = 1024;
+__global__ void __launch_bounds__(kMapsThreads) sparse_maps_lds_kernel(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits,
+                                                                       int nrb, int ncb, int rpq, int nqt, int ncw, int nrw,
+                                                                       const int32_t* order) {
+  __shared__ __attribute__((aligned(8))) uint32_t rl[kMapsRows * 2], cl[64 * (kMapsRows / 32)];
+  const int w = blockIdx.x, cb0 = w * 64, tid = threadIdx.x;
+  const int ncols = ncb - cb0 < 64 ? ncb - cb0 : 64;
+  for (int i = tid; i < nrb * 2; i += kMapsThreads) rl[i] = 0;
+  for (int i = tid; i < ncols * nrw * 2; i += kMapsThreads) cl[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < ncols * nrb; i += kMapsThreads) {
+    const int c = i / nrb, e = blockmask[(int64_t)cb0 * nrb + i];
+    const int rb = e >> 2;
+    if (e < 0 || rb >= nrb) continue;
+    atomicOr(rl + rb * 2 + (c >> 5), 1u << (c & 31));
+    atomicOr(cl + c * nrw * 2 + (rb >> 5), 1u << (rb & 31));
+  }
+  __syncthreads();
+  const uint64_t* const rw = reinterpret_cast<const uint64_t*>(rl);
+  const uint64_t* const cw = reinterpret_cast<const uint64_t*>(cl);
+  for (int i = tid; i < nrb; i += kMapsThreads) rbits[(int64_t)i * ncw + w] = rw[i];
+  for (int i = tid; i < ncols * nrw; i += kMapsThreads) cbits[(int64_t)cb0 * nrw + i] = cw[i];
+  for (int t = tid; t < nqt; t += kMapsThreads) {
+    uint64_t q = 0;
+    for (int j = 0; j < rpq; j++) {
+      const int pos = t * rpq + j;
+      int rb = pos < nrb ? (order ? order[pos] : pos) : -1;
+      if (rb >= 0 && rb < nrb) q |= rw[rb];
+    }
+    qbits[(int64_t)t * ncw + w] = q;
+  }
+}
+
 // One thread per (query row, key) element of S_dmask.  Slow scalar dot products: this path exists for tests
 // (flash_attn_interface.py:163-173).  The value is the normalised probability exp(scale*s - lse); its sign
 // bit is set when dropout dropped the element.
@@ -119,9 +157,18 @@ hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride,
 
 hipError_t launch_build_sparse_maps(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits, int nrb,
                                     int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv,
-                                    hipStream_t stream) {
+                                    void* maps, size_t maps_bytes, hipStream_t stream) {
   const int n = nrb * ncb;
-  if (order && inv) {  // (inv was cleared by the caller)
+  // us of one launch / of the three below, their gaps not counted: 64 x 4 blocks 2.9 / 5.9, 256 x 16 4.5 / 7.9, 512 x 32 9.4 / 17.2,
+  // 1024 x 64 27.4 / 23.1 (64 entries a thread of one workgroup)
+  if (nrb <= kMapsRows && n <= 16384) {
+    hipLaunchKernelGGL(sparse_maps_lds_kernel, dim3((unsigned)ncw), dim3(kMapsThreads), 0, stream, blockmask, rbits, qbits, cbits, nrb, ncb,
+                       rows_per_qt / 16, nqt, ncw, nrw, order);
+    return hipGetLastError();
+  }
+  const hipError_t e = launch_fill_f32(reinterpret_cast<float*>(maps), maps_bytes / 4, 0.f, stream);
+  if (e != hipSuccess) return e;
+  if (order && inv) {
     hipLaunchKernelGGL(invert_order_kernel, dim3((nrb + 255) / 256), dim3(256), 0, stream, order, inv, nrb);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -345,10 +345,11 @@ hipError_t launch_dump_probs(const DumpParams& p, int dtype, hipStream_t stream)
 // which: 0 = dQ kernel, 1 = dK/dV kernel
 hipError_t launch_bwd(const BwdParams& p, int which, int dtype, int head_dim, bool causal, bool dropout, bool sparse,
                       hipStream_t stream);
+// maps, maps_bytes: the scratch that holds all of them (cleared where they are built with atomics)
 // order / inv: null, or the row order (SparseMaps::order) and nrb ints of scratch for its inverse
 hipError_t launch_build_sparse_maps(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits, int nrb,
                                     int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv,
-                                    hipStream_t stream);
+                                    void* maps, size_t maps_bytes, hipStream_t stream);
 hipError_t launch_fill_f32(float* p, size_t n, float value, hipStream_t stream);
 // Zero a strided [total, H, D] tensor of 16-bit elements.
 hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride, int total, int H, int D,

@@ -1077,6 +1077,27 @@ def test_blocksparse_more_than_64_key_blocks():
     check_against_oracle({"out": out, "dq": dq, "dk": dk, "dv": dv}, ref, half, torch.float16, what="blocksparse 66 key blocks")
 
 
+def test_blocksparse_few_rows_many_key_blocks():
+    """Activity maps of two words a row block that are still built in one launch: 64 queries on 67 and on 128 key blocks."""
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
+    for ncb in (67, 128):
+        lens_q, lens_k, H, D = [64], [ncb * 256 - 9], 2, 16
+        layout = torch.rand(4, ncb, generator=torch.Generator().manual_seed(ncb)) < 0.3
+        layout[:, 0] = False
+        layout[:, 66] = True
+        q, k, v, do = _inputs(lens_q, lens_k, H, D, torch.float16, ncb)
+        cu_q, cu_k = _cu(lens_q, "cpu"), _cu(lens_k, "cpu")
+        ref = orc.varlen_attention(q, k, v, cu_q, cu_k, D ** -0.5, False, layout=layout.numpy(), dout=do)
+        half = half_attention(q.cuda(), k.cuda(), v.cuda(), cu_q.tolist(), cu_k.tolist(), D ** -0.5, False, layout=layout.numpy(), dout=do.cuda())
+        qg, kg, vg, dg = (x.cuda() for x in (q, k, v, do))
+        bm = convert_blockmask(layout.cuda(), causal=False)
+        out, lse = be.fwd_block(qg, kg, vg, cu_q.cuda(), cu_k.cuda(), bm, 64, lens_k[0], 0.0, D ** -0.5, False, False, None)
+        dq, dk, dv = torch.empty_like(qg), torch.empty_like(kg), torch.empty_like(vg)
+        be.bwd_block(dg, qg, kg, vg, out, lse, dq, dk, dv, cu_q.cuda(), cu_k.cuda(), bm, 64, lens_k[0], 0.0, D ** -0.5, False, None)
+        check_against_oracle(dict(out=out, dq=dq, dk=dk, dv=dv), ref, half, torch.float16, what="64 queries, %d key blocks" % ncb)
+
+
 def test_blocksparse_random_layouts_sweep():
     """Ten seeded random block-sparse cases: densities from 5 % to 90 % (with and without the diagonal band), ragged
     lengths up to 2100 (several activity words per key block on the backward side), every head dim, both dtypes, dropout."""
