@@ -696,10 +696,10 @@ int fa_scatter_rows(const void* src, void* dst, const int64_t* indices, int64_t 
   return FA_OK;
 }
 
-int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t batch, int32_t heads, int32_t rows,
+static int bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t batch, int32_t heads, int32_t rows,
                         int32_t cols, int64_t dbias_batch_stride, int64_t dbias_head_stride, int64_t dbias_row_stride,
                         int32_t sum_batch, int32_t sum_heads, int64_t out_batch_stride, int64_t out_head_stride,
-                        int64_t out_row_stride, void* stream) {
+                        int64_t out_row_stride, const fa::BiasGradLens& lens, void* stream) {
   FA_REQUIRE(dtype == 0 || dtype == 1, "fa_bias_grad_reduce: dtype must be 0 (fp16) or 1 (bf16)");
   FA_REQUIRE(batch >= 0 && heads >= 0 && rows >= 0 && cols >= 0, "fa_bias_grad_reduce: negative size");
   FA_REQUIRE(batch <= 65535 && heads <= 65535, "fa_bias_grad_reduce: more than 65535 batch entries or heads");
@@ -715,8 +715,27 @@ int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t bat
                          out_head_stride % 8 == 0 && out_row_stride % 8 == 0;
   FA_LAUNCH(fa::launch_bias_grad_reduce(dbias, out, dtype, batch, heads, rows, cols, dbias_batch_stride, dbias_head_stride,
                                         dbias_row_stride, sum_batch != 0, sum_heads != 0, out_batch_stride, out_head_stride,
-                                        out_row_stride, vec_store, reinterpret_cast<hipStream_t>(stream)));
+                                        out_row_stride, lens, vec_store, reinterpret_cast<hipStream_t>(stream)));
   return FA_OK;
+}
+
+int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t batch, int32_t heads, int32_t rows,
+                        int32_t cols, int64_t dbias_batch_stride, int64_t dbias_head_stride, int64_t dbias_row_stride,
+                        int32_t sum_batch, int32_t sum_heads, int64_t out_batch_stride, int64_t out_head_stride,
+                        int64_t out_row_stride, void* stream) {
+  return bias_grad_reduce(dbias, out, dtype, batch, heads, rows, cols, dbias_batch_stride, dbias_head_stride, dbias_row_stride, sum_batch,
+                          sum_heads, out_batch_stride, out_head_stride, out_row_stride, fa::BiasGradLens{}, stream);
+}
+
+int fa_bias_grad_reduce_ragged(const void* dbias, void* out, const fa_bwd_args* a, int32_t sum_batch, int32_t sum_heads,
+                               int64_t out_batch_stride, int64_t out_head_stride, int64_t out_row_stride) {
+  FA_REQUIRE(a && a->struct_bytes == sizeof(fa_bwd_args), "fa_bias_grad_reduce_ragged: struct size mismatch");
+  FA_REQUIRE(a->cu_seqlens_q && a->cu_seqlens_k, "fa_bias_grad_reduce_ragged: null pointer");
+  FA_REQUIRE(!a->blockmask, "fa_bias_grad_reduce_ragged: under a block layout only the listed blocks are written, clear dbias and use fa_bias_grad_reduce");
+  const fa::BiasGradLens lens{a->cu_seqlens_q, a->cu_seqlens_k, a->total_q, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0};
+  return bias_grad_reduce(dbias, out, a->dtype, a->batch, a->nheads, a->max_seqlen_q, a->max_seqlen_k, a->dbias_batch_stride,
+                          a->dbias_head_stride, a->dbias_row_stride, sum_batch, sum_heads, out_batch_stride, out_head_stride, out_row_stride,
+                          lens, a->stream);
 }
 
 int fa_rotary(const fa_rotary_args* a) {

@@ -338,9 +338,14 @@ hipError_t launch_scatter_rows(const void* src, void* dst, const int64_t* idx, i
 // From a (batch, seqlen) mask of bytes (nonzero: a token): row_of, row_info (FwdParams) and, if lens is not null, the lengths
 hipError_t launch_padding_rows(const unsigned char* mask, int64_t mask_stride, int batch, int seqlen, int32_t* row_of, int32_t* row_info,
                                int32_t* lens, hipStream_t stream);
+struct BiasGradLens {  // the batch's lengths as the backward had them (seq_extent); cu_q null: every element of the slices holds a gradient
+  const int32_t* cu_q;
+  const int32_t* cu_k;
+  int total_q, total_k, max_sq, max_sk, causal;
+};
 hipError_t launch_bias_grad_reduce(const void* in, void* out, int dtype, int nb, int nh, int rows, int cols, int64_t in_bs,
                                    int64_t in_hs, int64_t in_rs, int sum_batch, int sum_heads, int64_t out_bs, int64_t out_hs,
-                                   int64_t out_rs, bool vec_store, hipStream_t stream);
+                                   int64_t out_rs, const BiasGradLens& lens, bool vec_store, hipStream_t stream);
 hipError_t launch_dump_probs(const DumpParams& p, int dtype, hipStream_t stream);
 // which: 0 = dQ kernel, 1 = dK/dV kernel
 hipError_t launch_bwd(const BwdParams& p, int which, int dtype, int head_dim, bool causal, bool dropout, bool sparse,

@@ -120,7 +120,7 @@ EXPORTED_SYMBOLS = (
     "fa_fwd", "fa_bwd", "fa_fwd_block", "fa_bwd_block", "fa_fwd_block_noalloc", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes",
     "fa_round_seqlens", "fa_philox_offset_increment", "fa_last_error", "fa_abi_version",
     "fa_gather_rows", "fa_scatter_rows", "fa_scatter_rows_workspace_bytes", "fa_rotary", "fa_set_launch_policy",
-    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_padding_rows", "fa_fwd_padded",
+    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_bias_grad_reduce_ragged", "fa_padding_rows", "fa_fwd_padded",
 )
 # declared in include/flash_attn_gfx950_bench.h: instrumentation for bench.py, not part of the drop-in boundary
 BENCH_SYMBOLS = ("fa_bwd_profiled",)
@@ -174,6 +174,8 @@ def load_library():
         lib.fa_bias_grad_reduce.argtypes = ([ctypes.c_void_p] * 2 + [ctypes.c_int32] * 5 + [ctypes.c_int64] * 3 +
                                             [ctypes.c_int32] * 2 + [ctypes.c_int64] * 3 + [ctypes.c_void_p])
         lib.fa_bias_grad_reduce.restype = ctypes.c_int
+        lib.fa_bias_grad_reduce_ragged.argtypes = ([ctypes.c_void_p] * 2 + [ctypes.POINTER(BwdArgs)] + [ctypes.c_int32] * 2 + [ctypes.c_int64] * 3)
+        lib.fa_bias_grad_reduce_ragged.restype = ctypes.c_int
         lib.fa_padding_rows.argtypes = ([ctypes.c_void_p, ctypes.c_int64] + [ctypes.c_int32] * 2 + [ctypes.c_void_p] * 4)
         lib.fa_padding_rows.restype = ctypes.c_int
         lib.fa_fwd_padded.argtypes = [ctypes.POINTER(FwdArgs), ctypes.c_void_p, ctypes.c_void_p]
@@ -678,10 +680,12 @@ def gather_rows(input, indices):
     return out
 
 
-def reduce_bias_grad(dbias, out, sum_batch, sum_heads):
+def reduce_bias_grad(dbias, out, sum_batch, sum_heads, written=None):
     """out[...] = sum of the per-(batch, head) bias gradient `dbias` (batch, nheads, rows, cols padded to 8) over the
     batch entries (sum_batch) and / or heads (sum_heads), added in fp32 and rounded once, by fa_bias_grad_reduce.
-    out: a (1 or batch, 1 or nheads, rows, cols) view in dbias's dtype, cols <= dbias.shape[3], innermost stride 1."""
+    out: a (1 or batch, 1 or nheads, rows, cols) view in dbias's dtype, cols <= dbias.shape[3], innermost stride 1.
+    written: None if every element of dbias counts, or (cu_seqlens_q, cu_seqlens_k, total_q, total_k, causal) of the dense backward that
+    filled a dbias nobody had cleared: what it did not write counts as zero (fa_bias_grad_reduce_ragged)."""
     _check(dbias.dim() == 4 and out.dim() == 4 and dbias.is_cuda and out.device == dbias.device and out.dtype == dbias.dtype,
            "dbias and out must be 4-D tensors of one dtype on one GPU")
     batch, nheads, rows, _ = dbias.shape
@@ -689,6 +693,23 @@ def reduce_bias_grad(dbias, out, sum_batch, sum_heads):
            out.shape[3] <= dbias.shape[3] and dbias.stride(3) == 1 and (out.stride(3) == 1 or out.shape[3] <= 1),
            "out must be (1 or batch, 1 or nheads, rows, cols <= dbias's) with contiguous keys")
     lib = load_library()
+    if written is not None:
+        cu_q, cu_k, total_q, total_k, causal = written
+        _check_cu("cu_seqlens_q", cu_q, batch)
+        _check_cu("cu_seqlens_k", cu_k, batch)
+        a = BwdArgs()
+        a.struct_bytes = ctypes.sizeof(a)
+        a.dtype, a.batch, a.nheads = _dtype_code(dbias), batch, nheads
+        a.total_q, a.total_k, a.max_seqlen_q, a.max_seqlen_k = total_q, total_k, rows, out.shape[3]
+        a.cu_seqlens_q, a.cu_seqlens_k, a.is_causal = cu_q.data_ptr(), cu_k.data_ptr(), int(bool(causal))
+        a.dbias_batch_stride, a.dbias_head_stride, a.dbias_row_stride = dbias.stride()[:3]
+        a.stream = _stream_handle(dbias.device)
+        with _OnDevice(dbias.device):
+            rc = lib.fa_bias_grad_reduce_ragged(dbias.data_ptr(), out.data_ptr(), ctypes.byref(a), int(bool(sum_batch)), int(bool(sum_heads)),
+                                                out.stride(0), out.stride(1), out.stride(2))
+        if rc != 0:
+            _raise(rc, lib)
+        return out
     with _OnDevice(dbias.device):
         rc = lib.fa_bias_grad_reduce(dbias.data_ptr(), out.data_ptr(), _dtype_code(dbias), batch, nheads, rows, out.shape[3],
                                      dbias.stride(0), dbias.stride(1), dbias.stride(2), int(bool(sum_batch)),

@@ -115,7 +115,11 @@ def _backward(ctx, dout):
     grads = tuple(torch.empty_like(t) for t in tensors)
     dq, dk, dv = _split(ctx.packing, grads)
     dev = q.device
-    dbias = new_bias_grad(q, cu_seqlens_q.numel() - 1, ctx.max_seqlen_q, ctx.max_seqlen_k) if ctx.bias_needs_grad else None
+    dbias = written = None
+    if ctx.bias_needs_grad:
+        if cu_seqlens_q.numel() - 1 <= 65535 and q.shape[1] <= 65535:  # (the grid of the kernel that knows what was written)
+            written = (cu_seqlens_q, cu_seqlens_k, q.shape[0], k.shape[0], ctx.causal)
+        dbias = new_bias_grad(q, cu_seqlens_q.numel() - 1, ctx.max_seqlen_q, ctx.max_seqlen_k, cleared=written is None)
     if rng_state is not None:
         cur_rng_state = torch.cuda.get_rng_state(dev)
         torch.cuda.set_rng_state(rng_state, dev)
@@ -124,24 +128,28 @@ def _backward(ctx, dout):
                          ctx.alibi_slopes, ctx.keep_words, bias_t, dbias, ctx.rotary)
     if rng_state is not None:
         torch.cuda.set_rng_state(cur_rng_state, dev)
-    ctx.dbias = bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_seqlen_q, ctx.max_seqlen_k) if dbias is not None else None
+    ctx.dbias = None
+    if dbias is not None:
+        ctx.dbias = bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_seqlen_q, ctx.max_seqlen_k, written)
     return grads
 
 
-def new_bias_grad(q, batch, max_seqlen_q, max_seqlen_k):
-    """The tensor the backward kernels leave the bias gradient in: per (batch, head), rows padded to 8 keys, cleared (only
-    the tiles the kernels visit are written)."""
-    return torch.zeros((batch, q.shape[1], max_seqlen_q, (max_seqlen_k + 7) // 8 * 8), dtype=q.dtype, device=q.device)
+def new_bias_grad(q, batch, max_seqlen_q, max_seqlen_k, cleared=True):
+    """The tensor the backward kernels leave the bias gradient in: per (batch, head), rows padded to 8 keys; cleared (only
+    the tiles the kernels visit are written), unless what reads it knows what was written (bias_grad_in_shape)."""
+    return (torch.zeros if cleared else torch.empty)((batch, q.shape[1], max_seqlen_q, (max_seqlen_k + 7) // 8 * 8), dtype=q.dtype, device=q.device)
 
 
-def bias_grad_in_shape(dbias, shape, max_seqlen_q, max_seqlen_k):
+def bias_grad_in_shape(dbias, shape, max_seqlen_q, max_seqlen_k, written=None):
     """The gradient of an attn_bias of `shape` from the per-(batch, head) tensor of new_bias_grad(): summed over the batch
-    entries / heads that shared the bias (one pass, fp32 sums, one rounding); rows / keys beyond max_seqlen get none."""
-    full = torch.zeros(shape, dtype=dbias.dtype, device=dbias.device)
+    entries / heads that shared the bias (one pass, fp32 sums, one rounding); rows / keys beyond max_seqlen get none.
+    written: as in _backend.reduce_bias_grad (a dbias that was not cleared)."""
+    covered = tuple(shape[2:]) == (max_seqlen_q, max_seqlen_k)
+    full = (torch.empty if covered else torch.zeros)(shape, dtype=dbias.dtype, device=dbias.device)
     view = full[:, :, :max_seqlen_q, :max_seqlen_k]
     sum_batch, sum_heads = shape[0] == 1 and dbias.shape[0] > 1, shape[1] == 1 and dbias.shape[1] > 1
-    if sum_batch or sum_heads:
-        _backend.reduce_bias_grad(dbias, view, sum_batch, sum_heads)
+    if sum_batch or sum_heads or written is not None:
+        _backend.reduce_bias_grad(dbias, view, sum_batch, sum_heads, written)
     else:
         view.copy_(dbias[:, :, :, :max_seqlen_k])
     return full

@@ -278,6 +278,12 @@ int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t bat
                         int32_t cols, int64_t dbias_batch_stride, int64_t dbias_head_stride, int64_t dbias_row_stride,
                         int32_t sum_batch, int32_t sum_heads, int64_t out_batch_stride, int64_t out_head_stride,
                         int64_t out_row_stride, void* stream);
+/* The same behind a dense fa_bwd call whose dbias was NOT cleared: only the elements that call wrote are read (the queries and keys each
+ * sequence has, under a causal mask up to the diagonal), the others count as zero.  args: those of the fa_bwd call (dtype, batch, nheads,
+ * max_seqlen_q / k, total_q / k, cu_seqlens, is_causal, dbias strides and stream are read); dbias: its dbias; out:
+ * [sum_batch ? 1 : batch, sum_heads ? 1 : nheads, max_seqlen_q, max_seqlen_k]. */
+int fa_bias_grad_reduce_ragged(const void* dbias, void* out, const fa_bwd_args* args, int32_t sum_batch, int32_t sum_heads,
+                               int64_t out_batch_stride, int64_t out_head_stride, int64_t out_row_stride);
 
 /* Rotary position embedding of the query and key parts of a packed tensor in one pass: what
  * RotaryEmbedding.forward / apply_rotary_pos_emb compute with elementwise torch ops (flash_attn/rotary.py:22-42,

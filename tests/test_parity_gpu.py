@@ -913,6 +913,29 @@ def test_bias_grad_reduce_sums_in_fp32_and_rounds_once(dtype):
         be.reduce_bias_grad(dbias, torch.empty(2, 6, 8, 7, device="cuda", dtype=dtype), True, False)  # wrong batch extent
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("sum_batch,sum_heads", [(True, False), (True, True), (False, True), (False, False)])
+def test_bias_grad_reduce_reads_only_what_the_backward_wrote(causal, sum_batch, sum_heads):
+    """fa_bias_grad_reduce_ragged on slices full of NaN behind a backward: the same bits as the reduction of slices that were cleared before
+    it; lengths around the 64- and 128-row tiles, a sequence without tokens, more keys than queries."""
+    from flash_attn import flash_attn_gfx950 as be
+    for lens_q, lens_k, D in (([64, 129, 0, 33], [64, 129, 0, 33], 32), ([127, 1, 65], [130, 200, 7], 64)):
+        B, H, mq, mk = len(lens_q), 3, max(lens_q), max(lens_k)
+        q, k, v, do = (x.cuda() for x in _inputs(lens_q, lens_k, H, D, torch.float16, 3))
+        bias = be.prepare_attn_bias(torch.randn(1, H, mq, mk, device="cuda").half(), q, B, H, mq, mk)
+        cu_q, cu_k, cols = _cu(lens_q), _cu(lens_k), (mk + 7) // 8 * 8
+        out, lse = be.fwd(q, k, v, cu_q, cu_k, mq, mk, 0.0, D ** -0.5, False, causal, False, None, attn_bias=bias)
+        got = []
+        for fill in (0.0, float("nan")):
+            dbias = torch.full((B, H, mq, cols), fill, device="cuda", dtype=torch.float16)
+            be.bwd(do, q, k, v, out, lse, torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), cu_q, cu_k, mq, mk, 0.0, D ** -0.5,
+                   False, causal, None, attn_bias=bias, dbias=dbias)
+            r = torch.empty(1 if sum_batch else B, 1 if sum_heads else H, mq, mk, device="cuda", dtype=torch.float16)
+            be.reduce_bias_grad(dbias, r, sum_batch, sum_heads, None if fill == 0 else (cu_q, cu_k, q.shape[0], k.shape[0], causal))
+            got.append(r)
+        assert torch.equal(got[0], got[1]) and bool(got[0].isfinite().all()) and bool((got[0] != 0).any()), (lens_q, lens_k)
+
+
 @pytest.mark.parametrize("D,dtype,causal", [(64, torch.float16, False), (128, torch.bfloat16, True), (32, torch.float16, True)])
 def test_attn_bias_with_dropout(D, dtype, causal, dropout_path):
     """bias and dropout together (the backward reading the forward's keep words, or drawing again): the mask is the defined
