@@ -68,7 +68,8 @@ constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool
   if (!dropout && ((bias == 0 && sparse) || (d <= 64 && !(sparse && bias == kBiasAlibi)))) return 3;
   return 2;
 }
-// kRoomy (dense, d = 128, no dropout, no bias): launches of at most two workgroups per compute unit, which a third wave per SIMD does not help, keep
+// kRoomy (dense, d = 128, no dropout, no bias): launches of at most two workgroups per compute unit that do not run the half-size tiles
+// (small_launch_d128), which a third wave per SIMD does not help, keep
 // all K fragments of a tile in flight also where its scores are redone, at two waves per SIMD: us of that build / the other,
 // bf16, 64 workgroups (8 heads x 1000) 24.8 / 27.0, causal 26.5 / 27.8; 192 (16 x 1500) 34.8 / 38.1; 384 (16 x 3000) 92.5 / 95.3, causal 68.6 / 72.3;
 // 576 (64 x 1100) 61.5 / 54.5; 1536 (64 x 3000) 303 / 286.

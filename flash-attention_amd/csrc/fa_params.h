@@ -296,6 +296,18 @@ inline bool small_launch(int kernel, int BH, int max_s, bool causal, bool dropou
   return wgs >= 256 && wgs < 2 * 256 && (causal || dropout);
 }
 
+// The forward's half-size tiles at head dim 128 (64-key tiles, 64 KB of LDS: two workgroups a compute unit), for launches whose time is one
+// workgroup's walk over the keys.  By the workgroups that find query rows, about nheads * (tokens / 128 + batch / 2), and the longest sequence;
+// us of full-size / half-size tiles, bf16.  Causal: 8 heads x 2300 53.9 / 35.8, 16 x 3100 (400 workgroups) 72.7 / 58.0, 4 x 12 x 360 .. 1200 (312)
+// 32.7 / 24.8, 4 x 16 x 1200 (640) 40.7 / 43.5; short sequences fill the chip with fewer: 4 x 16 x 300 (192) 11.9 / 11.0, 16 x 12 x 52 .. 130 (204)
+// 8.7 / 9.3.  No mask: 8 x 1700 39.3 / 28.1, 8 x 2300 (144) 50.1 / 45.1, 4 x 12 x 500 (192) 16.3 / 17.2, 16 x 2300 (288) 72.6 / 75.0.
+inline bool small_launch_d128(int64_t live, int max_s, bool causal) {
+  const int policy = launch_policy() & 3;
+  if (policy != 0) return policy == 2;
+  if (causal) return max_s > 128 && live <= (max_s > 256 ? 384 : 192);
+  return max_s > 192 && live <= 150;
+}
+
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel): where the dQ kernel takes its half-size tiles
 // (small_launch), at head dim 64, dense, no score bias, no rotation, no key split, dropout off or read from the keep words.
 inline bool merged_backward_launch(int head_dim, int BH, int max_sq, bool causal, bool dropout, bool keep_words, bool sparse,
