@@ -296,6 +296,17 @@ inline bool small_launch(int kernel, int BH, int max_s, bool causal, bool dropou
   return wgs >= 256 && wgs < 2 * 256 && (causal || dropout);
 }
 
+// The forward at head dim 16 to 64 under a causal mask without dropout, longest sequence beyond 256: by the workgroups that find query rows
+// instead of the launched ones, half-size below 600 and, where the lengths differ (at most 0.85 of batch x longest are tokens: the last tiles of
+// the longest sequences decide), below 1000.  us of full-size / half-size tiles, fp16 and bf16, d = 64 (d = 16 and 32 alike): 3 x 8 x 2700 ..
+// 3479 (528 workgroups, 672 launched) 55.6 / 44.1, 6 x 12 x 260 .. 1631 (564, 936) 31.4 / 24.9, 3 x 12 x 1823 (540) 33.6 / 29.5, 16 x 8 x 480 .. 1200 (896,
+// 1280) 34.9 / 26.8, 3 x 12 x 1400 .. 2829 (624) 49.7 / 40.8; equal lengths 4 x 12 x 1700 (672) 32.3 / 33.0, 4 x 12 x 2300 (864) 47.8 / 51.2; uneven beyond
+// 3 x 16 x 2100 .. 3348 (1056) 69.5 / 69.8, 16 x 16 x 1262 (2112) 63.6 / 69.9.
+inline bool small_launch_causal(int64_t live, int BH, int max_s, int64_t total_q, int batch) {
+  if ((launch_policy() & 3) != 0 || max_s <= 256) return small_launch(kSmallLaunchFwd, BH, max_s, true, false);
+  return live < 600 || (live < 1000 && total_q * 20 <= (int64_t)17 * batch * max_s);
+}
+
 // The forward's half-size tiles at head dim 128 (64-key tiles, 64 KB of LDS: two workgroups a compute unit), for launches whose time is one
 // workgroup's walk over the keys.  By the workgroups that find query rows, about nheads * (tokens / 128 + batch / 2), and the longest sequence;
 // us of full-size / half-size tiles, bf16.  Causal: 8 heads x 2300 53.9 / 35.8, 16 x 3100 (400 workgroups) 72.7 / 58.0, 4 x 12 x 360 .. 1200 (312)
