@@ -517,7 +517,8 @@ int bwd_impl(const fa_bwd_args* a, bool want_block, void* ev_main_start = nullpt
     p.n_splits = sp.n_splits;
     p.dq_part = reinterpret_cast<float*>(a->workspace);
   }
-  if (!split && fa::merged_backward_launch(a->head_dim, a->batch * a->nheads, a->max_seqlen_q, a->is_causal != 0, dropout,
+  if (!split && fa::merged_backward_launch(a->head_dim, fa::live_row_tiles(a->nheads, a->total_q, a->batch), a->batch * a->nheads,
+                                           a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, dropout,
                                            p.keep_words != nullptr, sparse, p.alibi != nullptr || p.bias != nullptr,
                                            p.rot_cos != nullptr, sp.n_splits)) {
     if (ev_main_start) FA_LAUNCH(hipEventRecord(reinterpret_cast<hipEvent_t>(ev_main_start), stream));

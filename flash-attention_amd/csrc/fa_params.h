@@ -287,6 +287,8 @@ inline bool longest_first_launch(bool causal, bool sparse, int grid, int B) {
 // launch_policy() & 3: 0 = by this rule, 1 = always the full-size tiles, 2 = the half-size tiles wherever they exist
 // (fa_set_launch_policy; the parity tests run both shapes on the same inputs).
 int launch_policy();
+// About the workgroups of 128 query rows that find any: a sequence of n has n / 128 and half a tile more on average
+inline int64_t live_row_tiles(int nheads, int total_q, int batch) { return (int64_t)nheads * (total_q + (int64_t)64 * batch) / 128; }
 constexpr int kSmallLaunchFwd = 0, kSmallLaunchDq = 1;
 inline bool small_launch(int kernel, int BH, int max_s, bool causal, bool dropout) {
   const int policy = launch_policy() & 3;
@@ -319,13 +321,35 @@ inline bool small_launch_d128(int64_t live, int max_s, bool causal) {
   return max_s > 192 && live <= 150;
 }
 
-// Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel): where the dQ kernel takes its half-size tiles
-// (small_launch), at head dim 64, dense, no score bias, no rotation, no key split, dropout off or read from the keep words.
-inline bool merged_backward_launch(int head_dim, int BH, int max_sq, bool causal, bool dropout, bool keep_words, bool sparse,
-                                   bool bias, bool rotary, int n_splits) {
-  if ((launch_policy() & 0x30) == 0x10) return false;  // (the two-kernel plan was asked for)
-  return head_dim == 64 && !sparse && !bias && !rotary && n_splits <= 1 && (!dropout || keep_words) &&
-         small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
+// Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves
+// idle, one launch less): at head dim 64, dense, no score bias, no rotation, no key split, dropout off or read from the keep words.  By the
+// workgroups of 128 query rows that find any (live_row_tiles) and the longest sequence; us in two launches / merged.  Causal: 2 x 8 x 65 %
+// of 842 (76) 41.2 / 26.3, 12 x 1812 (175) 75.3 / 50.1, 3 x 12 x 78 % of 2283 (521) 106.8 / 79.2, 4 x 8 x 2383 (611) 136.5 / 124.0, 12 x 16 x 386 (675) 39.2 /
+// 42.0; with dropout 6 x 16 x 69 % of 1258 (701) 82.9 / 71.9.  No mask: 3 x 8 x 846 (113) 39.8 / 25.7, 3 x 16 x 641 (264) 46.5 / 35.4, 8 x 12 x 77 % of 731 (469)
+// 53.8 / 48.8, 16 x 16 x 204 (536) 30.6 / 30.5, 6 x 12 x 1631 (563) 105.6 / 110.6; with dropout 12 x 12 x 528 (666) 79.7 / 73.8.  Up to 128 tokens: causal
+// 16 x 12 x 97 (194) 16.4 / 10.6, 32 x 16 x 76 (528) 22.5 / 23.1; no mask 12 x 16 x 45 (163) 12.7 / 9.3, 16 x 12 x 70 (201) 15.7 / 16.4.
+// (policy 0x10, the two-kernel plan, runs the same tiles in two launches: same bits)
+inline bool merged_backward_shape(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words,
+                                  bool sparse, bool bias, bool rotary, int n_splits) {
+  if (head_dim != 64 || sparse || bias || rotary || n_splits > 1 || (dropout && !keep_words)) return false;
+  if ((launch_policy() & 3) != 0 || max_sk > 2 * max_sq) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
+  if (max_sq <= 128) return live <= (causal ? 500 : 190);
+  return live <= (causal ? (dropout ? 700 : 620) : (dropout ? 670 : 480));
+}
+inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words,
+                                   bool sparse, bool bias, bool rotary, int n_splits) {
+  return (launch_policy() & 0x30) != 0x10 &&
+         merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, sparse, bias, rotary, n_splits);
+}
+
+// The dQ kernel's half-size tiles in a launch of its own, dropout off (with dropout: small_launch): causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 /
+// 25.1 with the dK/dV kernel, 3 x 16 x 70 % of 1785 (494) 59.5 / 53.0, 12 x 16 x 336 (551) 23.7 / 23.3; d = 64 8 x 12 x 460 (393) 34.0 / 32.6, 12 x 8 x 609
+// (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.
+inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words, bool rotary,
+                            int n_splits) {
+  if (merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, false, false, rotary, n_splits)) return true;
+  if ((launch_policy() & 3) != 0 || dropout || max_sk > 2 * max_sq) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
+  return max_sq > 128 && live <= (causal ? (head_dim == 64 ? 400 : 500) : 130);
 }
 
 // Launchers (defined in fa_fwd.hip / fa_bwd.hip / fa_aux.hip).  Return hipError_t of the launch.
