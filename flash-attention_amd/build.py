@@ -17,6 +17,9 @@ LIB_PATH = os.path.join(HERE, "flash_attn", "libflash_attn_gfx950.so")
 EXAMPLE_SRC = os.path.join(HERE, "examples", "c_abi_caller.cpp")
 EXAMPLE_BIN = os.path.join(OBJ_DIR, "c_abi_caller")
 INCLUDE_DIR = os.path.join(os.path.dirname(HERE), "include")
+# the binding's native half (host/fa_host.cpp): a CPython extension against the installed torch, host code only
+HOST_SRC = os.path.join(HERE, "host", "fa_host.cpp")
+HOST_PATH = os.path.join(HERE, "flash_attn", "fa_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -41,16 +44,33 @@ def _compile(src):
     return src, obj, r.returncode, out
 
 
+def _build_host():
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+    cmd += [f for p in include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"] for f in ("-isystem", p)]
+    cmd += [HOST_SRC, "-o", HOST_PATH, "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building %s failed:\n%s" % (HOST_SRC, r.stdout))
+
+
 def build(jobs=8, verbose=False):
     os.makedirs(OBJ_DIR, exist_ok=True)
     objs = []
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host)
         for src, obj, rc, out in ex.map(_compile, sources()):
             if rc != 0:
                 raise RuntimeError("hipcc failed on %s:\n%s" % (src, out))
             if verbose and out.strip():
                 print(out)
             objs.append(obj)
+        host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH] + objs
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:

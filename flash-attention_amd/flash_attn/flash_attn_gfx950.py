@@ -18,6 +18,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libflash_attn_gfx950.so"
 LIB_PATH = os.path.join(_HERE, LIB_NAME)
+HOST_PATH = os.path.join(_HERE, "fa_host.so")
 
 FA_FP16, FA_BF16 = 0, 1
 FA_ABI_VERSION = 5
@@ -126,12 +127,28 @@ EXPORTED_SYMBOLS = (
 BENCH_SYMBOLS = ("fa_bwd_profiled",)
 
 _lib = None
+_host = None  # the binding's native half (host/fa_host.cpp), bound to _lib
 _lib_lock = threading.Lock()
+
+
+def _load_host(lib):
+    """The extension module that makes the fwd / bwd calls natively, bound to the library's entry points."""
+    import importlib.machinery
+    import importlib.util
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError("%s is not built; run `python flash-attention_amd/build.py`." % HOST_PATH)
+    spec = importlib.util.spec_from_file_location("fa_host", HOST_PATH, loader=importlib.machinery.ExtensionFileLoader("fa_host", HOST_PATH))
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    host.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
+        "fa_fwd", "fa_fwd_block", "fa_bwd", "fa_bwd_block", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes", "fa_round_seqlens",
+        "fa_last_error")))
+    return host
 
 
 def load_library():
     """dlopen the shared library once and declare the prototypes.  Raises if it has not been built."""
-    global _lib
+    global _lib, _host
     if _lib is not None:
         return _lib
     with _lib_lock:
@@ -190,6 +207,7 @@ def load_library():
         lib.fa_set_launch_policy.restype = ctypes.c_int
         if lib.fa_abi_version() != FA_ABI_VERSION:
             raise RuntimeError("%s has ABI version %d, binding expects %d" % (LIB_NAME, lib.fa_abi_version(), FA_ABI_VERSION))
+        _host = _load_host(lib)
         _lib = lib
     return _lib
 
@@ -245,16 +263,31 @@ def _check_cu(name, t, batch):
     _check(t.dim() == 1 and t.numel() == batch + 1, "%s must have shape (batch + 1,)" % name)  # :229-230
 
 
+class DrawnPhilox:
+    """In the place of a generator: the default one's (seed, offset) as the first call it is given to draws them, for the backward
+    of that call to use again."""
+    __slots__ = ("state",)
+
+    def __init__(self):
+        self.state = None
+
+
 def _philox_state(device, p_dropout, gen):
     """(seed, offset) of the device's generator, advanced the way philox_cuda_state(counter_offset) does
     (fmha_api.cpp:288-292).  Restoring the generator state reproduces the pair, which is how the backward
     regenerates the forward's mask (flash_attn_interface.py:43,61-63)."""
     if not p_dropout > 0.0:
         return 0, 0
-    if gen is None:
+    drawn = None
+    if gen is None or isinstance(gen, DrawnPhilox):
+        drawn = gen
         idx = device.index if device.index is not None else torch.cuda.current_device()
         gen = torch.cuda.default_generators[idx]
-    seed = gen.initial_seed()
+    seed = gen.initial_seed()  # (a generator refuses this under stream capture)
+    if drawn is not None:
+        if drawn.state is None:
+            drawn.state = _philox_state(device, p_dropout, None)
+        return drawn.state
     offset = gen.get_offset()
     gen.set_offset(offset + int(load_library().fa_philox_offset_increment()))
     return seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF
@@ -421,6 +454,13 @@ def _fwd_impl(q, k, v, cu_seqlens_q, cu_seqlens_k, blockmask, max_seqlen_q, max_
               zero_tensors, is_causal, return_softmax, gen, alibi_slopes=None, keep_words=None, attn_bias=None,
               row_order=None, rotary=None, q_rot=None):
     lib = load_library()
+    if not return_softmax:
+        cos, sin = rotary if rotary is not None else (None, None)
+        res = _host.fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale, zero_tensors, is_causal,
+                        (lambda: _philox_state(q.device, p_dropout, gen)) if p_dropout > 0.0 else None, alibi_slopes, keep_words, attn_bias,
+                        cos, sin, q_rot, blockmask, row_order)
+        if res is not None:  # (else: of a kind, or with a fault, that is dealt with here)
+            return list(res)
     code = _dtype_code(q)
     _check(q.dim() == 3, "q must be (total_q, nheads, head_size)")
     total_q, nheads, head_dim = q.shape
@@ -505,6 +545,14 @@ def _bwd_impl(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seql
               max_seqlen_k, p_dropout, softmax_scale, zero_tensors, is_causal, gen, main_kernel_events=None,
               alibi_slopes=None, keep_words=None, attn_bias=None, dbias=None, row_order=None, rotary=None):
     lib = load_library()
+    if main_kernel_events is None:
+        cos, sin = rotary if rotary is not None else (None, None)
+        softmax_d = _host.bwd(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, p_dropout,
+                              softmax_scale, zero_tensors, is_causal,
+                              (lambda: _philox_state(q.device, p_dropout, gen)) if p_dropout > 0.0 else None, alibi_slopes, keep_words,
+                              attn_bias, dbias, cos, sin, blockmask, row_order)
+        if softmax_d is not None:
+            return [dq, dk, dv, softmax_d]
     code = _dtype_code(q)
     _check(q.dim() == 3, "q must be (total_q, nheads, head_size)")
     total_q, nheads, head_dim = q.shape

@@ -17,17 +17,17 @@ def _get_block_size(device, head_dim, is_dropout):
 
 def _flash_attn_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                         softmax_scale, causal, return_softmax, alibi_slopes=None, keep_words=None, attn_bias=None,
-                        rotary=None, q_rot=None):
+                        rotary=None, q_rot=None, gen=None):
     res = _backend.fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale,
-                       False, causal, return_softmax, None, alibi_slopes, keep_words, attn_bias, rotary=rotary, q_rot=q_rot)
+                       False, causal, return_softmax, gen, alibi_slopes, keep_words, attn_bias, rotary=rotary, q_rot=q_rot)
     return res[0], res[1], (res[2] if return_softmax else None)
 
 
 def _flash_attn_backward(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k,
                          max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal, alibi_slopes=None,
-                         keep_words=None, attn_bias=None, dbias=None, rotary=None):
+                         keep_words=None, attn_bias=None, dbias=None, rotary=None, gen=None):
     _, _, _, softmax_d = _backend.bwd(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k,
-                                      max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, False, causal, None,
+                                      max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, False, causal, gen,
                                       alibi_slopes=alibi_slopes, keep_words=keep_words, attn_bias=attn_bias, dbias=dbias,
                                       rotary=rotary)
     return dq, dk, dv, softmax_d
@@ -72,8 +72,8 @@ def _forward(ctx, packing, tensors, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
     if rotary is not None:
         rot = _rotated_keys(tensors[0], cu_seqlens_q, int(max_seqlen_q), *rotary)
         q_rot, k = rot[:, 0], rot[:, 1]
-    # the dropout mask is a function of the generator state at this point; the backward rewinds to it
-    rng_state = torch.cuda.get_rng_state(q.device) if dropout_p > 0 else None
+    # the dropout mask is a function of the (seed, offset) the forward draws; the backward uses them again
+    philox = _backend.DrawnPhilox() if dropout_p > 0 else None
     if softmax_scale is None:
         softmax_scale = q.shape[-1] ** (-0.5)
     # with a backward to come, the forward leaves its dropout decisions (one bit per score) for it to read instead of
@@ -89,8 +89,9 @@ def _forward(ctx, packing, tensors, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
                                             int(max_seqlen_k))
     out, softmax_lse, S_dmask = _flash_attn_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                                                     dropout_p, softmax_scale, causal, return_softmax, alibi_slopes,
-                                                    keep_words, bias_t, rotary, q_rot)
-    ctx.save_for_backward(*tensors, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, rng_state, bias_t, rot)
+                                                    keep_words, bias_t, rotary, q_rot, philox)
+    ctx.save_for_backward(*tensors, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot)
+    ctx.philox = philox
     ctx.rotary = rotary  # constant tables, not differentiated
     ctx.bias_shape = tuple(attn_bias.shape) if attn_bias is not None else None
     ctx.bias_needs_grad = attn_bias is not None and attn_bias.requires_grad
@@ -108,26 +109,20 @@ def _forward(ctx, packing, tensors, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
 def _backward(ctx, dout):
     saved = ctx.saved_tensors
     tensors = saved[:ctx.n_in]
-    out, softmax_lse, cu_seqlens_q, cu_seqlens_k, rng_state, bias_t, rot = saved[ctx.n_in:]
+    out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot = saved[ctx.n_in:]
     q, k, v = _split(ctx.packing, tensors)
     if rot is not None:  # the kernels take the rotated q and k and turn dq and dk back themselves
         q, k = rot[:, 0], rot[:, 1]
     grads = tuple(torch.empty_like(t) for t in tensors)
     dq, dk, dv = _split(ctx.packing, grads)
-    dev = q.device
     dbias = written = None
     if ctx.bias_needs_grad:
         if cu_seqlens_q.numel() - 1 <= 65535 and q.shape[1] <= 65535:  # (the grid of the kernel that knows what was written)
             written = (cu_seqlens_q, cu_seqlens_k, q.shape[0], k.shape[0], ctx.causal)
         dbias = new_bias_grad(q, cu_seqlens_q.numel() - 1, ctx.max_seqlen_q, ctx.max_seqlen_k, cleared=written is None)
-    if rng_state is not None:
-        cur_rng_state = torch.cuda.get_rng_state(dev)
-        torch.cuda.set_rng_state(rng_state, dev)
     _flash_attn_backward(dout.contiguous(), q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k,
                          ctx.max_seqlen_q, ctx.max_seqlen_k, ctx.dropout_p, ctx.softmax_scale, ctx.causal,
-                         ctx.alibi_slopes, ctx.keep_words, bias_t, dbias, ctx.rotary)
-    if rng_state is not None:
-        torch.cuda.set_rng_state(cur_rng_state, dev)
+                         ctx.alibi_slopes, ctx.keep_words, bias_t, dbias, ctx.rotary, ctx.philox)
     ctx.dbias = None
     if dbias is not None:
         ctx.dbias = bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_seqlen_q, ctx.max_seqlen_k, written)

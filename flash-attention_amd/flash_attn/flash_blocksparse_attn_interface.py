@@ -63,26 +63,26 @@ def _row_order(blockmask, causal):
 
 
 def _flash_blocksparse_attn_forward(qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal,
-                                    return_softmax, alibi_slopes=None, attn_bias=None):
+                                    return_softmax, alibi_slopes=None, attn_bias=None, gen=None):
     res = _backend.fwd_block(qkv[:, 0], qkv[:, 1], qkv[:, 2], cu_seqlens, cu_seqlens, blockmask, max_s, max_s,
-                             dropout_p, softmax_scale, causal, return_softmax, None, row_order=_row_order(blockmask, causal),
+                             dropout_p, softmax_scale, causal, return_softmax, gen, row_order=_row_order(blockmask, causal),
                              alibi_slopes=alibi_slopes, attn_bias=attn_bias)
     return res[0], res[1], (res[2] if return_softmax else None)
 
 
 def _flash_blocksparse_attn_backward(dout, qkv, out, S_dmask, softmax_lse, cu_seqlens, blockmask, dropout_p, max_s,
-                                     softmax_scale, causal, alibi_slopes=None, attn_bias=None, dbias=None):
+                                     softmax_scale, causal, alibi_slopes=None, attn_bias=None, dbias=None, gen=None):
     dqkv = torch.empty_like(qkv)
     _backend.bwd_block(dout.contiguous(), qkv[:, 0], qkv[:, 1], qkv[:, 2], out, softmax_lse, dqkv[:, 0], dqkv[:, 1],
                        dqkv[:, 2], cu_seqlens, cu_seqlens, blockmask, max_s, max_s, dropout_p, softmax_scale, causal,
-                       None, row_order=_row_order(blockmask, causal), alibi_slopes=alibi_slopes, attn_bias=attn_bias,
+                       gen, row_order=_row_order(blockmask, causal), alibi_slopes=alibi_slopes, attn_bias=attn_bias,
                        dbias=dbias)
     return dqkv
 
 
 def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes,
                 attn_bias):
-    rng_state = torch.cuda.get_rng_state(qkv.device) if dropout_p > 0 else None
+    philox = _backend.DrawnPhilox() if dropout_p > 0 else None  # (seed, offset) of the forward, used again by the backward
     if softmax_scale is None:
         softmax_scale = qkv.shape[-1] ** (-0.5)
     # the bias in the form the kernels read (the caller's tensor itself if its layout allows, else a padded copy)
@@ -91,8 +91,10 @@ def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale
         bias_t = _backend.prepare_attn_bias(attn_bias.detach(), qkv[:, 0], cu_seqlens.numel() - 1, qkv.shape[2], int(max_s),
                                             int(max_s))
     context, softmax_lse, S_dmask = _flash_blocksparse_attn_forward(
-        qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes, bias_t)
-    ctx.save_for_backward(qkv, context, softmax_lse, cu_seqlens, blockmask, rng_state, bias_t)
+        qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes, bias_t,
+        philox)
+    ctx.save_for_backward(qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t)
+    ctx.philox = philox
     ctx.dropout_p = dropout_p
     ctx.max_s = max_s
     ctx.softmax_scale = softmax_scale
@@ -105,19 +107,13 @@ def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale
 
 def _bwd_common(ctx, dout):
     """(dqkv, gradient of attn_bias or None)"""
-    qkv, context, softmax_lse, cu_seqlens, blockmask, rng_state, bias_t = ctx.saved_tensors
-    dev = qkv.device
-    if rng_state is not None:
-        cur_rng_state = torch.cuda.get_rng_state(dev)
-        torch.cuda.set_rng_state(rng_state, dev)
+    qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t = ctx.saved_tensors
     dbias = None
     if ctx.bias_needs_grad:
         dbias = new_bias_grad(qkv[:, 0], cu_seqlens.numel() - 1, ctx.max_s, ctx.max_s)
     dqkv = _flash_blocksparse_attn_backward(dout, qkv, context, None, softmax_lse, cu_seqlens, blockmask,
                                             ctx.dropout_p, ctx.max_s, ctx.softmax_scale, ctx.causal, ctx.alibi_slopes,
-                                            bias_t, dbias)
-    if rng_state is not None:
-        torch.cuda.set_rng_state(cur_rng_state, dev)
+                                            bias_t, dbias, ctx.philox)
     return dqkv, (bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_s, ctx.max_s) if dbias is not None else None)
 
 

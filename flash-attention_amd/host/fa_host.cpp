@@ -1,0 +1,315 @@
+// The calls of flash_attn_gfx950.fwd / bwd (and their block-sparse forms) made natively: arguments checked, outputs and scratch
+// allocated, the argument struct of the C ABI filled and the entry point called, without Python in between.
+//
+// Every check the Python binding makes is made here too, but nothing is reported: a call that fails one, or that is of a kind
+// handled there (probabilities returned, profiling events, a device that is not current, tensors without memory of their own such as those of
+// functorch and of fake-tensor tracing), returns None and the binding runs it - and raises what it has to.  What the library itself refuses
+// is raised here with the binding's text.
+//
+// Bound by the interpreter.  us with the binding's own calls / with these: one forward of 12 heads x 61 tokens (kernel 6) 21.4 / 14.2; training
+// steps of 8 x 12 x 256 .. 512 with dropout (kernels 56; an empty autograd function with a backward takes 48) 159 / 101, 8 x 12 x 1024 rotary
+// (110) 175 / 118, 8 x 8 x 421 .. 701 with a bias (100) 203 / 120.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/flash_attn_gfx950.h"
+
+namespace {
+
+struct Library {
+  int (*fwd)(const fa_fwd_args*);
+  int (*fwd_block)(const fa_fwd_args*);
+  int (*bwd)(const fa_bwd_args*);
+  int (*bwd_block)(const fa_bwd_args*);
+  size_t (*fwd_workspace_bytes)(const fa_fwd_args*);
+  size_t (*bwd_workspace_bytes)(const fa_bwd_args*);
+  void (*round_seqlens)(int32_t, int32_t, int32_t, int32_t, int32_t*, int32_t*);
+  const char* (*last_error)();
+} g_lib;
+bool g_bound = false;
+
+// bind(addresses of the eight entry points above, in their order)
+PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 8) return PyErr_Format(PyExc_TypeError, "bind takes 8 addresses");
+  void* f[8];
+  for (int i = 0; i < 8; i++) {
+    f[i] = PyLong_AsVoidPtr(a[i]);
+    if (!f[i]) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
+      return nullptr;
+    }
+  }
+  static_assert(sizeof(g_lib) == sizeof(f), "eight pointers");
+  memcpy(&g_lib, f, sizeof(f));
+  g_bound = true;
+  Py_RETURN_NONE;
+}
+
+// A tensor argument; null for None.  ok is cleared for anything but a plain tensor (or parameter) with memory of its own.
+const at::Tensor* tensor(PyObject* o, bool& ok) {
+  if (o == Py_None) return nullptr;
+  if (!THPVariable_Check(o)) {
+    ok = false;
+    return nullptr;
+  }
+  const at::Tensor& t = THPVariable_Unpack(o);
+  constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::FuncTorchBatched});
+  if (!t.defined() || !t.has_storage() || t.key_set().has_any(wrapped) || t.layout() != at::kStrided) ok = false;
+  return &t;
+}
+bool as_int(PyObject* o, int64_t* v) {  // a Python int (what int() of anything else gives is left to the binding)
+  if (!PyLong_Check(o)) return false;
+  int overflow = 0;
+  *v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow == 0 && !(*v == -1 && PyErr_Occurred()) && *v >= INT32_MIN && *v <= INT32_MAX;
+}
+bool as_double(PyObject* o, double* v) {
+  if (PyFloat_Check(o)) *v = PyFloat_AS_DOUBLE(o);
+  else if (PyLong_Check(o)) *v = PyLong_AsDouble(o);
+  else return false;
+  return !PyErr_Occurred();
+}
+inline void* ptr(const at::Tensor& t) { return t.data_ptr(); }
+
+struct Shape {
+  at::ScalarType dtype;
+  c10::Device device{c10::kCPU};
+  int64_t heads, dim, batch, total_q, total_k;
+};
+bool rows_ok(const at::Tensor* t, const Shape& s, int64_t total) {
+  return t && t->is_cuda() && t->device() == s.device && t->scalar_type() == s.dtype && t->dim() == 3 && t->size(0) == total &&
+         t->size(1) == s.heads && t->size(2) == s.dim && t->stride(2) == 1;
+}
+bool cu_ok(const at::Tensor* t, const Shape& s) {
+  return t && t->is_cuda() && t->device() == s.device && t->scalar_type() == at::kInt && t->dim() == 1 && t->size(0) == s.batch + 1 && t->is_contiguous();
+}
+bool slopes_ok(const at::Tensor* t, const Shape& s) {
+  return !t || (t->device() == s.device && t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == s.heads && t->is_contiguous());
+}
+bool words_ok(const at::Tensor* t, const Shape& s) {
+  return !t || (t->device() == s.device && t->scalar_type() == at::kByte && t->is_contiguous());
+}
+bool bias_ok(const at::Tensor* t, const Shape& s, int64_t mq, int64_t mk) {  // what prepare_attn_bias() hands through
+  if (!t) return true;
+  return t->dim() == 4 && (t->size(0) == 1 || t->size(0) == s.batch) && (t->size(1) == 1 || t->size(1) == s.heads) && t->size(2) >= mq &&
+         t->size(3) >= mk && t->device() == s.device && t->scalar_type() == s.dtype && t->stride(3) == 1 && t->stride(2) % 8 == 0 &&
+         t->stride(2) >= mk && t->stride(0) % 8 == 0 && t->stride(1) % 8 == 0 && reinterpret_cast<uintptr_t>(ptr(*t)) % 16 == 0;
+}
+bool tables_ok(const at::Tensor* c, const at::Tensor* n, const Shape& s, int64_t rows) {
+  if (!c && !n) return true;
+  auto one = [&](const at::Tensor* t) {
+    return t && t->dim() == 2 && t->size(1) == s.dim / 2 && t->scalar_type() == s.dtype && t->is_contiguous() && t->device() == s.device && t->size(0) >= rows;
+  };
+  return one(c) && one(n) && c->size(0) == n->size(0);
+}
+bool blocks_ok(const at::Tensor* m, const at::Tensor* order, const Shape& s, int32_t sq_r, int32_t sk_r) {
+  if (!m) return true;
+  if (!(m->is_cuda() && m->device() == s.device && m->scalar_type() == at::kInt && m->is_contiguous() && m->dim() == 2 && m->size(0) == sk_r / 256 && m->size(1) == sq_r / 16))
+    return false;
+  return !order || (order->device() == s.device && order->scalar_type() == at::kInt && order->is_contiguous() && order->numel() == sq_r / 16);
+}
+
+bool common(const at::Tensor* q, const at::Tensor* k, const at::Tensor* cu_q, Shape* s) {
+  if (!g_bound || !q || !k || !cu_q || !q->is_cuda() || q->dim() != 3 || k->dim() != 3 || cu_q->dim() != 1) return false;
+  s->dtype = q->scalar_type();
+  if (s->dtype != at::kHalf && s->dtype != at::kBFloat16) return false;
+  s->device = q->device();
+  if (s->device.index() != c10::hip::current_device()) return false;
+  s->total_q = q->size(0);
+  s->total_k = k->size(0);
+  s->heads = q->size(1);
+  s->dim = q->size(2);
+  s->batch = cu_q->size(0) - 1;
+  return s->batch > 0 && (s->dim == 16 || s->dim == 32 || s->dim == 64 || s->dim == 128);
+}
+// (seed, offset) from a callable that draws them, called once nothing can be handed back to the binding any more; 0, 0 for None
+bool draw(PyObject* f, uint64_t* seed, uint64_t* offset) {
+  *seed = *offset = 0;
+  if (f == Py_None) return true;
+  PyObject* r = PyObject_CallNoArgs(f);
+  if (!r) return false;
+  if (PyTuple_Check(r) && PyTuple_GET_SIZE(r) == 2) {
+    *seed = PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(r, 0));
+    *offset = PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(r, 1));
+  } else {
+    PyErr_SetString(PyExc_TypeError, "(seed, offset) expected");
+  }
+  Py_DECREF(r);
+  return !PyErr_Occurred();
+}
+PyObject* refused(int rc) { return PyErr_Format(PyExc_RuntimeError, "flash_attn_gfx950 error %d: %s", rc, g_lib.last_error()); }
+
+// fwd(q, k, v, cu_q, cu_k, max_q, max_k, p, scale, zero, causal, draw, alibi, keep_words, bias, cos, sin, q_rot, blockmask, row_order)
+// -> (out, softmax_lse) or None
+PyObject* fwd(PyObject* const* a, Py_ssize_t n) {
+  if (n != 20) return PyErr_Format(PyExc_TypeError, "fwd takes 20 arguments");
+  bool ok = true;
+  const at::Tensor *q = tensor(a[0], ok), *k = tensor(a[1], ok), *v = tensor(a[2], ok), *cu_q = tensor(a[3], ok), *cu_k = tensor(a[4], ok);
+  const at::Tensor *alibi = tensor(a[12], ok), *words = tensor(a[13], ok), *bias = tensor(a[14], ok), *cos = tensor(a[15], ok), *sin = tensor(a[16], ok);
+  const at::Tensor *q_rot = tensor(a[17], ok), *mask = tensor(a[18], ok), *order = tensor(a[19], ok);
+  int64_t mq, mk;
+  double p, scale;
+  Shape s;
+  if (!ok || !as_int(a[5], &mq) || !as_int(a[6], &mk) || !as_double(a[7], &p) || !as_double(a[8], &scale) || mq <= 0 || mk <= 0 ||
+      !common(q, k, cu_q, &s) || s.total_q > INT32_MAX || s.total_k > INT32_MAX || s.batch > INT32_MAX || !rows_ok(q, s, s.total_q) ||
+      !rows_ok(k, s, s.total_k) || !rows_ok(v, s, s.total_k) || !cu_ok(cu_q, s) || !cu_ok(cu_k, s) || !slopes_ok(alibi, s) ||
+      !words_ok(words, s) || !bias_ok(bias, s, mq, mk) || !tables_ok(cos, sin, s, mq) || (q_rot && (!cos || !rows_ok(q_rot, s, s.total_q))))
+    Py_RETURN_NONE;
+  int32_t sq_r, sk_r;
+  g_lib.round_seqlens((int32_t)s.dim, (int32_t)mq, (int32_t)mk, mask != nullptr, &sq_r, &sk_r);
+  if (!blocks_ok(mask, order, s, sq_r, sk_r)) Py_RETURN_NONE;
+
+  at::Tensor o = at::empty({s.total_q, s.heads, s.dim}, q->options().memory_format(at::MemoryFormat::Contiguous).requires_grad(false));
+  at::Tensor lse = at::empty({s.batch, s.heads, (int64_t)sq_r}, o.options().dtype(at::kFloat));
+  fa_fwd_args f;
+  memset(&f, 0, sizeof(f));
+  f.struct_bytes = sizeof(f);
+  f.dtype = s.dtype == at::kHalf ? FA_FP16 : FA_BF16;
+  f.q = ptr(*q); f.k = ptr(*k); f.v = ptr(*v); f.o = ptr(o); f.softmax_lse = (float*)ptr(lse);
+  f.cu_seqlens_q = (const int32_t*)ptr(*cu_q); f.cu_seqlens_k = (const int32_t*)ptr(*cu_k);
+  f.q_row_stride = q->stride(0); f.q_head_stride = q->stride(1);
+  f.k_row_stride = k->stride(0); f.k_head_stride = k->stride(1);
+  f.v_row_stride = v->stride(0); f.v_head_stride = v->stride(1);
+  f.o_row_stride = s.heads * s.dim; f.o_head_stride = s.dim;
+  f.batch = (int32_t)s.batch; f.nheads = (int32_t)s.heads; f.head_dim = (int32_t)s.dim;
+  f.total_q = (int32_t)s.total_q; f.total_k = (int32_t)s.total_k;
+  f.max_seqlen_q = (int32_t)mq; f.max_seqlen_k = (int32_t)mk;
+  f.p_dropout = (float)p; f.softmax_scale = (float)scale;
+  f.zero_tensors = PyObject_IsTrue(a[9]); f.is_causal = PyObject_IsTrue(a[10]);
+  if (alibi) f.alibi_slopes = (const float*)ptr(*alibi);
+  if (words && !mask) { f.keep_words = ptr(*words); f.keep_words_bytes = (size_t)words->numel(); }
+  if (bias) {
+    f.attn_bias = ptr(*bias);
+    f.bias_batch_stride = bias->size(0) == 1 ? 0 : bias->stride(0);
+    f.bias_head_stride = bias->size(1) == 1 ? 0 : bias->stride(1);
+    f.bias_row_stride = bias->stride(2);
+  }
+  if (cos) { f.rotary_cos = ptr(*cos); f.rotary_sin = ptr(*sin); f.rotary_table_rows = (int32_t)cos->size(0); }
+  if (q_rot) { f.q_rot = ptr(*q_rot); f.q_rot_row_stride = q_rot->stride(0); f.q_rot_head_stride = q_rot->stride(1); }
+  if (mask) { f.blockmask = (const int32_t*)ptr(*mask); if (order) f.row_order = (const int32_t*)ptr(*order); }
+  at::Tensor ws;
+  f.workspace_bytes = g_lib.fwd_workspace_bytes(&f);
+  if (f.workspace_bytes) {
+    ws = at::empty({(int64_t)f.workspace_bytes}, o.options().dtype(at::kByte));
+    f.workspace = ptr(ws);
+  }
+  f.stream = c10::hip::getCurrentHIPStream(s.device.index()).stream();
+  if (!draw(a[11], &f.philox_seed, &f.philox_offset)) return nullptr;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = (mask ? g_lib.fwd_block : g_lib.fwd)(&f);
+  Py_END_ALLOW_THREADS
+  if (rc != 0) return refused(rc);
+  PyObject *po = THPVariable_Wrap(std::move(o)), *pl = THPVariable_Wrap(std::move(lse));
+  PyObject* r = po && pl ? PyTuple_Pack(2, po, pl) : nullptr;
+  Py_XDECREF(po);
+  Py_XDECREF(pl);
+  return r;
+}
+
+// bwd(dout, q, k, v, out, lse, dq, dk, dv, cu_q, cu_k, max_q, max_k, p, scale, zero, causal, draw, alibi, keep_words, bias, dbias, cos, sin,
+// blockmask, row_order) -> softmax_d or None
+PyObject* bwd(PyObject* const* a, Py_ssize_t n) {
+  if (n != 26) return PyErr_Format(PyExc_TypeError, "bwd takes 26 arguments");
+  bool ok = true;
+  const at::Tensor* t[11];
+  for (int i = 0; i < 11; i++) t[i] = tensor(a[i], ok);
+  const at::Tensor *dout = t[0], *q = t[1], *k = t[2], *v = t[3], *out = t[4], *lse = t[5], *dq = t[6], *dk = t[7], *dv = t[8], *cu_q = t[9], *cu_k = t[10];
+  const at::Tensor *alibi = tensor(a[18], ok), *words = tensor(a[19], ok), *bias = tensor(a[20], ok), *dbias = tensor(a[21], ok);
+  const at::Tensor *cos = tensor(a[22], ok), *sin = tensor(a[23], ok), *mask = tensor(a[24], ok), *order = tensor(a[25], ok);
+  int64_t mq, mk;
+  double p, scale;
+  Shape s;
+  if (!ok || !as_int(a[11], &mq) || !as_int(a[12], &mk) || !as_double(a[13], &p) || !as_double(a[14], &scale) || mq <= 0 || mk <= 0 ||
+      !common(q, k, cu_q, &s) || s.total_q > INT32_MAX || s.total_k > INT32_MAX || s.batch > INT32_MAX || !rows_ok(q, s, s.total_q) ||
+      !rows_ok(k, s, s.total_k) || !rows_ok(v, s, s.total_k) || !rows_ok(out, s, s.total_q) || !rows_ok(dout, s, s.total_q) ||
+      !rows_ok(dq, s, s.total_q) || !rows_ok(dk, s, s.total_k) || !rows_ok(dv, s, s.total_k) || !out->is_contiguous() || !dout->is_contiguous() ||
+      !cu_ok(cu_q, s) || !cu_ok(cu_k, s) || !lse || lse->device() != s.device || lse->scalar_type() != at::kFloat || lse->dim() != 3 ||
+      lse->size(0) != s.batch || lse->size(1) != s.heads || lse->size(2) > INT32_MAX || !lse->is_contiguous() || !slopes_ok(alibi, s) ||
+      !words_ok(words, s) || !bias_ok(bias, s, mq, mk) || !tables_ok(cos, sin, s, mq > mk ? mq : mk))
+    Py_RETURN_NONE;
+  if (dbias && !(bias && dbias->dim() == 4 && dbias->size(0) == s.batch && dbias->size(1) == s.heads && dbias->size(2) >= mq && dbias->size(3) >= mk &&
+                 dbias->stride(3) == 1 && dbias->scalar_type() == s.dtype && dbias->device() == s.device))
+    Py_RETURN_NONE;
+  int32_t sq_r, sk_r;
+  g_lib.round_seqlens((int32_t)s.dim, (int32_t)mq, (int32_t)mk, mask != nullptr, &sq_r, &sk_r);
+  if (!blocks_ok(mask, order, s, sq_r, sk_r)) Py_RETURN_NONE;
+
+  at::Tensor d = at::empty({s.batch, s.heads, (int64_t)sq_r}, lse->options().requires_grad(false));
+  fa_bwd_args f;
+  memset(&f, 0, sizeof(f));
+  f.struct_bytes = sizeof(f);
+  f.dtype = s.dtype == at::kHalf ? FA_FP16 : FA_BF16;
+  f.dout = ptr(*dout); f.q = ptr(*q); f.k = ptr(*k); f.v = ptr(*v); f.out = ptr(*out); f.softmax_lse = (const float*)ptr(*lse);
+  f.dq = ptr(*dq); f.dk = ptr(*dk); f.dv = ptr(*dv); f.softmax_d = (float*)ptr(d);
+  f.cu_seqlens_q = (const int32_t*)ptr(*cu_q); f.cu_seqlens_k = (const int32_t*)ptr(*cu_k);
+  f.do_row_stride = dout->stride(0); f.do_head_stride = dout->stride(1);
+  f.q_row_stride = q->stride(0); f.q_head_stride = q->stride(1);
+  f.k_row_stride = k->stride(0); f.k_head_stride = k->stride(1);
+  f.v_row_stride = v->stride(0); f.v_head_stride = v->stride(1);
+  f.o_row_stride = out->stride(0); f.o_head_stride = out->stride(1);
+  f.dq_row_stride = dq->stride(0); f.dq_head_stride = dq->stride(1);
+  f.dk_row_stride = dk->stride(0); f.dk_head_stride = dk->stride(1);
+  f.dv_row_stride = dv->stride(0); f.dv_head_stride = dv->stride(1);
+  f.lse_seq_stride = (int32_t)lse->size(2);
+  f.batch = (int32_t)s.batch; f.nheads = (int32_t)s.heads; f.head_dim = (int32_t)s.dim;
+  f.total_q = (int32_t)s.total_q; f.total_k = (int32_t)s.total_k;
+  f.max_seqlen_q = (int32_t)mq; f.max_seqlen_k = (int32_t)mk;
+  f.p_dropout = (float)p; f.softmax_scale = (float)scale;
+  f.zero_tensors = PyObject_IsTrue(a[15]); f.is_causal = PyObject_IsTrue(a[16]);
+  if (alibi) f.alibi_slopes = (const float*)ptr(*alibi);
+  if (words && !mask) { f.keep_words = ptr(*words); f.keep_words_bytes = (size_t)words->numel(); }
+  if (bias) {
+    f.attn_bias = ptr(*bias);
+    f.bias_batch_stride = bias->size(0) == 1 ? 0 : bias->stride(0);
+    f.bias_head_stride = bias->size(1) == 1 ? 0 : bias->stride(1);
+    f.bias_row_stride = bias->stride(2);
+  }
+  if (dbias) { f.dbias = ptr(*dbias); f.dbias_batch_stride = dbias->stride(0); f.dbias_head_stride = dbias->stride(1); f.dbias_row_stride = dbias->stride(2); }
+  if (cos) { f.rotary_cos = ptr(*cos); f.rotary_sin = ptr(*sin); f.rotary_table_rows = (int32_t)cos->size(0); }
+  if (mask) { f.blockmask = (const int32_t*)ptr(*mask); if (order) f.row_order = (const int32_t*)ptr(*order); }
+  at::Tensor ws;
+  f.workspace_bytes = g_lib.bwd_workspace_bytes(&f);
+  if (f.workspace_bytes) {
+    ws = at::empty({(int64_t)f.workspace_bytes}, q->options().memory_format(at::MemoryFormat::Contiguous).dtype(at::kByte).requires_grad(false));
+    f.workspace = ptr(ws);
+  }
+  f.stream = c10::hip::getCurrentHIPStream(s.device.index()).stream();
+  if (!draw(a[17], &f.philox_seed, &f.philox_offset)) return nullptr;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = (mask ? g_lib.bwd_block : g_lib.bwd)(&f);
+  Py_END_ALLOW_THREADS
+  if (rc != 0) return refused(rc);
+  return THPVariable_Wrap(std::move(d));
+}
+
+// C++ exceptions (an allocation that fails, memory that may not be touched under tracing) do not leave the module: the call is handed back and
+// the binding meets the same condition
+template <PyObject* (*F)(PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  try {
+    return F(a, n);
+  } catch (const std::exception&) {
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+  }
+}
+
+PyMethodDef methods[] = {
+    {"bind", (PyCFunction)(void (*)(void))py_bind, METH_FASTCALL, nullptr},
+    {"fwd", (PyCFunction)(void (*)(void))guarded<fwd>, METH_FASTCALL, nullptr},
+    {"bwd", (PyCFunction)(void (*)(void))guarded<bwd>, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_fa_host() { return PyModule_Create(&module); }

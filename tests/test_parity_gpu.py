@@ -1351,6 +1351,103 @@ def test_blocksparse_causal_sweep():
 # ------------------------------------------------------------------------------------------------
 # modules
 # ------------------------------------------------------------------------------------------------
+@pytest.fixture
+def binding_only():
+    """a context in which the binding makes its calls itself instead of through its native half"""
+    import contextlib
+    import types
+    from flash_attn import flash_attn_gfx950 as be
+
+    @contextlib.contextmanager
+    def cm():
+        host, be._host = be._host, types.SimpleNamespace(fwd=lambda *a: None, bwd=lambda *a: None)
+        try:
+            yield
+        finally:
+            be._host = host
+    be.load_library()
+    return cm
+
+
+@pytest.mark.parametrize("kind", ["plain", "causal", "dropout", "words", "alibi", "bias", "rotary", "block", "cross", "decode", "zero"])
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 64), (torch.bfloat16, 128), (torch.float16, 16)])
+def test_native_calls_equal_the_bindings(kind, dtype, D, binding_only):
+    """The native half of the binding makes the same call as the binding: every output equal bit for bit and the generator left where it was left,
+    for packed, separate and strided views, scratch (decode and cross splits, block layouts) and every optional argument."""
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
+    H, lens_q, lens_k = 3, [70, 129, 5], [70, 129, 5]
+    if kind == "cross":
+        lens_k = [900, 130, 700]
+    if kind == "decode":
+        lens_q, lens_k = [1, 1, 1], [3000, 400, 1200]
+    mq, mk, p = max(lens_q), max(lens_k), 0.2 if kind in ("dropout", "words") else 0.0
+    q, k, v, do = (x.cuda() for x in _inputs(lens_q, lens_k, H, D, dtype, 5))
+    if kind in ("plain", "words"):  # views of a packed tensor
+        q, k, v = torch.stack([q, k, v], 1).unbind(1)
+    if kind == "alibi":  # rows further apart than a row is wide
+        k = torch.stack([k, torch.zeros_like(k)], 1)[:, 0]
+    cu_q, cu_k, causal = _cu(lens_q), _cu(lens_k), kind in ("causal", "rotary", "alibi")
+    alibi = torch.tensor([0.5, 0.25, 0.1], device="cuda") if kind == "alibi" else None
+    bias = be.prepare_attn_bias(torch.randn(1, H, mq, mk, device="cuda").to(dtype), q, 3, H, mq, mk) if kind == "bias" else None
+    rot = tuple(torch.randn(mk, D // 2, device="cuda").to(dtype) for _ in range(2)) if kind == "rotary" else None
+    mask = None
+    if kind == "block":
+        sq_r, sk_r = be.round_seqlens(D, mq, mk, True)
+        mask = convert_blockmask(torch.ones(sq_r // 16, sk_r // 256, device="cuda").bool(), causal=False)
+
+    def step():
+        torch.cuda.manual_seed(11)
+        kw = be.new_keep_words(q, cu_q, mq, mk, p) if kind == "words" else None
+        q_rot = torch.zeros_like(q) if rot else None
+        dq, dk, dv = (torch.zeros_like(x, memory_format=torch.contiguous_format) for x in (q, k, v))
+        dbias = torch.zeros(3, H, mq, (mk + 7) // 8 * 8, dtype=dtype, device="cuda") if bias is not None else None
+        args = (0.1, kind == "zero", causal)
+        if mask is not None:
+            o, lse = be.fwd_block(q, k, v, cu_q, cu_k, mask, mq, mk, p, 0.1, causal, False)
+            d = be.bwd_block(do, q, k, v, o, lse, dq, dk, dv, cu_q, cu_k, mask, mq, mk, p, 0.1, causal)[3]
+        else:
+            o, lse = be.fwd(q, k, v, cu_q, cu_k, mq, mk, p, *args, False, None, alibi, kw, bias, rotary=rot, q_rot=q_rot)
+            state = torch.cuda.get_rng_state()
+            torch.cuda.manual_seed(11)
+            qb = q_rot if rot else q
+            d = be.bwd(do, qb, k, v, o, lse, dq, dk, dv, cu_q, cu_k, mq, mk, p, *args, None, alibi_slopes=alibi, keep_words=kw, attn_bias=bias,
+                       dbias=dbias, rotary=rot)[3]
+            assert torch.equal(state, torch.cuda.get_rng_state())
+        rows = [x[b, :, :L] for x in (lse, d) for b, L in enumerate(lens_q)]  # (what lies past a sequence's end is not written)
+        return [o, dq, dk, dv] + rows + [x for x in (q_rot, dbias) if x is not None] + [torch.cuda.get_rng_state()]
+
+    native = step()
+    with binding_only():
+        for i, (x, y) in enumerate(zip(native, step())):
+            assert torch.equal(x, y), i
+
+
+def test_native_calls_hand_back_what_the_binding_refuses(binding_only):
+    """the same exceptions with and without the native half"""
+    from flash_attn import flash_attn_gfx950 as be
+    x, cu = torch.randn(20, 3, 2, 64, device="cuda").half(), _cu([20])
+    q, k, v = x.unbind(1)
+    bad = [((q.float(), k, v, cu, cu, 20, 20, 0.0, 0.1), {}), ((q.cpu(), k, v, cu, cu, 20, 20, 0.0, 0.1), {}),
+           ((q, k[:, :1], v, cu, cu, 20, 20, 0.0, 0.1), {}), ((q, k, v, cu.long(), cu, 20, 20, 0.0, 0.1), {}),
+           ((q, k, v, cu, cu, 0, 20, 0.0, 0.1), {}), ((q, k, v, cu, cu, 20, 20, 1.5, 0.1), {}), ((q, k, v, cu, cu, 20, 20, 0.0, -1.0), {}),
+           ((q, k, v, cu, cu, 20, 20, 0.0, 0.1), {"alibi_slopes": torch.ones(3, device="cuda")}),
+           ((q, k, v, cu, cu, 20, 20, 0.0, 0.1), {"keep_words": torch.ones(3, device="cuda")}),
+           ((x[:, 0, :, :48], x[:, 1, :, :48], x[:, 2, :, :48], cu, cu, 20, 20, 0.0, 0.1), {}),
+           ((x.view(-1)[1:1 + 19 * 384].view(19, 3, 2, 64)[:, 0], k[:19], v[:19], cu, cu, 20, 20, 0.0, 0.1), {})]
+    for args, kw in bad:
+        said = []
+        for cm in (None, binding_only()):
+            with pytest.raises(RuntimeError) as e:
+                if cm is None:
+                    be.fwd(*args, False, False, False, None, **kw)
+                else:
+                    with cm:
+                        be.fwd(*args, False, False, False, None, **kw)
+            said.append(str(e.value))
+        assert said[0] == said[1] and said[0]
+
+
 def _padding_masks(B, S, seed):
     """(B, S) bool masks: right padding, left padding, holes, one run in the middle; entry 0 full, entry 1 (if there is one) without tokens."""
     g = torch.Generator().manual_seed(seed)
