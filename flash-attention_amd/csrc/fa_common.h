@@ -212,6 +212,36 @@ FA_DEVICE u32x4 philox4x32_7(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
   return r;
 }
 
+// The same output in two parts.  The counter is (c0, q4, bh, c3) with c0 by the key and q4 by the query: the first three rounds make
+// four words that depend on the key alone, two that depend on the query alone, and one product of both.  A tile's key words serve all its
+// query rows (the forward keeps them in LDS), a lane's query words all keys: nine multiplications are left of fourteen.
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u, kPhiloxM1 = 0xCD9E8D57u, kPhiloxW0 = 0x9E3779B9u, kPhiloxW1 = 0xBB67AE85u;
+FA_DEVICE u32x4 philox_key_words(const PhiloxKey& pk, uint32_t bh, uint32_t c0) {
+  const uint64_t a = (uint64_t)kPhiloxM0 * c0;
+  const uint64_t b = (uint64_t)kPhiloxM1 * xor3((uint32_t)(a >> 32), pk.c3, pk.k1);
+  const uint64_t d = (uint64_t)kPhiloxM0 * xor3((uint32_t)(b >> 32), kPhiloxM1 * bh, pk.k0 + kPhiloxW0);
+  return u32x4{(uint32_t)a ^ (pk.k1 + kPhiloxW1), (uint32_t)b ^ (pk.k0 + 2 * kPhiloxW0), (uint32_t)(d >> 32) ^ (pk.k1 + 2 * kPhiloxW1), (uint32_t)d};
+}
+FA_DEVICE uint64_t philox_query_words(const PhiloxKey& pk, uint32_t bh, uint32_t q4) {
+  return (uint64_t)kPhiloxM0 * xor3((uint32_t)(((uint64_t)kPhiloxM1 * bh) >> 32), q4, pk.k0);
+}
+FA_DEVICE u32x4 philox_finish(const PhiloxKey& pk, u32x4 key, uint64_t query) {
+  const uint64_t m = (uint64_t)kPhiloxM1 * ((uint32_t)(query >> 32) ^ key[0]);
+  uint32_t c0 = (uint32_t)(m >> 32) ^ key[1], c1 = (uint32_t)m, c2 = key[2] ^ (uint32_t)query, c3 = key[3];
+  uint32_t k0 = pk.k0 + 3 * kPhiloxW0, k1 = pk.k1 + 3 * kPhiloxW1;
+#pragma unroll
+  for (int i = 3; i < 7; i++) {
+    const uint64_t p0 = (uint64_t)kPhiloxM0 * c0, p1 = (uint64_t)kPhiloxM1 * c2;
+    c0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+    c1 = (uint32_t)p1;
+    c2 = xor3((uint32_t)(p0 >> 32), c3, k1);
+    c3 = (uint32_t)p0;
+    k0 += kPhiloxW0;
+    k1 += kPhiloxW1;
+  }
+  return u32x4{c0, c1, c2, c3};
+}
+
 // 16 keep bits of micro-block (Q4, K4): bit (4*(q%4) + key%4) set <=> keep.
 FA_DEVICE uint32_t dropout_keep_bits16(const PhiloxKey& pk, uint32_t bh, uint32_t Q4, uint32_t K4, uint32_t thr) {
   uint32_t bits = 0;
@@ -292,6 +322,22 @@ FA_DEVICE KeepFields keep_fields_row_layout(const PhiloxKey& pk, uint32_t bh, in
 #pragma unroll
   for (int m = 0; m < 2; m++) {  // micro-blocks m (odd lanes: 2 + m)
     const u32x4 a = philox4x32_7(c0 + 4 * m, (uint32_t)qrow >> 2, bh, pk.c3, pk.k0, pk.k1);
+    uint32_t lo[2] = {a[0], a[1]}, hi[2] = {a[2], a[3]};
+    exchange_in_lane_pair(lo, hi);
+    e.w[2 * m] = lo[0]; e.w[2 * m + 1] = lo[1];
+    e.w[4 + 2 * m] = hi[0]; e.w[5 + 2 * m] = hi[1];
+  }
+  return e;
+}
+// The same from words made before: words = philox_key_words of the 16 counters of the 32 keys, one after the other in LDS (counter c0 at
+// c0 - 2 * (key0 / 4)), query = this lane's philox_query_words.
+FA_DEVICE KeepFields keep_fields_row_layout(const PhiloxKey& pk, const u32x4* words, uint64_t query, int qrow, int hf) {
+  const uint32_t t = (uint32_t)qrow & 3u;
+  const u32x4* const w0 = words + (((hf + 4 * (t & 1)) << 1) | (t >> 1));
+  KeepFields e;
+#pragma unroll
+  for (int m = 0; m < 2; m++) {  // micro-blocks m (odd lanes: 2 + m)
+    const u32x4 a = philox_finish(pk, w0[4 * m], query);
     uint32_t lo[2] = {a[0], a[1]}, hi[2] = {a[2], a[3]};
     exchange_in_lane_pair(lo, hi);
     e.w[2 * m] = lo[0]; e.w[2 * m + 1] = lo[1];

@@ -95,8 +95,16 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
 
   // kTensorBias: behind the tiles, per wave 32 rows x BN keys of bias, rows padded by 8 bytes (see load_bias below)
   constexpr int kBiasRowBytes = BN * 2 + 8, kBiasWaveBytes = 32 * kBiasRowBytes;
+  // kKeyWords: behind everything else, for the staged and the next tile, the key words of its BN / 2 Philox counters (fa_common.h).  us of the
+  // forward with them / with whole outputs drawn, p = 0.1: 64 x 16 heads x 1004 .. 1023, d = 64, 535 / 551; 4 x 12 x 4096 313 / 319; 8 x 16 x
+  // 1000, d = 32, 60.6 / 63.0.  Not at d = 128 (8 x 12 x 2048: 316 / 301), nor where they cost a wave per SIMD
+  // or a spill: half-size at d = 16, over a block layout at d = 32.
+  // (Round keys stepped by the scalar unit in place of kept ones, which are parked in vector lanes: 550.)
+  constexpr bool kKeyWords = kDropout && !kSparse && kBias == 0 && (D == 32 || D == 64);
+  constexpr int kKeyWordBytes = BN / 2 * 16, kKeyWordOff = Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : 0);
   constexpr int kRowSlotBytes = 2 * 64 * 4;  // kRows: behind the tiles, per wave (see fetch_rows below)
-  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : kRows ? 4 * kRowSlotBytes : 0)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : kRows ? 4 * kRowSlotBytes : 0) +
+                                                                  (kKeyWords ? 2 * kKeyWordBytes : 0)];
 
   // Workgroup -> (batch, head, query tile), XCD-aware (see map_tile): the query tiles of one (batch, head) share
   // one XCD's L2 copy of K and V.
@@ -201,8 +209,14 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
         return;
       }
     }
+    if constexpr (kKeyWords) {  // the waves take turns, one tile each
+      if ((it & 3) == wave && lane < BN / 2)
+        *reinterpret_cast<u32x4*>(lds_raw + kKeyWordOff + buf * kKeyWordBytes + lane * 16) =
+            philox_key_words(p.pk, (uint32_t)bh, (uint32_t)(it * (BN / 2) + lane));
+    }
     stager.issue(lds_raw + buf * kBufBytes, it * BN, Lk);
   };
+  const uint64_t query_words = kKeyWords ? philox_query_words(p.pk, (uint32_t)bh, (uint32_t)qrow >> 2) : 0;
 
   // Sparse: tile `it` is computed iff its 256-key block is active for any 16-row block of this query tile.  The tile's
   // and this lane's row block's activity bits of 64 consecutive key blocks (16384 keys) sit in registers.
@@ -346,6 +360,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     }
     const T* Ks = reinterpret_cast<const T*>(lds_raw + buf * kBufBytes);
     const T* Vs = Ks + BN * D;
+    const u32x4* const key_words = reinterpret_cast<const u32x4*>(lds_raw + kKeyWordOff + buf * kKeyWordBytes);
     buf ^= 1;
 
     bool wave_work = wave_live;  // a wave whose 32 rows all lie past the sequence's end only helps with the staging
@@ -470,7 +485,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
         if (kDropout) {
 #pragma unroll
           for (int kb = 0; kb < KBW; kb++) {
-            const KeepFields keep = keep_fields_row_layout(p.pk, (uint32_t)bh, qrow, n0 + (kb0 + kb) * 32, hf);
+            KeepFields keep;
+            if constexpr (kKeyWords) keep = keep_fields_row_layout(p.pk, key_words + (kb0 + kb) * 16, query_words, qrow, hf);
+            else keep = keep_fields_row_layout(p.pk, (uint32_t)bh, qrow, n0 + (kb0 + kb) * 32, hf);
             // Dropped probabilities become 0 after the rounding, two a time: the keep decisions of a word of fields are 1 or 0 in each
             // half (two packed saturating subtractions), a packed 16-bit integer product applies them, and shifted together they are the
             // row's keep word.  Counted with SQ_INSTS_VALU over 64 x 16 heads x 1004 .. 1023, d = 64, p = 0.1, fp16, the forward issues 25.3 other
