@@ -284,6 +284,8 @@ inline bool longest_first_launch(bool causal, bool sparse, int grid, int B) {
 //   forward: half-size for x < 2 (more than one key tile pair to split: sequences beyond 128), and up to x < 3 with dropout
 //            (whose Philox work makes the serial walk longer);
 //   dQ:      half-size for 1 <= x < 2 under a causal mask or with dropout; the plain kernel gains nothing from it.
+// Where lengths differ, many launched workgroups find no rows: the rules that follow this one (causal forward, head dim 128, backward without
+// dropout) count those that do, and this one stays for the others.
 // launch_policy() & 3: 0 = by this rule, 1 = always the full-size tiles, 2 = the half-size tiles wherever they exist
 // (fa_set_launch_policy; the parity tests run both shapes on the same inputs).
 int launch_policy();
@@ -344,11 +346,15 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
 
 // The dQ kernel's half-size tiles in a launch of its own, dropout off (with dropout: small_launch): causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 /
 // 25.1 with the dK/dV kernel, 3 x 16 x 70 % of 1785 (494) 59.5 / 53.0, 12 x 16 x 336 (551) 23.7 / 23.3; d = 64 8 x 12 x 460 (393) 34.0 / 32.6, 12 x 8 x 609
-// (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.
+// (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
+// chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 3 x 16 x 1495 (292) 110.3 / 101.6, short sequences cross sooner: 6 x 16 x 183
+// (169) 25.6 / 27.1, 6 x 16 x 509 (345) 51.5 / 54.7; no mask 4 x 16 x 211 (134) 28.4 / 26.5, 2 x 8 x 1112 (133) 79.7 / 75.9, 3 x 16 x 789 (256) 70.7 / 75.7.
 inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words, bool rotary,
                             int n_splits) {
   if (merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, false, false, rotary, n_splits)) return true;
-  if ((launch_policy() & 3) != 0 || dropout || max_sk > 2 * max_sq) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
+  const bool swept = (launch_policy() & 3) == 0 && !dropout && max_sk <= 2 * max_sq;
+  if (head_dim == 128 && (launch_policy() & 3) == 0) return swept && max_sq > 128 && live <= (causal ? (max_sq > 450 ? 300 : 150) : 140);
+  if (!swept) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
   return max_sq > 128 && live <= (causal ? (head_dim == 64 ? 400 : 500) : 130);
 }
 

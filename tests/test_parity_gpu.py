@@ -235,6 +235,16 @@ def test_parity_ragged_shapes(lens_q, lens_k, causal, tile_shape):
     _parity_case(lens_q, lens_k, 2, 64, torch.float16, causal, packing="kv", seed=len(lens_q))
 
 
+@pytest.mark.parametrize("lens_q,lens_k", [
+    ([1, 63, 64, 65], [1, 63, 64, 65]),          # around a half-size tile of queries, one and two key tiles
+    ([129, 0, 191], [128, 40, 193]),             # an entry without queries, key counts across a tile's two halves
+    ([33, 300], [1, 31]),                        # fewer keys than one wave's block
+])
+@pytest.mark.parametrize("causal", [False, True])
+def test_d128_backward_tile_edges(lens_q, lens_k, causal, tile_shape):
+    _parity_case(lens_q, lens_k, 2, 128, torch.bfloat16, causal, packing="kv", seed=len(lens_q))
+
+
 def test_parity_separate_qkv_and_scale():
     _parity_case([100, 140], [90, 260], 4, 32, torch.bfloat16, False, packing="sep", seed=5, scale=0.3)
     _parity_case([100, 140], [100, 140], 4, 32, torch.float16, True, packing="sep", seed=6, scale=0.05)
