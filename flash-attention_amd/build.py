@@ -1,4 +1,4 @@
-"""Builds libflash_attn_gfx950.so (the C-ABI attention library) with hipcc for gfx950.
+"""Builds libflash_attn_gfx950.so (the C-ABI attention library) with hipcc for gfx950, and fa_host.so (the binding's native half) with g++.
 
 Usage:  python flash-attention_amd/build.py [-j JOBS]
 The translation units under csrc/ compile in parallel; objects go to build/ (git-ignored) and the
