@@ -720,6 +720,21 @@ static int bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t
   return FA_OK;
 }
 
+int fa_pad_bias_rows(const void* bias, void* out, int32_t batch, int32_t heads, int64_t rows, int64_t cols, int64_t batch_stride, int64_t head_stride,
+                     int64_t row_stride, int64_t key_stride, void* stream) {
+  FA_REQUIRE(batch >= 0 && heads >= 0 && rows >= 0 && cols >= 0, "fa_pad_bias_rows: negative size");
+  FA_REQUIRE(batch_stride >= 0 && head_stride >= 0 && row_stride >= 0 && key_stride >= 0, "fa_pad_bias_rows: negative stride");
+  if (batch == 0 || heads == 0 || rows == 0 || cols == 0) return FA_OK;
+  FA_REQUIRE(cols < ((int64_t)1 << 30) && rows < ((int64_t)1 << 31) && (int64_t)batch * heads < ((int64_t)1 << 31) &&
+             (int64_t)batch * heads <= ((int64_t)1 << 31) / rows, "fa_pad_bias_rows: too many rows");
+  FA_REQUIRE(bias && out, "fa_pad_bias_rows: null pointer");
+  FA_REQUIRE((reinterpret_cast<uintptr_t>(bias) & 1) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0,
+             "fa_pad_bias_rows: out must be 16-byte aligned, bias 2-byte aligned");
+  FA_LAUNCH(fa::launch_pad_bias_rows(bias, out, batch, heads, rows, cols, batch_stride, head_stride, row_stride, key_stride,
+                                     reinterpret_cast<hipStream_t>(stream)));
+  return FA_OK;
+}
+
 int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t batch, int32_t heads, int32_t rows,
                         int32_t cols, int64_t dbias_batch_stride, int64_t dbias_head_stride, int64_t dbias_row_stride,
                         int32_t sum_batch, int32_t sum_heads, int64_t out_batch_stride, int64_t out_head_stride,

@@ -1,4 +1,4 @@
-// Reduction of the bias gradient behind fa_bias_grad_reduce.  The dK/dV kernel writes the gradient of an attn_bias tensor
+// Reduction of the bias gradient behind fa_bias_grad_reduce, and the bias tensor's copy with padded rows (fa_pad_bias_rows).  The dK/dV kernel writes the gradient of an attn_bias tensor
 // per (batch, head); a bias that was broadcast over the batch and/or the heads wants the sum over the entries that shared
 // it.  One pass: every thread owns 8 consecutive keys of one output row, adds the slices in a fixed order (batch outer,
 // head inner) in fp32 and rounds once.  HBM-bound: each input element is read once, each output element written once.  With the batch's
@@ -59,7 +59,48 @@ __global__ void __launch_bounds__(256) bias_grad_reduce_kernel(const T* __restri
   }
 }
 
+// A bias tensor's rows copied to rows of whole 16-byte chunks, zeros behind the last key, for tensors whose rows the attention kernels cannot
+// read as they are (odd lengths, other strides).  HBM-bound: a thread moves one chunk, read whole where its eight keys are there and lie
+// together (a row of odd length starts at any even address: an unaligned 16-byte load; eight 2-byte loads took 85 us for 8 x 12 x 901
+// x 901), a workgroup the chunks of four rows (8 rows 69, 4 rows 66, 2 rows 74).  us of a clearing and a strided copy / this: 8 x 701 x 701
+// 8.0 / 6.2, 16 x 1100 x 1100 22.9 / 14.5, 12 x 2047 x 2047 52.6 / 40.4 (5.0 TB/s moved), 8 x 16 x 1101 x 1101 169 / 125.
+constexpr int kPadRows = 4;
+__global__ void __launch_bounds__(256) pad_bias_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int nh, int64_t rows,
+                                                            int64_t cols, int cpr, int64_t row_groups, int64_t s_bs, int64_t s_hs, int64_t s_rs,
+                                                            int64_t s_ks) {
+  const int64_t bh = blockIdx.x / row_groups, r0 = (blockIdx.x - bh * row_groups) * kPadRows;
+  const int nrows = (int)(rows - r0 < kPadRows ? rows - r0 : kPadRows);
+  src += bh / nh * s_bs + bh % nh * s_hs + r0 * s_rs;
+  dst += (bh * rows + r0) * cpr * 8;
+  const unsigned n = (unsigned)(nrows * cpr);
+  for (unsigned t = threadIdx.x; t < n; t += 256) {
+    const unsigned i = t / (unsigned)cpr;
+    const int64_t col0 = (int64_t)(t - i * (unsigned)cpr) * 8;
+    union { uint16_t e[8]; uint4 v; } c;
+    const uint16_t* const from = src + i * s_rs + col0 * s_ks;
+    if (s_ks == 1 && col0 + 8 <= cols) {
+      __builtin_memcpy(c.e, from, 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        c.e[j] = 0;
+        if (col0 + j < cols) c.e[j] = from[j * s_ks];
+      }
+    }
+    *reinterpret_cast<uint4*>(dst + (int64_t)t * 8) = c.v;
+  }
+}
+
 }  // namespace
+
+hipError_t launch_pad_bias_rows(const void* src, void* dst, int nb, int nh, int64_t rows, int64_t cols, int64_t s_bs, int64_t s_hs, int64_t s_rs,
+                                int64_t s_ks, hipStream_t stream) {
+  if (nb == 0 || nh == 0 || rows == 0 || cols == 0) return hipSuccess;
+  const int64_t groups = (rows + kPadRows - 1) / kPadRows;
+  hipLaunchKernelGGL(pad_bias_rows_kernel, dim3((unsigned)(groups * nb * nh)), dim3(256), 0, stream, reinterpret_cast<const uint16_t*>(src),
+                     reinterpret_cast<uint16_t*>(dst), nh, rows, cols, (int)((cols + 7) >> 3), groups, s_bs, s_hs, s_rs, s_ks);
+  return hipGetLastError();
+}
 
 hipError_t launch_bias_grad_reduce(const void* in, void* out, int dtype, int nb, int nh, int rows, int cols, int64_t in_bs,
                                    int64_t in_hs, int64_t in_rs, int sum_batch, int sum_heads, int64_t out_bs, int64_t out_hs,

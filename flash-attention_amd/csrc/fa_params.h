@@ -399,6 +399,8 @@ struct BiasGradLens {  // the batch's lengths as the backward had them (seq_exte
 hipError_t launch_bias_grad_reduce(const void* in, void* out, int dtype, int nb, int nh, int rows, int cols, int64_t in_bs,
                                    int64_t in_hs, int64_t in_rs, int sum_batch, int sum_heads, int64_t out_bs, int64_t out_hs,
                                    int64_t out_rs, const BiasGradLens& lens, bool vec_store, hipStream_t stream);
+hipError_t launch_pad_bias_rows(const void* src, void* dst, int nb, int nh, int64_t rows, int64_t cols, int64_t s_bs, int64_t s_hs, int64_t s_rs,
+                                int64_t s_ks, hipStream_t stream);
 hipError_t launch_dump_probs(const DumpParams& p, int dtype, hipStream_t stream);
 // which: 0 = dQ kernel, 1 = dK/dV kernel
 hipError_t launch_bwd(const BwdParams& p, int which, int dtype, int head_dim, bool causal, bool dropout, bool sparse,

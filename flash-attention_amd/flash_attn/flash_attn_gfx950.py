@@ -121,7 +121,7 @@ EXPORTED_SYMBOLS = (
     "fa_fwd", "fa_bwd", "fa_fwd_block", "fa_bwd_block", "fa_fwd_block_noalloc", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes",
     "fa_round_seqlens", "fa_philox_offset_increment", "fa_last_error", "fa_abi_version",
     "fa_gather_rows", "fa_scatter_rows", "fa_scatter_rows_workspace_bytes", "fa_rotary", "fa_set_launch_policy",
-    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_bias_grad_reduce_ragged", "fa_padding_rows", "fa_fwd_padded",
+    "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_bias_grad_reduce_ragged", "fa_pad_bias_rows", "fa_padding_rows", "fa_fwd_padded",
 )
 # declared in include/flash_attn_gfx950_bench.h: instrumentation for bench.py, not part of the drop-in boundary
 BENCH_SYMBOLS = ("fa_bwd_profiled",)
@@ -193,6 +193,8 @@ def load_library():
         lib.fa_bias_grad_reduce.restype = ctypes.c_int
         lib.fa_bias_grad_reduce_ragged.argtypes = ([ctypes.c_void_p] * 2 + [ctypes.POINTER(BwdArgs)] + [ctypes.c_int32] * 2 + [ctypes.c_int64] * 3)
         lib.fa_bias_grad_reduce_ragged.restype = ctypes.c_int
+        lib.fa_pad_bias_rows.argtypes = [ctypes.c_void_p] * 2 + [ctypes.c_int32] * 2 + [ctypes.c_int64] * 6 + [ctypes.c_void_p]
+        lib.fa_pad_bias_rows.restype = ctypes.c_int
         lib.fa_padding_rows.argtypes = ([ctypes.c_void_p, ctypes.c_int64] + [ctypes.c_int32] * 2 + [ctypes.c_void_p] * 4)
         lib.fa_padding_rows.restype = ctypes.c_int
         lib.fa_fwd_padded.argtypes = [ctypes.POINTER(FwdArgs), ctypes.c_void_p, ctypes.c_void_p]
@@ -372,6 +374,14 @@ def prepare_attn_bias(attn_bias, q, batch, nheads, max_seqlen_q, max_seqlen_k):
           attn_bias.data_ptr() % 16 == 0 and all(attn_bias.stride(i) % 8 == 0 for i in (0, 1)))
     if not ok:
         sk8 = (attn_bias.shape[3] + 7) // 8 * 8
+        if attn_bias.is_cuda and attn_bias.element_size() == 2:
+            lib = load_library()
+            with _OnDevice(attn_bias.device):
+                padded = torch.empty(attn_bias.shape[:3] + (sk8,), dtype=attn_bias.dtype, device=attn_bias.device)
+                rc = lib.fa_pad_bias_rows(attn_bias.data_ptr(), padded.data_ptr(), *attn_bias.shape, *attn_bias.stride(), _stream_handle(attn_bias.device))
+            if rc != 0:
+                _raise(rc, lib)
+            return padded
         padded = torch.zeros(attn_bias.shape[:3] + (sk8,), dtype=attn_bias.dtype, device=attn_bias.device)
         padded[..., :attn_bias.shape[3]] = attn_bias
         attn_bias = padded

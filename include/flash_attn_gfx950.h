@@ -285,6 +285,11 @@ int fa_bias_grad_reduce(const void* dbias, void* out, int32_t dtype, int32_t bat
 int fa_bias_grad_reduce_ragged(const void* dbias, void* out, const fa_bwd_args* args, int32_t sum_batch, int32_t sum_heads,
                                int64_t out_batch_stride, int64_t out_head_stride, int64_t out_row_stride);
 
+/* The copy of a bias tensor (16-bit elements, any strides, in elements) that fa_fwd and fa_bwd can read: out is contiguous, [batch, heads,
+ * rows, cols rounded up to 8], 16-byte aligned, with zeros behind column cols. */
+int fa_pad_bias_rows(const void* bias, void* out, int32_t batch, int32_t heads, int64_t rows, int64_t cols, int64_t batch_stride, int64_t head_stride,
+                     int64_t row_stride, int64_t key_stride, void* stream);
+
 /* Rotary position embedding of the query and key parts of a packed tensor in one pass: what
  * RotaryEmbedding.forward / apply_rotary_pos_emb compute with elementwise torch ops (flash_attn/rotary.py:22-42,
  * 89-100; FlashMHA applies it to q and k before attention, flash_attention.py:109-113).

@@ -923,6 +923,26 @@ def test_bias_grad_reduce_sums_in_fp32_and_rounds_once(dtype):
         be.reduce_bias_grad(dbias, torch.empty(2, 6, 8, 7, device="cuda", dtype=dtype), True, False)  # wrong batch extent
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 3, 7, 8), (1, 2, 9, 15), (2, 1, 33, 2049), (3, 2, 8, 701)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_prepare_attn_bias_pads_rows_on_the_gpu(shape, dtype):
+    """The copy with padded rows holds the tensor's own bits and zeros behind them, for every order and stride (keys not contiguous, heads
+    broadcast, axes swapped, a base that is only 2-byte aligned)."""
+    from flash_attn import flash_attn_gfx950 as be
+    B, H, R, C = shape
+    q = torch.empty(4, H, 64, device="cuda", dtype=dtype)
+    flat = torch.randint(-32768, 32768, (2 * B * H * R * C + 9,), device="cuda", dtype=torch.int16).view(dtype)
+    n = B * H * R * C
+    for t in (flat[1:1 + n].view(B, H, R, C), flat[:2 * n].view(B, H, R, 2 * C)[..., ::2], flat[1:1 + n].view(B, H, C, R).transpose(2, 3),
+              flat[1:1 + B * R * C].view(B, 1, R, C).expand(B, H, R, C), flat[3:3 + n].view(H, B, R, C).transpose(0, 1)):
+        p = be.prepare_attn_bias(t, q, B, H, R, C)
+        if p is t:
+            continue
+        assert tuple(p.shape) == (B, H, R, (C + 7) // 8 * 8) and p.is_contiguous()
+        assert torch.equal(p[..., :C].contiguous().view(torch.int16), t.contiguous().view(torch.int16))
+        assert not bool(p[..., C:].contiguous().view(torch.int16).any())
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("sum_batch,sum_heads", [(True, False), (True, True), (False, True), (False, False)])
 def test_bias_grad_reduce_reads_only_what_the_backward_wrote(causal, sum_batch, sum_heads):
