@@ -10,6 +10,7 @@ functions works but the first call raises.
 """
 import ctypes
 import functools
+import math
 import os
 import threading
 
@@ -802,9 +803,11 @@ def scatter_rows(values, indices, first_axis_dim):
 
 
 def padded_layout_ok(qkv, mask):
-    """Whether fwd_padded() takes this (batch, seqlen, 3, nheads, headdim) tensor and mask as they are: a bool mask of one byte a position,
-    rows of qkv one after the other, 16-byte aligned.  (Others are gathered and scattered, bert_padding.py.)"""
-    if not (qkv.is_cuda and qkv.dim() == 5 and qkv.shape[2] == 3 and mask.dtype == torch.bool and mask.device == qkv.device):
+    """Whether fwd_padded() takes this (batch, seqlen, 3, nheads, headdim) tensor and mask as they are: 16-bit elements, a bool mask of one
+    byte a position, rows of qkv one after the other, 16-byte aligned; no stream capture, which the wait for the lengths would break.
+    (Others are gathered and scattered, bert_padding.py, or refused on that way.)"""
+    if not (qkv.is_cuda and qkv.dim() == 5 and qkv.shape[2] == 3 and mask.dtype == torch.bool and mask.device == qkv.device and
+            qkv.dtype in (torch.float16, torch.bfloat16) and not torch.cuda.is_current_stream_capturing()):
         return False
     B, S, _, H, D = qkv.shape
     st = qkv.stride()
@@ -816,46 +819,51 @@ def padded_layout_ok(qkv, mask):
 def fwd_padded(qkv, mask, softmax_scale, is_causal):
     """Attention of a padded batch without gathering it first (fa_padding_rows, fa_fwd_padded): qkv (batch, seqlen, 3, nheads, headdim) and
     a (batch, seqlen) bool mask, True = token, for which padded_layout_ok() holds.  Returns (batch, seqlen, nheads, headdim) with zeros in
-    the padding, or None if the mask holds no token at all.  The lengths are read back for that while the attention kernel runs."""
+    the padding, or None if the mask holds no token at all or the scale is none the kernels take (nothing is enqueued then): the packed
+    call refuses both.  The lengths are read back while the attention kernel runs."""
     lib = load_library()
     B, S, _, H, D = qkv.shape
     st = qkv.stride()
     dev = qkv.device
+
+    def fill(a):
+        a.dtype = _dtype_code(qkv)
+        a.q_row_stride = a.k_row_stride = a.v_row_stride = st[1]
+        a.q_head_stride = a.k_head_stride = a.v_head_stride = st[3]
+        a.o_row_stride, a.o_head_stride = H * D, D
+        a.batch, a.nheads, a.head_dim = B, H, D
+        a.total_q = a.total_k = B * S
+        a.max_seqlen_q = a.max_seqlen_k = S
+        a.is_causal = int(bool(is_causal))
+        return 0
+
+    a, _ = _cached_args(("padded", qkv.dtype, qkv.shape, st, bool(is_causal)), FwdArgs, fill)
+    a.softmax_scale = float(softmax_scale)
+    if not 0.0 < a.softmax_scale < math.inf:  # (as rounded to fp32)
+        return None
     sq_r, _ = round_seqlens(D, S, S, False)
     with _OnDevice(dev):
         out = torch.empty((B, S, H, D), dtype=qkv.dtype, device=dev)
         lse = torch.empty((B, H, sq_r), dtype=torch.float32, device=dev)
         rows = torch.empty((B * (S + 4),), dtype=torch.int32, device=dev)
         lens = torch.empty((B,), dtype=torch.int32, pin_memory=True)
+        written = torch.cuda.Event()
         row_of, stream = rows.data_ptr(), _stream_handle(dev)
         row_info = row_of + 4 * B * S
-        rc = lib.fa_padding_rows(mask.data_ptr(), mask.stride(0), B, S, row_of, row_info, lens.data_ptr(), stream)
-        if rc != 0:
-            _raise(rc, lib)
-        written = torch.cuda.Event()
-        written.record()
-
-        def fill(a):
-            a.dtype = _dtype_code(qkv)
-            a.q_row_stride = a.k_row_stride = a.v_row_stride = st[1]
-            a.q_head_stride = a.k_head_stride = a.v_head_stride = st[3]
-            a.o_row_stride, a.o_head_stride = H * D, D
-            a.batch, a.nheads, a.head_dim = B, H, D
-            a.total_q = a.total_k = B * S
-            a.max_seqlen_q = a.max_seqlen_k = S
-            a.is_causal = int(bool(is_causal))
-            return 0
-
-        a, _ = _cached_args(("padded", qkv.dtype, qkv.shape, st, bool(is_causal)), FwdArgs, fill)
         a.q = qkv.data_ptr()
         a.k, a.v = a.q + 2 * st[2], a.q + 4 * st[2]
         a.o, a.softmax_lse = out.data_ptr(), lse.data_ptr()
-        a.softmax_scale = float(softmax_scale)
         a.stream = stream
-        rc = lib.fa_fwd_padded(ctypes.byref(a), row_of, row_info)
+        rc = lib.fa_padding_rows(mask.data_ptr(), mask.stride(0), B, S, row_of, row_info, lens.data_ptr(), stream)
         if rc != 0:
             _raise(rc, lib)
-        written.synchronize()
+        try:
+            written.record()
+            rc = lib.fa_fwd_padded(ctypes.byref(a), row_of, row_info)
+            if rc != 0:
+                _raise(rc, lib)
+        finally:  # (a kernel writes to lens, of which the pinned-memory allocator does not know)
+            written.synchronize()
     return out if lens.any() else None
 
 

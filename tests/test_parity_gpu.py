@@ -1524,6 +1524,49 @@ def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape):
             m(qkv, key_padding_mask=type("Mask", (), {"bool_matrix": torch.zeros(B, S, dtype=torch.bool, device="cuda")}), causal=causal)
 
 
+def test_padded_batch_is_refused_before_anything_is_enqueued(monkeypatch):
+    """What the packed call refuses is refused with no kernel of the in-place path in flight, which writes the lengths to host memory; a
+    launch that fails behind that kernel is waited for before the exception leaves."""
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.flash_attention import FlashAttention
+    lib, calls, events = be.load_library(), [], []
+
+    class Recorder:
+        def __getattr__(self, name):
+            calls.append(name)
+            return (lambda *a: 2) if name in fail else getattr(lib, name)
+
+    class Event(torch.cuda.Event):
+        def record(self, *a):
+            events.append("record")
+            return super().record(*a)
+
+        def synchronize(self):
+            events.append("synchronize")
+            return super().synchronize()
+
+    fail = ()
+    qkv = torch.randn(2, 70, 3, 2, 64, device="cuda").half()
+    kpm = type("Mask", (), {"bool_matrix": (torch.arange(70)[None] < torch.tensor([[70], [31]])).cuda()})
+    with torch.no_grad():
+        want = FlashAttention().eval()(qkv, key_padding_mask=kpm)[0]
+        monkeypatch.setattr(be, "_lib", Recorder())
+        for scale in (0.0, -0.1, float("nan"), float("inf"), 1e-60, 1e39):  # (the last two: 0 and inf in fp32)
+            with pytest.raises(RuntimeError, match="softmax_scale"):
+                FlashAttention(softmax_scale=scale).eval()(qkv, key_padding_mask=kpm)
+        assert "fa_padding_rows" not in calls and "fa_fwd_padded" not in calls
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)  # (no wait for lengths in a capture)
+        assert torch.equal(FlashAttention().eval()(qkv, key_padding_mask=kpm)[0], want)
+        assert "fa_padding_rows" not in calls
+        monkeypatch.undo()
+        monkeypatch.setattr(be, "_lib", Recorder())
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        fail = ("fa_fwd_padded",)
+        with pytest.raises(RuntimeError):
+            FlashAttention().eval()(qkv, key_padding_mask=kpm)
+        assert "fa_padding_rows" in calls and events == ["record", "synchronize"]
+
+
 def test_flash_attention_module_three_input_modes():
     from flash_attn.flash_attention import FlashAttention
     B, S, H, D = 3, 96, 2, 64
