@@ -725,8 +725,9 @@ int fa_pad_bias_rows(const void* bias, void* out, int32_t batch, int32_t heads, 
   FA_REQUIRE(batch >= 0 && heads >= 0 && rows >= 0 && cols >= 0, "fa_pad_bias_rows: negative size");
   FA_REQUIRE(batch_stride >= 0 && head_stride >= 0 && row_stride >= 0 && key_stride >= 0, "fa_pad_bias_rows: negative stride");
   if (batch == 0 || heads == 0 || rows == 0 || cols == 0) return FA_OK;
-  FA_REQUIRE(cols < ((int64_t)1 << 30) && rows < ((int64_t)1 << 31) && (int64_t)batch * heads < ((int64_t)1 << 31) &&
-             (int64_t)batch * heads <= ((int64_t)1 << 31) / rows, "fa_pad_bias_rows: too many rows");
+  // (a row's chunks are counted in 32 bits, all elements in 64)
+  FA_REQUIRE(cols < ((int64_t)1 << 32) && (int64_t)batch * heads <= ((int64_t)1 << 40) / rows &&
+             (int64_t)batch * heads * rows <= ((int64_t)1 << 60) / (cols + 7), "fa_pad_bias_rows: too many rows");
   FA_REQUIRE(bias && out, "fa_pad_bias_rows: null pointer");
   FA_REQUIRE((reinterpret_cast<uintptr_t>(bias) & 1) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0,
              "fa_pad_bias_rows: out must be 16-byte aligned, bias 2-byte aligned");

@@ -64,30 +64,32 @@ __global__ void __launch_bounds__(256) bias_grad_reduce_kernel(const T* __restri
 // together (a row of odd length starts at any even address: an unaligned 16-byte load; eight 2-byte loads took 85 us for 8 x 12 x 901
 // x 901), a workgroup the chunks of four rows (8 rows 69, 4 rows 66, 2 rows 74).  us of a clearing and a strided copy / this: 8 x 701 x 701
 // 8.0 / 6.2, 16 x 1100 x 1100 22.9 / 14.5, 12 x 2047 x 2047 52.6 / 40.4 (5.0 TB/s moved), 8 x 16 x 1101 x 1101 169 / 125.
-constexpr int kPadRows = 4;
+// (Groups of rows in a loop over a bounded grid, see pad_bias_grid.)
 __global__ void __launch_bounds__(256) pad_bias_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int nh, int64_t rows,
-                                                            int64_t cols, int cpr, int64_t row_groups, int64_t s_bs, int64_t s_hs, int64_t s_rs,
-                                                            int64_t s_ks) {
-  const int64_t bh = blockIdx.x / row_groups, r0 = (blockIdx.x - bh * row_groups) * kPadRows;
-  const int nrows = (int)(rows - r0 < kPadRows ? rows - r0 : kPadRows);
-  src += bh / nh * s_bs + bh % nh * s_hs + r0 * s_rs;
-  dst += (bh * rows + r0) * cpr * 8;
-  const unsigned n = (unsigned)(nrows * cpr);
-  for (unsigned t = threadIdx.x; t < n; t += 256) {
-    const unsigned i = t / (unsigned)cpr;
-    const int64_t col0 = (int64_t)(t - i * (unsigned)cpr) * 8;
-    union { uint16_t e[8]; uint4 v; } c;
-    const uint16_t* const from = src + i * s_rs + col0 * s_ks;
-    if (s_ks == 1 && col0 + 8 <= cols) {
-      __builtin_memcpy(c.e, from, 16);
-    } else {
+                                                            int64_t cols, int cpr, int64_t row_groups, int64_t groups, int64_t s_bs,
+                                                            int64_t s_hs, int64_t s_rs, int64_t s_ks) {
+  for (int64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+    const int64_t bh = g / row_groups, r0 = (g - bh * row_groups) * kPadBiasRows;
+    const int nrows = (int)(rows - r0 < kPadBiasRows ? rows - r0 : kPadBiasRows);
+    const uint16_t* const s = src + bh / nh * s_bs + bh % nh * s_hs + r0 * s_rs;
+    uint16_t* const d = dst + (bh * rows + r0) * cpr * 8;
+    const unsigned n = (unsigned)nrows * (unsigned)cpr;
+    for (unsigned t = threadIdx.x; t < n; t += 256) {
+      const unsigned i = t / (unsigned)cpr;
+      const int64_t col0 = (int64_t)(t - i * (unsigned)cpr) * 8;
+      union { uint16_t e[8]; uint4 v; } c;
+      const uint16_t* const from = s + i * s_rs + col0 * s_ks;
+      if (s_ks == 1 && col0 + 8 <= cols) {
+        __builtin_memcpy(c.e, from, 16);
+      } else {
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        c.e[j] = 0;
-        if (col0 + j < cols) c.e[j] = from[j * s_ks];
+        for (int j = 0; j < 8; j++) {
+          c.e[j] = 0;
+          if (col0 + j < cols) c.e[j] = from[j * s_ks];
+        }
       }
+      *reinterpret_cast<uint4*>(d + (int64_t)t * 8) = c.v;
     }
-    *reinterpret_cast<uint4*>(dst + (int64_t)t * 8) = c.v;
   }
 }
 
@@ -96,9 +98,9 @@ __global__ void __launch_bounds__(256) pad_bias_rows_kernel(const uint16_t* __re
 hipError_t launch_pad_bias_rows(const void* src, void* dst, int nb, int nh, int64_t rows, int64_t cols, int64_t s_bs, int64_t s_hs, int64_t s_rs,
                                 int64_t s_ks, hipStream_t stream) {
   if (nb == 0 || nh == 0 || rows == 0 || cols == 0) return hipSuccess;
-  const int64_t groups = (rows + kPadRows - 1) / kPadRows;
-  hipLaunchKernelGGL(pad_bias_rows_kernel, dim3((unsigned)(groups * nb * nh)), dim3(256), 0, stream, reinterpret_cast<const uint16_t*>(src),
-                     reinterpret_cast<uint16_t*>(dst), nh, rows, cols, (int)((cols + 7) >> 3), groups, s_bs, s_hs, s_rs, s_ks);
+  const PadBiasGrid g = pad_bias_grid(nb, nh, rows);
+  hipLaunchKernelGGL(pad_bias_rows_kernel, dim3(g.blocks), dim3(256), 0, stream, reinterpret_cast<const uint16_t*>(src),
+                     reinterpret_cast<uint16_t*>(dst), nh, rows, cols, (int)((cols + 7) >> 3), g.row_groups, g.groups, s_bs, s_hs, s_rs, s_ks);
   return hipGetLastError();
 }
 

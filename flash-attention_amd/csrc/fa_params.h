@@ -399,6 +399,20 @@ struct BiasGradLens {  // the batch's lengths as the backward had them (seq_exte
 hipError_t launch_bias_grad_reduce(const void* in, void* out, int dtype, int nb, int nh, int rows, int cols, int64_t in_bs,
                                    int64_t in_hs, int64_t in_rs, int sum_batch, int sum_heads, int64_t out_bs, int64_t out_hs,
                                    int64_t out_rs, const BiasGradLens& lens, bool vec_store, hipStream_t stream);
+// Its launch: a workgroup per kPadBiasRows rows of a slice, as far as a grid may hold them (fewer than 2^32 threads: above 2^22 workgroups
+// each takes several groups of rows)
+constexpr int kPadBiasRows = 4;
+struct PadBiasGrid {
+  int64_t row_groups, groups;  // of a (batch, head) slice, of all
+  unsigned blocks;
+};
+inline PadBiasGrid pad_bias_grid(int nb, int nh, int64_t rows) {
+  PadBiasGrid g;
+  g.row_groups = (rows + kPadBiasRows - 1) / kPadBiasRows;
+  g.groups = g.row_groups * ((int64_t)nb * nh);
+  g.blocks = (unsigned)(g.groups < (int64_t)1 << 22 ? g.groups : (int64_t)1 << 22);
+  return g;
+}
 hipError_t launch_pad_bias_rows(const void* src, void* dst, int nb, int nh, int64_t rows, int64_t cols, int64_t s_bs, int64_t s_hs, int64_t s_rs,
                                 int64_t s_ks, hipStream_t stream);
 hipError_t launch_dump_probs(const DumpParams& p, int dtype, hipStream_t stream);

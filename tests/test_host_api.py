@@ -550,6 +550,44 @@ def test_bias_grad_reduce_argument_checks(lib):
     assert call(None, None, 1, (2, 3, 16, 0, 0, 0, 0), ok_out) == 0
 
 
+def test_bias_rows_launch_fits_a_grid_at_every_size(tmp_path):
+    """The launch that pads a bias tensor's rows stays below the 2^32 threads a grid may hold and covers every group of rows once, up to
+    tensors of billions of rows (host code of the library's own header; nothing is launched)."""
+    import subprocess
+    import build as fa_build
+    src, exe = tmp_path / "grid.hip", tmp_path / "grid"
+    src.write_text("""#include <cstdio>
+#include "fa_params.h"
+int main() {
+  const int64_t sizes[][3] = {{1, 1, 1}, {1, 12, 333}, {8, 16, 1101}, {64, 16, 65535}, {64, 16, 65536}, {128, 16, 65537}, {1, 1, 3000000000}};
+  for (auto& s : sizes) {
+    const fa::PadBiasGrid g = fa::pad_bias_grid((int)s[0], (int)s[1], s[2]);
+    std::printf("%lld %lld %lld %lld %lld %u\\n", (long long)s[0], (long long)s[1], (long long)s[2], (long long)g.row_groups, (long long)g.groups, g.blocks);
+  }
+}
+""".replace("\\\\n", "\\n"))
+    cmd = [fa_build.HIPCC, "--offload-host-only", "-std=c++17", "-I", fa_build.CSRC, str(src), "-o", str(exe)]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout[-2000:]
+    lines = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, check=True).stdout.splitlines()
+    assert len(lines) == 7
+    for line in lines:
+        nb, nh, rows, row_groups, groups, blocks = map(int, line.split())
+        assert row_groups == -(-rows // 4) and groups == nb * nh * row_groups
+        assert 0 < blocks <= groups and blocks * 256 < 1 << 32
+        assert blocks == groups or blocks >= 1 << 20  # (one workgroup a group, as measured, unless there are more than a grid holds)
+
+
+def test_pad_bias_rows_argument_checks(lib):
+    """fa_pad_bias_rows: what it refuses, and that large tensors are not among it (a null pointer is what these are refused for)"""
+    call = lambda *sizes: lib.fa_pad_bias_rows(None, None, *sizes, 1, 1, 1, 1, None)
+    assert call(0, 3, 4, 5) == 0 and call(2, 3, 0, 5) == 0
+    for sizes in ((-1, 1, 1, 1), (1, 1, -1, 1), (1, 1, 1, 1 << 32), (1 << 30, 1 << 30, 9, 1)):
+        assert call(*sizes) == -1 and b"null" not in lib.fa_last_error(), sizes
+    for sizes in ((64, 16, 65536, 77), (64, 64, 1 << 20, 8), (1, 1, 1 << 31, 8), (1, 1, 1, 1 << 30)):
+        assert call(*sizes) == -1 and b"null" in lib.fa_last_error(), sizes
+
+
 def test_header_is_plain_c(tmp_path):
     """include/flash_attn_gfx950.h must be usable from C (the boundary a cgo / JNI / ctypes binding sees): it compiles as
     C99 with warnings as errors, and every declared entry point can be named."""
