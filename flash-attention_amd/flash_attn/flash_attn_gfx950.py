@@ -12,6 +12,7 @@ import ctypes
 import functools
 import math
 import os
+import struct
 import threading
 
 import torch
@@ -271,8 +272,32 @@ class DrawnPhilox:
     of that call to use again."""
     __slots__ = ("state",)
 
-    def __init__(self):
+    def __init__(self, saved=None):
         self.state = None
+        if saved is not None:
+            seed, offset = saved.tolist()
+            self.state = (seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF)
+
+    def saved(self):
+        """(seed, offset) as a host tensor"""
+        return torch.frombuffer(bytearray(struct.pack("=QQ", *self.state)), dtype=torch.int64)
+
+
+# Whether hooks see what an autograd function saves (a recomputed forward replaces all of it then): a private accessor, asked because
+# saving the dropout state as tensors costs a step 4 us; where it is gone, the state is always saved.
+_saved_tensor_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
+
+
+def pack_dropout(keep_words, philox):
+    """What a forward with dropout leaves its backward, as (tensors to save, object to keep): everything in one of the two."""
+    if philox is None or (_saved_tensor_hooks is not None and _saved_tensor_hooks(True) is None):
+        return (None, None), (keep_words, philox)
+    return (keep_words, philox.saved()), None
+
+
+def unpack_dropout(saved, kept):
+    """(keep_words, philox) from the two of pack_dropout()"""
+    return kept if kept is not None else (saved[0], DrawnPhilox(saved[1]))
 
 
 def _philox_state(device, p_dropout, gen):

@@ -90,12 +90,11 @@ def _forward(ctx, packing, tensors, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
     out, softmax_lse, S_dmask = _flash_attn_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                                                     dropout_p, softmax_scale, causal, return_softmax, alibi_slopes,
                                                     keep_words, bias_t, rotary, q_rot, philox)
-    ctx.save_for_backward(*tensors, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot)
-    ctx.philox = philox
+    dropout_saved, ctx.dropout_kept = _backend.pack_dropout(keep_words, philox)
+    ctx.save_for_backward(*tensors, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot, *dropout_saved)
     ctx.rotary = rotary  # constant tables, not differentiated
     ctx.bias_shape = tuple(attn_bias.shape) if attn_bias is not None else None
     ctx.bias_needs_grad = attn_bias is not None and attn_bias.requires_grad
-    ctx.keep_words = keep_words
     ctx.alibi_slopes = alibi_slopes  # fixed slopes, not differentiated
     ctx.packing = packing
     ctx.n_in = len(tensors)
@@ -109,7 +108,8 @@ def _forward(ctx, packing, tensors, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
 def _backward(ctx, dout):
     saved = ctx.saved_tensors
     tensors = saved[:ctx.n_in]
-    out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot = saved[ctx.n_in:]
+    out, softmax_lse, cu_seqlens_q, cu_seqlens_k, bias_t, rot, *dropout_saved = saved[ctx.n_in:]
+    keep_words, philox = _backend.unpack_dropout(dropout_saved, ctx.dropout_kept)
     q, k, v = _split(ctx.packing, tensors)
     if rot is not None:  # the kernels take the rotated q and k and turn dq and dk back themselves
         q, k = rot[:, 0], rot[:, 1]
@@ -122,7 +122,7 @@ def _backward(ctx, dout):
         dbias = new_bias_grad(q, cu_seqlens_q.numel() - 1, ctx.max_seqlen_q, ctx.max_seqlen_k, cleared=written is None)
     _flash_attn_backward(dout.contiguous(), q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k,
                          ctx.max_seqlen_q, ctx.max_seqlen_k, ctx.dropout_p, ctx.softmax_scale, ctx.causal,
-                         ctx.alibi_slopes, ctx.keep_words, bias_t, dbias, ctx.rotary, ctx.philox)
+                         ctx.alibi_slopes, keep_words, bias_t, dbias, ctx.rotary, philox)
     ctx.dbias = None
     if dbias is not None:
         ctx.dbias = bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_seqlen_q, ctx.max_seqlen_k, written)

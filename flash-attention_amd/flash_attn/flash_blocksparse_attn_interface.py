@@ -93,8 +93,8 @@ def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale
     context, softmax_lse, S_dmask = _flash_blocksparse_attn_forward(
         qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes, bias_t,
         philox)
-    ctx.save_for_backward(qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t)
-    ctx.philox = philox
+    dropout_saved, ctx.dropout_kept = _backend.pack_dropout(None, philox)
+    ctx.save_for_backward(qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t, *dropout_saved)
     ctx.dropout_p = dropout_p
     ctx.max_s = max_s
     ctx.softmax_scale = softmax_scale
@@ -107,13 +107,14 @@ def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale
 
 def _bwd_common(ctx, dout):
     """(dqkv, gradient of attn_bias or None)"""
-    qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t = ctx.saved_tensors
+    qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t, *dropout_saved = ctx.saved_tensors
+    _, philox = _backend.unpack_dropout(dropout_saved, ctx.dropout_kept)
     dbias = None
     if ctx.bias_needs_grad:
         dbias = new_bias_grad(qkv[:, 0], cu_seqlens.numel() - 1, ctx.max_s, ctx.max_s)
     dqkv = _flash_blocksparse_attn_backward(dout, qkv, context, None, softmax_lse, cu_seqlens, blockmask,
                                             ctx.dropout_p, ctx.max_s, ctx.softmax_scale, ctx.causal, ctx.alibi_slopes,
-                                            bias_t, dbias, ctx.philox)
+                                            bias_t, dbias, philox)
     return dqkv, (bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_s, ctx.max_s) if dbias is not None else None)
 
 

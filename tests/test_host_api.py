@@ -628,3 +628,28 @@ def test_prepare_attn_bias_layout_rules():
                      (torch.zeros(1, 3, 40, 48), "dtype and device")):                  # fp32 for fp16 inputs
         with pytest.raises(RuntimeError, match=msg):
             be.prepare_attn_bias(bad, q, 2, 3, 40, 48)
+
+
+def test_drawn_philox_state_survives_as_a_saved_tensor():
+    from flash_attn.flash_attn_gfx950 import DrawnPhilox
+    for state in ((0, 0), (5, 4), (1 << 63, 8), ((1 << 64) - 1, (1 << 63) + 12)):
+        d = DrawnPhilox()
+        d.state = state
+        t = d.saved()
+        assert t.device.type == "cpu" and t.dtype == torch.int64 and DrawnPhilox(t.clone()).state == state
+
+
+def test_dropout_state_is_saved_as_tensors_where_hooks_see_them(monkeypatch):
+    from flash_attn import flash_attn_gfx950 as be
+    d, words = be.DrawnPhilox(), torch.zeros(4, dtype=torch.uint8)
+    d.state = (7, 8)
+    saved, kept = be.pack_dropout(words, d)
+    assert be.unpack_dropout(saved, kept) == (words, d)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert be.pack_dropout(None, None) == ((None, None), (None, None))  # (no dropout: nothing to save)
+        saved, kept = be.pack_dropout(words, d)
+    assert kept is None and saved[0] is words
+    got = be.unpack_dropout(saved, kept)
+    assert got[0] is words and got[1].state == (7, 8)
+    monkeypatch.setattr(be, "_saved_tensor_hooks", None)
+    assert be.pack_dropout(words, d)[1] is None

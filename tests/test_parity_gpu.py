@@ -1478,6 +1478,39 @@ def test_native_calls_hand_back_what_the_binding_refuses(binding_only):
         assert said[0] == said[1] and said[0]
 
 
+@pytest.mark.parametrize("kind", ["dense", "redrawn", "block"])
+def test_recomputed_forward_replaces_the_dropout_of_the_first(kind, monkeypatch):
+    """Activation checkpointing that does not keep the generator's state draws another mask when it recomputes the forward: the backward then
+    takes everything - output, row statistics, decisions - from the recomputed one, and is that of a step drawn there."""
+    from torch.utils.checkpoint import checkpoint
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.flash_attn_interface import flash_attn_unpadded_qkvpacked_func
+    from flash_attn.flash_blocksparse_attn_interface import convert_blockmask, flash_blocksparse_attn_func
+    if kind == "redrawn":
+        monkeypatch.setattr(be, "KEEP_WORDS_MAX_BYTES", 0)
+    lens, H, D = [200, 77], 2, 64
+    cu = _cu(lens)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    qkv = torch.randn(sum(lens), 3, H, D, device="cuda", generator=g).half().requires_grad_()
+    do = torch.randn(sum(lens), H, D, device="cuda", generator=g).half()
+    layout = convert_blockmask(torch.ones(16, 1, device="cuda").bool(), causal=False)
+
+    def f(x):
+        if kind == "block":
+            return flash_blocksparse_attn_func(x, cu, layout, 0.3, 256, convert_mask=False)
+        return flash_attn_unpadded_qkvpacked_func(x, cu, 200, 0.3)
+
+    torch.cuda.manual_seed(21)
+    want = torch.autograd.grad(f(qkv), qkv, do)[0]
+    torch.cuda.manual_seed(20)
+    first = torch.autograd.grad(f(qkv), qkv, do, retain_graph=True)[0]
+    torch.cuda.manual_seed(20)
+    out = checkpoint(f, qkv, use_reentrant=False, preserve_rng_state=False)
+    torch.cuda.manual_seed(21)
+    got = torch.autograd.grad(out, qkv, do)[0]
+    assert torch.equal(got, want) and not torch.equal(got, first)
+
+
 def _padding_masks(B, S, seed):
     """(B, S) bool masks: right padding, left padding, holes, one run in the middle; entry 0 full, entry 1 (if there is one) without tokens."""
     g = torch.Generator().manual_seed(seed)
