@@ -291,6 +291,8 @@ inline bool longest_first_launch(bool causal, bool sparse, int grid, int B) {
 int launch_policy();
 // About the workgroups of 128 query rows that find any: a sequence of n has n / 128 and half a tile more on average
 inline int64_t live_row_tiles(int nheads, int total_q, int batch) { return (int64_t)nheads * (total_q + (int64_t)64 * batch) / 128; }
+// Pairs go to the 8 XCDs in turn (map_tile): of `live` workgroups, eight times what the fullest XCD gets (12 pairs load like 16)
+inline int64_t fullest_xcd(int64_t live, int BH) { return live * ((BH + 7) / 8 * 8) / BH; }
 constexpr int kSmallLaunchFwd = 0, kSmallLaunchDq = 1;
 inline bool small_launch(int kernel, int BH, int max_s, bool causal, bool dropout) {
   const int policy = launch_policy() & 3;
@@ -312,15 +314,19 @@ inline bool small_launch_causal(int64_t live, int BH, int max_s, int64_t total_q
 }
 
 // The forward's half-size tiles at head dim 128 (64-key tiles, 64 KB of LDS: two workgroups a compute unit), for launches whose time is one
-// workgroup's walk over the keys.  By the workgroups that find query rows, about nheads * (tokens / 128 + batch / 2), and the longest sequence;
-// us of full-size / half-size tiles, bf16.  Causal: 8 heads x 2300 53.9 / 35.8, 16 x 3100 (400 workgroups) 72.7 / 58.0, 4 x 12 x 360 .. 1200 (312)
-// 32.7 / 24.8, 4 x 16 x 1200 (640) 40.7 / 43.5; short sequences fill the chip with fewer: 4 x 16 x 300 (192) 11.9 / 11.0, 16 x 12 x 52 .. 130 (204)
-// 8.7 / 9.3.  No mask: 8 x 1700 39.3 / 28.1, 8 x 2300 (144) 50.1 / 45.1, 4 x 12 x 500 (192) 16.3 / 17.2, 16 x 2300 (288) 72.6 / 75.0.
-inline bool small_launch_d128(int64_t live, int max_s, bool causal) {
+// workgroup's walk over the keys.  By the workgroups that find query rows (live_row_tiles), on the fullest XCD (x below), and the longest
+// sequence: the longer the walk, the more of them may share the chip.  us of full-size / half-size tiles, fp16 and bf16.  Causal: 8 x 2300 53.9
+// / 35.8, 16 x 3100 (x = 400) 72.7 / 58.0, 4 x 12 x 360 .. 1200 (312) 32.7 / 24.8, 4 x 16 x 1200 (640) 40.7 / 43.5; 8 x 12 x 386 (317) 15.7 / 17.0, 10 x 8 x 405
+// (293) 15.5 / 15.9, 5 x 16 x 518 (363) 18.4 / 18.9; 8 x 16 x 281 (345) 12.8 / 15.7, 10 x 12 x 250 .. 337 (339) 14.9 / 17.4, 10 x 12 x 190 .. 287 (283) 12.0 /
+// 13.5, 4 x 16 x 300 (182) 11.9 / 11.0, 6 x 16 x 182 (184) 9.1 / 9.3, 16 x 12 x 52 .. 130 (204) 8.7 / 9.3.  No mask: 8 x 1700 39.3 / 28.1, 8 x 2300
+// (148) 50.1 / 45.1, 3 x 16 x 286 (131) 10.8 / 10.0, 6 x 8 x 323 (145) 12.4 / 13.9, 4 x 8 x 531 (148) 16.2 / 17.1, 4 x 12 x 500 (192) 16.3 / 17.2.
+inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
   const int policy = launch_policy() & 3;
   if (policy != 0) return policy == 2;
-  if (causal) return max_s > 128 && live <= (max_s > 256 ? 384 : 192);
-  return max_s > 192 && live <= 150;
+  const int64_t x = fullest_xcd(live, BH);
+  if (!causal) return max_s > 192 && x <= (max_s > 640 ? 150 : 140);
+  if (max_s <= 256) return max_s > 128 && x <= (max_s > 192 ? 192 : 125);
+  return live <= 384 && (max_s > 1100 || x <= (max_s > 768 ? 430 : max_s > 512 ? 360 : max_s > 384 ? 310 : 270));
 }
 
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves

@@ -653,3 +653,34 @@ def test_dropout_state_is_saved_as_tensors_where_hooks_see_them(monkeypatch):
     assert got[0] is words and got[1].state == (7, 8)
     monkeypatch.setattr(be, "_saved_tensor_hooks", None)
     assert be.pack_dropout(words, d)[1] is None
+
+
+def _launch_rules(tmp_path, expressions):
+    """Values of expressions over the launch rules of fa_params.h under the default policy (host code; nothing is launched)"""
+    import subprocess
+    import build as fa_build
+    src, exe = tmp_path / "rules.hip", tmp_path / "rules"
+    src.write_text('#include <cstdio>\n#include "fa_params.h"\nnamespace fa { int launch_policy() { return 0; } }\nusing namespace fa;\n'
+                   'int main() {\n' + "".join('  std::printf("%%d\\n", (int)(%s));\n' % e for e in expressions) + "}\n")
+    cmd = [fa_build.HIPCC, "--offload-host-only", "-std=c++17", "-I", fa_build.CSRC, str(src), "-o", str(exe)]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout[-2000:]
+    return [int(x) for x in subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, check=True).stdout.split()]
+
+
+def _spread(n, frac, batch):
+    """tokens of a batch whose lengths are spread evenly between frac * n and n"""
+    return sum(int(n - (n - frac * n) * i // max(1, batch - 1)) for i in range(batch))
+
+
+def test_d128_forward_tiles_follow_the_measurements(tmp_path):
+    """head dim 128: full- or half-size tiles by what was faster, us full / half, where the difference is more than the measurement's noise"""
+    cases = [  # batch, heads, longest, shortest / longest, causal, half-size?
+        (8, 16, 281, 1.0, 1, 0), (16, 8, 286, 1.0, 1, 0), (12, 12, 305, 0.55, 1, 0), (10, 12, 337, 0.77, 1, 0), (10, 12, 287, 0.66, 1, 0),  # 12.8 / 15.7 ..
+        (8, 12, 386, 0.86, 1, 0), (12, 8, 409, 1.0, 1, 0), (16, 8, 158, 0.53, 1, 0),  # 15.7 / 17.0, 16.0 / 18.0, 8.2 / 8.7
+        (6, 8, 323, 1.0, 0, 0), (3, 16, 325, 1.0, 0, 0), (4, 8, 531, 1.0, 0, 0),  # 12.4 / 13.9, 12.0 / 13.4, 16.1 / 17.1
+        (1, 8, 2300, 1.0, 1, 1), (4, 12, 1200, 0.3, 1, 1), (4, 16, 300, 1.0, 1, 1), (1, 16, 3000, 1.0, 1, 1),  # 53.9 / 35.8, 32.7 / 24.8, 11.9 / 11.0, 69.8 / 51.4
+        (1, 8, 1700, 1.0, 0, 1), (3, 16, 286, 1.0, 0, 1)]  # 39.3 / 28.1, 10.8 / 10.0
+    got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, c)
+                                   for b, h, n, f, c, _ in cases])
+    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
