@@ -330,19 +330,40 @@ inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
 }
 
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves
-// idle, one launch less): at head dim 64, dense, no score bias, no rotation, no key split, dropout off or read from the keep words.  By the
-// workgroups of 128 query rows that find any (live_row_tiles) and the longest sequence; us in two launches / merged.  Causal: 2 x 8 x 65 %
-// of 842 (76) 41.2 / 26.3, 12 x 1812 (175) 75.3 / 50.1, 3 x 12 x 78 % of 2283 (521) 106.8 / 79.2, 4 x 8 x 2383 (611) 136.5 / 124.0, 12 x 16 x 386 (675) 39.2 /
-// 42.0; with dropout 6 x 16 x 69 % of 1258 (701) 82.9 / 71.9.  No mask: 3 x 8 x 846 (113) 39.8 / 25.7, 3 x 16 x 641 (264) 46.5 / 35.4, 8 x 12 x 77 % of 731 (469)
-// 53.8 / 48.8, 16 x 16 x 204 (536) 30.6 / 30.5, 6 x 12 x 1631 (563) 105.6 / 110.6; with dropout 12 x 12 x 528 (666) 79.7 / 73.8.  Up to 128 tokens: causal
-// 16 x 12 x 97 (194) 16.4 / 10.6, 32 x 16 x 76 (528) 22.5 / 23.1; no mask 12 x 16 x 45 (163) 12.7 / 9.3, 16 x 12 x 70 (201) 15.7 / 16.4.
+// idle, one launch less; dQ at two waves per SIMD instead of three): at head dim 64, dense, no score bias, no rotation, no key split, dropout
+// off or read from the keep words.  By the workgroups of 128 query rows that find any (live_row_tiles, `live`), the longest sequence n and, where
+// the lengths are about equal, the launched workgroups on the fullest XCD (L): two launches are the better plan where L fills one or two rounds
+// of the chip's 256 compute units, the more so the longer the walk; one launch where it leaves the last round half empty.  us in two
+// launches / merged.
+// Causal: 2 x 8 x 65 % of 842 (live 76) 41.2 / 26.3, 12 x 1812 (175) 75.3 / 50.1, 3 x 12 x 78 % of 2283 (521) 106.8 / 79.2, 4 x 8 x 2383 (611) 136.5 / 124.0;
+// 27 x 8 x 273 (L 648) 30.5 / 33.4, 15 x 8 x 585 (600) 45.1 / 46.6, 16 x 16 x 219 (512) 26.6 / 27.6, 12 x 16 x 386 (live 675) 39.2 / 42.0; with
+// dropout 6 x 16 x 69 % of 1258 (701) 82.9 / 71.9, 16 x 8 x 602 (L 640) 48.1 / 51.1.
+// No mask: 3 x 8 x 846 (live 113) 39.8 / 25.7, 3 x 16 x 641 (264) 46.5 / 35.4, 8 x 12 x 77 % of 731 (469) 53.8 / 48.8; 7 x 16 x 239 (L 224) 20.4 / 21.6, 5 x 16 x
+// 277 (240) 23.2 / 24.1, 11 x 8 x 276 (264) 29.0 / 23.1; 8 x 16 x 392 (512) 36.7 / 38.5, 16 x 3616 (464) 195 / 219, 8 x 7464 (472) 410 / 454, 12 x
+// 3768 (480) 213 / 235, 3 x 16 x 1203 (480) 77 / 84, 8 x 6181 (392) 298 / 307, 12 x 4191 (528) 295 / 277; with dropout 7 x 16 x 380 .. 711 (533) 64.6 /
+// 59.8, 4 x 8 x 2013 (L 512) 142 / 150.
+// Up to 128 tokens: causal 16 x 12 x 97 (194) 16.4 / 10.6, 33 x 12 x 115 (553) 22.7 / 21.3, 32 x 16 x 76 (528) 22.5 / 23.1; no mask 12 x 16 x 45 (163) 12.7 /
+// 9.3, 16 x 12 x 70 (201) 15.7 / 16.4; with dropout 33 x 12 x 73 (423) 23.5 / 22.1, 17 x 16 x 123 (397) 22.8 / 19.4, 21 x 12 x 81 (278) 17.2 / 19.0.
 // (policy 0x10, the two-kernel plan, runs the same tiles in two launches: same bits)
 inline bool merged_backward_shape(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words,
                                   bool sparse, bool bias, bool rotary, int n_splits) {
   if (head_dim != 64 || sparse || bias || rotary || n_splits > 1 || (dropout && !keep_words)) return false;
   if ((launch_policy() & 3) != 0 || max_sk > 2 * max_sq) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
-  if (max_sq <= 128) return live <= (causal ? 500 : 190);
-  return live <= (causal ? (dropout ? 700 : 620) : (dropout ? 670 : 480));
+  const int64_t L = fullest_xcd((int64_t)BH * ((max_sq + 127) / 128), BH);
+  if (max_sq <= 128) {
+    if (causal) return live <= (max_sq <= 64 || dropout ? 500 : max_sq <= 96 ? 435 : 600) || (dropout && L <= 512);
+    return live <= 190 || (dropout && (max_sq <= 64 || BH > 256) && L <= 512);
+  }
+  if (live > (causal ? (dropout ? 700 : 620) : (dropout ? 670 : 480))) return false;
+  if ((128 * live - 64 * BH) * 10 <= (int64_t)9 * BH * max_sq) return true;  // lengths differ: at most 0.9 of batch x longest are tokens
+  if (causal) {
+    if (max_sq <= 192 || max_sq > 800) return true;
+    if (max_sq <= 256) return dropout || L <= 448;
+    return L <= (dropout ? 608 : max_sq <= 384 ? 544 : 576);
+  }
+  if (max_sq <= 400 && L > 192 && L <= 256) return L < 232 && (max_sq <= 192 || max_sq > 256);
+  if (L <= 512) return max_sq <= 384 || L <= (max_sq > 900 && !dropout ? 392 : 448);
+  return max_sq <= 384 || L <= (max_sq > 900 && !dropout ? 600 : 640);
 }
 inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words,
                                    bool sparse, bool bias, bool rotary, int n_splits) {
@@ -350,7 +371,9 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
          merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, sparse, bias, rotary, n_splits);
 }
 
-// The dQ kernel's half-size tiles in a launch of its own, dropout off (with dropout: small_launch): causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 /
+// The dQ kernel's half-size tiles in a launch of its own, dropout off (with dropout: small_launch; at head dim 64 with keep words only where
+// merged_backward_shape takes them, half-size tiles in two launches are the slowest plan there: 33 x 12 x 73 22.1 merged, 23.5 full-size, 29.1):
+// causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 /
 // 25.1 with the dK/dV kernel, 3 x 16 x 70 % of 1785 (494) 59.5 / 53.0, 12 x 16 x 336 (551) 23.7 / 23.3; d = 64 8 x 12 x 460 (393) 34.0 / 32.6, 12 x 8 x 609
 // (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
 // chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 3 x 16 x 1495 (292) 110.3 / 101.6, short sequences cross sooner: 6 x 16 x 183
@@ -358,8 +381,9 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
 inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words, bool rotary,
                             int n_splits) {
   if (merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, false, false, rotary, n_splits)) return true;
-  const bool swept = (launch_policy() & 3) == 0 && !dropout && max_sk <= 2 * max_sq;
+  const bool ruled = (launch_policy() & 3) == 0 && max_sk <= 2 * max_sq, swept = ruled && !dropout;
   if (head_dim == 128 && (launch_policy() & 3) == 0) return swept && max_sq > 128 && live <= (causal ? (max_sq > 450 ? 300 : 150) : 140);
+  if (ruled && head_dim == 64 && dropout && keep_words && !rotary) return false;
   if (!swept) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
   return max_sq > 128 && live <= (causal ? (head_dim == 64 ? 400 : 500) : 130);
 }

@@ -684,3 +684,26 @@ def test_d128_forward_tiles_follow_the_measurements(tmp_path):
     got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, c)
                                    for b, h, n, f, c, _ in cases])
     assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+
+
+def _rule_case(b, h, n, f):
+    return "live_row_tiles(%d, %d, %d), %d, %d, %d" % (h, _spread(n, f, b), b, b * h, n, n)
+
+
+def test_d64_backward_in_one_launch_where_measured(tmp_path):
+    """head dim 64: dQ and dK/dV in one launch or two by what was faster, us in two (full-size) / in one; where dropout is read from keep words, two
+    launches run the full-size tiles"""
+    cases = [  # batch, heads, longest, shortest / longest, causal, dropout, one launch?
+        (1, 16, 3616, 1.0, 0, 0, 0), (1, 8, 7464, 1.0, 0, 0, 0), (1, 12, 3768, 1.0, 0, 0, 0), (3, 16, 1203, 1.0, 0, 0, 0),  # 195 / 219 .. 77 / 84
+        (7, 16, 239, 1.0, 0, 0, 0), (5, 16, 277, 1.0, 0, 0, 0), (5, 16, 667, 1.0, 0, 0, 0), (8, 16, 392, 1.0, 0, 0, 0),  # 20.4 / 21.6 .. 36.7 / 38.5
+        (27, 8, 273, 1.0, 1, 0, 0), (15, 8, 585, 1.0, 1, 0, 0), (16, 16, 219, 1.0, 1, 0, 0), (16, 8, 602, 1.0, 1, 1, 0),  # 30.5 / 33.4 .. 48.1 / 51.1
+        (4, 8, 2013, 1.0, 0, 1, 0), (21, 12, 81, 0.905, 0, 1, 0), (32, 16, 76, 1.0, 1, 0, 0), (16, 12, 70, 1.0, 0, 0, 0),  # 142 / 150, 17.2 / 19.0
+        (33, 12, 73, 1.0, 0, 1, 1), (17, 16, 123, 1.0, 0, 1, 1), (36, 12, 108, 1.0, 0, 1, 1), (27, 16, 110, 1.0, 1, 1, 1),  # 23.5 / 22.1, 22.8 / 19.4
+        (33, 12, 115, 1.0, 1, 0, 1), (16, 12, 97, 1.0, 1, 0, 1), (12, 16, 45, 1.0, 0, 0, 1),  # 22.7 / 21.3, 16.4 / 10.6, 12.7 / 9.3
+        (1, 12, 1812, 1.0, 1, 0, 1), (4, 8, 2383, 1.0, 1, 0, 1), (3, 8, 846, 1.0, 0, 0, 1), (3, 16, 641, 1.0, 0, 0, 1),  # 75 / 50, 136 / 124, 40 / 26
+        (11, 8, 276, 1.0, 0, 0, 1), (7, 16, 711, 0.535, 0, 1, 1), (8, 12, 731, 0.54, 0, 0, 1), (2, 8, 3441, 0.34, 0, 0, 1)]  # 29.0 / 23.1, 64.6 / 59.8
+    one = _launch_rules(tmp_path, ["merged_backward_shape(64, %s, %d, %d, %d, 0, 0, 0, 1)" % (_rule_case(*c[:4]), c[4], c[5], c[5]) for c in cases])
+    assert one == [c[-1] for c in cases], [c for c, g in zip(cases, one) if g != c[-1]]
+    words = [c for c in cases if c[5]]
+    half = _launch_rules(tmp_path, ["small_launch_dq(64, %s, %d, 1, 1, 0, 1)" % (_rule_case(*c[:4]), c[4]) for c in words])
+    assert half == [c[-1] for c in words], [c for c, g in zip(words, half) if g != c[-1]]
