@@ -376,8 +376,8 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
 // causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 / 25.1 with the dK/dV kernel, 3 x 16 x 70 % of 1785 (494) 59.5 / 53.0, 12 x 16 x 336 (551) 23.7 / 23.3;
 // d = 16 2 x 8 x 3964 (503) 96.9 / 89.0; up to 128 tokens small_launch, 17 x 16 x 115 15.8 / 15.1; d = 64 8 x 12 x 460 (393) 34.0 / 32.6, 12 x 8 x 609
 // (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
-// chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 3 x 16 x 1495 (292) 110.3 / 101.6, short sequences cross sooner: 6 x 16 x 183
-// (169) 25.6 / 27.1, 6 x 16 x 509 (345) 51.5 / 54.7; no mask, on the fullest XCD, 2 x 8 x 1112 (133) 79.7 / 75.9, 3 x 16 x 789 (256) 70.7 / 75.7, 7 x 12 x 135
+// chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 2 x 12 x 1500 (293) 110.3 / 101.0, short sequences cross sooner: 6 x 16 x 183
+// (169) 25.6 / 27.1, 6 x 16 x 509 (345) 51.5 / 54.7; no mask, on the fullest XCD, 2 x 8 x 928 (124) 67.6 / 60.5, 3 x 16 x 789 (256) 70.7 / 75.7, 7 x 12 x 135
 // (136) 25.3 / 27.7, 9 x 8 x 80 .. 244 (127) 29.6 / 30.3.
 inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words, bool rotary,
                             int n_splits) {
