@@ -307,10 +307,16 @@ inline bool small_launch(int kernel, int BH, int max_s, bool causal, bool dropou
 // the longest sequences decide), below 1000.  us of full-size / half-size tiles, fp16 and bf16, d = 64 (d = 16 and 32 alike): 3 x 8 x 2700 ..
 // 3479 (528 workgroups, 672 launched) 55.6 / 44.1, 6 x 12 x 260 .. 1631 (564, 936) 31.4 / 24.9, 3 x 12 x 1823 (540) 33.6 / 29.5, 16 x 8 x 480 .. 1200 (896,
 // 1280) 34.9 / 26.8, 3 x 12 x 1400 .. 2829 (624) 49.7 / 40.8; equal lengths 4 x 12 x 1700 (672) 32.3 / 33.0, 4 x 12 x 2300 (864) 47.8 / 51.2; uneven beyond
-// 3 x 16 x 2100 .. 3348 (1056) 69.5 / 69.8, 16 x 16 x 1262 (2112) 63.6 / 69.9.
-inline bool small_launch_causal(int64_t live, int BH, int max_s, int64_t total_q, int batch) {
+// 3 x 16 x 2100 .. 3348 (1056) 69.5 / 69.8, 16 x 16 x 1262 (2112) 63.6 / 69.9.  At d = 64 shorter walks cross sooner (on the fullest XCD): 16 x 12 x 329
+// (589) 11.7 / 12.9, 11 x 16 x 355 (576) 11.5 / 12.4, 8 x 16 x 527 (591) 14.1 / 15.3, 7 x 12 x 838 (619) 19.7 / 21.1; uneven 21 x 12 x 290 (602) 11.4 / 12.9.
+inline bool small_launch_causal(int head_dim, int64_t live, int BH, int max_s, int64_t total_q, int batch) {
   if ((launch_policy() & 3) != 0 || max_s <= 256) return small_launch(kSmallLaunchFwd, BH, max_s, true, false);
-  return live < 600 || (live < 1000 && total_q * 20 <= (int64_t)17 * batch * max_s);
+  const bool uneven = total_q * 20 <= (int64_t)17 * batch * max_s;
+  if (head_dim == 64 && max_s <= 1000 && !(uneven && max_s > 400)) {
+    const int64_t x = fullest_xcd(live, BH);
+    return live < 600 && x <= (uneven || max_s > 640 ? 580 : max_s > 400 ? 560 : max_s > 320 ? 540 : 520);
+  }
+  return live < 600 || (live < 1000 && uneven);
 }
 
 // The forward's half-size tiles at head dim 128 (64-key tiles, 64 KB of LDS: two workgroups a compute unit), for launches whose time is one

@@ -717,3 +717,15 @@ def test_dq_tiles_follow_the_measurements(tmp_path):
         (128, 2, 8, 928, 1.0, 0, 1), (128, 1, 8, 974, 1.0, 1, 1), (128, 2, 12, 1500, 1.0, 1, 1), (32, 2, 16, 707, 0.46, 1, 1)]  # 67.6 / 60.5, 73.4 / 64.2
     half = _launch_rules(tmp_path, ["small_launch_dq(%d, %s, %d, 0, 0, 0, 1)" % (c[0], _rule_case(*c[1:5]), c[5]) for c in cases])
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
+
+
+def test_causal_forward_tiles_follow_the_measurements(tmp_path):
+    """head dim 16 to 64, causal: full- or half-size tiles by what was faster, us full / half"""
+    cases = [  # head dim, batch, heads, longest, shortest / longest, half-size?
+        (64, 16, 12, 329, 1.0, 0), (64, 11, 16, 355, 1.0, 0), (64, 8, 16, 527, 1.0, 0), (64, 7, 12, 838, 1.0, 0),  # 11.7 / 12.9 .. 19.7 / 21.1
+        (64, 21, 12, 290, 0.64, 0), (64, 13, 16, 266, 1.0, 0), (64, 4, 12, 2300, 1.0, 0), (64, 4, 12, 1700, 1.0, 0),  # 11.4 / 12.9, 10.9 / 11.9
+        (64, 20, 8, 364, 1.0, 1), (64, 3, 12, 1823, 1.0, 1), (64, 3, 12, 2829, 0.49, 1), (64, 6, 12, 1631, 0.16, 1),  # 11.2 / 10.5, 33.6 / 29.5
+        (64, 16, 8, 1200, 0.4, 1), (32, 24, 8, 330, 0.9, 1), (16, 21, 8, 317, 1.0, 1)]  # 34.9 / 26.8, 9.3 / 9.0, 8.5 / 7.4
+    half = _launch_rules(tmp_path, ["small_launch_causal(%d, live_row_tiles(%d, %d, %d), %d, %d, %d, %d)" % (
+        d, h, _spread(n, f, b), b, b * h, n, _spread(n, f, b), b) for d, b, h, n, f, _ in cases])
+    assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
