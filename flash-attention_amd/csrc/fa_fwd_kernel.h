@@ -98,9 +98,11 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   // kKeyWords: behind everything else, for the staged and the next tile, the key words of its BN / 2 Philox counters (fa_common.h).  us of the
   // forward with them / with whole outputs drawn, p = 0.1: 64 x 16 heads x 1004 .. 1023, d = 64, 535 / 551; 4 x 12 x 4096 313 / 319; 8 x 16 x
   // 1000, d = 32, 60.6 / 63.0.  Not at d = 128 (8 x 12 x 2048: 316 / 301), nor in the half-size tiles (causal, d = 64, 3 x 12 x 1200 24.8 / 23.4, 2 x 16 x
-  // 1600 30.4 / 28.5; d = 32, 16 x 2600 32.1 / 30.0), nor where they cost a wave per SIMD: over a block layout at d = 32.
+  // 1600 30.4 / 28.5; d = 32, 16 x 2600 32.1 / 30.0), nor where they cost a wave per SIMD: over a block layout at d = 32, nor under a causal mask
+  // where keep words are left (d = 64, 68 x 8 x 273 32.8 / 31.4, 50 x 12 x 1006 185.7 / 181.7, 17 x 16 x 103 11.0 / 10.5; between 0.96 and 1.05, 1.00 in the
+  // middle; without the words 0.97 to 0.99).
   // (Round keys stepped by the scalar unit in place of kept ones, which are parked in vector lanes: 550.)
-  constexpr bool kKeyWords = kDropout && !kSparse && kBias == 0 && KS == 1 && (D == 32 || D == 64);
+  constexpr bool kKeyWords = kDropout && !kSparse && kBias == 0 && KS == 1 && !(kCausal && kWords) && (D == 32 || D == 64);
   constexpr int kKeyWordBytes = BN / 2 * 16, kKeyWordOff = Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : 0);
   constexpr int kRowSlotBytes = 2 * 64 * 4;  // kRows: behind the tiles, per wave (see fetch_rows below)
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kTensorBias ? 4 * kBiasWaveBytes : kRows ? 4 * kRowSlotBytes : 0) +

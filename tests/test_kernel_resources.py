@@ -165,8 +165,8 @@ def test_forward_and_decode_variants_keep_their_waves_per_simd():
 
 @pytest.mark.timeout(600)
 def test_key_words_of_the_dropout_forward_only_where_they_pay():
-    """The Philox key words kept in LDS (1 KB of LDS, dense dropout forward): in the full-size tiles of d = 32 and 64, not in the half-size ones,
-    which they slow down; (waves per SIMD at least) of the variants that have them, and no vector register spilled."""
+    """The Philox key words kept in LDS (1 KB of LDS, dense dropout forward): in the full-size tiles of d = 32 and 64, not in the half-size ones nor
+    where a causal mask's keep words are left, which they slow down; (waves per SIMD at least) of the variants, and no vector register spilled."""
     with ThreadPoolExecutor(2) as ex:
         d32, d64 = ex.map(_resources, ("fa_fwd_d32.hip", "fa_fwd_d64.hip"))
     for dt in ("IDF16_", "IDF16b"):
@@ -177,5 +177,6 @@ def test_key_words_of_the_dropout_forward_only_where_they_pay():
                     full = _pick(res, name, causal + "Lb1ELb0ELi0ELi1E" + words + "EEv")
                     half = _pick(res, name, causal + "Lb1ELb0ELi0ELi2E" + words + "EEv")
                     tiles = 64 * d * 2 * 4  # two K and two V tiles of 64 keys
-                    assert full["Occupancy"] >= waves and full["VGPRs Spill"] == 0 and full["LDS Size"] == tiles + 1024, (dt, d, causal, words, full)
+                    key_words = 0 if causal == "Lb1E" and words == "Lb1E" else 1024
+                    assert full["Occupancy"] >= waves and full["VGPRs Spill"] == 0 and full["LDS Size"] == tiles + key_words, (dt, d, causal, words, full)
                     assert half["Occupancy"] >= 4 and half["VGPRs Spill"] == 0 and half["LDS Size"] == tiles, (dt, d, causal, words, half)
