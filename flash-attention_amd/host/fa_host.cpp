@@ -73,7 +73,15 @@ bool as_double(PyObject* o, double* v) {
   if (PyFloat_Check(o)) *v = PyFloat_AS_DOUBLE(o);
   else if (PyLong_Check(o)) *v = PyLong_AsDouble(o);
   else return false;
-  return !PyErr_Occurred();
+  if (!PyErr_Occurred()) return true;
+  PyErr_Clear();  // (an int beyond a double: the binding meets it again)
+  return false;
+}
+bool as_flag(PyObject* o, int32_t* v) {
+  const int r = PyObject_IsTrue(o);
+  if (r < 0) PyErr_Clear();  // (something without a truth value, as above)
+  *v = r > 0;
+  return r >= 0;
 }
 inline void* ptr(const at::Tensor& t) { return t.data_ptr(); }
 
@@ -154,9 +162,11 @@ PyObject* fwd(PyObject* const* a, Py_ssize_t n) {
   const at::Tensor *alibi = tensor(a[12], ok), *words = tensor(a[13], ok), *bias = tensor(a[14], ok), *cos = tensor(a[15], ok), *sin = tensor(a[16], ok);
   const at::Tensor *q_rot = tensor(a[17], ok), *mask = tensor(a[18], ok), *order = tensor(a[19], ok);
   int64_t mq, mk;
+  int32_t zero, causal;
   double p, scale;
   Shape s;
-  if (!ok || !as_int(a[5], &mq) || !as_int(a[6], &mk) || !as_double(a[7], &p) || !as_double(a[8], &scale) || mq <= 0 || mk <= 0 ||
+  if (!ok || !as_int(a[5], &mq) || !as_int(a[6], &mk) || !as_double(a[7], &p) || !as_double(a[8], &scale) || !as_flag(a[9], &zero) ||
+      !as_flag(a[10], &causal) || mq <= 0 || mk <= 0 ||
       !common(q, k, cu_q, &s) || s.total_q > INT32_MAX || s.total_k > INT32_MAX || s.batch > INT32_MAX || !rows_ok(q, s, s.total_q) ||
       !rows_ok(k, s, s.total_k) || !rows_ok(v, s, s.total_k) || !cu_ok(cu_q, s) || !cu_ok(cu_k, s) || !slopes_ok(alibi, s) ||
       !words_ok(words, s) || !bias_ok(bias, s, mq, mk) || !tables_ok(cos, sin, s, mq) || (q_rot && (!cos || !rows_ok(q_rot, s, s.total_q))))
@@ -181,7 +191,7 @@ PyObject* fwd(PyObject* const* a, Py_ssize_t n) {
   f.total_q = (int32_t)s.total_q; f.total_k = (int32_t)s.total_k;
   f.max_seqlen_q = (int32_t)mq; f.max_seqlen_k = (int32_t)mk;
   f.p_dropout = (float)p; f.softmax_scale = (float)scale;
-  f.zero_tensors = PyObject_IsTrue(a[9]); f.is_causal = PyObject_IsTrue(a[10]);
+  f.zero_tensors = zero; f.is_causal = causal;
   if (alibi) f.alibi_slopes = (const float*)ptr(*alibi);
   if (words && !mask) { f.keep_words = ptr(*words); f.keep_words_bytes = (size_t)words->numel(); }
   if (bias) {
@@ -224,9 +234,11 @@ PyObject* bwd(PyObject* const* a, Py_ssize_t n) {
   const at::Tensor *alibi = tensor(a[18], ok), *words = tensor(a[19], ok), *bias = tensor(a[20], ok), *dbias = tensor(a[21], ok);
   const at::Tensor *cos = tensor(a[22], ok), *sin = tensor(a[23], ok), *mask = tensor(a[24], ok), *order = tensor(a[25], ok);
   int64_t mq, mk;
+  int32_t zero, causal;
   double p, scale;
   Shape s;
-  if (!ok || !as_int(a[11], &mq) || !as_int(a[12], &mk) || !as_double(a[13], &p) || !as_double(a[14], &scale) || mq <= 0 || mk <= 0 ||
+  if (!ok || !as_int(a[11], &mq) || !as_int(a[12], &mk) || !as_double(a[13], &p) || !as_double(a[14], &scale) || !as_flag(a[15], &zero) ||
+      !as_flag(a[16], &causal) || mq <= 0 || mk <= 0 ||
       !common(q, k, cu_q, &s) || s.total_q > INT32_MAX || s.total_k > INT32_MAX || s.batch > INT32_MAX || !rows_ok(q, s, s.total_q) ||
       !rows_ok(k, s, s.total_k) || !rows_ok(v, s, s.total_k) || !rows_ok(out, s, s.total_q) || !rows_ok(dout, s, s.total_q) ||
       !rows_ok(dq, s, s.total_q) || !rows_ok(dk, s, s.total_k) || !rows_ok(dv, s, s.total_k) || !out->is_contiguous() || !dout->is_contiguous() ||
@@ -262,7 +274,7 @@ PyObject* bwd(PyObject* const* a, Py_ssize_t n) {
   f.total_q = (int32_t)s.total_q; f.total_k = (int32_t)s.total_k;
   f.max_seqlen_q = (int32_t)mq; f.max_seqlen_k = (int32_t)mk;
   f.p_dropout = (float)p; f.softmax_scale = (float)scale;
-  f.zero_tensors = PyObject_IsTrue(a[15]); f.is_causal = PyObject_IsTrue(a[16]);
+  f.zero_tensors = zero; f.is_causal = causal;
   if (alibi) f.alibi_slopes = (const float*)ptr(*alibi);
   if (words && !mask) { f.keep_words = ptr(*words); f.keep_words_bytes = (size_t)words->numel(); }
   if (bias) {

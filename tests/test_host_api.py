@@ -729,3 +729,15 @@ def test_causal_forward_tiles_follow_the_measurements(tmp_path):
     half = _launch_rules(tmp_path, ["small_launch_causal(%d, live_row_tiles(%d, %d, %d), %d, %d, %d, %d)" % (
         d, h, _spread(n, f, b), b, b * h, n, _spread(n, f, b), b) for d, b, h, n, f, _ in cases])
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
+
+
+def test_native_calls_leave_no_exception_behind_what_they_hand_back():
+    """numbers a double cannot hold and flags without a truth value are handed back to the binding, which raises for them"""
+    import numpy as np
+    from flash_attn import flash_attn_gfx950 as be
+    be.load_library()
+    x, cu = torch.zeros(4, 2, 16, dtype=torch.half), torch.tensor([0, 4], dtype=torch.int32)
+    for p, scale, zero, causal in ((10 ** 400, 0.1, False, False), (0.0, 10 ** 400, False, False), (0.0, 0.1, np.ones(2), False),
+                                   (0.0, 0.1, False, np.ones(2))):
+        assert be._host.fwd(x, x, x, cu, cu, 4, 4, p, scale, zero, causal, *[None] * 9) is None
+        assert be._host.bwd(x, x, x, x, x, None, x, x, x, cu, cu, 4, 4, p, scale, zero, causal, *[None] * 9) is None

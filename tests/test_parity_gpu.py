@@ -1476,6 +1476,15 @@ def test_native_calls_hand_back_what_the_binding_refuses(binding_only):
                         be.fwd(*args, False, False, False, None, **kw)
             said.append(str(e.value))
         assert said[0] == said[1] and said[0]
+    import numpy as np
+    for causal in (np.ones(2), torch.ones(2)):  # (no truth value: what bool() raises)
+        for cm in (None, binding_only()):
+            with pytest.raises((ValueError, RuntimeError), match="ambiguous"):
+                if cm is None:
+                    be.fwd(q, k, v, cu, cu, 20, 20, 0.0, 0.1, False, causal, False, None)
+                else:
+                    with cm:
+                        be.fwd(q, k, v, cu, cu, 20, 20, 0.0, 0.1, False, causal, False, None)
 
 
 @pytest.mark.parametrize("kind", ["dense", "redrawn", "block"])
