@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   auto stage = [&](int it, int buf) {
     if constexpr (kRows) {
       if (listed) {
-        stager.issue_listed(lds_raw + buf * kBufBytes, row_slots + (it & 1) * 64);
+        stager.template issue_listed<D == 128 && KS == 1 && !kRoomy>(lds_raw + buf * kBufBytes, row_slots + (it & 1) * 64);
         if (it + 1 < ntiles) {
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the list has been read (and the slot of it + 1 was before it)
           fetch_rows(it + 1);

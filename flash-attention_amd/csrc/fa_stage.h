@@ -142,13 +142,17 @@ struct TilePairStager {
     }
   }
 
-  // The same for a tile whose row r is tensor row list[r] (list: LDS, one entry per tile row, all of them valid rows).
+  // The same for a tile whose row r is tensor row list[r] (list: LDS, one entry per tile row, all of them valid rows), by way of the offsets that
+  // issue() keeps: chunk offsets of its own, hoisted out of the caller's main loop, cost the forward six registers in scratch at d = 64.
+  // kTight: the row behind an opaque copy, so that differences with it are not hoisted either (at d = 128 they cost the third wave per SIMD, us
+  // with it / without 16 x 1500 rows x 8 heads 108 / 115, causal 63.1 / 73.8; where two waves run anyway it is 3 % slower).
+  template <bool kTight>
   FA_DEVICE void issue_listed(unsigned char* lds, const int32_t* list) const {
+    int rlv = rl;
+    if constexpr (kTight) asm volatile("" : "+v"(rlv));
 #pragma unroll
-    for (int i = 0; i < NI; i++) {
-      const int r = row0 + i * RPI + rl;
-      dma16(base, (uint32_t)list[r] * (uint32_t)rsb + 16u * (uint32_t)(pch ^ swz(r)), lds + dst0 + i * 1024);
-    }
+    for (int i = 0; i < NI; i++)
+      dma16(base, (uint32_t)(list[row0 + i * RPI + rlv] - rlv) * (uint32_t)rsb + src_off[i % NOFF], lds + dst0 + i * 1024);
   }
 
   // The same for a tile whose rows are gathered from 16-row blocks of the tensors: tile rows 16 j .. 16 j + 15 are tensor

@@ -4,6 +4,7 @@ The d = 64 kernels are tuned to the register counts at which one more wave fits 
 One extra live register in a main loop silently costs a wave per SIMD or turns into scratch traffic, so the counts the
 compiler reports (-Rpass-analysis=kernel-resource-usage) are pinned here for the variants the headline workloads run.
 """
+import functools
 import os
 import re
 import subprocess
@@ -17,6 +18,7 @@ sys.path.insert(0, os.path.join(ROOT, "flash-attention_amd"))
 import build as fa_build  # noqa: E402
 
 
+@functools.lru_cache(maxsize=None)
 def _resources(src):
     cmd = [fa_build.HIPCC] + fa_build.FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-c",
                                                os.path.join(fa_build.CSRC, src), "-o", os.devnull]
@@ -180,3 +182,23 @@ def test_key_words_of_the_dropout_forward_only_where_they_pay():
                     key_words = 0 if causal == "Lb1E" and words == "Lb1E" else 1024
                     assert full["Occupancy"] >= waves and full["VGPRs Spill"] == 0 and full["LDS Size"] == tiles + key_words, (dt, d, causal, words, full)
                     assert half["Occupancy"] >= 4 and half["VGPRs Spill"] == 0 and half["LDS Size"] == tiles, (dt, d, causal, words, half)
+
+
+@pytest.mark.timeout(600)
+def test_padded_rows_and_d128_half_size_variants_keep_their_waves_per_simd():
+    """The forward over a padded batch (three as score-bias parameter) keeps the waves per SIMD of the dense variant it is bounded like, nothing in
+    scratch; the half-size tiles of d = 128, forward and dQ, run two waves per SIMD and two workgroups' LDS on a compute unit."""
+    with ThreadPoolExecutor(5) as ex:
+        d16, d32, d64, d128, bwd = ex.map(_resources, ("fa_fwd_d16.hip", "fa_fwd_d32.hip", "fa_fwd_d64.hip", "fa_fwd_d128.hip", "fa_bwd_d128.hip"))
+    for dt in ("IDF16_", "IDF16b"):
+        for causal in ("Lb0E", "Lb1E"):
+            rows, dense = causal + "Lb0ELb0ELi3ELi%dELb0EEEv", causal + "Lb0ELb0ELi0ELi2ELb0EEEv"
+            for res, d, bn, roomy, ks, waves in ((d16, 16, 64, 0, 1, 5), (d16, 16, 64, 0, 2, 7), (d32, 32, 64, 0, 1, 4), (d32, 32, 64, 0, 2, 6),
+                                                 (d64, 64, 64, 0, 1, 4), (d64, 64, 64, 0, 2, 4), (d128, 128, 32, 0, 1, 3), (d128, 128, 32, 1, 1, 2),
+                                                 (d128, 128, 64, 0, 2, 2)):
+                k = _pick(res, "fa_fwd_kernel%sLi%dELi%dELb%dE" % (dt, d, bn, roomy), rows % ks)
+                assert k["Occupancy"] >= waves and k["VGPRs Spill"] == 0, ("padded rows", d, dt, causal, roomy, ks, k)
+            k = _pick(d128, "fa_fwd_kernel%sLi128ELi64ELb0E" % dt, dense)
+            assert k["Occupancy"] >= 2 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 80 * 1024, ("forward, half-size", dt, causal, k)
+            k = _pick(bwd, "fa_bwd_dq_kernel%sLi128E" % dt, causal + "Li0ELb0ELi0ELi2EEEv")
+            assert k["Occupancy"] >= 2 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 80 * 1024, ("dq, half-size", dt, causal, k)
