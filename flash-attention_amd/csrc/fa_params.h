@@ -335,6 +335,16 @@ inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
   return live <= 384 && (max_s > 1100 || x <= (max_s > 768 ? 430 : max_s > 512 ? 360 : max_s > 384 ? 310 : 270));
 }
 
+// The forward over a padded batch, whose number of tokens is not known here: at head dim 128 as if three quarters of the rows were tokens, of
+// short rows all; us of full-size / half-size tiles over 30 % .. 100 % of the rows, causal, 6 x 16 x 400 16.1 / 14.4, 4 x 12 x 1079 31.4 / 23.5, all rows tokens
+// 2 x 12 x 1217 33.8 / 24.0, 8 x 16 x 218 .. 272 13.5 / 15.6 (over 1000 drawn shapes 2 % over the better of both, none 3 % slower than
+// full-size throughout); below by the launched workgroups.
+inline bool small_launch_rows(int head_dim, int batch, int nheads, int max_s, bool causal) {
+  if (head_dim <= 64) return small_launch(kSmallLaunchFwd, batch * nheads, max_s, causal, false);
+  const int64_t rows = (int64_t)batch * max_s;
+  return small_launch_d128(live_row_tiles(nheads, (int)(max_s > 384 ? rows * 3 / 4 : rows), batch), batch * nheads, max_s, causal);
+}
+
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves
 // idle, one launch less; dQ at two waves per SIMD instead of three): at head dim 64, dense, no score bias, no rotation, no key split, dropout
 // off or read from the keep words.  By the workgroups of 128 query rows that find any (live_row_tiles, `live`), the longest sequence n and, where

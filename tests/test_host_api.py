@@ -741,3 +741,12 @@ def test_native_calls_leave_no_exception_behind_what_they_hand_back():
                                    (0.0, 0.1, False, np.ones(2))):
         assert be._host.fwd(x, x, x, cu, cu, 4, 4, p, scale, zero, causal, *[None] * 9) is None
         assert be._host.bwd(x, x, x, x, x, None, x, x, x, cu, cu, 4, 4, p, scale, zero, causal, *[None] * 9) is None
+
+
+def test_padded_forward_tiles_follow_the_measurements(tmp_path):
+    """padded batches: full- or half-size tiles by what was faster over batches of 30 % to 100 % tokens"""
+    cases = [  # head dim, batch, heads, rows, causal, half-size?
+        (128, 6, 16, 400, 1, 1), (128, 4, 12, 1079, 1, 1), (128, 2, 12, 1217, 1, 1), (128, 1, 16, 1376, 0, 1),  # us full / half: 16.1 / 14.4 .. 36.2 / 31.2
+        (128, 8, 12, 156, 0, 0), (128, 12, 16, 209, 0, 0), (128, 8, 16, 272, 1, 0), (128, 16, 8, 1500, 1, 0), (64, 32, 16, 512, 0, 0), (64, 8, 8, 512, 0, 1)]  # 10.3 / 11.7, 13.5 / 15.6
+    half = _launch_rules(tmp_path, ["small_launch_rows(%d, %d, %d, %d, %d)" % c[:-1] for c in cases])
+    assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
