@@ -41,8 +41,8 @@ def _need_gpu(lib):
 
 @pytest.fixture(params=[1, 2], ids=["full-size tiles", "half-size tiles"])
 def tile_shape(request):
-    """Runs a test with both tile shapes of the dense kernels (the library picks per launch by default; the half-size
-    variants exist for head dims up to 64): fa_set_launch_policy."""
+    """Runs a test with both tile shapes of the dense kernels (the library picks per launch by default; the half-size variants
+    exist without a score bias, at head dim 128 without dropout): fa_set_launch_policy."""
     from flash_attn import flash_attn_gfx950 as be
     be.set_launch_policy(request.param)
     yield request.param
@@ -1401,9 +1401,10 @@ def binding_only():
 
 @pytest.mark.parametrize("kind", ["plain", "causal", "dropout", "words", "alibi", "bias", "rotary", "block", "cross", "decode", "zero"])
 @pytest.mark.parametrize("dtype,D", [(torch.float16, 64), (torch.bfloat16, 128), (torch.float16, 16)])
-def test_native_calls_equal_the_bindings(kind, dtype, D, binding_only):
-    """The native half of the binding makes the same call as the binding: every output equal bit for bit and the generator left where it was left,
-    for packed, separate and strided views, scratch (decode and cross splits, block layouts) and every optional argument."""
+def test_native_calls_equal_the_bindings(kind, dtype, D, binding_only, monkeypatch):
+    """The native half of the binding makes the same call as the binding, and takes every kind: every output equal bit for bit and the generator
+    left where it was left, for packed, separate and strided views, scratch (decode and cross splits, block layouts) and every optional argument."""
+    import types
     from flash_attn import flash_attn_gfx950 as be
     from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
     H, lens_q, lens_k = 3, [70, 129, 5], [70, 129, 5]
@@ -1447,7 +1448,19 @@ def test_native_calls_equal_the_bindings(kind, dtype, D, binding_only):
         rows = [x[b, :, :L] for x in (lse, d) for b, L in enumerate(lens_q)]  # (what lies past a sequence's end is not written)
         return [o, dq, dk, dv] + rows + [x for x in (q_rot, dbias) if x is not None] + [torch.cuda.get_rng_state()]
 
+    host, taken = be._host, []
+
+    def noted(name):
+        def call(*a):
+            res = getattr(host, name)(*a)
+            taken.append((name, res is not None))
+            return res
+        return call
+
+    monkeypatch.setattr(be, "_host", types.SimpleNamespace(fwd=noted("fwd"), bwd=noted("bwd")))
     native = step()
+    assert taken == [("fwd", True), ("bwd", True)]
+    monkeypatch.undo()
     with binding_only():
         for i, (x, y) in enumerate(zip(native, step())):
             assert torch.equal(x, y), i
@@ -1536,14 +1549,16 @@ def _padding_masks(B, S, seed):
 
 @pytest.mark.parametrize("D", [16, 32, 64, 128])
 @pytest.mark.parametrize("causal", [False, True])
-def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape):
+def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape, monkeypatch):
     """Evaluation of a padded batch reads q, k, v where they lie and writes the padded output at once (fa_padding_rows, fa_fwd_padded).
     With one entry full both ways run the same tiles over the same tokens in the same order (beyond the decode kernel's 32 rows): equal bit
     for bit to unpad, packed attention, pad.  Lengths around the 64- and 128-row tiles, tokens in one run or anywhere, entries without any."""
     from flash_attn.bert_padding import pad_input, unpad_input
     from flash_attn.flash_attention import FlashAttention
     from flash_attn.flash_attn_interface import flash_attn_unpadded_qkvpacked_func
-    m = FlashAttention(attention_dropout=0.3).eval()
+    from flash_attn import flash_attn_gfx950 as be
+    m, in_place, fwd_padded = FlashAttention(attention_dropout=0.3).eval(), [], be.fwd_padded
+    monkeypatch.setattr(be, "fwd_padded", lambda *a: in_place.append(fwd_padded(*a)) or in_place[-1])
     for S, B, H in ((1, 1, 2), (33, 3, 2), (64, 2, 3), (127, 4, 1), (129, 5, 2), (200, 9, 3), (513, 3, 4)):
         g = torch.Generator(device="cuda").manual_seed(S)
         wide = torch.randn(B, S, 4, H, D, generator=g, device="cuda").half()
@@ -1551,7 +1566,9 @@ def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape):
             qkv = wide[:, :, :3] if i % 2 else wide[:, :, :3].contiguous()  # rows apart by more than their width, or packed
             kpm = type("Mask", (), {"bool_matrix": mask.cuda()})
             with torch.no_grad():
+                del in_place[:]
                 got = m(qkv, key_padding_mask=kpm, causal=causal)[0]
+                assert len(in_place) == 1 and in_place[0] is got
                 rows, idx, cu, mx = unpad_input(qkv.reshape(B, S, -1), kpm.bool_matrix)
                 out = flash_attn_unpadded_qkvpacked_func(rows.view(-1, 3, H, D), cu, mx, 0.0, causal=causal)
                 want = pad_input(out.view(-1, H * D), idx, B, S).view(B, S, H, D)
@@ -1564,6 +1581,35 @@ def test_padded_batch_in_place_equals_gathered(D, causal, tile_shape):
     with pytest.raises(RuntimeError):  # a batch without a token is refused
         with torch.no_grad():
             m(qkv, key_padding_mask=type("Mask", (), {"bool_matrix": torch.zeros(B, S, dtype=torch.bool, device="cuda")}), causal=causal)
+
+
+@pytest.mark.parametrize("B,S,H,D,dtype", [
+    (70, 300, 3, 128, torch.bfloat16),   # more than 64 entries (their order is kept) and 512 workgroups
+    (4, 900, 12, 128, torch.float16),    # without a mask the build for few workgroups
+    (3, 700, 4, 128, torch.bfloat16),    # half-size tiles
+    (9, 600, 12, 64, torch.bfloat16), (65, 130, 4, 64, torch.bfloat16), (5, 200, 3, 32, torch.bfloat16), (66, 70, 2, 16, torch.bfloat16)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_padded_rows_against_fp32(B, S, H, D, dtype, causal):
+    """fwd_padded with the tiles it picks by itself, both element types.  Probabilities and result are rounded once each and the row sum is that
+    of the rounded probabilities: three half units in the last place of the largest value."""
+    from flash_attn import flash_attn_gfx950 as be
+    g = torch.Generator(device="cuda").manual_seed(S)
+    qkv = torch.randn(B, S, 3, H, D, generator=g, device="cuda").to(dtype)
+    future = torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1)
+    for mask in list(_padding_masks(B, S, D))[::2]:  # tokens in front, tokens anywhere
+        mask = mask.cuda()
+        assert be.padded_layout_ok(qkv, mask)
+        got = be.fwd_padded(qkv, mask, D ** -0.5, causal)
+        assert (got[~mask] == 0).all()
+        for b in range(B):
+            q, k, v = qkv[b, mask[b]].float().permute(1, 2, 0, 3).contiguous()
+            if q.shape[1] == 0:
+                continue
+            s = torch.matmul(q, k.transpose(1, 2).contiguous()) * D ** -0.5
+            if causal:
+                s = s.masked_fill(future[:q.shape[1], :q.shape[1]], float("-inf"))
+            want = torch.matmul(s.softmax(-1), v).transpose(0, 1)
+            assert (got[b, mask[b]].float() - want).abs().max() <= 3 * HALF_ULP[dtype] * v.abs().max(), b
 
 
 def test_padded_batch_is_refused_before_anything_is_enqueued(monkeypatch):
