@@ -302,8 +302,9 @@ def unpack_dropout(saved, kept):
 
 def _philox_state(device, p_dropout, gen):
     """(seed, offset) of the device's generator, advanced the way philox_cuda_state(counter_offset) does
-    (fmha_api.cpp:288-292).  Restoring the generator state reproduces the pair, which is how the backward
-    regenerates the forward's mask (flash_attn_interface.py:43,61-63)."""
+    (fmha_api.cpp:288-292).  gen: a generator, None (the device's default one), or a DrawnPhilox, which keeps the pair a forward
+    drew for its backward to regenerate the mask with (the reference restores the generator's state for that,
+    flash_attn_interface.py:43,61-63)."""
     if not p_dropout > 0.0:
         return 0, 0
     drawn = None
@@ -846,6 +847,9 @@ def fwd_padded(qkv, mask, softmax_scale, is_causal):
     a (batch, seqlen) bool mask, True = token, for which padded_layout_ok() holds.  Returns (batch, seqlen, nheads, headdim) with zeros in
     the padding, or None if the mask holds no token at all or the scale is none the kernels take (nothing is enqueued then): the packed
     call refuses both.  The lengths are read back while the attention kernel runs."""
+    scale = ctypes.c_float(softmax_scale).value
+    if not 0.0 < scale < math.inf:
+        return None
     lib = load_library()
     B, S, _, H, D = qkv.shape
     st = qkv.stride()
@@ -862,28 +866,25 @@ def fwd_padded(qkv, mask, softmax_scale, is_causal):
         a.is_causal = int(bool(is_causal))
         return 0
 
-    a, _ = _cached_args(("padded", qkv.dtype, qkv.shape, st, bool(is_causal)), FwdArgs, fill)
-    a.softmax_scale = float(softmax_scale)
-    if not 0.0 < a.softmax_scale < math.inf:  # (as rounded to fp32)
-        return None
-    sq_r, _ = round_seqlens(D, S, S, False)
     with _OnDevice(dev):
-        out = torch.empty((B, S, H, D), dtype=qkv.dtype, device=dev)
-        lse = torch.empty((B, H, sq_r), dtype=torch.float32, device=dev)
         rows = torch.empty((B * (S + 4),), dtype=torch.int32, device=dev)
         lens = torch.empty((B,), dtype=torch.int32, pin_memory=True)
         written = torch.cuda.Event()
         row_of, stream = rows.data_ptr(), _stream_handle(dev)
         row_info = row_of + 4 * B * S
-        a.q = qkv.data_ptr()
-        a.k, a.v = a.q + 2 * st[2], a.q + 4 * st[2]
-        a.o, a.softmax_lse = out.data_ptr(), lse.data_ptr()
-        a.stream = stream
         rc = lib.fa_padding_rows(mask.data_ptr(), mask.stride(0), B, S, row_of, row_info, lens.data_ptr(), stream)
         if rc != 0:
             _raise(rc, lib)
-        try:
+        try:  # (the rest is prepared while that kernel runs)
             written.record()
+            out = torch.empty((B, S, H, D), dtype=qkv.dtype, device=dev)
+            lse = torch.empty((B, H, round_seqlens(D, S, S, False)[0]), dtype=torch.float32, device=dev)
+            a, _ = _cached_args(("padded", qkv.dtype, qkv.shape, st, bool(is_causal)), FwdArgs, fill)
+            a.softmax_scale = scale
+            a.q = qkv.data_ptr()
+            a.k, a.v = a.q + 2 * st[2], a.q + 4 * st[2]
+            a.o, a.softmax_lse = out.data_ptr(), lse.data_ptr()
+            a.stream = stream
             rc = lib.fa_fwd_padded(ctypes.byref(a), row_of, row_info)
             if rc != 0:
                 _raise(rc, lib)
