@@ -76,8 +76,8 @@ constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool
 // kWords (dropout, dense): the keep decisions are also left in p.keep_words for the backward (fa_common.h)
 // kBias = kPaddedRows (dense, no dropout): q, k, v and o are a padded batch, (batch, max_sq) rows of which p.row_of and p.row_info name the
 // tokens; these attend each other, counted in their own order, and the padding rows of o are written as zeros.  32 x 512 rows, 256 .. 512 of
-// them tokens, 16 heads, d = 64: one launch of 47 us in place of gather 29, forward 40 and scatter 15,
-// and tokens anywhere in their row instead of in one run cost it 6 % (the module call 49 and 52 us, 175 gathered).
+// them tokens, 16 heads, d = 64: one launch of 43 us in place of gather 29, forward 40 and scatter 15, 42 with tokens anywhere in their row (the
+// module call 52 us, 175 gathered).
 template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
           bool kWords = false>
 __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % kPaddedRows, KS, kWords)) fa_fwd_kernel(const FwdParams p) {

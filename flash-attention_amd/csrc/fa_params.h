@@ -163,8 +163,8 @@ struct BwdParams {
   const float* alibi;  // as in FwdParams
   const void* bias;    // as in FwdParams
   int64_t bias_bs, bias_hs, bias_rs;
-  void* dbias;         // null, or where the dK/dV kernel leaves d(loss)/d(bias) = dS / keep: [b, h, query, key], written for the
-  int64_t dbias_bs, dbias_hs, dbias_rs;  // (query, key) tiles it visits (the caller clears the tensor)
+  void* dbias;         // null, or where the dK/dV kernel leaves d(loss)/d(bias) = dS / keep: [b, h, query, key], written for the queries and
+  int64_t dbias_bs, dbias_hs, dbias_rs;  // keys a sequence has (causal: up to the diagonal; block layout: listed blocks); the rest is left as it is
   // Rotary position embedding (as in FwdParams; null: none): q and k are the rotated tensors, and dq and dk are turned back
   // by the opposite angles in the kernels' epilogues, before they are rounded
   const void* rot_cos;
@@ -283,9 +283,9 @@ inline bool longest_first_launch(bool causal, bool sparse, int grid, int B) {
 // workgroups per compute unit,
 //   forward: half-size for x < 2 (more than one key tile pair to split: sequences beyond 128), and up to x < 3 with dropout
 //            (whose Philox work makes the serial walk longer);
-//   dQ:      half-size for 1 <= x < 2 under a causal mask or with dropout; the plain kernel gains nothing from it.
-// Where lengths differ, many launched workgroups find no rows: the rules that follow this one (causal forward, head dim 128, backward without
-// dropout) count those that do, and this one stays for the others.
+//   dQ:      half-size for 1 <= x < 2 under a causal mask or with dropout.
+// Where lengths differ, many launched workgroups find no rows: the rules that follow this one (causal forward, head dim 128, dQ without
+// dropout, the backward in one launch) count those that do, and this one stays for the others.
 // launch_policy() & 3: 0 = by this rule, 1 = always the full-size tiles, 2 = the half-size tiles wherever they exist
 // (fa_set_launch_policy; the parity tests run both shapes on the same inputs).
 int launch_policy();
@@ -337,7 +337,7 @@ inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
 
 // The forward over a padded batch, whose number of tokens is not known here: at head dim 128 as if three quarters of the rows were tokens, of
 // short rows all; us of full-size / half-size tiles over 30 % .. 100 % of the rows, causal, 6 x 16 x 400 16.1 / 14.4, 4 x 12 x 1079 31.4 / 23.5, all rows tokens
-// 2 x 12 x 1217 33.8 / 24.0, 8 x 16 x 218 .. 272 13.5 / 15.6 (over 1000 drawn shapes 2 % over the better of both, none 3 % slower than
+// 2 x 12 x 1217 33.8 / 24.0, 8 x 16 x 218 .. 272 13.5 / 15.6 (over 1000 drawn shapes 2 % over the better of both, none more than 5 % slower than
 // full-size throughout); below by the launched workgroups.
 inline bool small_launch_rows(int head_dim, int batch, int nheads, int max_s, bool causal) {
   if (head_dim <= 64) return small_launch(kSmallLaunchFwd, batch * nheads, max_s, causal, false);

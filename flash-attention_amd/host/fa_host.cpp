@@ -8,7 +8,8 @@
 //
 // Bound by the interpreter.  us with the binding's own calls / with these: one forward of 12 heads x 61 tokens (kernel 6) 21.4 / 14.2; training
 // steps of 8 x 12 x 256 .. 512 with dropout (kernels 56; an empty autograd function with a backward takes 48) 159 / 101, 8 x 12 x 1024 rotary
-// (110) 175 / 118, 8 x 8 x 421 .. 701 with a bias (100) 203 / 120.
+// (110) 175 / 118, 8 x 8 x 421 .. 701 with a bias (100) 208 / 149 - 100 where both host threads, the
+// caller's and the autograd engine's, run on one core: handing over to another core is what the rest goes to.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
