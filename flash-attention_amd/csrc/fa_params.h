@@ -326,10 +326,17 @@ inline bool small_launch_causal(int head_dim, int64_t live, int BH, int max_s, i
 // (293) 15.5 / 15.9, 5 x 16 x 518 (363) 18.4 / 18.9; 8 x 16 x 281 (345) 12.8 / 15.7, 10 x 12 x 250 .. 337 (339) 14.9 / 17.4, 10 x 12 x 190 .. 287 (283) 12.0 /
 // 13.5, 4 x 16 x 300 (182) 11.9 / 11.0, 6 x 16 x 182 (184) 9.1 / 9.3, 16 x 12 x 52 .. 130 (204) 8.7 / 9.3.  No mask: 8 x 1700 39.3 / 28.1, 8 x 2300
 // (148) 50.1 / 45.1, 3 x 16 x 286 (131) 10.8 / 10.0, 6 x 8 x 323 (145) 12.4 / 13.9, 4 x 8 x 531 (148) 16.2 / 17.1, 4 x 12 x 500 (192) 16.3 / 17.2.
-inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
+// With rotary, which every workgroup's prologue pays for, they cross sooner: causal 12 x 8 x 150 .. 197 (x = 177) 12.0 / 14.4, 6 x 16 x 276 (255) 15.4 / 16.4; no
+// mask 9 x 8 x 98 .. 229 (128) 13.5 / 15.3, 3 x 8 x 640 .. 706 (138) 23.1 / 24.7.
+inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal, bool rotary) {
   const int policy = launch_policy() & 3;
   if (policy != 0) return policy == 2;
   const int64_t x = fullest_xcd(live, BH);
+  if (rotary) {
+    if (!causal) return max_s > 192 && x <= (max_s > 768 ? 140 : 120);
+    if (max_s <= 256) return max_s > 128 && x <= (max_s > 192 ? 140 : 125);
+    return live <= 384 && (max_s > 2500 || x <= (max_s > 1100 ? 430 : max_s > 768 ? 360 : max_s > 512 ? 310 : max_s > 384 ? 200 : 150));
+  }
   if (!causal) return max_s > 192 && x <= (max_s > 640 ? 150 : 140);
   if (max_s <= 256) return max_s > 128 && x <= (max_s > 192 ? 192 : 125);
   return live <= 384 && (max_s > 1100 || x <= (max_s > 768 ? 430 : max_s > 512 ? 360 : max_s > 384 ? 310 : 270));
@@ -342,7 +349,7 @@ inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal) {
 inline bool small_launch_rows(int head_dim, int batch, int nheads, int max_s, bool causal) {
   if (head_dim <= 64) return small_launch(kSmallLaunchFwd, batch * nheads, max_s, causal, false);
   const int64_t rows = (int64_t)batch * max_s;
-  return small_launch_d128(live_row_tiles(nheads, (int)(max_s > 384 ? rows * 3 / 4 : rows), batch), batch * nheads, max_s, causal);
+  return small_launch_d128(live_row_tiles(nheads, (int)(max_s > 384 ? rows * 3 / 4 : rows), batch), batch * nheads, max_s, causal, false);
 }
 
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves

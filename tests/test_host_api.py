@@ -681,9 +681,12 @@ def test_d128_forward_tiles_follow_the_measurements(tmp_path):
         (6, 8, 323, 1.0, 0, 0), (3, 16, 325, 1.0, 0, 0), (4, 8, 531, 1.0, 0, 0),  # 12.4 / 13.9, 12.0 / 13.4, 16.1 / 17.1
         (1, 8, 2300, 1.0, 1, 1), (4, 12, 1200, 0.3, 1, 1), (4, 16, 300, 1.0, 1, 1), (1, 16, 3000, 1.0, 1, 1),  # 53.9 / 35.8, 32.7 / 24.8, 11.9 / 11.0, 69.8 / 51.4
         (1, 8, 1700, 1.0, 0, 1), (3, 16, 286, 1.0, 0, 1)]  # 39.3 / 28.1, 10.8 / 10.0
-    got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, c)
-                                   for b, h, n, f, c, _ in cases])
-    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+    rotary = [(12, 8, 197, 0.75, 1, 0), (6, 16, 276, 1.0, 1, 0), (9, 8, 229, 0.43, 0, 0), (3, 8, 706, 0.91, 0, 0),  # 12.0 / 14.4 .. 23.1 / 24.7
+              (1, 8, 2300, 1.0, 1, 1), (1, 8, 1100, 1.0, 0, 1), (2, 8, 500, 1.0, 1, 1)]
+    for rot, cs in ((0, cases), (1, rotary)):
+        got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, c, rot)
+                                       for b, h, n, f, c, _ in cs])
+        assert got == [c[-1] for c in cs], [c for c, g in zip(cs, got) if g != c[-1]]
 
 
 def _rule_case(b, h, n, f):
