@@ -398,7 +398,8 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
 // merged_backward_shape takes them, half-size tiles in two launches are the slowest plan there: 33 x 12 x 73 22.1 merged, 23.5 full-size, 29.1):
 // causal d = 32 2 x 16 x 73 % of 707 (145) 27.6 / 25.1 with the dK/dV kernel, 3 x 16 x 70 % of 1785 (494) 59.5 / 53.0, 12 x 16 x 336 (551) 23.7 / 23.3;
 // d = 16 2 x 8 x 3964 (503) 96.9 / 89.0; up to 128 tokens small_launch, 17 x 16 x 115 15.8 / 15.1; d = 64 8 x 12 x 460 (393) 34.0 / 32.6, 12 x 8 x 609
-// (504) 40.5 / 42.7; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
+// (504) 40.5 / 42.7, with rotary (on the fullest XCD) 6 x 8 x 1012 (403) 57.6 / 53.1, 3 x 8 x 2177 (420) 102.6 / 96.5, 16 x 3394 (432) 144.8 / 135.1, 18 x 16 x 126
+// (427) 26.3 / 25.4; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
 // chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 2 x 12 x 1500 (293) 110.3 / 101.0, short sequences cross sooner: 6 x 16 x 183
 // (169) 25.6 / 27.1, 6 x 16 x 509 (345) 51.5 / 54.7; no mask, on the fullest XCD, 2 x 8 x 928 (124) 67.6 / 60.5, 3 x 16 x 789 (256) 70.7 / 75.7, 7 x 12 x 135
 // (136) 25.3 / 27.7, 9 x 8 x 80 .. 244 (127) 29.6 / 30.3.
@@ -412,7 +413,12 @@ inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int 
   }
   if (ruled && head_dim == 64 && dropout && keep_words && !rotary) return false;
   if (!swept || (head_dim < 64 && max_sq <= 128)) return small_launch(kSmallLaunchDq, BH, max_sq, causal, dropout);
-  return max_sq > 128 && live <= (causal ? (head_dim == 64 ? 400 : 520) : 130);
+  if (head_dim == 64 && causal) {
+    const int64_t x = fullest_xcd(live, BH);
+    if (max_sq <= 128) return rotary && max_sq > 96 && x <= 470;
+    return x <= (max_sq > 1800 ? 520 : max_sq > 1200 ? 460 : max_sq > 800 ? 430 : max_sq > 384 ? 410 : 400);
+  }
+  return max_sq > 128 && live <= (causal ? 520 : 130);
 }
 
 // Launchers (defined in fa_fwd.hip / fa_bwd.hip / fa_aux.hip).  Return hipError_t of the launch.

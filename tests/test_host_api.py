@@ -720,6 +720,10 @@ def test_dq_tiles_follow_the_measurements(tmp_path):
         (128, 2, 8, 928, 1.0, 0, 1), (128, 1, 8, 974, 1.0, 1, 1), (128, 2, 12, 1500, 1.0, 1, 1), (32, 2, 16, 707, 0.46, 1, 1)]  # 67.6 / 60.5, 73.4 / 64.2
     half = _launch_rules(tmp_path, ["small_launch_dq(%d, %s, %d, 0, 0, 0, 1)" % (c[0], _rule_case(*c[1:5]), c[5]) for c in cases])
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
+    rotary = [(6, 8, 1012, 1.0, 1, 1), (3, 8, 2177, 1.0, 1, 1), (1, 16, 3394, 1.0, 1, 1), (18, 16, 126, 1.0, 1, 1),  # 57.6 / 53.1 .. 26.3 / 25.4
+              (27, 16, 90, 1.0, 1, 0), (12, 8, 609, 1.0, 1, 0), (8, 12, 460, 1.0, 1, 1)]
+    half = _launch_rules(tmp_path, ["small_launch_dq(64, %s, %d, 0, 0, 1, 1)" % (_rule_case(*c[:4]), c[4]) for c in rotary])
+    assert half == [c[-1] for c in rotary], [c for c, g in zip(rotary, half) if g != c[-1]]
 
 
 def test_causal_forward_tiles_follow_the_measurements(tmp_path):
