@@ -328,9 +328,13 @@ inline bool small_launch_causal(int head_dim, int64_t live, int BH, int max_s, i
 // (148) 50.1 / 45.1, 3 x 16 x 286 (131) 10.8 / 10.0, 6 x 8 x 323 (145) 12.4 / 13.9, 4 x 8 x 531 (148) 16.2 / 17.1, 4 x 12 x 500 (192) 16.3 / 17.2.
 // With rotary, which every workgroup's prologue pays for, they cross sooner: causal 12 x 8 x 150 .. 197 (x = 177) 12.0 / 14.4, 6 x 16 x 276 (255) 15.4 / 16.4; no
 // mask 9 x 8 x 98 .. 229 (128) 13.5 / 15.3, 3 x 8 x 640 .. 706 (138) 23.1 / 24.7.
-inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal, bool rotary) {
+// Where keys are fewer than queries the walk is over them: causal 12 x 2413 over 603 keys 20.3 / 26.0, 3 x 8 x 1736 over 868 27.9 / 31.1; no mask 2 x 16 x
+// 352 over 88 7.5 / 8.0.
+inline bool small_launch_d128(int64_t live, int BH, int max_sq, int max_sk, bool causal, bool rotary) {
   const int policy = launch_policy() & 3;
   if (policy != 0) return policy == 2;
+  if (causal && 4 * (int64_t)max_sk < 3 * (int64_t)max_sq) return false;
+  const int max_s = max_sk < max_sq ? max_sk : max_sq;
   const int64_t x = fullest_xcd(live, BH);
   if (rotary) {
     if (!causal) return max_s > 192 && x <= (max_s > 768 ? 140 : 120);
@@ -349,7 +353,7 @@ inline bool small_launch_d128(int64_t live, int BH, int max_s, bool causal, bool
 inline bool small_launch_rows(int head_dim, int batch, int nheads, int max_s, bool causal) {
   if (head_dim <= 64) return small_launch(kSmallLaunchFwd, batch * nheads, max_s, causal, false);
   const int64_t rows = (int64_t)batch * max_s;
-  return small_launch_d128(live_row_tiles(nheads, (int)(max_s > 384 ? rows * 3 / 4 : rows), batch), batch * nheads, max_s, causal, false);
+  return small_launch_d128(live_row_tiles(nheads, (int)(max_s > 384 ? rows * 3 / 4 : rows), batch), batch * nheads, max_s, max_s, causal, false);
 }
 
 // Short backward launches run dQ and dK/dV as one grid (fa_bwd_merged_kernel: half-size dQ tiles, each part fills what the other leaves
@@ -402,13 +406,13 @@ inline bool merged_backward_launch(int head_dim, int64_t live, int BH, int max_s
 // (427) 26.3 / 25.4; no mask d = 64 2 x 12 x 615 (118) 30.5 / 27.8, 4 x 16 x 335 (199) 24.8 / 25.0.  d = 128 (the dK/dV kernel fills more of the
 // chip there) causal 1 x 8 x 974 (64) 73.4 / 64.2, 4 x 12 x 272 (104) 31.4 / 28.8, 2 x 12 x 1500 (293) 110.3 / 101.0, short sequences cross sooner: 6 x 16 x 183
 // (169) 25.6 / 27.1, 6 x 16 x 509 (345) 51.5 / 54.7; no mask, on the fullest XCD, 2 x 8 x 928 (124) 67.6 / 60.5, 3 x 16 x 789 (256) 70.7 / 75.7, 7 x 12 x 135
-// (136) 25.3 / 27.7, 9 x 8 x 80 .. 244 (127) 29.6 / 30.3.
+// (136) 25.3 / 27.7, 9 x 8 x 80 .. 244 (127) 29.6 / 30.3; over a quarter as many keys as queries, causal 2 x 16 x 1109 67.5 / 74.4.
 inline bool small_launch_dq(int head_dim, int64_t live, int BH, int max_sq, int max_sk, bool causal, bool dropout, bool keep_words, bool rotary,
                             int n_splits) {
   if (merged_backward_shape(head_dim, live, BH, max_sq, max_sk, causal, dropout, keep_words, false, false, rotary, n_splits)) return true;
   const bool ruled = (launch_policy() & 3) == 0 && max_sk <= 2 * max_sq, swept = ruled && !dropout;
   if (head_dim == 128 && (launch_policy() & 3) == 0) {
-    if (!swept || max_sq <= 128) return false;
+    if (!swept || max_sq <= 128 || 2 * max_sk < max_sq) return false;
     return causal ? live <= (max_sq > 450 ? 300 : 150) : fullest_xcd(live, BH) <= (max_sq > 640 ? 140 : 120);
   }
   if (ruled && head_dim == 64 && dropout && keep_words && !rotary) return false;

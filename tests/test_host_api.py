@@ -684,9 +684,13 @@ def test_d128_forward_tiles_follow_the_measurements(tmp_path):
     rotary = [(12, 8, 197, 0.75, 1, 0), (6, 16, 276, 1.0, 1, 0), (9, 8, 229, 0.43, 0, 0), (3, 8, 706, 0.91, 0, 0),  # 12.0 / 14.4 .. 23.1 / 24.7
               (1, 8, 2300, 1.0, 1, 1), (1, 8, 1100, 1.0, 0, 1), (2, 8, 500, 1.0, 1, 1)]
     for rot, cs in ((0, cases), (1, rotary)):
-        got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, c, rot)
+        got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d, %d, %d)" % (h, _spread(n, f, b), b, b * h, n, n, c, rot)
                                        for b, h, n, f, c, _ in cs])
         assert got == [c[-1] for c in cs], [c for c, g in zip(cs, got) if g != c[-1]]
+    # fewer keys than queries: us full / half 20.3 / 26.0, 27.9 / 31.1, 7.5 / 8.0; as many or more keys as above
+    got = _launch_rules(tmp_path, ["small_launch_d128(live_row_tiles(%d, %d, %d), %d, %d, %d, %d, 0)" % (h, b * n, b, b * h, n, k, c) for b, h, n, k, c in (
+        (1, 12, 2413, 603, 1), (3, 8, 1736, 868, 1), (2, 16, 352, 88, 0), (1, 8, 2300, 4600, 1), (1, 8, 1700, 1700, 0))])
+    assert got == [0, 0, 0, 1, 1]
 
 
 def _rule_case(b, h, n, f):
@@ -720,6 +724,7 @@ def test_dq_tiles_follow_the_measurements(tmp_path):
         (128, 2, 8, 928, 1.0, 0, 1), (128, 1, 8, 974, 1.0, 1, 1), (128, 2, 12, 1500, 1.0, 1, 1), (32, 2, 16, 707, 0.46, 1, 1)]  # 67.6 / 60.5, 73.4 / 64.2
     half = _launch_rules(tmp_path, ["small_launch_dq(%d, %s, %d, 0, 0, 0, 1)" % (c[0], _rule_case(*c[1:5]), c[5]) for c in cases])
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
+    assert _launch_rules(tmp_path, ["small_launch_dq(128, live_row_tiles(16, 2218, 2), 32, 1109, %d, 1, 0, 0, 0, 1)" % k for k in (277, 1109)]) == [0, 1]
     rotary = [(6, 8, 1012, 1.0, 1, 1), (3, 8, 2177, 1.0, 1, 1), (1, 16, 3394, 1.0, 1, 1), (18, 16, 126, 1.0, 1, 1),  # 57.6 / 53.1 .. 26.3 / 25.4
               (27, 16, 90, 1.0, 1, 0), (12, 8, 609, 1.0, 1, 0), (8, 12, 460, 1.0, 1, 1)]
     half = _launch_rules(tmp_path, ["small_launch_dq(64, %s, %d, 0, 0, 1, 1)" % (_rule_case(*c[:4]), c[4]) for c in rotary])
