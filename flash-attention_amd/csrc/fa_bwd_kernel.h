@@ -70,6 +70,12 @@ struct BwdCfg {
   static constexpr int kBiasTileBytes = BM * 32 * 2;  // per wave, behind everything else: the bias-tensor variants' tile
 };
 
+// The variants that know kLiveOrder (map_live): the dense ones but those whose main loop it would cost registers
+template <bool kSparse, int kBias>
+struct DkdvLive {
+  static constexpr bool value = !kSparse && kBias != kBiasTensor;
+};
+
 // kDrop: 0 = no dropout; 1 = the keep decisions are drawn here (Philox); 2 = they are read from the keep words the
 // forward left (fa_common.h; dense only): the kernel then has the tile shape of the one without dropout.
 // kBias: as in fa_fwd_kernel; with a bias tensor the kernel also leaves d(loss)/d(bias) in p.dbias if that is not null
@@ -99,16 +105,25 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   static_assert(kBiasTileBytes == BwdCfg<T, D, kDrop == 1>::kBiasTileBytes, "LDS size of the kernel");
 
   // XCD-aware id map (see map_tile): the key tiles of one (batch, head) share one XCD's L2 copy of Q and dO.
-  int bh, kt;  // under a causal mask the first key tiles see the most query rows: rank order is already heavy-first
-  if (!map_tile<kCausal>(block, p.nk_tiles, p.B * p.H, &bh, &kt, p.tile_group)) return;
-  const int h = bh % p.H;
-  // (dense, no mask: the batch entries are taken longest first - here by their queries, which a key tile walks; longest_first)
-  const int b = (!kCausal && !kSparse && p.tile_group < 0) ? longest_first(p.cu_q, p.B, bh / p.H) : bh / p.H;
-  bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
+  int q_begin = 0, Lq = 0, k_begin = 0, Lk = 0;
+  int b, h, kt;  // under a causal mask the first key tiles see the most query rows: rank order is already heavy-first
+  if (DkdvLive<kSparse, kBias>::value && p.tile_group == kLiveOrder) {
+    TileId id;
+    if (!map_live<kCausal>(block, p.cu_k, p.total_k, p.max_sk, p.cu_q, p.total_q, p.max_sq, BN, p.nk_tiles, true, p.B, p.H, nullptr,
+                           lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
+    b = id.b; h = id.h; kt = id.tile;
+    k_begin = id.own_begin; Lk = id.own_len; q_begin = id.walk_begin; Lq = id.walk_len;
+  } else {
+    int bh;
+    if (!map_tile<kCausal>(block, p.nk_tiles, p.B * p.H, &bh, &kt, p.tile_group)) return;
+    h = bh % p.H;
+    // (dense, no mask: the batch entries are taken longest first - here by their queries, which a key tile walks; longest_first)
+    b = (!kCausal && !kSparse && p.tile_group == kLongestFirst) ? longest_first(p.cu_q, p.B, bh / p.H) : bh / p.H;
+    if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) return;
+    if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) Lq = 0;  // no queries: dK = dV = 0
+  }
+  const int bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
 
-  int q_begin = 0, Lq = 0, k_begin, Lk;
-  if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) return;
-  if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) Lq = 0;  // no queries: dK = dV = 0
   const int n0 = kt * BN;
   if (n0 >= Lk) return;
 
@@ -861,20 +876,29 @@ FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char
   constexpr int kBiasRowBytes = BN * 2 + 8, kBiasWaveBytes = 32 * kBiasRowBytes;
   static_assert(kBiasWaveBytes == Cfg::kBiasWaveBytes, "LDS size of the kernel");
 
-  int bh, rank;
+  int b, h, qt, split = 0;
+  int q_begin = 0, Lq = 0, k_begin = 0, Lk = 0;
   const int n_splits = p.n_splits > 1 ? p.n_splits : 1;  // key splits per query tile (see BwdParams)
-  if (!map_tile<kCausal>(block, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
-  const int split = rank % n_splits;
-  rank /= n_splits;
-  const int qt = kCausal ? p.nq_tiles - 1 - rank : rank;
-  const int h = bh % p.H;
-  // (dense, no mask: the batch entries are taken longest keys first, see longest_first)
-  const int b = (!kCausal && !kSparse && p.tile_group < 0) ? longest_first(p.cu_k, p.B, bh / p.H) : bh / p.H;
-  bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
+  if (!kSparse && p.tile_group == kLiveOrder) {
+    TileId id;
+    if (!map_live<kCausal>(block, p.cu_q, p.total_q, p.max_sq, p.cu_k, p.total_k, p.max_sk, BM, p.nq_tiles, false, p.B, p.H, nullptr,
+                           lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
+    b = id.b; h = id.h; qt = id.tile;
+    q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
+  } else {
+    int bh, rank;
+    if (!map_tile<kCausal>(block, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
+    split = rank % n_splits;
+    rank /= n_splits;
+    qt = kCausal ? p.nq_tiles - 1 - rank : rank;
+    h = bh % p.H;
+    // (dense, no mask: the batch entries are taken longest keys first, see longest_first)
+    b = (!kCausal && !kSparse && p.tile_group == kLongestFirst) ? longest_first(p.cu_k, p.B, bh / p.H) : bh / p.H;
+    if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
+    if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: dQ = 0
+  }
+  const int bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
 
-  int q_begin, Lq, k_begin = 0, Lk = 0;
-  if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
-  if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: dQ = 0
   const int m0 = qt * BM;
 
   const int tid = threadIdx.x, lane = tid & 63;

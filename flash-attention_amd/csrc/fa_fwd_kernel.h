@@ -55,6 +55,12 @@ struct FwdCfg {
   static constexpr int CH = D / 8;
 };
 
+// The variants that know kLiveOrder (map_live): the dense ones but those whose main loop it would cost registers
+template <int D, bool kSparse, int kBias>
+struct FwdLive {
+  static constexpr bool value = !kSparse && kBias != kBiasTensor && !(kBias == kPaddedRows && D == 128);
+};
+
 // kBias (fa_params.h): 1 = ALiBi, the score of (query i, key j) gets -slope[head] * |i - j| added after scaling; 2 = it gets
 // bias[b, h, i, j] of a tensor added.  The scores are then moved to the softmax's own units (base-2 exponent) before the row
 // maximum is taken, and the running maximum is kept in those units.
@@ -110,18 +116,29 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
 
   // Workgroup -> (batch, head, query tile), XCD-aware (see map_tile): the query tiles of one (batch, head) share
   // one XCD's L2 copy of K and V.
-  int bh, rank;
-  const int n_splits = p.n_splits > 1 ? p.n_splits : 1;   // key splits per query tile (see FwdParams)
-  if (!map_tile<kCausal>(blockIdx.x, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
-  const int split = rank % n_splits;
-  rank /= n_splits;
-  const int qt = kCausal ? p.nq_tiles - 1 - rank : rank;  // under a causal mask the last query tiles cost most
-  const int h = bh % p.H;
-  // (dense, no mask: the batch entries are taken longest keys first, see longest_first)
-  const int b = (!kCausal && !kSparse && p.tile_group < 0) ? longest_first(p.cu_k, p.B, bh / p.H, kRows ? p.row_info : nullptr) : bh / p.H;
-  bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
-
+  int b, h, qt, split = 0;
   int q_begin, Lq, k_begin = 0, Lk = 0;
+  const int n_splits = p.n_splits > 1 ? p.n_splits : 1;   // key splits per query tile (see FwdParams)
+  bool mapped = false;
+  if constexpr (FwdLive<D, kSparse, kBias>::value) mapped = p.tile_group == kLiveOrder;
+  if (mapped) {
+    TileId id;
+    if (!map_live<kCausal>(blockIdx.x, p.cu_q, p.total_q, p.max_sq, p.cu_k, p.total_k, p.max_sk, BM, p.nq_tiles, false, p.B, p.H,
+                           kRows ? p.row_info : nullptr, lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
+    b = id.b; h = id.h; qt = id.tile;
+    q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
+  } else {
+    int bh, rank;
+    if (!map_tile<kCausal>(blockIdx.x, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
+    split = rank % n_splits;
+    rank /= n_splits;
+    qt = kCausal ? p.nq_tiles - 1 - rank : rank;  // under a causal mask the last query tiles cost most
+    h = bh % p.H;
+    // (dense, no mask: the batch entries are taken longest keys first, see longest_first)
+    b = (!kCausal && !kSparse && p.tile_group == kLongestFirst) ? longest_first(p.cu_k, p.B, bh / p.H, kRows ? p.row_info : nullptr) : bh / p.H;
+  }
+  const int bh = b * p.H + h;  // (what the dropout counters and the keep words are indexed by)
+
   // kRows: this entry's slice of row_of; its tokens lie one after the other (from row q_begin on) or, `listed`, anywhere in it
   const int32_t* const row_of = kRows ? p.row_of + (int64_t)b * p.max_sq : nullptr;
   bool listed = false;
@@ -129,7 +146,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     Lq = Lk = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b]);
     listed = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 2]) == 0;
     q_begin = k_begin = b * p.max_sq + (listed ? 0 : __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 1]));
-  } else {
+  } else if (!mapped) {
     if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
     if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: o = 0, lse = -inf
   }

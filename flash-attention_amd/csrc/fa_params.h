@@ -64,7 +64,7 @@ struct FwdParams {
   int max_sq, max_sk;  // caller's bounds on the sequence lengths; longer sequences are truncated to them
   int sq_r;  // rounded max_seqlen_q = innermost extent of lse
   int nq_tiles;
-  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all
+  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst, kLiveOrder
   float scale;       // softmax_scale
   float scale_log2;  // softmax_scale * log2(e)
   float rp_keep;     // 1 / keep probability
@@ -148,7 +148,7 @@ struct BwdParams {
   int nk_tiles;      // key tiles of the dK/dV kernel
   int merged_dkdv_blocks, merged_nq_tiles;  // fa_bwd_merged_kernel: its dK/dV workgroups come first; query tiles of the dQ part
   int nq_tiles;      // query tiles of the dQ kernel
-  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all
+  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst, kLiveOrder
   float scale;
   float scale_log2;
   float p_keep;
@@ -200,7 +200,7 @@ FA_DEVICE bool seq_extent(const int32_t* cu, int b, int total, int max_len, int*
 // equal lengths keeps its order).  Every wave finds the entry itself: lane i holds entry i's length, counts the entries
 // that precede it (one readlane and compare per entry), and the lane whose count is `slot` is the answer.  Batches of
 // more than 64 entries keep their order.  The search costs every workgroup's prologue a few instructions per batch entry,
-// so the launchers ask for it (tile_group < 0 in a launch without a mask) only for grids that are resident all at once
+// so the launchers ask for it (tile_group == kLongestFirst in a launch without a mask) only for grids that are resident all at once
 // (longest_first_launch), where the spreading is what it buys.
 // (info: the lengths stand in row_info instead, see FwdParams)
 FA_DEVICE int longest_first(const int32_t* cu, int B, int slot, const int32_t* info = nullptr) {
@@ -267,6 +267,140 @@ FA_DEVICE bool map_tile(int block, int tiles_per_bh, int BH, int* bh, int* rank,
   *rank = (j - q * tiles_per_bh + q) % tiles_per_bh;
   return *bh < BH;
 }
+// Ragged batches (tile_group == kLiveOrder): workgroup ids enumerate the tiles that hold rows, the dearest first, and behind them the ones
+// that hold none.  The other two orders deal out (pair, rank) slots as if every sequence were the longest: the slots past a shorter one's end
+// exit at once, but the dispatcher gives the ids of an XCD to its shader engines strictly in turn, so where the live slots recur with a
+// period of 2 or 4 half of the compute units hold every live workgroup and the rest stand idle until the ids have passed (4 x 16 heads x 600 ..
+// 3001, d = 128, causal: 65 of 100 us); and the longest walks come where their pair comes.  us of the kernels in the other orders / here, same
+// bits: forward 4 x 16 x 600 .. 3001 d = 128 causal 102 / 90, 4 x 12 x 1800 .. 6000 d = 64 causal 186 / 146 (backward 567 / 438), 12 x 12 x 214 ..
+// 550 15.9 / 13.5, 64 x 8 x 36 .. 129 13.6 / 7.7; backward 7 x 12 x 1051 .. 2132 d = 128 causal 321 / 250, 57 x 8 x 55 .. 139 41.2 / 22.2.
+//
+// Lane i of a wave holds batch entry i (at most 64).  Every tile falls into one of 64 buckets, bucket 0 the dearest; a histogram in LDS and a
+// prefix sum over it find the bucket that a workgroup id falls into, and a prefix sum over the entries the tile in it: some 0.4 us, whatever
+// the batch (ranking the entries by readlanes took 1.5 us at 64 of them).
+//   kByTile (causal): cost grows with the tile's distance from the cheap end (its level); bucket = level, a lane's weight its pairs on this XCD;
+//   otherwise: bucket = length of the walk (cu_walk: the side that a tile walks over), weight = pairs x tiles, a pair's tiles one after the other.
+// The pairs of an entry go to the XCDs in turn and stay there.  Where the heads are no multiple of 8, the entries (up to 16) take their turns
+// longest first, so that neighbours in length share the rounding.
+// A launch that is resident all at once (at most four workgroups on each of an XCD's 32 compute units, which get ids in turn) walks every other
+// group of 32 backwards: the unit with the dearest of one group gets the cheapest of the next.
+// info: null, or the lengths of a padded batch (FwdParams::row_info), whose `tiles` tiles a pair are all visited (rows to be zeroed).
+// lds_wave: 256 bytes of the wave's own.
+constexpr int kLongestFirst = -1, kLiveOrder = -2;
+struct TileId {
+  int b, h, tile;
+  int own_begin, own_len, walk_begin, walk_len;  // as seq_extent has them (walk: 0 keys or queries where it skips the entry)
+};
+FA_DEVICE int wave_prefix_sum(int x) {  // inclusive
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+template <bool kByTile>
+FA_DEVICE bool map_live(int block, const int32_t* cu_own, int total_own, int max_own, const int32_t* cu_walk, int total_walk, int max_walk, int rows,
+                        int tiles, bool cheap_last, int B, int H, const int32_t* info, void* lds_wave, TileId* id) {
+  const int lane = threadIdx.x & 63;
+  const int i = lane < B ? lane : B - 1;
+  int begin = 0, n, walk_begin = 0, walk;
+  if (info) {
+    n = walk = info[kRowInfo * i];
+  } else {
+    begin = cu_own[i];
+    walk_begin = cu_walk[i];
+    const int e = cu_own[i + 1], we = cu_walk[i + 1];
+    n = e - begin;
+    if (begin < 0 || n <= 0 || e > total_own) n = 0;
+    n = n < max_own ? n : max_own;
+    walk = we - walk_begin;
+    if (walk_begin < 0 || walk <= 0 || we > total_walk) walk = 0;
+    walk = walk < max_walk ? walk : max_walk;
+  }
+  const int x = block & 7;
+  int j = block >> 3;
+  const int t = (int)(((uint32_t)n + rows - 1) / (uint32_t)rows);
+  int turn = i;
+  if ((H & 7) != 0 && B <= 16) {
+    const int key = walk << 4 | (15 - (i & 15));
+    turn = 0;
+    for (int e = 0; e < B; e++) turn += __builtin_amdgcn_readlane(key, e) > key ? 1 : 0;
+  }
+  // this XCD's pairs of entry i: heads h0, h0 + 8, ...
+  const int h0 = (x - turn * H) & 7, cnt = lane < B ? (H + 7 - h0) >> 3 : 0;
+  const int weight = kByTile ? cnt : cnt * t;
+  const int bucket = kByTile ? 64 - t : 63 - (int)((float)walk * (63.5f / (float)max_walk));  // 0: the dearest
+  volatile FA_LDS int* const hist = (volatile FA_LDS int*)lds_wave;
+  hist[lane] = 0;
+  if (t > 0) __hip_atomic_fetch_add((FA_LDS int*)lds_wave + bucket, weight, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  int size = hist[lane];
+  if (kByTile) size = wave_prefix_sum(size);  // pairs that reach level 63 - lane
+  const int end = wave_prefix_sum(size);
+  const int live = __builtin_amdgcn_readlane(end, 63);
+  if (j >= live) {
+    if (!info) return false;
+    j -= live;
+    const int rest = (tiles - t) * cnt, rest_end = wave_prefix_sum(rest);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(rest_end > j);
+    if (hit == 0) return false;
+    const int k = (int)__builtin_ctzll(hit);
+    const uint32_t r = (uint32_t)(j - (__builtin_amdgcn_readlane(rest_end, k) - __builtin_amdgcn_readlane(rest, k)));
+    const int tk = __builtin_amdgcn_readlane(t, k);
+    const uint32_t per = (uint32_t)(tiles - tk), q = r / per;
+    id->tile = tk + (int)(r - q * per);
+    id->h = __builtin_amdgcn_readlane(h0, k) + 8 * (int)q;
+    id->b = k;
+  } else {
+    if (live <= 4 * 32 && (j & 32)) {
+      const int left = live - (j & ~31);
+      j = (j & ~31) + (left < 32 ? left : 32) - 1 - (j & 31);
+    }
+    const int l = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(end > j));
+    int r = j - (__builtin_amdgcn_readlane(end, l) - __builtin_amdgcn_readlane(size, l));
+    const int mine = (kByTile ? bucket <= l : bucket == l) && t > 0 ? weight : 0;
+    const int mine_end = wave_prefix_sum(mine);
+    const int k = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(mine_end > r));
+    r -= __builtin_amdgcn_readlane(mine_end, k) - __builtin_amdgcn_readlane(mine, k);
+    const uint32_t tk = (uint32_t)__builtin_amdgcn_readlane(t, k);
+    uint32_t q = (uint32_t)r;
+    if (kByTile) {
+      id->tile = cheap_last ? (int)tk - 64 + l : 63 - l;
+    } else {
+      q = (uint32_t)r / tk;
+      id->tile = (int)((uint32_t)r - q * tk);
+    }
+    id->h = __builtin_amdgcn_readlane(h0, k) + 8 * (int)q;
+    id->b = k;
+  }
+  id->own_begin = __builtin_amdgcn_readlane(begin, id->b);
+  id->own_len = __builtin_amdgcn_readlane(n, id->b);
+  id->walk_begin = __builtin_amdgcn_readlane(walk_begin, id->b);
+  id->walk_len = __builtin_amdgcn_readlane(walk, id->b);
+  return true;
+}
+// Who takes it: dense launches of at most 64 batch entries (lanes) and 64 tiles a pair (buckets) whose lengths differ, at most 0.95 of batch x
+// longest being tokens; below that nothing is gained and the prologue costs up to 2 %.
+// - Without a mask all of them (0.54 to 1.04 of the time over 100 drawn shapes, 0.92 in the middle), but dQ and dK/dV in one launch only
+//   where it is not resident at once: 3 x 12 x 414 .. 910 35.3 / 38.8, 2 x 16 x 728 .. 1234 48.1 / 51.7; 8 x 12 x 256 .. 512 33.4 / 31.8.
+// - Under a causal mask the other orders have their empty slots at one end.  The forward and dQ take it where at most nine tenths of the slots hold
+//   rows (38 x 16 x 414 .. 628 46.1 / 48.8) of more than 256-token sequences (64 x 8 x 42 .. 109 7.9 / 8.2, 64 x 16 x 172 .. 202 d = 128 42.4 /
+//   44.7) in more than 150 workgroups (2 x 12 x 553 .. 787 14.8 / 15.4), dK/dV, whose empty slots come last, where its pairs are taken in groups
+//   (causal_tile_group; 3 x 16 x 2821 .. 5841 dQ alone 481, both 441; 14 x 16 x 471 .. 703, no groups, 82.0 / 86.1).  At d = 32 many
+//   pairs in groups stay with them, whose K and V it would read again: 64 x 16 x 509 .. 926 100.9 / 122.5, 38 x 12 x 353 .. 1766 91.2 / 101.2.
+enum LiveKernel { kLiveFwd, kLiveDq, kLiveDkdv, kLiveMerged };
+inline bool live_order_launch(LiveKernel kernel, int head_dim, bool causal, int B, int H, int total, int max_s, int n_splits, int tiles, int tile_group,
+                              int grid) {
+  if (n_splits > 1 || B > 64 || tiles > 64 || (int64_t)total * 20 > (int64_t)19 * B * max_s) return false;
+  if (kernel == kLiveMerged) return !causal && grid > 1024;
+  if (!causal) return true;
+  if (kernel == kLiveDkdv && (tile_group <= 0 || max_s <= 640)) return false;
+  if (head_dim <= 32 && tile_group > 0 && B * H >= 256) return false;
+  const int64_t live = (int64_t)H * (total + (int64_t)64 * B) / 128;
+  return max_s > 256 && live > 150 && 10 * live <= (int64_t)9 * B * H * ((max_s + 127) / 128);
+}
+inline bool live_order_rows(int B, int tiles) { return B <= 64 && tiles <= 64; }
 inline int tile_grid(bool tile_major, int tiles_per_bh, int BH) {
   return ((BH + 7) & ~7) * tiles_per_bh;
 }

@@ -762,3 +762,19 @@ def test_padded_forward_tiles_follow_the_measurements(tmp_path):
         (128, 8, 12, 156, 0, 0), (128, 12, 16, 209, 0, 0), (128, 8, 16, 272, 1, 0), (128, 16, 8, 1500, 1, 0), (64, 32, 16, 512, 0, 0), (64, 8, 8, 512, 0, 1)]  # 10.3 / 11.7, 13.5 / 15.6
     half = _launch_rules(tmp_path, ["small_launch_rows(%d, %d, %d, %d, %d)" % c[:-1] for c in cases])
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
+
+
+def test_live_order_where_measured(tmp_path):
+    """ragged launches whose workgroups enumerate the tiles that hold rows, and those that keep the slot orders"""
+    cases = [  # kernel, head dim, causal, batch, heads, longest, shortest / longest, tile_group, grid, live order?
+        ("kLiveFwd", 128, 1, 4, 16, 3001, 0.2, 4, 1536, 1), ("kLiveFwd", 64, 0, 12, 12, 550, 0.39, 0, 720, 1), ("kLiveDq", 64, 1, 4, 12, 6000, 0.3, 4, 2256, 1),
+        ("kLiveDkdv", 64, 1, 3, 16, 5841, 0.483, 4, 2208, 1), ("kLiveMerged", 64, 0, 8, 12, 512, 0.5, 0, 1152, 1), ("kLiveDkdv", 64, 0, 57, 8, 139, 0.39, 0, 912, 1),
+        ("kLiveFwd", 64, 0, 64, 16, 1023, 0.982, 0, 8192, 0), ("kLiveFwd", 64, 0, 65, 8, 500, 0.5, 0, 2080, 0), ("kLiveFwd", 64, 0, 2, 8, 8193, 0.5, 0, 1040, 0),
+        ("kLiveMerged", 64, 0, 3, 12, 910, 0.455, 0, 960, 0), ("kLiveMerged", 64, 1, 8, 12, 512, 0.5, 0, 1152, 0), ("kLiveFwd", 64, 1, 38, 16, 628, 0.66, 0, 3040, 0),
+        ("kLiveFwd", 64, 1, 64, 8, 109, 0.383, 0, 512, 0), ("kLiveFwd", 64, 1, 2, 12, 787, 0.703, 0, 168, 0), ("kLiveDkdv", 64, 1, 14, 16, 703, 0.67, 0, 1344, 0),
+        ("kLiveFwd", 32, 1, 64, 16, 926, 0.55, 53, 8192, 0)]
+    got = _launch_rules(tmp_path, ["live_order_launch(%s, %d, %d, %d, %d, %d, %d, 1, %d, %d, %d)" % (
+        k, d, c, b, h, _spread(n, f, b), n, -(-n // 128), group, grid) for k, d, c, b, h, n, f, group, grid, _ in cases])
+    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+    assert _launch_rules(tmp_path, ["live_order_launch(kLiveFwd, 64, 0, 4, 8, 1000, 1000, 2, 8, 0, 256)", "live_order_rows(64, 64)", "live_order_rows(65, 1)",
+                                    "live_order_rows(1, 65)"]) == [0, 1, 0, 0]

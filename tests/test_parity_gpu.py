@@ -2732,3 +2732,64 @@ def test_key_split_backward(lens_q, lens_k, D, p):
     for got in (dq_s, dq_1):
         check_against_oracle({"dq": got}, ref, half, dtype, names=("dq",), what="key-split backward")
     assert (dq_s.float() - dq_1.float()).abs().max() <= 2.0 ** -10 * max(1.0, ref["dq"].abs().max().item())
+
+
+# lengths of ragged batches at the edges of the live order (map_live): 64 entries, heads that are no multiple of 8, empty sequences, one long
+# entry among short ones, 64 tiles a pair (no sequence within the decode kernel's 32 rows, which would take it alone), grids beyond and within what is resident at once; (heads, head dim, lengths)
+LIVE_ORDER_BATCHES = [(12, 64, [700, 33, 0, 129, 512, 640, 64, 385]), (16, 64, [1500] + [300 + 7 * i for i in range(31)]), (8, 128, [2000, 0, 900, 257, 1300, 128]),
+                      (3, 32, [(97 * i) % 330 + 33 for i in range(64)]), (5, 16, [8192, 100, 4000]), (12, 64, [3000, 1100, 2100])]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("H, D, lens", LIVE_ORDER_BATCHES)
+def test_live_order_reaches_every_tile(H, D, lens, causal, full_size_tiles):
+    """A ragged batch is, sequence by sequence and bit for bit, what the sequences give alone (launches of one length, in the slot order): no tile
+    is left out and none is computed with another entry's rows."""
+    from flash_attn import flash_attn_gfx950 as be
+    N, cu, dtype = max(lens), _cu(lens), torch.float16
+    q, k, v, do = (x.cuda() for x in _inputs(lens, lens, H, D, dtype, 7))
+
+    def both(q, k, v, do, cu, n):
+        out, lse = be.fwd(q, k, v, cu, cu, n, n, 0.0, D ** -0.5, False, causal, False, None)
+        dq, dk, dv = (torch.full_like(q, float("nan")) for _ in range(3))
+        be.bwd(do, q, k, v, out, lse, dq, dk, dv, cu, cu, n, n, 0.0, D ** -0.5, False, causal, None)
+        return out, dq, dk, dv
+
+    whole = both(q, k, v, do, cu, N)
+    for b, n in enumerate(lens):
+        if n == 0:
+            continue
+        a = sum(lens[:b])
+        alone = both(*(x[a:a + n] for x in (q, k, v, do)), _cu([n]), n)
+        for name, x, y in zip(("out", "dq", "dk", "dv"), whole, alone):
+            assert torch.equal(x[a:a + n], y), (name, b, n)
+
+
+@pytest.mark.parametrize("listed", [False, True])
+@pytest.mark.parametrize("B, H, D, N, causal", [(64, 3, 64, 200, False), (5, 12, 32, 700, True), (3, 16, 64, 1100, False)])
+def test_padded_batches_in_live_order_write_every_row(B, H, D, N, causal, listed):
+    """A padded batch in place: token rows are those of a launch that holds nothing but its sequence (one entry, lengths equal), padding rows are
+    zeros, entries without any token included."""
+    from flash_attn.flash_attention import FlashAttention
+    g = torch.Generator(device="cuda").manual_seed(3)
+    qkv = torch.randn(B, N, 3, H, D, device="cuda", generator=g).half()
+    lens = torch.randint(0, N + 1, (B,), generator=g, device="cuda")
+    lens[0], lens[-1] = N, 0
+    mask = torch.arange(N, device="cuda")[None] < lens[:, None]
+    if listed:
+        mask = mask & (torch.rand(B, N, device="cuda", generator=g) < 0.8)
+    module = FlashAttention().eval()
+    with torch.no_grad():
+        out = module(qkv, key_padding_mask=type("Mask", (), {"bool_matrix": mask}), causal=causal)[0]
+    assert out[~mask].abs().max() == 0
+    for b in range(B):
+        x = qkv[b][mask[b]].float()
+        if x.shape[0] == 0:
+            continue
+        qh, kh, vh = (x[:, i].transpose(0, 1).contiguous() for i in range(3))
+        s = torch.matmul(qh, kh.transpose(1, 2).contiguous()) * D ** -0.5
+        if causal:
+            s = s.masked_fill(torch.ones_like(s[0], dtype=torch.bool).triu(1), float("-inf"))
+        ref = torch.matmul(s.softmax(-1), vh).transpose(0, 1)
+        # probabilities and outputs are rounded to 11 bits: 2^-11 of values up to max |v|, twice, and the fp32 sums
+        assert (out[b][mask[b]].float() - ref).abs().max() <= 3 * HALF_ULP[torch.float16] * x[:, 2].abs().max(), b
