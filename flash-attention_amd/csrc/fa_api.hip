@@ -80,6 +80,7 @@ Rounded round_seqlens(int head_dim, int max_sq, int max_sk, bool blocksparse) {
 struct SparseLayout {
   int nrb, ncb, nqt, ncw, nrw;
   size_t offr, offq, offc, offi, bytes;
+  size_t offs, bytes_sorted;  // the tiles dearest first, behind what the maps need: scratch for them is asked for, but may be missing
 };
 
 SparseLayout sparse_layout(const Rounded& r) {
@@ -94,6 +95,8 @@ SparseLayout sparse_layout(const Rounded& r) {
   s.offc = s.offq + align16((size_t)s.nqt * s.ncw * 8);
   s.offi = s.offc + align16((size_t)s.ncb * s.nrw * 8);  // inverse of the row order
   s.bytes = s.offi + align16((size_t)s.nrb * 4);
+  s.offs = s.bytes;
+  s.bytes_sorted = s.offs + align16(((size_t)s.nqt * (fa::kFwdBM / 16) + s.ncb) * 4);
   return s;
 }
 
@@ -170,13 +173,20 @@ bool decode_needs_splits(int batch, int nheads, int head_dim, int max_sk) {
   return head_dim == 64 && (int64_t)batch * nheads < 448 && max_sk > 512;
 }
 
-int build_maps(const int32_t* blockmask, const int32_t* row_order, unsigned char* ws, const SparseLayout& sl,
+// (ws_bytes: at least sl.bytes)
+int build_maps(const int32_t* blockmask, const int32_t* row_order, bool causal, unsigned char* ws, size_t ws_bytes, const SparseLayout& sl,
                fa::SparseMaps* out, hipStream_t stream) {
+  if (causal) row_order = nullptr;  // (the tile ranges there follow the rows' positions)
+  int32_t* const sorted = !causal && ws_bytes >= sl.bytes_sorted ? reinterpret_cast<int32_t*>(ws + sl.offs) : nullptr;
+  bool is_sorted = false;
   FA_LAUNCH(fa::launch_build_sparse_maps(blockmask, reinterpret_cast<uint64_t*>(ws + sl.offr),
                                          reinterpret_cast<uint64_t*>(ws + sl.offq),
                                          reinterpret_cast<uint64_t*>(ws + sl.offc), sl.nrb, sl.ncb, fa::kFwdBM, sl.nqt,
-                                         sl.ncw, sl.nrw, row_order, reinterpret_cast<int32_t*>(ws + sl.offi), ws, sl.bytes, stream));
-  out->order = row_order;
+                                         sl.ncw, sl.nrw, row_order, reinterpret_cast<int32_t*>(ws + sl.offi), sorted, &is_sorted, ws, sl.bytes,
+                                         stream));
+  out->order = is_sorted ? sorted : row_order;
+  out->n_order = is_sorted ? sl.nqt * (fa::kFwdBM / 16) : sl.nrb;
+  out->corder = is_sorted ? sorted + out->n_order : nullptr;
   out->rbits = reinterpret_cast<const uint64_t*>(ws + sl.offr);
   out->qbits = reinterpret_cast<const uint64_t*>(ws + sl.offq);
   out->cbits = reinterpret_cast<const uint64_t*>(ws + sl.offc);
@@ -260,7 +270,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block, const int32_t* row_of = null
       return fail(FA_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", sl.bytes, a->workspace_bytes);
     FA_REQUIRE(aligned16(a->workspace), "workspace must be 16-byte aligned");
     FA_REQUIRE(!a->row_order || (reinterpret_cast<uintptr_t>(a->row_order) & 3) == 0, "row_order must be 4-byte aligned");
-    rc = build_maps(a->blockmask, a->is_causal ? nullptr : a->row_order, reinterpret_cast<unsigned char*>(a->workspace), sl,
+    rc = build_maps(a->blockmask, a->row_order, a->is_causal != 0, reinterpret_cast<unsigned char*>(a->workspace), a->workspace_bytes, sl,
                     &p.sp, stream);
     if (rc) return rc;
   }
@@ -284,7 +294,7 @@ int fwd_impl(const fa_fwd_args* a, bool want_block, const int32_t* row_of = null
   p.max_sq = a->max_seqlen_q; p.max_sk = a->max_seqlen_k;
   p.sq_r = r.sq_r;
   p.nq_tiles = (a->max_seqlen_q + fa::kFwdBM - 1) / fa::kFwdBM;
-  p.tile_group = a->is_causal ? causal_tile_group(a->batch, a->nheads, a->head_dim, a->max_seqlen_k) : 0;
+  p.tile_group = a->is_causal || p.sp.corder ? causal_tile_group(a->batch, a->nheads, a->head_dim, a->max_seqlen_k) : 0;
   p.scale = a->softmax_scale;
   p.scale_log2 = a->softmax_scale * fa::kLog2e;
   p.rp_keep = 1.f / p_keep;
@@ -422,7 +432,7 @@ int bwd_impl(const fa_bwd_args* a, bool want_block, void* ev_main_start = nullpt
   memset(&p, 0, sizeof(p));
   if (sparse) {
     FA_REQUIRE(!a->row_order || (reinterpret_cast<uintptr_t>(a->row_order) & 3) == 0, "row_order must be 4-byte aligned");
-    rc = build_maps(a->blockmask, a->is_causal ? nullptr : a->row_order, ws, sl, &p.sp, stream);
+    rc = build_maps(a->blockmask, a->row_order, a->is_causal != 0, ws, a->workspace_bytes, sl, &p.sp, stream);
     if (rc) return rc;
   }
   if (a->zero_tensors) {  // fmha_api.cpp:406-411
@@ -447,9 +457,10 @@ int bwd_impl(const fa_bwd_args* a, bool want_block, void* ev_main_start = nullpt
   p.total_q = a->total_q; p.total_k = a->total_k;
   p.max_sq = a->max_seqlen_q; p.max_sk = a->max_seqlen_k;
   p.sq_r = r.sq_r; p.lse_stride = a->lse_seq_stride;
-  p.nk_tiles = (a->max_seqlen_k + fa::kBwdBN - 1) / fa::kBwdBN;
+  // (key blocks in an order of their own: two tiles each, the last one's second may lie past the last key)
+  p.nk_tiles = p.sp.corder ? 256 / fa::kBwdBN * sl.ncb : (a->max_seqlen_k + fa::kBwdBN - 1) / fa::kBwdBN;
   p.nq_tiles = (a->max_seqlen_q + fa::kFwdBM - 1) / fa::kFwdBM;
-  p.tile_group = a->is_causal ? causal_tile_group(a->batch, a->nheads, a->head_dim, a->max_seqlen_k) : 0;
+  p.tile_group = a->is_causal || p.sp.corder ? causal_tile_group(a->batch, a->nheads, a->head_dim, a->max_seqlen_k) : 0;
   p.scale = a->softmax_scale;
   p.scale_log2 = a->softmax_scale * fa::kLog2e;
   p.p_keep = p_keep;
@@ -619,7 +630,7 @@ int fa_bwd_block(const fa_bwd_args* args) { return bwd_impl(args, true); }
 
 size_t fa_fwd_workspace_bytes(const fa_fwd_args* a) {
   if (!a) return 0;
-  if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes;
+  if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes_sorted;
   const Rounded r = round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, false);
   if (decode_launch(a->batch, a->nheads, a->head_dim, a->total_k, a->max_seqlen_q, a->max_seqlen_k, a->is_causal != 0, false,
                     a->p_dropout > 0.f, a->alibi_slopes || a->attn_bias)) {
@@ -632,7 +643,7 @@ size_t fa_fwd_workspace_bytes(const fa_fwd_args* a) {
 
 size_t fa_bwd_workspace_bytes(const fa_bwd_args* a) {
   if (!a) return 0;
-  if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes;
+  if (a->blockmask) return sparse_layout(round_seqlens(a->head_dim, a->max_seqlen_q, a->max_seqlen_k, true)).bytes_sorted;
   // optional: the fp32 dQ and counters of the one-kernel backward, or the partial dQ of the key-split dQ kernel (same plan as
   // the forward's; o_bytes is n_splits fp32 copies of dq)
   const size_t fused = fused_bwd_bytes(a);

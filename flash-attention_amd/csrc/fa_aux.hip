@@ -59,11 +59,15 @@ __global__ void sparse_maps_kernel(const int32_t* blockmask, uint32_t* rbits, ui
 // owns once; a query tile's bits are the OR of its row blocks', read off the order as it is.  Latency-bound; with many entries one workgroup
 // per 64 key blocks is too few, see launch_build_sparse_maps.  (A training step builds them twice: 4 x 16 heads x 4096, a quarter of the
 // blocks, 508 -> 501 us.)
-constexpr int kMapsRows = 2048, kMapsThreads = 1024;
+// sorted: null, or (one workgroup holds the whole layout) where the query tiles are listed dearest first - qbits in that order, and the row
+// blocks of each, -1 where it has fewer than eight, as a row order of 8 nqt entries - and behind them the key blocks, those with the most row
+// blocks first.  A tile's cost: the key blocks its workgroup stages and those its waves (two row blocks each) compute on.
+constexpr int kMapsRows = 2048, kMapsThreads = 1024, kMapsRowsPerTile = kFwdBM / 16;
 __global__ void __launch_bounds__(kMapsThreads) sparse_maps_lds_kernel(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits,
                                                                        int nrb, int ncb, int rpq, int nqt, int ncw, int nrw,
-                                                                       const int32_t* order) {
+                                                                       const int32_t* order, int32_t* sorted) {
   __shared__ __attribute__((aligned(8))) uint32_t rl[kMapsRows * 2], cl[64 * (kMapsRows / 32)];
+  __shared__ int qcost[kMapsRows / kMapsRowsPerTile], kcost[64];
   const int w = blockIdx.x, cb0 = w * 64, tid = threadIdx.x;
   const int ncols = ncb - cb0 < 64 ? ncb - cb0 : 64;
   for (int i = tid; i < nrb * 2; i += kMapsThreads) rl[i] = 0;
@@ -81,15 +85,66 @@ __global__ void __launch_bounds__(kMapsThreads) sparse_maps_lds_kernel(const int
   const uint64_t* const cw = reinterpret_cast<const uint64_t*>(cl);
   for (int i = tid; i < nrb; i += kMapsThreads) rbits[(int64_t)i * ncw + w] = rw[i];
   for (int i = tid; i < ncols * nrw; i += kMapsThreads) cbits[(int64_t)cb0 * nrw + i] = cw[i];
-  for (int t = tid; t < nqt; t += kMapsThreads) {
-    uint64_t q = 0;
-    for (int j = 0; j < rpq; j++) {
-      const int pos = t * rpq + j;
-      int rb = pos < nrb ? (order ? order[pos] : pos) : -1;
-      if (rb >= 0 && rb < nrb) q |= rw[rb];
+  auto row_at = [&](int pos) {  // the row block at a position of the order, -1: none
+    const int rb = pos < nrb ? (order ? order[pos] : pos) : -1;
+    return rb < nrb ? rb : -1;
+  };
+  if (sorted == nullptr) {
+    for (int t = tid; t < nqt; t += kMapsThreads) {
+      uint64_t q = 0;
+      for (int j = 0; j < rpq; j++) {
+        const int rb = row_at(t * rpq + j);
+        if (rb >= 0) q |= rw[rb];
+      }
+      qbits[(int64_t)t * ncw + w] = q;
     }
-    qbits[(int64_t)t * ncw + w] = q;
+    return;
   }
+  // A thread per position of the order (two of them beyond 1024 row blocks): the eight lanes of a tile share its sums, and the comparisons
+  // that rank it; then 16 lanes per key block
+  constexpr int R = kMapsRowsPerTile, kRounds = kMapsRows / kMapsThreads;
+  static_assert(R == 8, "a tile is eight lanes");
+  int rb[kRounds], cost[kRounds];
+  uint64_t q[kRounds];
+#pragma unroll
+  for (int n = 0; n < kRounds; n++) {
+    const int pos = tid + n * kMapsThreads;
+    rb[n] = row_at(pos);
+    const uint64_t bits = rb[n] >= 0 ? rw[rb[n]] : 0;
+    const uint64_t slab = bits | __shfl_xor(bits, 1);
+    q[n] = slab | __shfl_xor(slab, 2);
+    q[n] |= __shfl_xor(q[n], 4);
+    int c = __popcll(slab);
+    c += __shfl_xor(c, 2);
+    c += __shfl_xor(c, 4);
+    cost[n] = c + __popcll(q[n]);
+    if (pos % R == 0 && pos / R < nqt) qcost[pos / R] = cost[n];
+  }
+  const int cb = tid >> 4, l = tid & 15;
+  int kc = 0;
+  if (cb < ncb)
+    for (int i = l; i < nrw; i += 16) kc += __popcll(cw[cb * nrw + i]);
+#pragma unroll
+  for (int d = 1; d < 16; d *= 2) kc += __shfl_xor(kc, d);
+  if (l == 0 && cb < ncb) kcost[cb] = kc;
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < kRounds; n++) {
+    const int pos = tid + n * kMapsThreads, t = pos / R;
+    int rank = 0;
+    for (int u = pos % R; u < nqt; u += R) rank += (qcost[u] > cost[n] || (qcost[u] == cost[n] && u < t)) ? 1 : 0;
+#pragma unroll
+    for (int d = 1; d < R; d *= 2) rank += __shfl_xor(rank, d);
+    if (t < nqt) {
+      if (pos % R == 0) qbits[rank] = q[n];
+      sorted[rank * R + pos % R] = rb[n];
+    }
+  }
+  int rank = 0;
+  for (int u = l; u < ncb; u += 16) rank += (kcost[u] > kc || (kcost[u] == kc && u < cb)) ? 1 : 0;
+#pragma unroll
+  for (int d = 1; d < 16; d *= 2) rank += __shfl_xor(rank, d);
+  if (l == 0 && cb < ncb) sorted[R * nqt + rank] = cb;
 }
 
 // One thread per (query row, key) element of S_dmask.  Slow scalar dot products: this path exists for tests
@@ -156,14 +211,16 @@ hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride,
 }
 
 hipError_t launch_build_sparse_maps(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits, int nrb,
-                                    int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv,
-                                    void* maps, size_t maps_bytes, hipStream_t stream) {
+                                    int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv, int32_t* sorted,
+                                    bool* is_sorted, void* maps, size_t maps_bytes, hipStream_t stream) {
   const int n = nrb * ncb;
-  // us of one launch / of the three below, their gaps not counted: 64 x 4 blocks 2.9 / 5.9, 256 x 16 4.5 / 7.9, 512 x 32 9.4 / 17.2,
+  // us of one launch (the ranking, some 1, not counted) / of the three below, their gaps not counted: 64 x 4 blocks 2.9 / 5.9, 256 x 16 4.5 / 7.9, 512 x 32 9.4 / 17.2,
   // 1024 x 64 27.4 / 23.1 (64 entries a thread of one workgroup)
+  *is_sorted = false;
   if (nrb <= kMapsRows && n <= 16384) {
+    *is_sorted = sorted != nullptr && ncw == 1;
     hipLaunchKernelGGL(sparse_maps_lds_kernel, dim3((unsigned)ncw), dim3(kMapsThreads), 0, stream, blockmask, rbits, qbits, cbits, nrb, ncb,
-                       rows_per_qt / 16, nqt, ncw, nrw, order);
+                       rows_per_qt / 16, nqt, ncw, nrw, order, *is_sorted ? sorted : nullptr);
     return hipGetLastError();
   }
   const hipError_t e = launch_fill_f32(reinterpret_cast<float*>(maps), maps_bytes / 4, 0.f, stream);

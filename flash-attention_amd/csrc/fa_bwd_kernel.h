@@ -115,7 +115,12 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
     k_begin = id.own_begin; Lk = id.own_len; q_begin = id.walk_begin; Lq = id.walk_len;
   } else {
     int bh;
-    if (!map_tile<kCausal>(block, p.nk_tiles, p.B * p.H, &bh, &kt, p.tile_group)) return;
+    if (kSparse && p.sp.corder != nullptr) {
+      if (!map_tile<true>(block, p.nk_tiles, p.B * p.H, &bh, &kt, p.tile_group)) return;
+      kt = (256 / Cfg::BN) * p.sp.corder[kt / (256 / Cfg::BN)] + kt % (256 / Cfg::BN);
+    } else if (!map_tile<kCausal>(block, p.nk_tiles, p.B * p.H, &bh, &kt, p.tile_group)) {
+      return;
+    }
     h = bh % p.H;
     // (dense, no mask: the batch entries are taken longest first - here by their queries, which a key tile walks; longest_first)
     b = (!kCausal && !kSparse && p.tile_group == kLongestFirst) ? longest_first(p.cu_q, p.B, bh / p.H) : bh / p.H;
@@ -887,7 +892,9 @@ FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char
     q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
   } else {
     int bh, rank;
-    if (!map_tile<kCausal>(block, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
+    if (kSparse && p.sp.corder != nullptr ? !map_tile<true>(block, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)
+                                          : !map_tile<kCausal>(block, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group))
+      return;
     split = rank % n_splits;
     rank /= n_splits;
     qt = kCausal ? p.nq_tiles - 1 - rank : rank;

@@ -129,7 +129,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
   } else {
     int bh, rank;
-    if (!map_tile<kCausal>(blockIdx.x, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)) return;
+    if (kSparse && p.sp.corder != nullptr ? !map_tile<true>(blockIdx.x, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group)
+                                          : !map_tile<kCausal>(blockIdx.x, p.nq_tiles * n_splits, p.B * p.H, &bh, &rank, p.tile_group))
+      return;
     split = rank % n_splits;
     rank /= n_splits;
     qt = kCausal ? p.nq_tiles - 1 - rank : rank;  // under a causal mask the last query tiles cost most

@@ -27,13 +27,20 @@ struct SparseMaps {
   // blocks next to each other makes a workgroup stage few tiles that only one of its row blocks needs.  Not used under a
   // causal mask (the tile ranges there follow the rows' positions).
   const int32_t* order;
+  int n_order;  // its entries, -1 for none (nrb without an order)
+  // The key blocks, those with the most row blocks first (or null).  Where it is given the query tiles are in such an order, too (order and
+  // qbits are), and workgroup ids enumerate ranks outermost, as under a causal mask: tiles differ in cost by a factor of two, and a launch that
+  // ends on a dear one leaves a fifth of the compute units idle over its length.  us before / now, fp16, 16 queries x 256 keys blocks a
+  // quarter full: 4 x 16 heads x 4096 forward 172 / 157, dQ 211 / 200, dK/dV 159 / 156; 8 x 12 x 1033 (bf16, 35 %) 38 / 28, 42 / 33,
+  // 38 / 34; 256 x 256 blocks, 4 x 16 x 4096 121 / 110, 149 / 138, 194 / 176.  25 drawn shapes, step: 0.92 of the time, none above 1.012.
+  const int32_t* corder;
 };
 
 // The two 16-row blocks of the 32-row slab `slab` (0 .. 3) of query tile qt: positions 8 qt + 2 slab and + 1 of the row
 // order; -1 = none (past the last row block, or an entry that is not a row block).
 FA_DEVICE void slab_row_blocks(const SparseMaps& sp, bool ordered, int qt, int slab, int* a, int* b) {
   const int pos = 8 * qt + 2 * slab;
-  int ra = pos < sp.nrb ? pos : -1, rb = pos + 1 < sp.nrb ? pos + 1 : -1;
+  int ra = pos < sp.n_order ? pos : -1, rb = pos + 1 < sp.n_order ? pos + 1 : -1;
   if (ordered) {
     if (ra >= 0) ra = sp.order[pos];
     if (rb >= 0) rb = sp.order[pos + 1];
@@ -622,9 +629,10 @@ hipError_t launch_bwd(const BwdParams& p, int which, int dtype, int head_dim, bo
                       hipStream_t stream);
 // maps, maps_bytes: the scratch that holds all of them (cleared where they are built with atomics)
 // order / inv: null, or the row order (SparseMaps::order) and nrb ints of scratch for its inverse
+// sorted: null, or scratch for SparseMaps::order and corder, dearest first; *is_sorted: whether they were left there
 hipError_t launch_build_sparse_maps(const int32_t* blockmask, uint64_t* rbits, uint64_t* qbits, uint64_t* cbits, int nrb,
-                                    int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv,
-                                    void* maps, size_t maps_bytes, hipStream_t stream);
+                                    int ncb, int rows_per_qt, int nqt, int ncw, int nrw, const int32_t* order, int32_t* inv, int32_t* sorted,
+                                    bool* is_sorted, void* maps, size_t maps_bytes, hipStream_t stream);
 hipError_t launch_fill_f32(float* p, size_t n, float value, hipStream_t stream);
 // Zero a strided [total, H, D] tensor of 16-bit elements.
 hipError_t launch_zero_rows(void* base, int64_t row_stride, int64_t head_stride, int total, int H, int D,

@@ -200,7 +200,7 @@ int fa_bwd_block(const fa_bwd_args* args);
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the block activity maps that
  * fa_fwd_block keeps in `workspace` live in a device array inside the library instead (FA_NOALLOC_SCRATCH_BYTES, held by
  * every GPU the library runs on until the process ends).  args->workspace / workspace_bytes are ignored; inputs and
- * outputs are the caller's as usual.  Layouts whose maps need more (fa_fwd_workspace_bytes() > FA_NOALLOC_SCRATCH_BYTES;
+ * outputs are the caller's as usual.  Layouts whose maps need more (about what fa_fwd_workspace_bytes() says;
  * the limit is reached between 16384 and 32768 tokens) are refused with FA_ERR_WORKSPACE.  The call allocates nothing
  * and the maps are rebuilt by every call, but all calls on one GPU share the one array: calls that overlap on a GPU
  * (different streams or host threads) race; serialise them.  The first call on a device looks up the array's device
@@ -211,7 +211,7 @@ int fa_fwd_block_noalloc(const fa_fwd_args* args);
 
 /* Scratch the caller provides.  The dense forward and backward need none to be correct
  * (there is no o_tmp / dq_tmp, fmha_api.cpp:247,403-404).  The block-sparse paths need room for their block activity
- * maps (an error without it).  For a dense, non-causal forward with few query rows (max_seqlen_q <= 128: decoding and cross-attention
+ * maps (an error without it) and are asked for that of an order of their tiles (taken in any order without it).  For a dense, non-causal forward with few query rows (max_seqlen_q <= 128: decoding and cross-attention
  * shapes) and more keys than its (batch, head) pairs alone would spread over the GPU, fa_fwd_workspace_bytes() returns the size of
  * the partial results of a key-split pass: if `workspace` holds that much, fa_fwd shares the keys of each query tile
  * among several workgroups and merges their results; if not, it runs the single pass.  Arguments that fa_fwd refuses need none.  fa_bwd_workspace_bytes() does the

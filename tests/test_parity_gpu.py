@@ -1312,6 +1312,30 @@ def test_blocksparse_row_order(D, N, dtype):
         be.fwd_block(qg, kg, vg, cug, cug, conv, N, N, 0.0, D ** -0.5, False, False, None, row_order=bad)
 
 
+@pytest.mark.parametrize("Sq,Sk,H,B", [(16, 100, 1, 1), (300, 257, 3, 3), (130, 15900, 2, 2), (16390, 300, 1, 1)])
+def test_blocksparse_tiles_dearest_first(Sq, Sk, H, B):
+    """Workgroups take a layout's query tiles and key blocks dearest first: one tile of each, a last key block half of whose keys have no
+    tile, heads that are no multiple of the XCDs, 63 key blocks, and more row blocks than the kernel that ranks them has threads"""
+    from flash_attn import flash_attn_gfx950 as be
+    from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
+    D, dtype = 64, torch.float16
+    lens_q, lens_k = [Sq - 37 * i for i in range(B)], [Sk - 129 * i if Sk > 300 else Sk - 20 * i for i in range(B)]
+    sq_r, sk_r = be.round_seqlens(D, Sq, Sk, True)
+    layout = _layout(sq_r // 16, sk_r // 256, 0.4, Sq + Sk)
+    q, k, v, do = _inputs(lens_q, lens_k, H, D, dtype, Sq)
+    cu_q, cu_k = _cu(lens_q, "cpu"), _cu(lens_k, "cpu")
+    ref = orc.varlen_attention(q, k, v, cu_q, cu_k, None, False, layout=layout.numpy(), dout=do)
+    qg, kg, vg, dog = q.cuda(), k.cuda(), v.cuda(), do.cuda()
+    half = half_attention(qg, kg, vg, cu_q.tolist(), cu_k.tolist(), D ** -0.5, False, layout=layout.numpy(), dout=dog)
+    conv = convert_blockmask(layout.cuda(), causal=False)
+    for order in (None, be.blockmask_row_order(layout.cuda())):
+        o, lse = be.fwd_block(qg, kg, vg, cu_q.cuda(), cu_k.cuda(), conv, Sq, Sk, 0.0, D ** -0.5, False, False, None, row_order=order)
+        dq, dk, dv = (torch.full_like(x, float("nan")) for x in (qg, kg, vg))
+        be.bwd_block(dog, qg, kg, vg, o, lse, dq, dk, dv, cu_q.cuda(), cu_k.cuda(), conv, Sq, Sk, 0.0, D ** -0.5, False, None, row_order=order)
+        torch.cuda.synchronize()
+        check_against_oracle({"out": o, "dq": dq, "dk": dk, "dv": dv}, ref, half, dtype, what="block layout %d x %d" % (Sq, Sk))
+
+
 def test_blocksparse_full_layout_equals_dense(full_size_tiles):
     from flash_attn.flash_blocksparse_attn_interface import flash_blocksparse_attn_func
     from flash_attn.flash_attn_interface import flash_attn_unpadded_qkvpacked_func
