@@ -429,6 +429,15 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
         // not masked score by score: its lanes' exponentials are taken against +inf below.)
         const bool need_mask = (n0 + BN > Lk) || (kCausal && (n0 + BN - 1 > mw));
         if (need_mask) {
+          // kFewMasks: keys from `limit` on are dead, counted from the lane's register 0, behind an opaque copy and four registers at a time.
+          // Left alone the compiler holds the 32 compare masks of a tile in scalar registers, also for the case that its scores are redone,
+          // and what it moves to vector lanes for them it reads back in every step: in the d = 64 forward with dropout 16 of them and a
+          // scalar load (64 x 16 heads x 1004 .. 1023, p = 0.1, step 1670 / 1656 us), in the causal one 5 (8 x 12 x 4096 bf16, step 900 / 894; 13 x 16 x
+          // 1380 forward 88.5 / 85.8), in the padded one 4 (63 x 8 x 867 .. 1352 222 / 216).  Not where it costs
+          // registers instead: ALiBi terms or a block layout under a causal mask two to eight in scratch, the half-size tiles (one block a wave).
+          constexpr bool kFewMasks = KS == 1 && KBW == 2 && !kAlibi && !(kSparse && kCausal);
+          int limit = (kCausal && qrow < Lk ? qrow + 1 : Lk) - (n0 + kb0 * 32 + hf * 4);
+          if constexpr (kFewMasks) asm volatile("" : "+v"(limit));
 #pragma unroll
           for (int kb = 0; kb < KBW; kb++)
 #pragma unroll
@@ -436,7 +445,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
               const int key = n0 + (kb0 + kb) * 32 + (r >> 2) * 8 + hf * 4 + (r & 3);
               bool dead = key >= Lk;
               if (kCausal) dead = dead || key > qrow;
+              if (kFewMasks) dead = kb * 32 + (r >> 2) * 8 + (r & 3) >= limit;
               if (dead) s[kb][r] = -INFINITY;
+              if (kFewMasks && (r & 3) == 3) __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (kTensorBias) {  // s <- s * scale * log2(e) + bias * log2(e)
