@@ -259,6 +259,17 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   const int nwords = kSparse ? (((nrb_q < p.sp.nrb ? nrb_q : p.sp.nrb) + 63) >> 6) : 0;
   int wi = (rb_first >> 6) - 1;
   auto next_tile = [&](BlockTile& t) -> bool {  // the next RBT listed blocks; false if there is none
+    // All in the word in hand: no branch per block.  (With both slabs of a tile in one piece of code for the scheduler, as the dense kernel has
+    // them - a slab without blocks runs with its rows switched off -, d = 64, 1 x 16 heads x 7701, bf16: 209.8 -> 199.6 us, 4 x 16 x 4096 with
+    // all blocks active 616 -> 585.)
+    if (__builtin_popcountll(word) >= RBT) {
+#pragma unroll
+      for (int j = 0; j < RBT; j++) {
+        t.rb[j] = wi * 64 + (int)__builtin_ctzll(word);
+        word &= word - 1;
+      }
+      return true;
+    }
 #pragma unroll
     for (int j = 0; j < RBT; j++) {
       while (word == 0 && wi + 1 < nwords) {
@@ -277,15 +288,16 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   };
   auto stage_blocks = [&](const BlockTile& t, int buf) {
     if (tid < 2 * BM) {
-      const int tr = tid < BM ? tid : tid - BM;
-      int blk = -1;
+      // (rows of 64: wave 0 fetches lse and wave 1 Dk, from a wave-uniform base)
+      const bool second = BM == 64 ? wave != 0 : tid >= BM;
+      const int tr = tid & (BM - 1);
+      int blk = t.rb[0];
 #pragma unroll
-      for (int j = 0; j < RBT; j++)
-        if ((tr >> 4) == j) blk = t.rb[j];
+      for (int j = 1; j < RBT; j++)
+        if (tr >= 16 * j) blk = t.rb[j];
       const int row = blk * 16 + (tr & 15);
-      const bool live = blk >= 0 && row < Lq;
-      statpre = tid < BM ? INFINITY : 0.f;  // rows of no block or past the end are switched off (P = 0)
-      if (live) statpre = tid < BM ? lsebase[row] : dsbase[row];
+      statpre = second ? 0.f : INFINITY;  // rows of no block or past the end are switched off (P = 0)
+      if (blk >= 0 && row < Lq) statpre = (second ? dsbase : lsebase)[(uint32_t)row];
     }
     stager.issue_blocks(lds_raw + buf * kBufBytes, t.rb, Lq);
   };
@@ -316,13 +328,13 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   T* const bias_lds = reinterpret_cast<T*>(lds_raw + Cfg::kLdsBytes + wave * kBiasTileBytes);
   constexpr int kBiasNLD = BM * 4 / 64;  // 16-byte loads per lane and tile
   u32x4 bpre[kTensorBias ? kBiasNLD : 1];
-  // (q_first: the tile's first query row; sparse: the packed tile's list of 16-row blocks instead, -1 = no block)
+  // (q_first: the tile's first query row; sparse: the packed tile's list of 16-row blocks instead, -1 = no block, the first is one)
   auto load_bias = [&](int q_first, const int* rb) {
 #pragma unroll
     for (int i = 0; i < kBiasNLD; i++) {
       const int k0 = n0 + wave * 32 + (lane & 3) * 8;
       int qr = q_first + i * 16 + (lane >> 2);
-      if (kSparse) qr = rb[i] >= 0 ? rb[i] * 16 + (lane >> 2) : Lq;
+      if (kSparse) qr = (rb[i] >= 0 ? rb[i] : rb[0]) * 16 + (lane >> 2);  // (no block: the first one's rows again, as the stager has it)
       bpre[i] = u32x4{0, 0, 0, 0};  // chunks that begin past the last key are not read; rows past the end read the last row
       if (k0 < Lk) bpre[i] = ld_global16(bias_bh + (uint32_t)(qr < Lq ? qr : Lq - 1) * bias_rs + (uint32_t)k0);
     }
@@ -409,7 +421,6 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
       // first query rows of the slab's two 16-row halves (sparse: of the two listed blocks; ascending)
       const int q_lo = kSparse ? tc.rb[2 * qb] * 16 : m0 + qb * 32;
       const int q_hi = kSparse ? tc.rb[2 * qb + 1] * 16 : q_lo + 16;
-      if (kSparse && q_lo < 0) continue;  // the last tile's list ended before this slab
       const bool diag = kCausal && ((kSparse ? q_lo : m0) < n0 + wave * 32 + 32);  // some (q, key) of the wave's has key > q
       // ---- S = Q K^T and dP = dO V^T for 32 query rows x this wave's 32 keys
       // dP starts from -Dk of its query row (fmha_dgrad_kernel_1xN_loop.h:361-371), so the MFMA delivers dP - Dk

@@ -239,33 +239,40 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   };
   const uint64_t query_words = kKeyWords ? philox_query_words(p.pk, (uint32_t)bh, (uint32_t)qrow >> 2) : 0;
 
-  // Sparse: tile `it` is computed iff its 256-key block is active for any 16-row block of this query tile.  The tile's
-  // and this lane's row block's activity bits of 64 consecutive key blocks (16384 keys) sit in registers.
-  uint64_t tile_bits = 0, row_bits = 0;
+  // Sparse: tile `it` is computed iff its 256-key block is active for any 16-row block of this query tile.  Everything about it is
+  // wave-uniform and kept in scalar registers: the activity bits of 64 consecutive key blocks (16384 keys) for the query tile and for
+  // the wave's two row blocks, and the lanes whose row block attends the tile in hand.  The search sits in front of the next tile's loads
+  // in every wave, a chain of dependent scalar instructions and branches, so it runs once per key block: within one the next tile is the
+  // next (d = 64, a quarter to a third of the 16 x 256 blocks, 1 x 8 heads x 4959 70.3 / 66.3 us, 2 x 16 x 5584 148 / 140; the dQ kernel, with no
+  // register to spare from spilling, is 1 % slower for it and searches tile by tile).
+  uint64_t tile_bits = 0, bits_a = 0, bits_b = 0;
   int bits_word = -1;
   const int qt_u = __builtin_amdgcn_readfirstlane(qt);
+  uint64_t row_mask_next = ~uint64_t(0);  // lanes whose row block attends the tile the last search found
   // First tile >= it whose 256-key block is active (ntiles if none): the bits of the loaded word are searched with a
   // count-trailing-zeros, not tile by tile.
-  bool row_on_next = true;  // this lane's row block attends the tile the last next_active() found
-  auto next_active = [&](int it) -> int {
-    if (!kSparse) return it;
+  auto find_active = [&](int it) -> int {
     constexpr int kTilesPerBlock = 256 / BN;
     while (it < ntiles) {
       const int cb = __builtin_amdgcn_readfirstlane((it * BN) >> 8);
       if ((cb >> 6) != bits_word) {
         bits_word = cb >> 6;
         tile_bits = uniform64(p.sp.qbits[(int64_t)qt_u * p.sp.ncw + bits_word]);
-        const int rbl = c < 16 ? rb_a : rb_b;
-        row_bits = rbl >= 0 ? p.sp.rbits[(int64_t)rbl * p.sp.ncw + bits_word] : 0;
+        bits_a = rb_a >= 0 ? uniform64(p.sp.rbits[(int64_t)rb_a * p.sp.ncw + bits_word]) : 0;
+        bits_b = rb_b >= 0 ? uniform64(p.sp.rbits[(int64_t)rb_b * p.sp.ncw + bits_word]) : 0;
       }
       const uint64_t rest = tile_bits >> (cb & 63);  // bit 0: this tile's block
-      if (rest & 1) break;
+      if (rest & 1) {
+        row_mask_next = half_slab_lanes((bits_a >> (cb & 63)) & 1, (bits_b >> (cb & 63)) & 1);
+        return it;
+      }
       // first tile of the next active block of this word, or of the next word
       it = (rest ? cb + (int)__builtin_ctzll(rest) : (cb | 63) + 1) * kTilesPerBlock;
     }
-    if (it > ntiles) it = ntiles;
-    if (it < ntiles) row_on_next = (row_bits >> (((it * BN) >> 8) & 63)) & 1;
-    return it;
+    return ntiles;
+  };
+  auto next_active = [&](int it) -> int {  // the tile after `it`, which is active
+    return !kSparse || (it + 1) % (256 / BN) != 0 ? it + 1 : find_active(it + 1);
   };
 
   f32x16 o_acc[DV / 32];
@@ -332,8 +339,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     }
   };
 
-  int it = next_active(tile0);
-  bool row_on_cur = row_on_next;
+  int it = kSparse ? find_active(tile0) : tile0;
   if (it < ntiles) {
     if constexpr (kRows) {
       if (listed) {
@@ -373,7 +379,8 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
       flush_keep_words();
       __syncthreads();                   // so is everyone else's, and nobody still reads the other buffer
     }
-    const int it_next = next_active(it + 1);
+    const uint64_t row_mask = row_mask_next;  // (of this tile: the search below moves on)
+    const int it_next = next_active(it);
     if (it_next < ntiles) stage(it_next, buf ^ 1);
     if (kTensorBias) {  // (the wave's own reads of the last tile's values are behind it: LDS operations of a wave stay in order)
       bias_to_lds();
@@ -387,12 +394,8 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     bool wave_work = wave_live;  // a wave whose 32 rows all lie past the sequence's end only helps with the staging
     if (kCausal && n0 + kh * 32 * KBW > mw + 31) wave_work = false;  // every key of the wave's share is above its diagonal
     if (KS > 1 && n0 + kh * 32 * KBW >= Lk) wave_work = false;       // ... or past the last key
-    bool row_on = true;
-    if (kSparse) {
-      row_on = row_on_cur;
-      row_on_cur = row_on_next;  // next_active(it + 1) above has set it
-      if (__ballot(row_on) == 0) wave_work = false;
-    }
+    if (kSparse && row_mask == 0) wave_work = false;
+    const bool row_on = !kSparse || lane_bit(row_mask);
 
     if (wave_work) {
       // this wave's 32-key blocks of the tile: kb0, kb0 + 1, ... (all of them without a key split)

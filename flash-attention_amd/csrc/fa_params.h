@@ -51,6 +51,11 @@ FA_DEVICE void slab_row_blocks(const SparseMaps& sp, bool ordered, int qt, int s
   *b = __builtin_amdgcn_readfirstlane(rb);
 }
 
+// The lanes of a 32-row slab whose row block (of its two) is on: lane l owns row l % 32
+FA_DEVICE uint64_t half_slab_lanes(bool a, bool b) {
+  return (a ? 0x0000ffff0000ffffull : 0) | (b ? 0xffff0000ffff0000ull : 0);
+}
+
 // What is added to the scaled scores before the softmax (template parameter kBias of the kernels)
 constexpr int kBiasNone = 0;    // nothing
 constexpr int kBiasAlibi = 1;   // -slope[head] * |query - key| (alibi)

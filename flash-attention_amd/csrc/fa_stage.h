@@ -156,11 +156,25 @@ struct TilePairStager {
   }
 
   // The same for a tile whose rows are gathered from 16-row blocks of the tensors: tile rows 16 j .. 16 j + 15 are tensor
-  // rows 16 blk[j] .. 16 blk[j] + 15 (blk[j] wave-uniform; < 0: no block - some valid row is fetched and the caller
+  // rows 16 blk[j] .. 16 blk[j] + 15 (blk[j] wave-uniform; < 0: no block - the first one, which there always is, is fetched again and the caller
   // switches those tile rows off).  Rows >= n_rows re-read the last valid row.
   FA_DEVICE void issue_blocks(unsigned char* lds, const int (&blk)[ROWS / 16], int n_rows) const {
     constexpr int SEG = RPI < 16 ? RPI : 16;  // rows of one block that one instruction covers
     const int jb = row0 >> 4;                 // first block this wave fetches from
+    if constexpr (RPI <= 16 && ROWS == 64) {  // this wave's two blocks, whole and inside the tensor (all but a list's last ones)
+      int l[4];  // (by value: a choice between array elements would keep the list in memory)
+#pragma unroll
+      for (int j = 0; j < 4; j++) l[j] = __builtin_amdgcn_readfirstlane(blk[j]);
+      const int b0 = jb == 0 ? l[0] : l[2], b1 = jb == 0 ? l[1] : l[3];  // (ascending where b1 is a block)
+      if (__builtin_expect(b1 >= 0 && (b1 + 1) * 16 <= n_rows, 1)) {
+        const char* const t0 = base + (int64_t)b0 * 16 * rsb;
+        const char* const t1 = base + (int64_t)b1 * 16 * rsb;
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+          dma16((i * RPI < 16 ? t0 : t1) + (i * RPI % 16) * rsb, src_off[i % NOFF], lds + dst0 + i * 1024);
+        return;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NI; i++) {
 #pragma unroll
@@ -170,15 +184,16 @@ struct TilePairStager {
 #pragma unroll
         for (int j = 0; j < ROWS / 16; j++)
           if (jb + (tr >> 4) == j) b = blk[j];
-        int srow = (b < 0 ? 0 : b * 16) + (tr & 15);  // tensor row of the segment's first tile row
+        int srow = (b < 0 ? blk[0] : b) * 16 + (tr & 15);  // tensor row of the segment's first tile row
         if (srow > n_rows - 1) srow = n_rows - 1;
         const bool mine = RPI / SEG == 1 || (rl >> 4) == sg;
         if (__builtin_expect(srow + SEG <= n_rows, 1)) {
           // lane offsets count rows from the instruction's first tile row: rl rows (sg * 16 of them before this segment)
           if (mine) dma16(base + ((int64_t)srow - sg * 16) * rsb, src_off[i % NOFF], lds + dst0 + i * 1024);
         } else {
-          int rlv = rl, pchv = pch;
-          asm volatile("" : "+v"(rlv), "+v"(pchv));
+          int ln = (int)threadIdx.x;  // (opaque: formed here and not kept in registers through the caller's main loop)
+          asm volatile("" : "+v"(ln));
+          const int rlv = (ln & 63) / CH, pchv = ln % CH;
           const int within = rlv - sg * 16;
           const int rc = srow + within < n_rows ? within : n_rows - 1 - srow;
           if (mine)

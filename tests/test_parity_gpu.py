@@ -1336,6 +1336,32 @@ def test_blocksparse_tiles_dearest_first(Sq, Sk, H, B):
         check_against_oracle({"out": o, "dq": dq, "dk": dk, "dv": dv}, ref, half, dtype, what="block layout %d x %d" % (Sq, Sk))
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("listed", [1, 2, 3, 5])
+def test_blocksparse_rows_outside_a_key_blocks_list_do_not_reach_its_gradients(D, listed):
+    """Tiles of four 16-row blocks at the end of a key block's list are filled up with rows it does list, switched off: a row that is NaN and
+    attends another key block only leaves this one's gradients as they are without it"""
+    from flash_attn.flash_blocksparse_attn_interface import flash_blocksparse_attn_func
+    N, H = 512, 2
+    layout = torch.zeros(N // 16, N // 256, device="cuda")
+    layout[:16, 0] = 1
+    layout[16:16 + listed, 1] = 1
+    g = torch.Generator("cuda").manual_seed(listed)
+    qkv = torch.randn(N, 3, H, D, device="cuda", dtype=torch.float16, generator=g)
+    dout = torch.randn(N, H, D, device="cuda", dtype=torch.float16, generator=g)
+    grads = []
+    for bad in (False, True):
+        x = qkv.clone()
+        if bad:
+            x[:16, 0] = float("nan")
+            x[-16:, 0] = float("inf")  # (attends nothing)
+        x.requires_grad_()
+        flash_blocksparse_attn_func(x, _cu([N]), layout, 0.0, N).backward(dout)
+        torch.cuda.synchronize()
+        grads.append(x.grad[256:, 1:])
+    assert torch.isfinite(grads[0]).all() and torch.equal(grads[0], grads[1])
+
+
 def test_blocksparse_full_layout_equals_dense(full_size_tiles):
     from flash_attn.flash_blocksparse_attn_interface import flash_blocksparse_attn_func
     from flash_attn.flash_attn_interface import flash_attn_unpadded_qkvpacked_func
