@@ -243,8 +243,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   // wave-uniform and kept in scalar registers: the activity bits of 64 consecutive key blocks (16384 keys) for the query tile and for
   // the wave's two row blocks, and the lanes whose row block attends the tile in hand.  The search sits in front of the next tile's loads
   // in every wave, a chain of dependent scalar instructions and branches, so it runs once per key block: within one the next tile is the
-  // next (d = 64, a quarter to a third of the 16 x 256 blocks, 1 x 8 heads x 4959 70.3 / 66.3 us, 2 x 16 x 5584 148 / 140; the dQ kernel, with no
-  // register to spare from spilling, is 1 % slower for it and searches tile by tile).
+  // next (d = 64, a quarter to a third of the 16 x 256 blocks, 1 x 8 heads x 4959 70.3 / 66.3 us, 2 x 16 x 5584 148 / 140).
   uint64_t tile_bits = 0, bits_a = 0, bits_b = 0;
   int bits_word = -1;
   const int qt_u = __builtin_amdgcn_readfirstlane(qt);
@@ -362,11 +361,6 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     for (int ks = 0; ks < D / 16; ks++)
       qreg[ks] = rotate8<T>(qreg[ks], *reinterpret_cast<const typename E::vec4*>(ct + ks * 8),
                             *reinterpret_cast<const typename E::vec4*>(st + ks * 8), false);
-    if (p.q_rot != nullptr && kh == 0 && split == 0 && qrow < Lq) {
-      T* const qo = reinterpret_cast<T*>(p.q_rot) + (int64_t)(q_begin + qrow) * p.qr_rs + (int64_t)h * p.qr_hs + hf * 8;
-#pragma unroll
-      for (int ks = 0; ks < D / 16; ks++) st_global16(qo + ks * 16, bitcast<u32x4>(qreg[ks]));
-    }
   }
   while (it < ntiles) {
     const int n0 = it * BN;
@@ -603,6 +597,14 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     it = it_next;
   }
   flush_keep_words();
+  // (the fragments are still there; stored in front of the loop, whose first step waits for everything outstanding, the rotated rows cost
+  // every workgroup a store's latency: us of the kernel there / here, causal bf16, 8 x 12 x 1024 d = 64 27.0 / 26.6, d = 128 47.8 / 46.2, 2 x 16 x 2000 d = 128
+  // 56.8 / 55.8; 23.3, 39 and 53.5 without rotary)
+  if (!kSparse && !kBiased && p.q_rot != nullptr && kh == 0 && split == 0 && qrow < Lq) {
+    T* const qo = reinterpret_cast<T*>(p.q_rot) + (int64_t)(q_begin + qrow) * p.qr_rs + (int64_t)h * p.qr_hs + hf * 8;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ks++) st_global16(qo + ks * 16, bitcast<u32x4>(qreg[ks]));
+  }
 
   // ---- key split: the waves kh > 0 hand their partial (O, maximum, sum) to the wave kh == 0 of their rows, in the
   // accumulator's own register order (word (rs * (16 DV/32 + 2) + j) * 64 + lane: consecutive lanes, no bank conflicts)
