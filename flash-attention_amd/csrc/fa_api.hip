@@ -795,6 +795,16 @@ int fa_rotary(const fa_rotary_args* a) {
   return FA_OK;
 }
 
+int fa_token_positions(const int32_t* cu_seqlens, int32_t batch, int32_t total, int32_t* positions, void* stream) {
+  FA_REQUIRE(batch > 0 && total >= 0, "fa_token_positions: bad sizes");
+  if (total == 0) return FA_OK;
+  FA_REQUIRE(cu_seqlens && positions, "fa_token_positions: null pointer");
+  FA_REQUIRE(((reinterpret_cast<uintptr_t>(cu_seqlens) | reinterpret_cast<uintptr_t>(positions)) & 3) == 0,
+             "fa_token_positions: pointers must be 4-byte aligned");
+  FA_LAUNCH(fa::launch_token_positions(cu_seqlens, batch, total, positions, reinterpret_cast<hipStream_t>(stream)));
+  return FA_OK;
+}
+
 int fa_set_launch_policy(int policy) {
   FA_REQUIRE((policy & ~0x73) == 0 && (policy & 3) != 3 && (policy & 0x30) != 0x30,
              "launch policy: tile shape 0 (automatic), 1 (full-size) or 2 (half-size), plus 0x10 (two-kernel backward) or 0x20 "

@@ -596,6 +596,8 @@ struct RotaryParams {
   int64_t row_offset;  // set by launch_rotary: index of this launch's first row in the caller's tensor (position = row % seqlen)
 };
 hipError_t launch_rotary(const RotaryParams& p, int dtype, hipStream_t stream);
+// positions[i] = i - cu[b], b the sequence that packed row i lies in
+hipError_t launch_token_positions(const int32_t* cu, int batch, int total, int32_t* positions, hipStream_t stream);
 hipError_t launch_gather_rows(const void* src, void* dst, const int64_t* idx, int64_t n_idx, int64_t n_src,
                               int64_t row_bytes, int64_t src_stride, int64_t dst_stride, int vec, hipStream_t stream);
 hipError_t launch_scatter_rows(const void* src, void* dst, const int64_t* idx, int64_t n_idx, int64_t n_dst,

@@ -68,7 +68,29 @@ __global__ void __launch_bounds__(512) rotary_kernel(const RotaryParams p, int w
   }
 }
 
+// The position of every packed row inside its sequence, by a binary search over the batch.  Bound by latency (a handful of dependent reads of
+// an array that stays in cache); it replaces seven launches of tensor arithmetic, 13 us
+// and the host's time for them: 2.5 us; forward and backward with rotary, causal bf16, us a step 8 x 12 heads x 717 .. 1024 d = 64 179 / 132,
+// 4 x 16 x 450 .. 900 d = 128 177 / 129, 40 x 12 x 280 .. 700 205 / 189.
+__global__ void __launch_bounds__(256) token_positions_kernel(const int32_t* __restrict__ cu, int batch, int total, int32_t* __restrict__ positions) {
+  const int row = blockIdx.x * 256 + threadIdx.x;
+  if (row >= total) return;
+  int lo = 0, hi = batch;  // the last entry that begins at or before the row (behind empty ones), whatever cu holds inside [0, batch]
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (cu[mid] <= row) lo = mid;
+    else hi = mid - 1;
+  }
+  positions[row] = row - cu[lo];
+}
+
 }  // namespace
+
+hipError_t launch_token_positions(const int32_t* cu, int batch, int total, int32_t* positions, hipStream_t stream) {
+  if (total <= 0) return hipSuccess;
+  hipLaunchKernelGGL(token_positions_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, cu, batch, total, positions);
+  return hipGetLastError();
+}
 
 hipError_t launch_rotary(const RotaryParams& p, int dtype, hipStream_t stream) {
   const bool in_place = p.src == p.dst && p.src_row_stride == p.dst_row_stride && p.src_part_stride == p.dst_part_stride &&

@@ -124,6 +124,7 @@ EXPORTED_SYMBOLS = (
     "fa_round_seqlens", "fa_philox_offset_increment", "fa_last_error", "fa_abi_version",
     "fa_gather_rows", "fa_scatter_rows", "fa_scatter_rows_workspace_bytes", "fa_rotary", "fa_set_launch_policy",
     "fa_keep_words_bytes", "fa_blocksparse_row_order", "fa_bias_grad_reduce", "fa_bias_grad_reduce_ragged", "fa_pad_bias_rows", "fa_padding_rows", "fa_fwd_padded",
+    "fa_token_positions",
 )
 # declared in include/flash_attn_gfx950_bench.h: instrumentation for bench.py, not part of the drop-in boundary
 BENCH_SYMBOLS = ("fa_bwd_profiled",)
@@ -205,6 +206,8 @@ def load_library():
         lib.fa_scatter_rows_workspace_bytes.restype = ctypes.c_size_t
         lib.fa_rotary.argtypes = [ctypes.POINTER(RotaryArgs)]
         lib.fa_rotary.restype = ctypes.c_int
+        lib.fa_token_positions.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
+        lib.fa_token_positions.restype = ctypes.c_int
         lib.fa_blocksparse_row_order.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
         lib.fa_blocksparse_row_order.restype = ctypes.c_int
         lib.fa_set_launch_policy.argtypes = [ctypes.c_int]
@@ -891,6 +894,20 @@ def fwd_padded(qkv, mask, softmax_scale, is_causal):
         finally:  # (a kernel writes to lens, of which the pinned-memory allocator does not know)
             written.synchronize()
     return out if lens.any() else None
+
+
+def token_positions(cu_seqlens, total):
+    """(total,) int32: the position of every row of a packed batch inside its sequence (fa_token_positions)."""
+    batch = cu_seqlens.numel() - 1
+    _check(batch > 0, "batch size must be positive")
+    _check_cu("cu_seqlens", cu_seqlens, batch)
+    lib = load_library()
+    with _OnDevice(cu_seqlens.device):
+        positions = torch.empty((total,), dtype=torch.int32, device=cu_seqlens.device)
+        rc = lib.fa_token_positions(cu_seqlens.data_ptr(), batch, total, positions.data_ptr(), _stream_handle(cu_seqlens.device))
+    if rc != 0:
+        _raise(rc, lib)
+    return positions
 
 
 def rotary(src, dst, cos, sin, n_rotated, conjugate=False, positions=None):

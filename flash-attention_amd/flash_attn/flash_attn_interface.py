@@ -41,9 +41,7 @@ def _rotated_keys(qkv, cu_seqlens, max_seqlen, cos_half, sin_half):
     rot = torch.empty((total, 2, nheads, headdim), dtype=qkv.dtype, device=qkv.device)
     positions = None
     if total != batch * max_seqlen:  # ragged: every row's position inside its sequence
-        lens = (cu_seqlens[1:] - cu_seqlens[:-1]).long()
-        positions = (torch.arange(total, device=qkv.device, dtype=torch.int32)
-                     - torch.repeat_interleave(cu_seqlens[:-1], lens, output_size=total))
+        positions = _backend.token_positions(cu_seqlens, total)
         src, dst = qkv[None, :, 1:2], rot[None, :, 1:2]
     else:
         src = qkv.reshape(batch, max_seqlen, 3, nheads, headdim)[:, :, 1:2]

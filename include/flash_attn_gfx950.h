@@ -317,6 +317,9 @@ typedef struct fa_rotary_args {
   void* stream;
 } fa_rotary_args;
 int fa_rotary(const fa_rotary_args* args);
+/* The `positions` of fa_rotary for a packed batch (no counterpart in the reference): positions[i] = i - cu_seqlens[b] for the
+ * total rows, b the sequence row i lies in (rows behind the last sequence count on from its end).  cu_seqlens: batch + 1 int32. */
+int fa_token_positions(const int32_t* cu_seqlens, int32_t batch, int32_t total, int32_t* positions, void* stream);
 
 /* Host-side helper of the block-sparse entry points (no GPU work, no counterpart in the reference): an order of the 16-row
  * blocks for fa_fwd_args.row_order / fa_bwd_args.row_order that puts row blocks with similar key-block lists into the same

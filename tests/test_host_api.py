@@ -533,6 +533,10 @@ def test_rows_and_rotary_argument_checks(lib):
     assert lib.fa_rotary(ctypes.byref(r)) == -1 and b"null" in lib.fa_last_error()
     r.n_rows = 0
     assert lib.fa_rotary(ctypes.byref(r)) == 0
+    assert lib.fa_token_positions(0x1000, 0, 4, 0x2000, None) == -1 and b"sizes" in lib.fa_last_error()
+    assert lib.fa_token_positions(None, 1, 4, 0x2000, None) == -1 and b"null" in lib.fa_last_error()
+    assert lib.fa_token_positions(0x1000, 1, 4, 0x2002, None) == -1 and b"aligned" in lib.fa_last_error()
+    assert lib.fa_token_positions(None, 1, 0, None, None) == 0
 
 
 def test_bias_grad_reduce_argument_checks(lib):

@@ -2271,6 +2271,16 @@ def _rotary_attention_fp32(qkv, cos_h, sin_h, lens, scale, causal, dout):
     return out.detach(), x.grad
 
 
+@pytest.mark.parametrize("lens", [[1], [700], [0, 0, 3, 0, 255, 256, 257, 0], [1] * 300, [5, 4000, 0]])
+def test_token_positions(lens):
+    """the positions of a packed batch's rows: empty entries at either end and in between, more entries than a wave has lanes, whole numbers"""
+    from flash_attn import flash_attn_gfx950 as be
+    want = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
+    assert torch.equal(be.token_positions(_cu(lens), sum(lens)).cpu(), want)
+    with pytest.raises(RuntimeError, match="int32"):
+        be.token_positions(_cu(lens).long(), sum(lens))
+
+
 @pytest.mark.parametrize("D,dtype,causal,lens", [
     (64, torch.float16, False, [256, 256]),
     (64, torch.float16, True, [200, 37, 129]),
