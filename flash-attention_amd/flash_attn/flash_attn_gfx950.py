@@ -131,6 +131,7 @@ BENCH_SYMBOLS = ("fa_bwd_profiled",)
 
 _lib = None
 _host = None  # the binding's native half (host/fa_host.cpp), bound to _lib
+_passes = None  # the same module, for its calls around fwd and bwd
 _lib_lock = threading.Lock()
 
 
@@ -145,13 +146,13 @@ def _load_host(lib):
     spec.loader.exec_module(host)
     host.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
         "fa_fwd", "fa_fwd_block", "fa_bwd", "fa_bwd_block", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes", "fa_round_seqlens",
-        "fa_last_error")))
+        "fa_last_error", "fa_pad_bias_rows", "fa_bias_grad_reduce_ragged", "fa_rotary", "fa_token_positions")))
     return host
 
 
 def load_library():
     """dlopen the shared library once and declare the prototypes.  Raises if it has not been built."""
-    global _lib, _host
+    global _lib, _host, _passes
     if _lib is not None:
         return _lib
     with _lib_lock:
@@ -214,7 +215,7 @@ def load_library():
         lib.fa_set_launch_policy.restype = ctypes.c_int
         if lib.fa_abi_version() != FA_ABI_VERSION:
             raise RuntimeError("%s has ABI version %d, binding expects %d" % (LIB_NAME, lib.fa_abi_version(), FA_ABI_VERSION))
-        _host = _load_host(lib)
+        _host = _passes = _load_host(lib)
         _lib = lib
     return _lib
 
@@ -403,6 +404,10 @@ def prepare_attn_bias(attn_bias, q, batch, nheads, max_seqlen_q, max_seqlen_k):
     ok = (attn_bias.stride(3) == 1 and attn_bias.stride(2) % 8 == 0 and attn_bias.stride(2) >= max_seqlen_k and
           attn_bias.data_ptr() % 16 == 0 and all(attn_bias.stride(i) % 8 == 0 for i in (0, 1)))
     if not ok:
+        load_library()
+        padded = _passes.pad_bias(attn_bias)
+        if padded is not None:
+            return padded
         sk8 = (attn_bias.shape[3] + 7) // 8 * 8
         if attn_bias.is_cuda and attn_bias.element_size() == 2:
             lib = load_library()
@@ -783,6 +788,8 @@ def reduce_bias_grad(dbias, out, sum_batch, sum_heads, written=None):
     lib = load_library()
     if written is not None:
         cu_q, cu_k, total_q, total_k, causal = written
+        if _passes.reduce_bias_grad(dbias, out, sum_batch, sum_heads, cu_q, cu_k, total_q, total_k, causal):
+            return out
         _check_cu("cu_seqlens_q", cu_q, batch)
         _check_cu("cu_seqlens_k", cu_k, batch)
         a = BwdArgs()
@@ -894,6 +901,13 @@ def fwd_padded(qkv, mask, softmax_scale, is_causal):
         finally:  # (a kernel writes to lens, of which the pinned-memory allocator does not know)
             written.synchronize()
     return out if lens.any() else None
+
+
+def rotated_keys(qkv, cu_seqlens, max_seqlen, cos_half, sin_half):
+    """(total, 2, nheads, headdim) with the keys of a packed (total, 3, nheads, headdim) qkv, turned by their positions, as part 1; None for what
+    is to be rotated by way of rotary()."""
+    load_library()
+    return _passes.rotated_keys(qkv, cu_seqlens, max_seqlen, cos_half, sin_half)
 
 
 def token_positions(cu_seqlens, total):

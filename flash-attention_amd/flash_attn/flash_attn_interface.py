@@ -36,6 +36,9 @@ def _flash_attn_backward(dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens
 def _rotated_keys(qkv, cu_seqlens, max_seqlen, cos_half, sin_half):
     """(total, 2, nheads, headdim) buffer whose part 1 holds the rotated keys of a packed qkv (part 0 is left for the
     rotated queries, which the attention kernel writes): one pass of the rotary kernel over the k third only."""
+    rot = _backend.rotated_keys(qkv, cu_seqlens, max_seqlen, cos_half, sin_half)
+    if rot is not None:
+        return rot
     total, _, nheads, headdim = qkv.shape
     batch = cu_seqlens.numel() - 1
     rot = torch.empty((total, 2, nheads, headdim), dtype=qkv.dtype, device=qkv.device)
@@ -139,7 +142,7 @@ def bias_grad_in_shape(dbias, shape, max_seqlen_q, max_seqlen_k, written=None):
     written: as in _backend.reduce_bias_grad (a dbias that was not cleared)."""
     covered = tuple(shape[2:]) == (max_seqlen_q, max_seqlen_k)
     full = (torch.empty if covered else torch.zeros)(shape, dtype=dbias.dtype, device=dbias.device)
-    view = full[:, :, :max_seqlen_q, :max_seqlen_k]
+    view = full if covered else full[:, :, :max_seqlen_q, :max_seqlen_k]
     sum_batch, sum_heads = shape[0] == 1 and dbias.shape[0] > 1, shape[1] == 1 and dbias.shape[1] > 1
     if sum_batch or sum_heads or written is not None:
         _backend.reduce_bias_grad(dbias, view, sum_batch, sum_heads, written)

@@ -1,4 +1,4 @@
-// The calls of flash_attn_gfx950.fwd / bwd (and their block-sparse forms) made natively: arguments checked, outputs and scratch
+// The calls of flash_attn_gfx950.fwd / bwd (and their block-sparse forms), and of the passes around them, made natively: arguments checked, outputs and scratch
 // allocated, the argument struct of the C ABI filled and the entry point called, without Python in between.
 //
 // Every check the Python binding makes is made here too, but nothing is reported: a call that fails one, or that is of a kind
@@ -31,21 +31,26 @@ struct Library {
   size_t (*bwd_workspace_bytes)(const fa_bwd_args*);
   void (*round_seqlens)(int32_t, int32_t, int32_t, int32_t, int32_t*, int32_t*);
   const char* (*last_error)();
+  int (*pad_bias_rows)(const void*, void*, int32_t, int32_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, void*);
+  int (*bias_grad_reduce_ragged)(const void*, void*, const fa_bwd_args*, int32_t, int32_t, int64_t, int64_t, int64_t);
+  int (*rotary)(const fa_rotary_args*);
+  int (*token_positions)(const int32_t*, int32_t, int32_t, int32_t*, void*);
 } g_lib;
 bool g_bound = false;
 
-// bind(addresses of the eight entry points above, in their order)
+// bind(addresses of the twelve entry points above, in their order)
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 8) return PyErr_Format(PyExc_TypeError, "bind takes 8 addresses");
-  void* f[8];
-  for (int i = 0; i < 8; i++) {
+  constexpr int kEntries = 12;
+  if (n != kEntries) return PyErr_Format(PyExc_TypeError, "bind takes %d addresses", kEntries);
+  void* f[kEntries];
+  for (int i = 0; i < kEntries; i++) {
     f[i] = PyLong_AsVoidPtr(a[i]);
     if (!f[i]) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
       return nullptr;
     }
   }
-  static_assert(sizeof(g_lib) == sizeof(f), "eight pointers");
+  static_assert(sizeof(g_lib) == sizeof(f), "a pointer each");
   memcpy(&g_lib, f, sizeof(f));
   g_bound = true;
   Py_RETURN_NONE;
@@ -303,6 +308,118 @@ PyObject* bwd(PyObject* const* a, Py_ssize_t n) {
   return THPVariable_Wrap(std::move(d));
 }
 
+// The calls around the attention itself: the keys' rotation, the copy of a bias with padded rows, the sum of its gradient.  us with the binding's
+// own calls / with these: 14.3 / 4.1, 9.9 / 6.2 and 11.8 / 7.4 of the host's time for one; a step of 8 x 12 heads x 1024 with rotary 122.8 / 107.6 (kernels 107),
+// of 8 x 8 x 421 .. 701 with a bias 151.6 / 124.6 (102).
+hipStream_t stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+bool on_current_device(const at::Tensor* t) { return g_bound && t && t->is_cuda() && t->device().index() == c10::hip::current_device(); }
+bool is_cu(const at::Tensor* t, const at::Tensor& like) {
+  return t && t->is_cuda() && t->device() == like.device() && t->scalar_type() == at::kInt && t->dim() == 1 && t->size(0) > 1 && t->size(0) <= INT32_MAX &&
+         t->is_contiguous();
+}
+
+// rotated_keys(qkv, cu, max_seqlen, cos, sin) -> (total, 2, nheads, headdim) with the rotated keys as part 1, or None
+PyObject* rotated_keys(PyObject* const* a, Py_ssize_t n) {
+  if (n != 5) return PyErr_Format(PyExc_TypeError, "rotated_keys takes 5 arguments");
+  bool ok = true;
+  const at::Tensor *qkv = tensor(a[0], ok), *cu = tensor(a[1], ok), *cos = tensor(a[3], ok), *sin = tensor(a[4], ok);
+  int64_t ms;
+  if (!ok || !as_int(a[2], &ms) || ms <= 0 || !on_current_device(qkv) || !is_cu(cu, *qkv) || !cos || !sin) Py_RETURN_NONE;
+  const at::ScalarType type = qkv->scalar_type();
+  if ((type != at::kHalf && type != at::kBFloat16) || qkv->dim() != 4 || qkv->size(0) <= 0 || qkv->size(0) > INT32_MAX || qkv->size(1) != 3 ||
+      qkv->stride(3) != 1 || qkv->size(2) <= 0 || qkv->size(2) > INT32_MAX || qkv->size(3) <= 0 || qkv->size(3) % 8 != 0 || qkv->size(3) > INT32_MAX)
+    Py_RETURN_NONE;
+  const int64_t total = qkv->size(0), heads = qkv->size(2), dim = qkv->size(3), batch = cu->size(0) - 1;
+  auto table = [&](const at::Tensor* t) {
+    return t->dim() == 2 && t->size(1) == dim / 2 && t->scalar_type() == type && t->is_contiguous() && t->device() == qkv->device() && t->size(0) > 0 &&
+           t->size(0) <= INT32_MAX && reinterpret_cast<uintptr_t>(ptr(*t)) % 8 == 0;
+  };
+  const bool ragged = total != batch * ms;
+  if (!table(cos) || !table(sin) || cos->size(0) != sin->size(0) || (!ragged && cos->size(0) < ms)) Py_RETURN_NONE;
+  const char* const k = static_cast<const char*>(ptr(*qkv)) + 2 * qkv->stride(1);
+  if (reinterpret_cast<uintptr_t>(k) % 16 != 0 || qkv->stride(0) < 0 || qkv->stride(0) % 8 != 0 || qkv->stride(2) < 0 || qkv->stride(2) % 8 != 0 ||
+      qkv->stride(1) < 0 || qkv->stride(1) % 8 != 0)
+    Py_RETURN_NONE;
+  at::Tensor rot = at::empty({total, 2, heads, dim}, qkv->options().memory_format(at::MemoryFormat::Contiguous).requires_grad(false)), pos;
+  fa_rotary_args f;
+  memset(&f, 0, sizeof(f));
+  f.struct_bytes = sizeof(f);
+  f.dtype = type == at::kHalf ? FA_FP16 : FA_BF16;
+  f.src = k;
+  f.dst = static_cast<char*>(ptr(rot)) + 2 * heads * dim;
+  f.cos_table = ptr(*cos); f.sin_table = ptr(*sin);
+  f.n_rows = total;
+  f.src_row_stride = qkv->stride(0); f.src_part_stride = qkv->stride(1); f.src_head_stride = qkv->stride(2);
+  f.dst_row_stride = 2 * heads * dim; f.dst_part_stride = heads * dim; f.dst_head_stride = dim;
+  f.n_parts = f.n_rotated = 1;
+  f.n_heads = (int32_t)heads; f.head_dim = (int32_t)dim;
+  f.seqlen = (int32_t)ms; f.table_rows = (int32_t)cos->size(0);
+  f.stream = stream_of(*qkv);
+  if (ragged) {
+    pos = at::empty({total}, cu->options().requires_grad(false));
+    f.positions = (const int32_t*)ptr(pos);
+  }
+  int rc = 0;
+  Py_BEGIN_ALLOW_THREADS
+  if (ragged) rc = g_lib.token_positions((const int32_t*)ptr(*cu), (int32_t)batch, (int32_t)total, (int32_t*)ptr(pos), f.stream);
+  if (rc == 0) rc = g_lib.rotary(&f);
+  Py_END_ALLOW_THREADS
+  return rc != 0 ? refused(rc) : THPVariable_Wrap(std::move(rot));
+}
+
+// pad_bias(bias): the copy with rows of a multiple of 8 keys that fa_fwd can read, or None
+PyObject* pad_bias(PyObject* const* a, Py_ssize_t n) {
+  if (n != 1) return PyErr_Format(PyExc_TypeError, "pad_bias takes 1 argument");
+  bool ok = true;
+  const at::Tensor* t = tensor(a[0], ok);
+  if (!ok || !on_current_device(t) || (t->scalar_type() != at::kHalf && t->scalar_type() != at::kBFloat16) || t->dim() != 4 || t->size(0) > INT32_MAX ||
+      t->size(1) > INT32_MAX)
+    Py_RETURN_NONE;
+  at::Tensor out = at::empty({t->size(0), t->size(1), t->size(2), (t->size(3) + 7) / 8 * 8},
+                             t->options().memory_format(at::MemoryFormat::Contiguous).requires_grad(false));
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = g_lib.pad_bias_rows(ptr(*t), ptr(out), (int32_t)t->size(0), (int32_t)t->size(1), t->size(2), t->size(3), t->stride(0), t->stride(1), t->stride(2),
+                           t->stride(3), stream_of(*t));
+  Py_END_ALLOW_THREADS
+  return rc != 0 ? refused(rc) : THPVariable_Wrap(std::move(out));
+}
+
+// reduce_bias_grad(dbias, out, sum_batch, sum_heads, cu_q, cu_k, total_q, total_k, causal) -> True or None
+PyObject* reduce_bias_grad(PyObject* const* a, Py_ssize_t n) {
+  if (n != 9) return PyErr_Format(PyExc_TypeError, "reduce_bias_grad takes 9 arguments");
+  bool ok = true;
+  const at::Tensor *d = tensor(a[0], ok), *o = tensor(a[1], ok), *cu_q = tensor(a[4], ok), *cu_k = tensor(a[5], ok);
+  int32_t sum_b, sum_h, causal;
+  int64_t tq, tk;
+  if (!ok || !on_current_device(d) || !o || !as_flag(a[2], &sum_b) || !as_flag(a[3], &sum_h) || !as_int(a[6], &tq) || !as_int(a[7], &tk) ||
+      !as_flag(a[8], &causal) || (d->scalar_type() != at::kHalf && d->scalar_type() != at::kBFloat16) || d->dim() != 4 || o->dim() != 4 ||
+      o->device() != d->device() || o->scalar_type() != d->scalar_type() || !is_cu(cu_q, *d) || !is_cu(cu_k, *d))
+    Py_RETURN_NONE;
+  const int64_t batch = d->size(0), heads = d->size(1), rows = d->size(2), cols = o->size(3);
+  if (o->size(0) != (sum_b ? 1 : batch) || o->size(1) != (sum_h ? 1 : heads) || o->size(2) != rows || cols > d->size(3) || d->stride(3) != 1 ||
+      (o->stride(3) != 1 && cols > 1) || cu_q->size(0) != batch + 1 || cu_k->size(0) != batch + 1 || heads > INT32_MAX || rows > INT32_MAX ||
+      cols > INT32_MAX)
+    Py_RETURN_NONE;
+  fa_bwd_args f;
+  memset(&f, 0, sizeof(f));
+  f.struct_bytes = sizeof(f);
+  f.dtype = d->scalar_type() == at::kHalf ? FA_FP16 : FA_BF16;
+  f.batch = (int32_t)batch; f.nheads = (int32_t)heads;
+  f.total_q = (int32_t)tq; f.total_k = (int32_t)tk;
+  f.max_seqlen_q = (int32_t)rows; f.max_seqlen_k = (int32_t)cols;
+  f.cu_seqlens_q = (const int32_t*)ptr(*cu_q); f.cu_seqlens_k = (const int32_t*)ptr(*cu_k);
+  f.is_causal = causal;
+  f.dbias_batch_stride = d->stride(0); f.dbias_head_stride = d->stride(1); f.dbias_row_stride = d->stride(2);
+  f.stream = stream_of(*d);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = g_lib.bias_grad_reduce_ragged(ptr(*d), ptr(*o), &f, sum_b, sum_h, o->stride(0), o->stride(1), o->stride(2));
+  Py_END_ALLOW_THREADS
+  if (rc != 0) return refused(rc);
+  Py_RETURN_TRUE;
+}
+
 // C++ exceptions (an allocation that fails, memory that may not be touched under tracing) do not leave the module: the call is handed back and
 // the binding meets the same condition
 template <PyObject* (*F)(PyObject* const*, Py_ssize_t)>
@@ -319,6 +436,9 @@ PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))py_bind, METH_FASTCALL, nullptr},
     {"fwd", (PyCFunction)(void (*)(void))guarded<fwd>, METH_FASTCALL, nullptr},
     {"bwd", (PyCFunction)(void (*)(void))guarded<bwd>, METH_FASTCALL, nullptr},
+    {"rotated_keys", (PyCFunction)(void (*)(void))guarded<rotated_keys>, METH_FASTCALL, nullptr},
+    {"pad_bias", (PyCFunction)(void (*)(void))guarded<pad_bias>, METH_FASTCALL, nullptr},
+    {"reduce_bias_grad", (PyCFunction)(void (*)(void))guarded<reduce_bias_grad>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "fa_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -1516,6 +1516,68 @@ def test_native_calls_equal_the_bindings(kind, dtype, D, binding_only, monkeypat
             assert torch.equal(x, y), i
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form", ["packed", "ragged", "wide rows", "odd cols", "transposed", "broadcast", "one head"])
+def test_native_passes_equal_the_bindings(form, dtype, monkeypatch):
+    """the keys' rotation, the bias copy and the sum of its gradient through the native half and without it: the same bits, whatever the
+    strides, and the native half takes them"""
+    import types
+    from flash_attn import flash_attn_gfx950 as be, flash_attn_interface as fi
+    torch.manual_seed(5)
+    lens, H, D = ([40, 7, 65] if form == "ragged" else [33, 33, 33]), 4, 32
+    N, B = max(lens), len(lens)
+    cu, total = _cu(lens), sum(lens)
+    wide = torch.randn(total, 4, H, D + 8, device="cuda").to(dtype)
+    qkv = wide[:, 1:, :, :D] if form == "wide rows" else torch.randn(total, 3, H, D, device="cuda").to(dtype)
+    cos, sin = (torch.randn(N + 2, D // 2, device="cuda").to(dtype) for _ in range(2))
+    bias = torch.randn(B, H, N + 3, N + 3, device="cuda").to(dtype)
+    if form == "transposed":
+        bias = bias.transpose(2, 3)
+    elif form == "broadcast":
+        bias = bias[:1, :1, :1].expand(1, H, N, N + 3)
+    elif form == "one head":
+        bias = bias[:, :1]
+    bias = bias[:, :, :N, :N]
+    dbias = torch.randn(B, H, N, (N + 7) // 8 * 8, device="cuda").to(dtype)
+
+    def passes():
+        rot = fi._rotated_keys(qkv, cu, N, cos, sin)[:, 1]
+        padded = be.prepare_attn_bias(bias, qkv[:, 0], B, H, N, N)
+        grads = [fi.bias_grad_in_shape(dbias, shape, N, N, (cu, cu, total, total, causal))
+                 for shape in ((1, H, N, N), (B, 1, N, N + 1), (B, H, N, N)) for causal in (False, True)]
+        torch.cuda.synchronize()
+        return [rot, padded[..., :N]] + grads
+
+    be.load_library()
+    native, taken = be._passes, []
+
+    def noted(name):
+        def call(*a):
+            res = getattr(native, name)(*a)
+            taken.append(res is not None)
+            return res
+        return call
+
+    names = ("rotated_keys", "pad_bias", "reduce_bias_grad")
+    monkeypatch.setattr(be, "_passes", types.SimpleNamespace(**{n: noted(n) for n in names}))
+    want = passes()
+    assert len(taken) == 8 and all(taken)
+    monkeypatch.setattr(be, "_passes", types.SimpleNamespace(**{n: (lambda *a: None) for n in names}))
+    for i, (x, y) in enumerate(zip(want, passes())):
+        assert torch.equal(x, y), i
+
+
+def test_native_passes_hand_back_what_the_binding_refuses():
+    """the binding's own exceptions, from tables that are too short, lengths of another type and strides that no kernel reads"""
+    from flash_attn import flash_attn_interface as fi
+    qkv, cu = torch.randn(40, 3, 2, 32, device="cuda").half(), _cu([20, 20])
+    table = torch.randn(20, 16, device="cuda").half()
+    for args in ((qkv, cu, 20, table[:19], table[:19]), (qkv, cu.long(), 25, table, table), (qkv, cu, 20, table.float(), table.float()),
+                 (qkv[..., :20], cu, 20, table[:, :10].contiguous(), table[:, :10].contiguous()), (qkv, cu, 20, table, table[:10])):
+        with pytest.raises(RuntimeError):
+            fi._rotated_keys(*args)
+
+
 def test_native_calls_hand_back_what_the_binding_refuses(binding_only):
     """the same exceptions with and without the native half"""
     from flash_attn import flash_attn_gfx950 as be
