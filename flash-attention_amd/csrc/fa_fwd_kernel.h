@@ -599,8 +599,9 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   flush_keep_words();
   // (the fragments are still there; stored in front of the loop, whose first step waits for everything outstanding, the rotated rows cost
   // every workgroup a store's latency: us of the kernel there / here, causal bf16, 8 x 12 x 1024 d = 64 27.0 / 26.6, d = 128 47.8 / 46.2, 2 x 16 x 2000 d = 128
-  // 56.8 / 55.8; 23.3, 39 and 53.5 without rotary)
-  if (!kSparse && !kBiased && p.q_rot != nullptr && kh == 0 && split == 0 && qrow < Lq) {
+  // 56.8 / 55.8; 23.3, 39 and 53.5 without rotary; kept out of the variants that take no rotary tables: a padded batch at d = 128 has no
+  // register to spare, 169 are two waves per SIMD and 168 three: 16 x 16 heads x 512 .. 1024 fp16 130 / 119)
+  if (!kSparse && kBias == 0 && p.q_rot != nullptr && kh == 0 && split == 0 && qrow < Lq) {
     T* const qo = reinterpret_cast<T*>(p.q_rot) + (int64_t)(q_begin + qrow) * p.qr_rs + (int64_t)h * p.qr_hs + hf * 8;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ks++) st_global16(qo + ks * 16, bitcast<u32x4>(qreg[ks]));
