@@ -202,3 +202,19 @@ def test_padded_rows_and_d128_half_size_variants_keep_their_waves_per_simd():
             assert k["Occupancy"] >= 2 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 80 * 1024, ("forward, half-size", dt, causal, k)
             k = _pick(bwd, "fa_bwd_dq_kernel%sLi128E" % dt, causal + "Li0ELb0ELi0ELi2EEEv")
             assert k["Occupancy"] >= 2 and k["VGPRs Spill"] == 0 and k["LDS Size"] <= 80 * 1024, ("dq, half-size", dt, causal, k)
+
+
+@pytest.mark.timeout(600)
+def test_block_layout_dkdv_keeps_its_block_list_in_registers():
+    """dK/dV over a block layout at d = 16, whose tiles gather four 16-row blocks: the list is neither in scratch nor in LDS beside the tiles."""
+    bwd = _resources("fa_bwd_d16.hip")
+    for dt in ("IDF16_", "IDF16b"):
+        for causal in ("Lb0E", "Lb1E"):
+            for drop in ("Li0E", "Li1E"):
+                lds = []
+                for bias in ("Li0E", "Li1E", "Li2E"):
+                    k = _pick(bwd, "fa_bwd_dkdv_kernel%sLi16E" % dt, "Li16E" + causal + drop + "Lb1E" + bias + "Lb0EEEv")
+                    assert k["ScratchSize"] == 0, (dt, causal, drop, bias, k)
+                    lds.append(k["LDS Size"])
+                # two buffers of 64 rows of Q and dO, 16 elements of 2 bytes, and the rows' statistics, and less than the list's 32 bytes a thread more
+                assert lds[0] == lds[1] < 2 * 64 * (2 * 16 * 2 + 2 * 4) + 256 * 32 and lds[2] > lds[0], (dt, causal, drop, lds)
