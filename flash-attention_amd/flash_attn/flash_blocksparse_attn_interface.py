@@ -43,7 +43,8 @@ _ROW_ORDERS = {}  # converted blockmask (address, shape, version) -> row order
 def _row_order(blockmask, causal):
     """The order of the 16-row blocks the kernels' workgroups take them in (flash_attn_gfx950.blockmask_row_order), worked
     out once per converted blockmask (the first call reads the blockmask back to the host).  Any order gives the same
-    results; a cache entry that outlived its tensor costs speed at worst."""
+    results but for rounding (the reference point of a row's exponentials depends on the rows beside it: up to 2.4e-4 in
+    fp16, 2 x 512 tokens); a cache entry that outlived its tensor costs speed and that."""
     if causal:
         return None
     key = (blockmask.data_ptr(), tuple(blockmask.shape), blockmask._version, str(blockmask.device))
