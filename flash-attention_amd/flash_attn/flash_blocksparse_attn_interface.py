@@ -6,7 +6,10 @@ reference's Python at this commit calls its extension with an argument list its 
 (:45-47,56-58 vs fmha_api.cpp:451-464,575-594); here the public signature is kept and the native call uses the
 C++ argument order.
 """
+from collections import OrderedDict
+
 import torch
+from torch.utils.weak import WeakTensorKeyDictionary
 
 from . import flash_attn_gfx950 as _backend
 from .flash_attn_interface import bias_grad_in_shape, new_bias_grad
@@ -37,55 +40,86 @@ def convert_blockmask(blockmask, causal):
     return torch.gather(code, 0, order).T.contiguous().to(torch.int32)
 
 
-_ROW_ORDERS = {}  # converted blockmask (address, shape, version) -> row order
+_ORDERS_OF_MASKS = WeakTensorKeyDictionary()  # a caller's mask (of a view: its base) -> {what it looked like: row order}
+_ORDERS_OF_CONTENTS = OrderedDict()  # (shape, device, values) of a converted mask -> row order, the most recently used last
+_ORDERS_KEPT = 64
 
 
-def _row_order(blockmask, causal):
-    """The order of the 16-row blocks the kernels' workgroups take them in (flash_attn_gfx950.blockmask_row_order), worked
-    out once per converted blockmask (the first call reads the blockmask back to the host).  Any order gives the same
-    results but for rounding (the reference point of a row's exponentials depends on the rows beside it: up to 2.4e-4 in
-    fp16, 2 x 512 tokens); a cache entry that outlived its tensor costs speed and that."""
+def _row_order(blockmask, causal, source=None):
+    """The order of the 16-row blocks the kernels' workgroups take them in (flash_attn_gfx950.blockmask_row_order): a function of
+    the blockmask's values alone, so that a call's results, which follow the order in their last bits (the reference point of a
+    row's exponentials depends on the rows beside it: up to 2.4e-4 in fp16, 2 x 512 tokens), do not depend on earlier calls.
+
+    It takes milliseconds to work out and the blockmask's values on the host, so it is kept for as long as the caller's mask
+    lives - `source`, the 0 / 1 layout that blockmask was converted from, or blockmask itself -, by that tensor (weakly) and its
+    version; for any other mask the values are read back and compared with those of the last 64.  (Writes that bypass
+    the version counter, as through .data, are not seen: the order is then another one, and valid.)"""
     if causal:
         return None
-    key = (blockmask.data_ptr(), tuple(blockmask.shape), blockmask._version, str(blockmask.device))
-    order = _ROW_ORDERS.get(key)
+    mask = blockmask if source is None else source
+    orders = None
+    if not mask.is_inference():
+        base = mask if mask._base is None else mask._base
+        look = (mask._version, mask.data_ptr(), mask.storage_offset(), tuple(mask.shape), mask.stride(), mask.dtype, mask.device,
+                source is None)
+        orders = _ORDERS_OF_MASKS.setdefault(base, {})
+        order = orders.get(look)
+    if orders is None or order is None:
+        order = _row_order_of_values(blockmask)
+        if orders is not None:
+            if len(orders) >= _ORDERS_KEPT:
+                orders.clear()
+            orders[look] = order
+    if order.is_cuda:  # (kept across streams: memory that a kernel on this one still reads is not given away)
+        order.record_stream(torch.cuda.current_stream(order.device))
+    return order
+
+
+def _row_order_of_values(blockmask):
+    conv = blockmask.cpu()
+    key = (tuple(conv.shape), conv.dtype, str(blockmask.device), conv.numpy().tobytes())
+    order = _ORDERS_OF_CONTENTS.pop(key, None)
     if order is None:
-        conv = blockmask.cpu()
         ncol, nrow = conv.shape
         layout = torch.zeros(nrow, ncol, dtype=torch.bool)
         cols = torch.arange(ncol)[:, None].expand(ncol, nrow)
         live = (conv >= 0) & ((conv >> 2) < nrow)
         layout[(conv >> 2)[live].long(), cols[live]] = True
         order = _backend.blockmask_row_order(layout).to(blockmask.device)
-        if len(_ROW_ORDERS) >= 64:
-            _ROW_ORDERS.clear()
-        _ROW_ORDERS[key] = order
+    while len(_ORDERS_OF_CONTENTS) >= _ORDERS_KEPT:
+        try:
+            _ORDERS_OF_CONTENTS.popitem(last=False)
+        except KeyError:  # (another thread took the last one)
+            break
+    _ORDERS_OF_CONTENTS[key] = order
     return order
 
 
 def _flash_blocksparse_attn_forward(qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal,
-                                    return_softmax, alibi_slopes=None, attn_bias=None, gen=None):
+                                    return_softmax, alibi_slopes=None, attn_bias=None, gen=None, row_order=None):
     res = _backend.fwd_block(qkv[:, 0], qkv[:, 1], qkv[:, 2], cu_seqlens, cu_seqlens, blockmask, max_s, max_s,
-                             dropout_p, softmax_scale, causal, return_softmax, gen, row_order=_row_order(blockmask, causal),
+                             dropout_p, softmax_scale, causal, return_softmax, gen, row_order=row_order,
                              alibi_slopes=alibi_slopes, attn_bias=attn_bias)
     return res[0], res[1], (res[2] if return_softmax else None)
 
 
 def _flash_blocksparse_attn_backward(dout, qkv, out, S_dmask, softmax_lse, cu_seqlens, blockmask, dropout_p, max_s,
-                                     softmax_scale, causal, alibi_slopes=None, attn_bias=None, dbias=None, gen=None):
+                                     softmax_scale, causal, alibi_slopes=None, attn_bias=None, dbias=None, gen=None, row_order=None):
     dqkv = torch.empty_like(qkv)
     _backend.bwd_block(dout.contiguous(), qkv[:, 0], qkv[:, 1], qkv[:, 2], out, softmax_lse, dqkv[:, 0], dqkv[:, 1],
                        dqkv[:, 2], cu_seqlens, cu_seqlens, blockmask, max_s, max_s, dropout_p, softmax_scale, causal,
-                       gen, row_order=_row_order(blockmask, causal), alibi_slopes=alibi_slopes, attn_bias=attn_bias,
+                       gen, row_order=row_order, alibi_slopes=alibi_slopes, attn_bias=attn_bias,
                        dbias=dbias)
     return dqkv
 
 
 def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes,
-                attn_bias):
+                attn_bias, row_order):
     philox = _backend.DrawnPhilox() if dropout_p > 0 else None  # (seed, offset) of the forward, used again by the backward
     if softmax_scale is None:
         softmax_scale = qkv.shape[-1] ** (-0.5)
+    if row_order is None:
+        row_order = _row_order(blockmask, causal)
     # the bias in the form the kernels read (the caller's tensor itself if its layout allows, else a padded copy)
     bias_t = None
     if attn_bias is not None:
@@ -93,8 +127,9 @@ def _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale
                                             int(max_s))
     context, softmax_lse, S_dmask = _flash_blocksparse_attn_forward(
         qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, return_softmax, alibi_slopes, bias_t,
-        philox)
+        philox, row_order)
     dropout_saved, ctx.dropout_kept = _backend.pack_dropout(None, philox)
+    ctx.row_order = row_order
     ctx.save_for_backward(qkv, context, softmax_lse, cu_seqlens, blockmask, bias_t, *dropout_saved)
     ctx.dropout_p = dropout_p
     ctx.max_s = max_s
@@ -115,39 +150,41 @@ def _bwd_common(ctx, dout):
         dbias = new_bias_grad(qkv[:, 0], cu_seqlens.numel() - 1, ctx.max_s, ctx.max_s)
     dqkv = _flash_blocksparse_attn_backward(dout, qkv, context, None, softmax_lse, cu_seqlens, blockmask,
                                             ctx.dropout_p, ctx.max_s, ctx.softmax_scale, ctx.causal, ctx.alibi_slopes,
-                                            bias_t, dbias, philox)
+                                            bias_t, dbias, philox, ctx.row_order)
     return dqkv, (bias_grad_in_shape(dbias, ctx.bias_shape, ctx.max_s, ctx.max_s) if dbias is not None else None)
 
 
 class FlashBlocksparseAttnFun(torch.autograd.Function):
-    """apply(qkv, cu_seqlens, blockmask_converted, dropout_p, max_s, softmax_scale, causal, alibi_slopes, attn_bias)
+    """apply(qkv, cu_seqlens, blockmask_converted, dropout_p, max_s, softmax_scale, causal, alibi_slopes, attn_bias, row_order)
     -> context"""
 
     @staticmethod
-    def forward(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes=None, attn_bias=None):
+    def forward(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes=None, attn_bias=None,
+                row_order=None):
         return _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, False, alibi_slopes,
-                           attn_bias)[0]
+                           attn_bias, row_order)[0]
 
     @staticmethod
     def backward(ctx, dout):
         dqkv, dbias = _bwd_common(ctx, dout)
-        return dqkv, None, None, None, None, None, None, None, dbias
+        return dqkv, None, None, None, None, None, None, None, dbias, None
 
 
 class FlashBlocksparseAttnFunWithS(torch.autograd.Function):
     """Same, returning (context, S_dmask, softmax_lse) for tests."""
 
     @staticmethod
-    def forward(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes=None, attn_bias=None):
+    def forward(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes=None, attn_bias=None,
+                row_order=None):
         context, S_dmask, softmax_lse = _fwd_common(ctx, qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale,
-                                                    causal, True, alibi_slopes, attn_bias)
+                                                    causal, True, alibi_slopes, attn_bias, row_order)
         ctx.mark_non_differentiable(S_dmask, softmax_lse)
         return context, S_dmask, softmax_lse
 
     @staticmethod
     def backward(ctx, dout, _dS_dmask_ignored, _dsoftmax_sum_ignored):
         dqkv, dbias = _bwd_common(ctx, dout)
-        return dqkv, None, None, None, None, None, None, None, dbias
+        return dqkv, None, None, None, None, None, None, None, dbias, None
 
 
 def flash_blocksparse_attn_func(qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale=None,
@@ -159,6 +196,8 @@ def flash_blocksparse_attn_func(qkv, cu_seqlens, blockmask, dropout_p, max_s, so
     alibi_slopes, attn_bias (extensions, as in flash_attn_unpadded_qkvpacked_func): a score bias inside the active
     blocks; attn_bias is differentiable."""
     func = FlashBlocksparseAttnFun if not return_attn_probs else FlashBlocksparseAttnFunWithS
+    row_order = None
     if convert_mask:
-        blockmask = convert_blockmask(blockmask, causal=causal)
-    return func.apply(qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes, attn_bias)
+        layout, blockmask = blockmask, convert_blockmask(blockmask, causal=causal)
+        row_order = _row_order(blockmask, causal, layout)
+    return func.apply(qkv, cu_seqlens, blockmask, dropout_p, max_s, softmax_scale, causal, alibi_slopes, attn_bias, row_order)

@@ -253,6 +253,69 @@ def test_blockmask_row_order_is_a_permutation_that_groups_similar_rows():
 
 
 # ---------------------------------------------------------------- host helpers
+def _layouts_to_order(n):
+    """0 / 1 layouts whose row orders are not the plain one and differ"""
+    g = torch.Generator().manual_seed(3)
+    return [torch.rand(64, 16, generator=g) < 0.3 for _ in range(n)]
+
+
+def test_row_order_follows_the_masks_values_not_its_address():
+    """A converted mask at the address of one that is gone, with the same shape and version, has its own order; so does a mask after a write to it."""
+    from flash_attn import flash_attn_gfx950 as be, flash_blocksparse_attn_interface as bi
+    a, b, c = _layouts_to_order(3)
+    want = [be.blockmask_row_order(m) for m in (a, b, c)]
+    assert not torch.equal(want[0], want[1]) and not torch.equal(want[1], want[2])
+    memory = np.empty((16, 64), dtype=np.int32)
+    at = None
+    for m, order in ((a, want[0]), (b, want[1])):
+        memory[:] = bi.convert_blockmask(m, causal=False).numpy()
+        conv = torch.from_numpy(memory)
+        assert at in (None, conv.data_ptr()) and conv._version == 0
+        at = conv.data_ptr()
+        assert torch.equal(bi._row_order(conv, False), order)
+        del conv
+    conv = bi.convert_blockmask(b, causal=False)
+    assert torch.equal(bi._row_order(conv, False), want[1])
+    conv.copy_(bi.convert_blockmask(c, causal=False))
+    assert torch.equal(bi._row_order(conv, False), want[2])
+    assert bi._row_order(conv, True) is None
+
+
+def test_row_order_is_worked_out_once_per_mask(monkeypatch):
+    """Kept with the caller's layout (whose converted form is a new tensor in every call), with views of it, and by its values where a call
+    makes a new layout; nothing is kept for a layout that is gone but the last 64 values."""
+    import gc
+    from flash_attn import flash_attn_gfx950 as be, flash_blocksparse_attn_interface as bi
+    calls, reads = [], []
+    worked_out, read = be.blockmask_row_order, bi._row_order_of_values
+    monkeypatch.setattr(be, "blockmask_row_order", lambda m: calls.append(1) or worked_out(m))
+    monkeypatch.setattr(bi, "_row_order_of_values", lambda m: reads.append(1) or read(m))
+    bi._ORDERS_OF_CONTENTS.clear()
+    gc.collect()
+    kept = len(bi._ORDERS_OF_MASKS)
+    layout, = _layouts_to_order(1)
+
+    def order(m):
+        return bi._row_order(bi.convert_blockmask(m, causal=False), False, m)
+
+    first = order(layout)
+    assert all(order(layout) is first for _ in range(3)) and (len(calls), len(reads)) == (1, 1)
+    part = order(layout[:32, :8])
+    assert order(layout[:32, :8]) is part and part.numel() == 32 and (len(calls), len(reads)) == (2, 2)
+    assert torch.equal(order(layout.clone()), first) and (len(calls), len(reads)) == (2, 3)
+    with torch.inference_mode():
+        assert order(layout) is first and order(layout[:32, :8]) is part and len(reads) == 3
+        assert torch.equal(order(layout.clone()), first) and len(calls) == 2 and len(reads) == 4  # (an inference tensor has no version)
+    layout[0] = ~layout[0]
+    assert not torch.equal(order(layout), first) and len(calls) == 3
+    for i in range(70):
+        order(torch.rand(16, 4, generator=torch.Generator().manual_seed(i)) < 0.5)
+    assert len(bi._ORDERS_OF_CONTENTS) <= 64
+    del layout
+    gc.collect()
+    assert len(bi._ORDERS_OF_MASKS) == kept
+
+
 def test_convert_blockmask_matches_spec():
     from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
     g = torch.Generator().manual_seed(0)

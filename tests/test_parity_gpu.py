@@ -1312,6 +1312,30 @@ def test_blocksparse_row_order(D, N, dtype):
         be.fwd_block(qg, kg, vg, cug, cug, conv, N, N, 0.0, D ** -0.5, False, False, None, row_order=bad)
 
 
+def test_blocksparse_results_do_not_follow_earlier_layouts():
+    """Converted masks made, used and freed one after the other lie at the same addresses: each call's bits are those of its own layout"""
+    from flash_attn import flash_blocksparse_attn_interface as bi
+    N, H, D = 1024, 2, 64
+    g = torch.Generator("cuda").manual_seed(11)
+    qkv = torch.randn(N, 3, H, D, device="cuda", dtype=torch.float16, generator=g)
+    dout = torch.randn(N, H, D, device="cuda", dtype=torch.float16, generator=g)
+
+    def run(seed):
+        layout = torch.rand(N // 16, N // 256, device="cuda", generator=torch.Generator("cuda").manual_seed(seed)) < 0.4
+        x = qkv.clone().requires_grad_()
+        out = bi.flash_blocksparse_attn_func(x, _cu([N]), layout, 0.0, N)
+        return (out.detach(),) + torch.autograd.grad(out, x, dout)
+
+    want = {}
+    for seed in range(6):
+        bi._ORDERS_OF_MASKS.clear()
+        bi._ORDERS_OF_CONTENTS.clear()
+        want[seed] = run(seed)
+    for seed in (3, 1, 4, 1, 5, 0, 2, 3, 0):
+        for x, y in zip(run(seed), want[seed]):
+            assert torch.equal(x, y), seed
+
+
 @pytest.mark.parametrize("Sq,Sk,H,B", [(16, 100, 1, 1), (300, 257, 3, 3), (130, 15900, 2, 2), (16390, 300, 1, 1)])
 def test_blocksparse_tiles_dearest_first(Sq, Sk, H, B):
     """Workgroups take a layout's query tiles and key blocks dearest first: one tile of each, a last key block half of whose keys have no
