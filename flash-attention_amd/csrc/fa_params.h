@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "fa_common.h"
 
 namespace fa {
@@ -400,8 +402,27 @@ FA_DEVICE bool map_live(int block, const int32_t* cu_own, int total_own, int max
 //   rows (38 x 16 x 414 .. 628 46.1 / 48.8) of more than 256-token sequences (64 x 8 x 42 .. 109 7.9 / 8.2, 64 x 16 x 172 .. 202 d = 128 42.4 /
 //   44.7) in more than 150 workgroups (2 x 12 x 553 .. 787 14.8 / 15.4), dK/dV, whose empty slots come last, where its pairs are taken in groups
 //   (causal_tile_group; 3 x 16 x 2821 .. 5841 dQ alone 481, both 441; 14 x 16 x 471 .. 703, no groups, 82.0 / 86.1).  At d = 32 many
-//   pairs in groups stay with them, whose K and V it would read again: 64 x 16 x 509 .. 926 100.9 / 122.5, 38 x 12 x 353 .. 1766 91.2 / 101.2.
+//   pairs in groups stay with them, whose K and V it would read again: 64 x 16 x 509 .. 926 100.9 / 122.5, 38 x 12 x 353 .. 1766 91.2 / 101.2;
+//   and so does what live_order_rereads names.
+//
+// Under a causal mask the live order has all of an XCD's pairs in flight and reads their K and V (dK/dV: Q and dO) past its L2 for every level; the
+// other one takes them in groups that fit.  The more pairs share the L2 and the more the batch holds beyond the 256 MB of the memory-side cache,
+// the more that costs, and the fuller the slots, the less the empty ones did.  Lines through the times of 1238 grouped shapes (d = 16 .. 128, 2 to
+// 64 entries, 270 .. 7986 tokens, shortest 0.2 .. 0.9 of the longest).  Over 900 others a step's kernels take 0.92 (d = 64), 0.91 (128), 0.98 (32) of the
+// groups' time, at most 1.03, and over 500 a forward alone 0.93, 0.93 and 0.98, at most 1.06; the live order regardless 0.93, 0.92, 0.99, at most
+// 1.24, and 0.95, 0.97, 1.01, at most 1.51.
+// us in groups / live: forward d = 128 64 x 16 x 614 .. 1024 286 / 409, 32 x 16 x 1229 .. 2048 459 / 541, 28 x 12 x 938 .. 1537 183 / 196, 16 x 8 x 1229 .. 4096 (live) 366 / 271, d = 64
+// 64 x 16 x 1229 .. 2048 509 / 640, 63 x 8 x 1970 .. 2463 383 / 444, 32 x 16 x 614 .. 2048 (live) 215 / 192, d = 32 20 x 12 x 2458 .. 4096 281 / 366; dQ d = 64
+// 64 x 16 x 1229 .. 2048 699 / 822, d = 128 41 x 16 x 1650 .. 2261 1142 / 1443, 64 x 12 x 416 .. 520 (live) 185 / 159; dK/dV d = 64 36 x 16 x 1785 .. 3719 1299 / 1407.
 enum LiveKernel { kLiveFwd, kLiveDq, kLiveDkdv, kLiveMerged };
+inline bool live_order_rereads(LiveKernel kernel, int head_dim, int64_t live, int64_t slots, int B, int H, int total) {
+  const bool fwd = kernel == kLiveFwd, dq = kernel == kLiveDq;
+  const double mb = (double)total * H * head_dim * 4 / (1 << 20), pairs = (B * H + 7) / 8;
+  if (!fwd && head_dim >= 64 && mb <= 256) return false;
+  const double most = head_dim == 16 ? (fwd || dq ? 1.5 : 2.0) : head_dim == 32 ? (fwd || dq ? 1.86 : 2.32)
+                      : fwd ? (head_dim == 64 ? 2.28 : 2.16) : dq || head_dim == 64 ? 2.3 : 2.48;
+  return (double)live / slots + 0.08 * std::log2(pairs * pairs * mb) > most;
+}
 inline bool live_order_launch(LiveKernel kernel, int head_dim, bool causal, int B, int H, int total, int max_s, int n_splits, int tiles, int tile_group,
                               int grid) {
   if (n_splits > 1 || B > 64 || tiles > 64 || (int64_t)total * 20 > (int64_t)19 * B * max_s) return false;
@@ -409,8 +430,9 @@ inline bool live_order_launch(LiveKernel kernel, int head_dim, bool causal, int 
   if (!causal) return true;
   if (kernel == kLiveDkdv && (tile_group <= 0 || max_s <= 640)) return false;
   if (head_dim <= 32 && tile_group > 0 && B * H >= 256) return false;
-  const int64_t live = (int64_t)H * (total + (int64_t)64 * B) / 128;
-  return max_s > 256 && live > 150 && 10 * live <= (int64_t)9 * B * H * ((max_s + 127) / 128);
+  const int64_t live = (int64_t)H * (total + (int64_t)64 * B) / 128, slots = (int64_t)B * H * ((max_s + 127) / 128);
+  if (tile_group > 0 && live_order_rereads(kernel, head_dim, live, slots, B, H, total)) return false;
+  return max_s > 256 && live > 150 && 10 * live <= 9 * slots;
 }
 inline bool live_order_rows(int B, int tiles) { return B <= 64 && tiles <= 64; }
 inline int tile_grid(bool tile_major, int tiles_per_bh, int BH) {

@@ -831,6 +831,27 @@ def test_padded_forward_tiles_follow_the_measurements(tmp_path):
     assert half == [c[-1] for c in cases], [c for c, g in zip(cases, half) if g != c[-1]]
 
 
+def test_live_order_not_where_it_reads_keys_again(tmp_path):
+    """ragged causal launches of many pairs, whose K and V the groups of the other order keep in L2: us in groups / live"""
+    cases = [  # kernel, head dim, batch, heads, longest, shortest / longest, live order?
+        ("kLiveFwd", 128, 64, 16, 1024, 0.6, 0), ("kLiveFwd", 128, 64, 16, 2048, 0.3, 0), ("kLiveFwd", 128, 32, 16, 2048, 0.6, 0),  # 286 / 409, 675 / 953, 459 / 541
+        ("kLiveFwd", 64, 64, 16, 2048, 0.6, 0), ("kLiveFwd", 64, 63, 8, 2463, 0.8, 0), ("kLiveFwd", 32, 20, 12, 4096, 0.6, 0),  # 509 / 640, 383 / 444, 281 / 366
+        ("kLiveFwd", 16, 20, 12, 7900, 0.6, 0), ("kLiveDq", 16, 20, 12, 7900, 0.6, 0), ("kLiveDq", 32, 20, 12, 4096, 0.6, 0),  # 1009 / 1216, 1026 / 1314, 331 / 396
+        ("kLiveDq", 64, 64, 16, 2048, 0.6, 0), ("kLiveDq", 128, 64, 16, 2048, 0.3, 0), ("kLiveDq", 128, 41, 16, 2261, 0.73, 0),  # 699 / 822, 992 / 1254, 1142 / 1443
+        ("kLiveDkdv", 64, 31, 16, 3723, 0.65, 0), ("kLiveDkdv", 64, 36, 16, 3719, 0.48, 0),  # 1324 / 1440, 1299 / 1407
+        ("kLiveFwd", 64, 32, 16, 2048, 0.3, 1), ("kLiveFwd", 128, 16, 8, 4096, 0.3, 1), ("kLiveFwd", 32, 7, 12, 7900, 0.3, 1),  # 215 / 192, 366 / 271, 279 / 246
+        ("kLiveDq", 128, 64, 12, 520, 0.8, 1), ("kLiveDq", 64, 32, 16, 2048, 0.3, 1), ("kLiveDkdv", 128, 64, 8, 1024, 0.3, 1),  # 185 / 159, 292 / 239, 235 / 191
+        ("kLiveDkdv", 64, 64, 16, 1024, 0.3, 1), ("kLiveDkdv", 128, 20, 12, 4096, 0.3, 1)]  # 219 / 195, 1327 / 1061
+
+    def group(d, b, h, n):  # causal_tile_group
+        kv, pairs = 4 * n * d, -(-b * h // 8)
+        return 0 if pairs * kv <= 8 << 20 else max(4, (6 << 20) // kv)
+
+    got = _launch_rules(tmp_path, ["live_order_launch(%s, %d, 1, %d, %d, %d, %d, 1, %d, %d, %d)" % (
+        k, d, b, h, _spread(n, f, b), n, -(-n // 128), group(d, b, h, n), -(-b * h // 8) * 8 * -(-n // 128)) for k, d, b, h, n, f, _ in cases])
+    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+
+
 def test_live_order_where_measured(tmp_path):
     """ragged launches whose workgroups enumerate the tiles that hold rows, and those that keep the slot orders"""
     cases = [  # kernel, head dim, causal, batch, heads, longest, shortest / longest, tile_group, grid, live order?
