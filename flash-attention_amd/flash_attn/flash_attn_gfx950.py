@@ -150,6 +150,20 @@ def _load_host(lib):
     return host
 
 
+def _check_library(lib):
+    """Raises if lib is not the library this binding was written for: another version of the structs, or one built before an entry point was added
+    (the version counts changes of what was there, so it does not tell)."""
+    if not hasattr(lib, "fa_abi_version"):
+        raise RuntimeError("%s has no fa_abi_version: not this binding's library" % LIB_NAME)
+    lib.fa_abi_version.argtypes = []
+    lib.fa_abi_version.restype = ctypes.c_int
+    if lib.fa_abi_version() != FA_ABI_VERSION:
+        raise RuntimeError("%s has ABI version %d, binding expects %d" % (LIB_NAME, lib.fa_abi_version(), FA_ABI_VERSION))
+    missing = [name for name in EXPORTED_SYMBOLS + BENCH_SYMBOLS if not hasattr(lib, name)]
+    if missing:
+        raise RuntimeError("%s lacks %s; build it again with `python flash-attention_amd/build.py`." % (LIB_NAME, ", ".join(missing)))
+
+
 def load_library():
     """dlopen the shared library once and declare the prototypes.  Raises if it has not been built."""
     global _lib, _host, _passes
@@ -163,6 +177,7 @@ def load_library():
                 "%s is not built (expected at %s); run `python flash-attention_amd/build.py`. "
                 "There is no non-HIP fallback." % (LIB_NAME, LIB_PATH))
         lib = ctypes.CDLL(LIB_PATH)
+        _check_library(lib)
         for name in ("fa_fwd", "fa_fwd_block", "fa_fwd_block_noalloc"):
             fn = getattr(lib, name)
             fn.argtypes = [ctypes.POINTER(FwdArgs)]
@@ -185,8 +200,6 @@ def load_library():
         lib.fa_philox_offset_increment.restype = ctypes.c_uint64
         lib.fa_last_error.argtypes = []
         lib.fa_last_error.restype = ctypes.c_char_p
-        lib.fa_abi_version.argtypes = []
-        lib.fa_abi_version.restype = ctypes.c_int
         lib.fa_gather_rows.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int64] * 5 + [ctypes.c_void_p]
         lib.fa_gather_rows.restype = ctypes.c_int
         lib.fa_scatter_rows.argtypes = ([ctypes.c_void_p] * 3 + [ctypes.c_int64] * 5 +
@@ -213,8 +226,6 @@ def load_library():
         lib.fa_blocksparse_row_order.restype = ctypes.c_int
         lib.fa_set_launch_policy.argtypes = [ctypes.c_int]
         lib.fa_set_launch_policy.restype = ctypes.c_int
-        if lib.fa_abi_version() != FA_ABI_VERSION:
-            raise RuntimeError("%s has ABI version %d, binding expects %d" % (LIB_NAME, lib.fa_abi_version(), FA_ABI_VERSION))
         _host = _passes = _load_host(lib)
         _lib = lib
     return _lib

@@ -29,6 +29,25 @@ def test_library_exports_every_declared_symbol(lib):
     assert lib.fa_abi_version() == be.FA_ABI_VERSION == 5
 
 
+@pytest.mark.parametrize("version, says", [(4, "has ABI version 4, binding expects 5"), (5, "lacks fa_fwd, .*fa_token_positions.*build it again"),
+                                           (None, "has no fa_abi_version")])
+def test_another_library_is_named_as_such(lib, tmp_path, monkeypatch, version, says):
+    """a library of another version, or one built before an entry point was added, is refused with a message, not by a missing symbol; the one in
+    use stays in use"""
+    import subprocess
+    from flash_attn import flash_attn_gfx950 as be
+    src, so = tmp_path / "other.c", tmp_path / "other.so"
+    src.write_text("int nothing;" if version is None else "int fa_abi_version(void) { return %d; }" % version)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    for name, value in (("_lib", None), ("_host", None), ("_passes", None), ("LIB_PATH", str(so))):
+        monkeypatch.setattr(be, name, value)
+    with pytest.raises(RuntimeError, match=says):
+        be.load_library()
+    assert be._lib is None and be._host is None
+    monkeypatch.undo()
+    assert be.load_library() is lib
+
+
 def test_struct_layout_matches_library(lib):
     """a wrong struct size is reported as an ABI mismatch; the right size passes that check"""
     from flash_attn import flash_attn_gfx950 as be
