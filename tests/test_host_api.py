@@ -885,3 +885,19 @@ def test_live_order_where_measured(tmp_path):
     assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
     assert _launch_rules(tmp_path, ["live_order_launch(kLiveFwd, 64, 0, 4, 8, 1000, 1000, 2, 8, 0, 256)", "live_order_rows(64, 64)", "live_order_rows(65, 1)",
                                     "live_order_rows(1, 65)"]) == [0, 1, 0, 0]
+
+
+def test_live_order_batches_of_the_gpu_tests_take_it(tmp_path):
+    """forward, dQ and dK/dV of the batch on which the variants are compared (16 heads, 1500 tokens and 31 sequences of 300 to 510), in full-size and
+    half-size tiles, with a causal mask and without; not with 33 empty sequences behind it"""
+    lens = [1500] + [300 + 7 * i for i in range(31)]
+    n, total, expressions = max(lens), sum(lens), []
+    for d in (64, 128):
+        group = max(4, (6 << 20) // (4 * n * d))  # causal_tile_group: 64 pairs of an XCD are beyond its L2
+        for causal in (0, 1):
+            for rows in (128, 64):
+                tiles = -(-n // rows)
+                for kernel in ("kLiveFwd", "kLiveDq") + (("kLiveDkdv",) if rows == 128 else ()):
+                    expressions += ["live_order_launch(%s, %d, %d, %d, 16, %d, %d, 1, %d, %d, %d)" % (
+                        kernel, d, causal, b, total, n, tiles, group * causal, b * 16 * tiles) for b in (32, 65)]
+    assert _launch_rules(tmp_path, expressions) == [1, 0] * (len(expressions) // 2)

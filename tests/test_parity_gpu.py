@@ -2911,6 +2911,38 @@ def test_live_order_reaches_every_tile(H, D, lens, causal, full_size_tiles):
             assert torch.equal(x[a:a + n], y), (name, b, n)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kind", ["plain", "ALiBi", "rotary", "keep words", "redrawn", "ALiBi, keep words"])
+def test_live_order_in_every_variant(kind, D, causal, tile_shape):
+    """A step of a ragged batch that forward, dQ and dK/dV take in the live order, bit for bit as with 33 empty sequences behind it: 65 entries, which
+    go in the slot order, with the same batch index (that of the dropout counters and keep words) for every row."""
+    from flash_attn import flash_attn_gfx950 as be, flash_attn_interface as fi
+    H, _, lens = LIVE_ORDER_BATCHES[1]
+    N, dtype = max(lens), torch.float16
+    q, k, v, do = (x.cuda() for x in _inputs(lens, lens, H, D, dtype, 13))
+    qkv = torch.stack([q, k, v], 1)
+    slopes = 2.0 ** (-8.0 * torch.arange(1, H + 1, device="cuda") / H) if "ALiBi" in kind else None
+    angle = torch.outer(torch.arange(N, device="cuda").float(), 10000.0 ** (-torch.arange(0, D, 2, device="cuda").float() / D))
+    p = 0.2 if "words" in kind or kind == "redrawn" else 0.0
+    old = be.KEEP_WORDS_MAX_BYTES, be.KEEP_WORDS_MAX_INPUT_RATIO
+    be.KEEP_WORDS_MAX_BYTES, be.KEEP_WORDS_MAX_INPUT_RATIO = (0 if kind == "redrawn" else 1 << 30), None
+    try:
+        results = []
+        for cu in (_cu(lens), _cu(lens + [0] * 33)):
+            x = qkv.clone().requires_grad_()
+            torch.manual_seed(5)
+            if kind == "rotary":
+                out = fi.flash_attn_unpadded_qkvpacked_rotary_func(x, torch.cos(angle).to(dtype), torch.sin(angle).to(dtype), cu, N, p, causal=causal)
+            else:
+                out = fi.flash_attn_unpadded_qkvpacked_func(x, cu, N, p, causal=causal, alibi_slopes=slopes)
+            results.append((out.detach(),) + torch.autograd.grad(out, x, do))
+    finally:
+        be.KEEP_WORDS_MAX_BYTES, be.KEEP_WORDS_MAX_INPUT_RATIO = old
+    for name, x, y in zip(("out", "dqkv"), *results):
+        assert x.isfinite().all() and torch.equal(x, y), name
+
+
 @pytest.mark.parametrize("listed", [False, True])
 @pytest.mark.parametrize("B, H, D, N, causal", [(64, 3, 64, 200, False), (5, 12, 32, 700, True), (3, 16, 64, 1100, False)])
 def test_padded_batches_in_live_order_write_every_row(B, H, D, N, causal, listed):
