@@ -435,6 +435,19 @@ inline bool live_order_launch(LiveKernel kernel, int head_dim, bool causal, int 
   return max_s > 256 && live > 150 && 10 * live <= 9 * slots;
 }
 inline bool live_order_rows(int B, int tiles) { return B <= 64 && tiles <= 64; }
+// The forward over a padded batch, whose number of tokens is not known here (map_live's info).  Without a mask wherever there is more than one entry to
+// order (one: 12.5 / 12.7 us at 12 heads x 860, 17.3 / 17.7 at 5 x 1865; over 300 others at most 1.01 of the slot order's time, 0.95 in the mean).  Under a
+// causal mask from two workgroups a compute unit on (16 x 3 heads x 172 6.4 / 7.0 us, 14 x 12 x 300 9.8 / 10.2), and not where its pairs, all in
+// flight, read their K and V past the L2 (live_order_rereads, here by the rows there may be): all rows tokens, d = 64 64 x 16 x 2048 728 / 1028 us,
+// 32 x 24 x 2197 654 / 839, 16 x 16 x 4096 (live) 688 / 674, d = 32 36 x 16 x 3218 718 / 983, 33 x 8 x 4321 543 / 661, d = 16 44 x 8 x 5687 1129 / 1459,
+// 40 x 16 x 533 42.9 / 45.8.  700 drawn shapes: 0.94 (d = 64), 0.98 (32, 16), at most 1.01; given up where many rows are padding (32 x 16 x 2048, 30 %
+// to all tokens, 231 / 203).
+inline bool live_order_padded(int head_dim, bool causal, int B, int H, int max_s, int tiles) {
+  if (!live_order_rows(B, tiles)) return false;
+  if (!causal) return B > 1;
+  const double mb = (double)B * max_s * H * head_dim * 4 / (1 << 20), pairs = (B * H + 7) / 8;
+  return (int64_t)B * H * ((max_s + 127) / 128) >= 512 && pairs * pairs * mb <= (head_dim <= 16 ? 16384 : head_dim == 32 ? 32768 : 440000);
+}
 inline int tile_grid(bool tile_major, int tiles_per_bh, int BH) {
   return ((BH + 7) & ~7) * tiles_per_bh;
 }

@@ -901,3 +901,18 @@ def test_live_order_batches_of_the_gpu_tests_take_it(tmp_path):
                     expressions += ["live_order_launch(%s, %d, %d, %d, 16, %d, %d, 1, %d, %d, %d)" % (
                         kernel, d, causal, b, total, n, tiles, group * causal, b * 16 * tiles) for b in (32, 65)]
     assert _launch_rules(tmp_path, expressions) == [1, 0] * (len(expressions) // 2)
+
+
+def test_live_order_of_padded_batches_where_measured(tmp_path):
+    """the forward over a padded batch: us in the slot order (groups) / live, all rows tokens or 30 % of them and more"""
+    cases = [  # head dim, causal, batch, heads, rows, live order?
+        (64, 1, 64, 16, 2048, 0), (64, 1, 32, 24, 2197, 0), (32, 1, 36, 16, 3218, 0), (32, 1, 33, 8, 4321, 0),  # 728 / 1028, 654 / 839, 718 / 983, 543 / 661
+        (32, 1, 21, 16, 3933, 0), (16, 1, 7, 24, 7411, 0), (16, 1, 44, 8, 5687, 0), (16, 1, 40, 16, 533, 0),  # 590 / 785, 858 / 1131, 1129 / 1459, 42.9 / 45.8
+        (64, 1, 16, 3, 172, 0), (64, 1, 14, 12, 300, 0), (16, 1, 28, 8, 183, 0), (64, 1, 4, 3, 162, 0),  # 6.4 / 7.0, 9.8 / 10.2, 5.9 / 6.3, 6.2 / 6.5
+        (64, 0, 1, 5, 1865, 0), (32, 0, 1, 8, 795, 0), (64, 1, 65, 16, 512, 0), (64, 0, 65, 16, 512, 0),  # 21.1 / 21.7, 9.6 / 9.8
+        (64, 1, 8, 12, 2048, 1), (64, 1, 16, 16, 4096, 1), (64, 1, 30, 12, 786, 1),  # 70.3 / 67.8, 688 / 674, 62.0 / 54.5
+        (16, 1, 4, 8, 4720, 1), (64, 0, 64, 16, 512, 1), (64, 0, 46, 3, 197, 1), (32, 0, 62, 8, 2120, 1)]  # 70.1 / 51.9, 75.6 / 68.5, ..
+    got = _launch_rules(tmp_path, ["live_order_padded(%d, %d, %d, %d, %d, %d)" % (d, c, b, h, n, -(-n // 128)) for d, c, b, h, n, _ in cases])
+    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+    # the GPU test of the order, whose causal batches are to take it
+    assert _launch_rules(tmp_path, ["live_order_padded(32, 1, 12, 8, 700, 11)", "live_order_padded(64, 1, 9, 16, 600, 10)"]) == [1, 1]

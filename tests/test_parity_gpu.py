@@ -2944,7 +2944,8 @@ def test_live_order_in_every_variant(kind, D, causal, tile_shape):
 
 
 @pytest.mark.parametrize("listed", [False, True])
-@pytest.mark.parametrize("B, H, D, N, causal", [(64, 3, 64, 200, False), (5, 12, 32, 700, True), (3, 16, 64, 1100, False)])
+@pytest.mark.parametrize("B, H, D, N, causal", [(64, 3, 64, 200, False), (5, 12, 32, 700, True), (3, 16, 64, 1100, False),
+                                               (12, 8, 32, 700, True), (9, 16, 64, 600, True)])
 def test_padded_batches_in_live_order_write_every_row(B, H, D, N, causal, listed):
     """A padded batch in place: token rows are those of a launch that holds nothing but its sequence (one entry, lengths equal), padding rows are
     zeros, entries without any token included."""
