@@ -70,7 +70,7 @@ struct BwdCfg {
   static constexpr int kBiasTileBytes = BM * 32 * 2;  // per wave, behind everything else: the bias-tensor variants' tile
 };
 
-// The variants that know kLiveOrder (map_live): the dense ones but those whose main loop it would cost registers
+// The variants that come in the live order, too (kLive below, map_live)
 template <bool kSparse, int kBias>
 struct DkdvLive {
   static constexpr bool value = !kSparse && kBias != kBiasTensor;
@@ -85,7 +85,8 @@ struct DkdvLive {
 // kOwnD: the kernel forms Dk = keep * rowsum(dO o O) of every tile's rows itself instead of reading what the dQ kernel left in
 // p.dsoftmax (four threads per row, 16 elements each, fetched with the tile): it then depends on nothing the dQ kernel writes,
 // and the two can share one launch (fa_bwd_merged_kernel).  64-row tiles, head dim 64.
-template <typename T, int D, bool kCausal, int kDrop, bool kSparse, int kBias = 0, bool kRot = false, bool kOwnD = false>
+// kLive: as in fa_fwd_body
+template <typename T, int D, bool kCausal, int kDrop, bool kSparse, int kBias, bool kRot, bool kOwnD, bool kLive>
 FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned char* const lds_raw) {
   static_assert(!kRot || (!kSparse && kBias == 0), "rotary: dense variants without score bias");
   static_assert(!kOwnD || (D == 64 && !kSparse && kBias == 0 && BwdCfg<T, D, kDrop == 1>::BM == 64), "own Dk: d = 64, dense");
@@ -107,7 +108,7 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   // XCD-aware id map (see map_tile): the key tiles of one (batch, head) share one XCD's L2 copy of Q and dO.
   int q_begin = 0, Lq = 0, k_begin = 0, Lk = 0;
   int b, h, kt;  // under a causal mask the first key tiles see the most query rows: rank order is already heavy-first
-  if (DkdvLive<kSparse, kBias>::value && p.tile_group == kLiveOrder) {
+  if constexpr (kLive) {
     TileId id;
     if (!map_live<kCausal>(block, p.cu_k, p.total_k, p.max_sk, p.cu_q, p.total_q, p.max_sq, BN, p.nk_tiles, true, p.B, p.H, nullptr,
                            lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
@@ -365,6 +366,7 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   }
   finish_kv();
   if (kTensorBias && more) load_bias(mt * BM, tc.rb);
+  asm volatile(".p2align 7");  // (as in fa_fwd_body: d = 64 causal 4 x 8 heads x 1000 and its like 1.008 / 0.998 of the time without the live order's code)
   while (more) {
     const int m0 = mt * BM;
     if constexpr ((FA_ABLATE_DKDV & 1) == 0) wait_vmem();  // this thread's share of the tile has arrived (LDS) / is in statpre
@@ -603,7 +605,12 @@ template <typename T, int D, bool kCausal, int kDrop, bool kSparse, int kBias = 
 __global__ void __launch_bounds__(256, (kDrop == 0 && D <= 64 && kBias != kBiasTensor) ? 3 : ((D == 128 && kBias == kBiasTensor) ? 1 : BwdCfg<T, D, kDrop == 1>::kMinBlocks)) fa_bwd_dkdv_kernel(const BwdParams p) {
   using Cfg = BwdCfg<T, D, kDrop == 1>;
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kBias == kBiasTensor ? 4 * Cfg::kBiasTileBytes : 0)];
-  fa_bwd_dkdv_body<T, D, kCausal, kDrop, kSparse, kBias, kRot>(p, blockIdx.x, lds_raw);
+  fa_bwd_dkdv_body<T, D, kCausal, kDrop, kSparse, kBias, kRot, false, false>(p, blockIdx.x, lds_raw);
+}
+template <typename T, int D, bool kCausal, int kDrop, int kBias, bool kRot>
+__global__ void __launch_bounds__(256, ((kDrop == 0 && D <= 64) ? 3 : BwdCfg<T, D, kDrop == 1>::kMinBlocks)) fa_bwd_dkdv_live_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[BwdCfg<T, D, kDrop == 1>::kLdsBytes];
+  fa_bwd_dkdv_body<T, D, kCausal, kDrop, false, kBias, kRot, false, true>(p, blockIdx.x, lds_raw);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -876,7 +883,7 @@ struct DqCfg {
 
 // kDrop: as in fa_bwd_dkdv_kernel
 // (the kernel proper is fa_bwd_dq_kernel below: `block` is its workgroup id, `lds_raw` its LDS)
-template <typename T, int D, int BN, bool kCausal, int kDrop, bool kSparse, int kBias = 0, int KS = 1>
+template <typename T, int D, int BN, bool kCausal, int kDrop, bool kSparse, int kBias, int KS, bool kLive>
 FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char* const lds_raw) {
   constexpr bool kDropout = kDrop == 1, kStored = kDrop == 2;
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
@@ -895,11 +902,12 @@ FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char
   int b, h, qt, split = 0;
   int q_begin = 0, Lq = 0, k_begin = 0, Lk = 0;
   const int n_splits = p.n_splits > 1 ? p.n_splits : 1;  // key splits per query tile (see BwdParams)
-  if (!kSparse && p.tile_group == kLiveOrder) {
+  if constexpr (kLive) {
     TileId id;
     if (!map_live<kCausal>(block, p.cu_q, p.total_q, p.max_sq, p.cu_k, p.total_k, p.max_sk, BM, p.nq_tiles, false, p.B, p.H, nullptr,
                            lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
     b = id.b; h = id.h; qt = id.tile;
+    asm volatile("" : "+s"(split));  // (as in fa_fwd_body; causal d = 128 2 x 8 x 1200 .. 2000, backward, 144.9 us for 119.1)
     q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
   } else {
     int bh, rank;
@@ -1101,6 +1109,7 @@ FA_DEVICE void fa_bwd_dq_body(const BwdParams& p, const int block, unsigned char
   }
 #pragma unroll
   for (int r = 0; r < 16; r++) negd[r] = kInitNegD ? -dkv : 0.f;
+  asm volatile(".p2align 7");  // (as in fa_fwd_body)
   while (it < ntiles) {
     const int n0 = it * BN;
     // Opaque redefinition of the accumulators (keeps the register allocator from copying them around the loop)
@@ -1293,7 +1302,13 @@ template <typename T, int D, int BN, bool kCausal, int kDrop, bool kSparse, int 
 __global__ void __launch_bounds__(256, (D <= 64 && kDrop != 2 && kBias != kBiasTensor) ? 3 : 2) fa_bwd_dq_kernel(const BwdParams p) {
   using Cfg = DqCfg<T, D, BN, KS>;
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kBias == kBiasTensor ? 4 * Cfg::kBiasWaveBytes : 0)];
-  fa_bwd_dq_body<T, D, BN, kCausal, kDrop, kSparse, kBias, KS>(p, blockIdx.x, lds_raw);
+  fa_bwd_dq_body<T, D, BN, kCausal, kDrop, kSparse, kBias, KS, false>(p, blockIdx.x, lds_raw);
+}
+template <typename T, int D, int BN, bool kCausal, int kDrop, int kBias, int KS>
+__global__ void __launch_bounds__(256, (D <= 64 && kDrop != 2 && kBias != kBiasTensor) ? 3 : 2) fa_bwd_dq_live_kernel(const BwdParams p) {
+  using Cfg = DqCfg<T, D, BN, KS>;
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kBias == kBiasTensor ? 4 * Cfg::kBiasWaveBytes : 0)];
+  fa_bwd_dq_body<T, D, BN, kCausal, kDrop, false, kBias, KS, true>(p, blockIdx.x, lds_raw);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1303,8 +1318,8 @@ __global__ void __launch_bounds__(256, (D <= 64 && kDrop != 2 && kBias != kBiasT
 // pays that twice.  Here the workgroups of the dK/dV kernel (ids below p.merged_dkdv_blocks; they form their own Dk, kOwnD) and
 // the half-size workgroups of the dQ kernel (the ids after them) make one grid: one fill, one drain, and the two kinds run
 // side by side.  Head dim 64, dense, no score bias; kDrop 0 or 2.
-template <typename T, bool kCausal, int kDrop>
-__global__ void __launch_bounds__(256, 2) fa_bwd_merged_kernel(const BwdParams p) {
+template <typename T, bool kCausal, int kDrop, bool kLive>
+FA_DEVICE void fa_bwd_merged_body(const BwdParams& p) {
   constexpr int D = 64;
   using CfgK = BwdCfg<T, D, kDrop == 1>;
   using CfgQ = DqCfg<T, D, 64, 2>;
@@ -1312,12 +1327,20 @@ __global__ void __launch_bounds__(256, 2) fa_bwd_merged_kernel(const BwdParams p
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[kLds];
   const int block = blockIdx.x;
   if (block < p.merged_dkdv_blocks) {
-    fa_bwd_dkdv_body<T, D, kCausal, kDrop, false, 0, false, true>(p, block, lds_raw);
+    fa_bwd_dkdv_body<T, D, kCausal, kDrop, false, 0, false, true, kLive>(p, block, lds_raw);
   } else {
     BwdParams pq = p;
     pq.nq_tiles = p.merged_nq_tiles;
-    fa_bwd_dq_body<T, D, 64, kCausal, kDrop, false, 0, 2>(pq, block - p.merged_dkdv_blocks, lds_raw);
+    fa_bwd_dq_body<T, D, 64, kCausal, kDrop, false, 0, 2, kLive>(pq, block - p.merged_dkdv_blocks, lds_raw);
   }
+}
+template <typename T, bool kCausal, int kDrop>
+__global__ void __launch_bounds__(256, 2) fa_bwd_merged_kernel(const BwdParams p) {
+  fa_bwd_merged_body<T, kCausal, kDrop, false>(p);
+}
+template <typename T, int kDrop>
+__global__ void __launch_bounds__(256, 2) fa_bwd_merged_live_kernel(const BwdParams p) {
+  fa_bwd_merged_body<T, false, kDrop, true>(p);
 }
 
 }  // namespace fa

@@ -55,7 +55,7 @@ struct FwdCfg {
   static constexpr int CH = D / 8;
 };
 
-// The variants that know kLiveOrder (map_live): the dense ones but those whose main loop it would cost registers
+// The variants that come in the live order, too (kLive below, map_live)
 template <int D, bool kSparse, int kBias>
 struct FwdLive {
   static constexpr bool value = !kSparse && kBias != kBiasTensor && !(kBias == kPaddedRows && D == 128);
@@ -84,9 +84,12 @@ constexpr int fwd_waves(int d, bool dropout, bool sparse, int bias, int ks, bool
 // tokens; these attend each other, counted in their own order, and the padding rows of o are written as zeros.  32 x 512 rows, 256 .. 512 of
 // them tokens, 16 heads, d = 64: one launch of 43 us in place of gather 29, forward 40 and scatter 15, 42 with tokens anywhere in their row (the
 // module call 52 us, 175 gathered).
-template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
-          bool kWords = false>
-__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % kPaddedRows, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
+// kLive: the workgroups' ids enumerate the tiles that hold rows (map_live).  A kernel of its own: with both orders' code in one, launches in the slot order
+// paid for the other's, in registers, parked scalars and arguments loaded again in the main loop.  us, both in one / apart, equal lengths: backward
+// without a mask, d = 64 16 x 1500 45.2 / 41.5, 2 x 8 x 2000 72.9 / 69.5, 8 x 12 x 512 37.5 / 35.2; causal 7 x 24 x 132 .. 268 19.4 / 18.8; forward d = 16
+// causal 3 x 3 x 4049 30.4 / 28.9, d = 128 causal with keep words 2 x 12 x 3218 108.9 / 106.1.
+template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias, int KS, bool kWords, bool kLive>
+FA_DEVICE void fa_fwd_body(const FwdParams& p) {
   constexpr bool kRows = kBias == kPaddedRows;
   constexpr bool kBiased = kBias != 0 && !kRows;
   constexpr bool kAlibi = kBias == kBiasAlibi, kTensorBias = kBias == kBiasTensor;
@@ -118,14 +121,15 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
   // one XCD's L2 copy of K and V.
   int b, h, qt, split = 0;
   int q_begin, Lq, k_begin = 0, Lk = 0;
-  const int n_splits = p.n_splits > 1 ? p.n_splits : 1;   // key splits per query tile (see FwdParams)
-  bool mapped = false;
-  if constexpr (FwdLive<D, kSparse, kBias>::value) mapped = p.tile_group == kLiveOrder;
-  if (mapped) {
+  const int n_splits = p.n_splits > 1 ? p.n_splits : 1;  // key splits per query tile (see FwdParams)
+  if constexpr (kLive) {
     TileId id;
     if (!map_live<kCausal>(blockIdx.x, p.cu_q, p.total_q, p.max_sq, p.cu_k, p.total_k, p.max_sk, BM, p.nq_tiles, false, p.B, p.H,
                            kRows ? p.row_info : nullptr, lds_raw + kBufBytes + (threadIdx.x >> 6) * 256, &id)) return;
     b = id.b; h = id.h; qt = id.tile;
+    // (opaque: known to be 0 the first step over the keys is peeled off the loop, for 20 to 50 registers: the half-size tiles went to scratch, causal
+    // d = 64 2 x 12 x 500 .. 1000 17.1 us for 13.4)
+    asm volatile("" : "+s"(split));
     q_begin = id.own_begin; Lq = id.own_len; k_begin = id.walk_begin; Lk = id.walk_len;
   } else {
     int bh, rank;
@@ -148,7 +152,7 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
     Lq = Lk = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b]);
     listed = __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 2]) == 0;
     q_begin = k_begin = b * p.max_sq + (listed ? 0 : __builtin_amdgcn_readfirstlane(p.row_info[kRowInfo * b + 1]));
-  } else if (!mapped) {
+  } else if constexpr (!kLive) {
     if (!seq_extent(p.cu_q, b, p.total_q, p.max_sq, &q_begin, &Lq)) return;
     if (!seq_extent(p.cu_k, b, p.total_k, p.max_sk, &k_begin, &Lk)) Lk = 0;  // no keys: o = 0, lse = -inf
   }
@@ -362,6 +366,10 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
       qreg[ks] = rotate8<T>(qreg[ks], *reinterpret_cast<const typename E::vec4*>(ct + ks * 8),
                             *reinterpret_cast<const typename E::vec4*>(st + ks * 8), false);
   }
+  // Aligned, so that what precedes it does not move it against the instruction cache's lines: with one or two waves on a SIMD the loop waits for its
+  // own instructions, and the same code elsewhere took up to 8 % longer (us, d = 32 causal 3 x 3 heads x 4049 33.3 / 31.2, 2 x 8 x 2000 18.1 / 17.4, d = 128
+  // 2 x 8 x 2000 47.3 / 45.8, with keep words 2 x 12 x 1189 43.5 / 41.7; 300 drawn launches 0.996 in the mean).
+  asm volatile(".p2align 7");
   while (it < ntiles) {
     const int n0 = it * BN;
     // Opaque redefinition of the accumulators at the top of every iteration: without it the register allocator
@@ -700,6 +708,16 @@ __global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % k
       st_global16(obase + (int64_t)orow * p.o_rs + col, val);
     }
   }
+}
+
+template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias = 0, int KS = 1,
+          bool kWords = false>
+__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % kPaddedRows, KS, kWords)) fa_fwd_kernel(const FwdParams p) {
+  fa_fwd_body<T, D, BN, kRoomy, kCausal, kDropout, kSparse, kBias, KS, kWords, false>(p);
+}
+template <typename T, int D, int BN, bool kRoomy, bool kCausal, bool kDropout, bool kSparse, int kBias, int KS, bool kWords>
+__global__ void __launch_bounds__(256, fwd_waves(D, kDropout, kSparse, kBias % kPaddedRows, KS, kWords)) fa_fwd_live_kernel(const FwdParams p) {
+  fa_fwd_body<T, D, BN, kRoomy, kCausal, kDropout, kSparse, kBias, KS, kWords, true>(p);
 }
 
 }  // namespace fa

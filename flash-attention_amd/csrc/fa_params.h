@@ -78,7 +78,7 @@ struct FwdParams {
   int max_sq, max_sk;  // caller's bounds on the sequence lengths; longer sequences are truncated to them
   int sq_r;  // rounded max_seqlen_q = innermost extent of lse
   int nq_tiles;
-  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst, kLiveOrder
+  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst
   float scale;       // softmax_scale
   float scale_log2;  // softmax_scale * log2(e)
   float rp_keep;     // 1 / keep probability
@@ -162,7 +162,7 @@ struct BwdParams {
   int nk_tiles;      // key tiles of the dK/dV kernel
   int merged_dkdv_blocks, merged_nq_tiles;  // fa_bwd_merged_kernel: its dK/dV workgroups come first; query tiles of the dQ part
   int nq_tiles;      // query tiles of the dQ kernel
-  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst, kLiveOrder
+  int tile_group;    // causal launches: (batch, head) pairs of an XCD in flight together (map_tile); 0 = all; or kLongestFirst
   float scale;
   float scale_log2;
   float p_keep;
@@ -281,7 +281,7 @@ FA_DEVICE bool map_tile(int block, int tiles_per_bh, int BH, int* bh, int* rank,
   *rank = (j - q * tiles_per_bh + q) % tiles_per_bh;
   return *bh < BH;
 }
-// Ragged batches (tile_group == kLiveOrder): workgroup ids enumerate the tiles that hold rows, the dearest first, and behind them the ones
+// Ragged batches (the kernels' kLive variants): workgroup ids enumerate the tiles that hold rows, the dearest first, and behind them the ones
 // that hold none.  The other two orders deal out (pair, rank) slots as if every sequence were the longest: the slots past a shorter one's end
 // exit at once, but the dispatcher gives the ids of an XCD to its shader engines strictly in turn, so where the live slots recur with a
 // period of 2 or 4 half of the compute units hold every live workgroup and the rest stand idle until the ids have passed (4 x 16 heads x 600 ..
@@ -300,7 +300,7 @@ FA_DEVICE bool map_tile(int block, int tiles_per_bh, int BH, int* bh, int* rank,
 // group of 32 backwards: the unit with the dearest of one group gets the cheapest of the next.
 // info: null, or the lengths of a padded batch (FwdParams::row_info), whose `tiles` tiles a pair are all visited (rows to be zeroed).
 // lds_wave: 256 bytes of the wave's own.
-constexpr int kLongestFirst = -1, kLiveOrder = -2;
+constexpr int kLongestFirst = -1;
 struct TileId {
   int b, h, tile;
   int own_begin, own_len, walk_begin, walk_len;  // as seq_extent has them (walk: 0 keys or queries where it skips the entry)

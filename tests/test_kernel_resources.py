@@ -218,3 +218,35 @@ def test_block_layout_dkdv_keeps_its_block_list_in_registers():
                     lds.append(k["LDS Size"])
                 # two buffers of 64 rows of Q and dO, 16 elements of 2 bytes, and the rows' statistics, and less than the list's 32 bytes a thread more
                 assert lds[0] == lds[1] < 2 * 64 * (2 * 16 * 2 + 2 * 4) + 256 * 32 and lds[2] > lds[0], (dt, causal, drop, lds)
+
+
+@pytest.mark.timeout(600)
+def test_live_order_variants_are_bounded_like_the_slot_order():
+    """The kernels whose workgroups enumerate the tiles that hold rows keep the waves per SIMD of the same variant in the slot order and put at most
+    two registers more in scratch (the first step over the keys peeled off the loop took 20 to 50); at d = 16 dQ with a bias under a causal mask takes two
+    registers more than its waves allow.  The merged causal backward, which has no such variant, does not carry its code: few of its scalars are parked."""
+    units = ["fa_fwd_d64.hip", "fa_fwd_d128.hip", "fa_fwd_d16.hip", "fa_bwd_d64.hip", "fa_bwd_d128.hip", "fa_bwd_d16.hip"]
+    with ThreadPoolExecutor(6) as ex:
+        all_res = dict(zip(units, ex.map(_resources, units)))
+    pairs = 0
+    for unit, res in all_res.items():
+        for name, k in res.items():
+            if "_live_kernel" not in name:
+                continue
+            m = re.match(r"_ZN2fa\d+fa_(fwd|bwd_dq|bwd_dkdv|bwd_merged)_live_kernelI(.*)EEEvNS", name)
+            kind, args = m.group(1), m.group(2)
+            if kind == "bwd_dq":
+                args = re.sub(r"^(\w+?Li\d+ELi\d+ELb[01]ELi\d)E(Li\dELi\d)$", r"\1ELb0E\2", args)
+            elif kind == "bwd_dkdv":
+                args = re.sub(r"^(\w+?Li\d+ELb[01]ELi\d)E(Li\dELb[01])$", r"\1ELb0E\2", args)
+            elif kind == "bwd_merged":
+                args = re.sub(r"Li", "Lb0ELi", args, count=1)
+            slot = _pick(res, "fa_%s_kernelI%sEEEv" % (kind, args))
+            waves = slot["Occupancy"] - (1 if kind == "bwd_dq" and re.search(r"Li16ELi64ELb1ELi0ELb0ELi[12]E", args) else 0)
+            assert k["Occupancy"] >= waves and k["VGPRs Spill"] <= slot["VGPRs Spill"] + 2 and k["LDS Size"] == slot["LDS Size"], (unit, name, k, slot)
+            pairs += 1
+    assert pairs > 200, pairs
+    for dt in ("IDF16_", "IDF16b"):
+        for drop in ("Li0E", "Li2E"):
+            k = _pick(all_res["fa_bwd_d64.hip"], "fa_bwd_merged_kernel" + dt, "Lb1E" + drop + "EEv")
+            assert k["VGPRs Spill"] == 0 and k["SGPRs Spill"] <= 20, ("merged causal", dt, drop, k)
