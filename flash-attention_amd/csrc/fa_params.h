@@ -399,9 +399,17 @@ FA_DEVICE bool map_live(int block, const int32_t* cu_own, int total_own, int max
 // - Without a mask all of them (0.54 to 1.04 of the time over 100 drawn shapes, 0.92 in the middle), but dQ and dK/dV in one launch only
 //   where it is not resident at once: 3 x 12 x 414 .. 910 35.3 / 38.8, 2 x 16 x 728 .. 1234 48.1 / 51.7; 8 x 12 x 256 .. 512 33.4 / 31.8.
 // - Under a causal mask the other orders have their empty slots at one end.  The forward and dQ take it where at most nine tenths of the slots hold
-//   rows (38 x 16 x 414 .. 628 46.1 / 48.8) of more than 256-token sequences (64 x 8 x 42 .. 109 7.9 / 8.2, 64 x 16 x 172 .. 202 d = 128 42.4 /
-//   44.7) in more than 150 workgroups (2 x 12 x 553 .. 787 14.8 / 15.4), dK/dV, whose empty slots come last, where its pairs are taken in groups
-//   (causal_tile_group; 3 x 16 x 2821 .. 5841 dQ alone 481, both 441; 14 x 16 x 471 .. 703, no groups, 82.0 / 86.1).  At d = 32 many
+//   rows (38 x 16 x 414 .. 628 46.1 / 48.8), eight tenths at d = 128 without groups (forward 4 x 8 x 1836 .. 2384 61.3 / 63.8, 8 x 8 x 932 .. 1195 35.4 / 37.1;
+//   backward 8 x 5 x 773 .. 920 67.5 / 70.3), of more than 256-token sequences (64 x 8 x 42 .. 109 7.9 / 8.2, 64 x 16 x 172 .. 202 d = 128 42.4 / 44.7),
+//   in more workgroups with rows than `least`, below which the longer prologue is all there is: forward d = 64 4 x 12 x 344 .. 400 (163 of them) 8.1 / 8.5,
+//   d = 16 12 x 3 x 631 .. 1147 (268) 10.7 / 11.2, d = 32 6 x 5 x 750 .. 1056 (226) 10.6 / 11.3, 8 x 12 x 181 .. 464 (290) 7.5 / 7.9; backward d = 32 2 x 12 x
+//   1362 .. 2671 (390) 69.5 / 73.5, d = 128 12 x 3 x 385 .. 593 (155) 48.3 / 49.4; and not half-size tiles of the d = 64 forward from 640 on, over a round
+//   of what is resident at once, but for long walks (12 x 12 x 204 .. 928 18.9 / 20.6, 5 x 24 x 268 .. 1115 19.2 / 20.6, 3 x 24 x 578 .. 1864 28.8 / 31.2;
+//   2 x 24 x 471 .. 3139 51.5 / 45.5).  Over 900 drawn shapes without groups a forward takes 0.95 (d = 16 to 64), 0.99 (128), at most 1.06, a backward 0.99, at
+//   most 1.06.  dK/dV, whose empty slots come last, takes it where its pairs are taken in groups
+//   (causal_tile_group; 3 x 16 x 2821 .. 5841 dQ alone 481, both 441; 14 x 16 x 471 .. 703, no groups, 82.0 / 86.1) of more than 640 tokens (backward
+//   d = 128 48 x 12 x 183 .. 262 90.2 / 94.3, 48 x 12 x 226 .. 452 164.8 / 170.2, d = 64 64 x 24 x 147 .. 587 261 / 270; up to 8 % given up where one of the
+//   sequences is long, 16 x 16 x 82 .. 631 89.3 / 82.0).  At d = 32 many
 //   pairs in groups stay with them, whose K and V it would read again: 64 x 16 x 509 .. 926 100.9 / 122.5, 38 x 12 x 353 .. 1766 91.2 / 101.2;
 //   and so does what live_order_rereads names.
 //
@@ -432,7 +440,10 @@ inline bool live_order_launch(LiveKernel kernel, int head_dim, bool causal, int 
   if (head_dim <= 32 && tile_group > 0 && B * H >= 256) return false;
   const int64_t live = (int64_t)H * (total + (int64_t)64 * B) / 128, slots = (int64_t)B * H * ((max_s + 127) / 128);
   if (tile_group > 0 && live_order_rereads(kernel, head_dim, live, slots, B, H, total)) return false;
-  return max_s > 256 && live > 150 && 10 * live <= 9 * slots;
+  const bool fwd = kernel == kLiveFwd, half_size = tiles > (max_s + 127) / 128;
+  const int least = fwd ? (head_dim == 16 ? 300 : head_dim == 32 ? 330 : 200) : head_dim == 32 ? 450 : head_dim == 128 ? 200 : 150;
+  if (tile_group <= 0 && fwd && head_dim == 64 && half_size && live >= 640 && max_s < 2000) return false;
+  return max_s > 256 && live > least && 10 * live <= (tile_group <= 0 && head_dim == 128 ? 8 : 9) * slots;
 }
 inline bool live_order_rows(int B, int tiles) { return B <= 64 && tiles <= 64; }
 // The forward over a padded batch, whose number of tokens is not known here (map_live's info).  Without a mask wherever there is more than one entry to

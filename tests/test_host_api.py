@@ -887,6 +887,20 @@ def test_live_order_where_measured(tmp_path):
                                     "live_order_rows(1, 65)"]) == [0, 1, 0, 0]
 
 
+def test_live_order_not_where_launches_are_short(tmp_path):
+    """ragged causal launches without groups: of few workgroups, of half-size tiles just over a round of the chip, of fuller slots at head dim 128"""
+    cases = [  # kernel, head dim, batch, heads, longest, shortest / longest, rows of a tile, live order?
+        ("kLiveFwd", 64, 4, 12, 400, 0.86, 64, 0), ("kLiveFwd", 16, 12, 3, 1147, 0.55, 64, 0), ("kLiveFwd", 16, 12, 5, 557, 0.26, 64, 0),  # us in the slot order / live:
+        ("kLiveFwd", 32, 6, 5, 1056, 0.71, 64, 0), ("kLiveFwd", 32, 8, 12, 464, 0.39, 64, 0), ("kLiveDq", 32, 2, 12, 2671, 0.51, 64, 0),  # 8.1 / 8.5, 10.7 / 11.2, 7.2 / 7.7,
+        ("kLiveDq", 128, 12, 3, 593, 0.65, 64, 0), ("kLiveFwd", 64, 12, 12, 928, 0.22, 64, 0), ("kLiveFwd", 64, 3, 24, 1864, 0.31, 64, 0),  # 10.6 / 11.3, 7.5 / 7.9, 69.5 / 73.5,
+        ("kLiveFwd", 128, 4, 8, 2384, 0.77, 128, 0), ("kLiveFwd", 128, 8, 8, 1195, 0.78, 128, 0), ("kLiveDq", 128, 8, 5, 920, 0.84, 64, 0),  # 48.3 / 49.4, 18.9 / 20.6, 28.8 / 31.2, ..
+        ("kLiveFwd", 64, 2, 24, 3139, 0.15, 64, 1), ("kLiveFwd", 64, 5, 12, 3299, 0.3, 128, 1), ("kLiveFwd", 128, 12, 5, 1209, 0.2, 64, 1),  # 51.5 / 45.5, 81.0 / 61.0, 32.2 / 24.6
+        ("kLiveFwd", 32, 12, 5, 1738, 0.2, 64, 1), ("kLiveFwd", 64, 6, 5, 3653, 0.17, 64, 1), ("kLiveDq", 32, 12, 12, 1230, 0.4, 64, 1)]
+    got = _launch_rules(tmp_path, ["live_order_launch(%s, %d, 1, %d, %d, %d, %d, 1, %d, 0, %d)" % (
+        k, d, b, h, _spread(n, f, b), n, -(-n // rows), -(-b * h // 8) * 8 * -(-n // rows)) for k, d, b, h, n, f, rows, _ in cases])
+    assert got == [c[-1] for c in cases], [c for c, g in zip(cases, got) if g != c[-1]]
+
+
 def test_live_order_batches_of_the_gpu_tests_take_it(tmp_path):
     """forward, dQ and dK/dV of the batch on which the variants are compared (16 heads, 1500 tokens and 31 sequences of 300 to 510), in full-size and
     half-size tiles, with a causal mask and without; not with 33 empty sequences behind it"""
