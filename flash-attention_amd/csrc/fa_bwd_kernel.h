@@ -601,14 +601,21 @@ FA_DEVICE void fa_bwd_dkdv_body(const BwdParams& p, const int block, unsigned ch
   }
 }
 
+// Waves per SIMD that the variants are bounded to.  Four where the compiler takes a register or a few more than they allow (128) and has them to
+// spare, without a mask: over a block layout at d = 16, with keep words and rotary at d = 32.
+constexpr int dkdv_waves(int d, bool causal, int drop, bool sparse, int bias, bool rot, int min_blocks) {
+  if (!causal && bias == 0 && ((d == 16 && sparse && drop == 0) || (d == 32 && drop == 2 && rot))) return 4;
+  if (drop == 0 && d <= 64 && bias != kBiasTensor) return 3;
+  return d == 128 && bias == kBiasTensor ? 1 : min_blocks;
+}
 template <typename T, int D, bool kCausal, int kDrop, bool kSparse, int kBias = 0, bool kRot = false>
-__global__ void __launch_bounds__(256, (kDrop == 0 && D <= 64 && kBias != kBiasTensor) ? 3 : ((D == 128 && kBias == kBiasTensor) ? 1 : BwdCfg<T, D, kDrop == 1>::kMinBlocks)) fa_bwd_dkdv_kernel(const BwdParams p) {
+__global__ void __launch_bounds__(256, (dkdv_waves(D, kCausal, kDrop, kSparse, kBias, kRot, BwdCfg<T, D, kDrop == 1>::kMinBlocks))) fa_bwd_dkdv_kernel(const BwdParams p) {
   using Cfg = BwdCfg<T, D, kDrop == 1>;
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[Cfg::kLdsBytes + (kBias == kBiasTensor ? 4 * Cfg::kBiasTileBytes : 0)];
   fa_bwd_dkdv_body<T, D, kCausal, kDrop, kSparse, kBias, kRot, false, false>(p, blockIdx.x, lds_raw);
 }
 template <typename T, int D, bool kCausal, int kDrop, int kBias, bool kRot>
-__global__ void __launch_bounds__(256, ((kDrop == 0 && D <= 64) ? 3 : BwdCfg<T, D, kDrop == 1>::kMinBlocks)) fa_bwd_dkdv_live_kernel(const BwdParams p) {
+__global__ void __launch_bounds__(256, (dkdv_waves(D, kCausal, kDrop, false, kBias, kRot, BwdCfg<T, D, kDrop == 1>::kMinBlocks))) fa_bwd_dkdv_live_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[BwdCfg<T, D, kDrop == 1>::kLdsBytes];
   fa_bwd_dkdv_body<T, D, kCausal, kDrop, false, kBias, kRot, false, true>(p, blockIdx.x, lds_raw);
 }

@@ -250,3 +250,24 @@ def test_live_order_variants_are_bounded_like_the_slot_order():
         for drop in ("Li0E", "Li2E"):
             k = _pick(all_res["fa_bwd_d64.hip"], "fa_bwd_merged_kernel" + dt, "Lb1E" + drop + "EEv")
             assert k["VGPRs Spill"] == 0 and k["SGPRs Spill"] <= 20, ("merged causal", dt, drop, k)
+
+
+@pytest.mark.timeout(600)
+def test_small_head_dkdv_variants_keep_four_waves():
+    """dK/dV over a block layout at d = 16: four waves per SIMD without dropout, as with ALiBi; the LDS of all its variants is two buffers of a pair of 64 x 16
+    tiles, 64 bytes that the wider transposed reads run past a row and the rows' statistics, with a bias tensor 4 KB a wave more and nothing for
+    the block list (2 KB or more wherever it was).  With keep words and rotary at d = 32: four waves."""
+    with ThreadPoolExecutor(2) as ex:
+        d16, d32 = ex.map(_resources, ("fa_bwd_d16.hip", "fa_bwd_d32.hip"))
+    tiles = 2 * 2 * 64 * 16 * 2 + 64 + 2 * 2 * 64 * 4
+    for dt in ("IDF16_", "IDF16b"):
+        for causal in ("Lb0E", "Lb1E"):
+            for bias, waves in (("Li0E", 4), ("Li1E", 4), ("Li2E", 3)):
+                for drop in ("Li0E", "Li1E"):
+                    k = _pick(d16, "fa_bwd_dkdv_kernel%sLi16E" % dt, "Li16E" + causal + drop + "Lb1E" + bias + "Lb0EEEv")
+                    assert k["LDS Size"] == tiles + (4 * 64 * 32 * 2 if bias == "Li2E" else 0), (dt, causal, drop, bias, k)
+                    if drop == "Li0E":
+                        assert k["Occupancy"] >= waves and k["VGPRs Spill"] == 0, (dt, causal, bias, k)
+        for name, flags in (("fa_bwd_dkdv_kernel%sLi32E", "Lb0ELi2ELb0ELi0ELb1EEEv"), ("fa_bwd_dkdv_live_kernel%sLi32E", "Lb0ELi2ELi0ELb1EEEv")):
+            k = _pick(d32, name % dt, flags)
+            assert k["Occupancy"] >= 4 and k["VGPRs Spill"] == 0, (name, dt, k)
