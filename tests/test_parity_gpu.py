@@ -1336,10 +1336,12 @@ def test_blocksparse_results_do_not_follow_earlier_layouts():
             assert torch.equal(x, y), seed
 
 
-@pytest.mark.parametrize("Sq,Sk,H,B", [(16, 100, 1, 1), (300, 257, 3, 3), (130, 15900, 2, 2), (16390, 300, 1, 1)])
+@pytest.mark.parametrize("Sq,Sk,H,B", [(16, 100, 1, 1), (300, 257, 3, 3), (130, 15900, 2, 2), (16390, 300, 1, 1),
+                                        (16, 100, 129, 1), (300, 257, 9, 8)])
 def test_blocksparse_tiles_dearest_first(Sq, Sk, H, B):
     """Workgroups take a layout's query tiles and key blocks dearest first: one tile of each, a last key block half of whose keys have no
-    tile, heads that are no multiple of the XCDs, 63 key blocks, and more row blocks than the kernel that ranks them has threads"""
+    tile, heads that are no multiple of the XCDs, 63 key blocks, and more row blocks than the kernel that ranks them has threads (and in their own
+    order where no compute unit has two: the first two)"""
     from flash_attn import flash_attn_gfx950 as be
     from flash_attn.flash_blocksparse_attn_interface import convert_blockmask
     D, dtype = 64, torch.float16
