@@ -1362,7 +1362,7 @@ def test_blocksparse_tiles_dearest_first(Sq, Sk, H, B):
         check_against_oracle({"out": o, "dq": dq, "dk": dk, "dv": dv}, ref, half, dtype, what="block layout %d x %d" % (Sq, Sk))
 
 
-@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
 @pytest.mark.parametrize("listed", [1, 2, 3, 5])
 def test_blocksparse_rows_outside_a_key_blocks_list_do_not_reach_its_gradients(D, listed):
     """Tiles of four 16-row blocks at the end of a key block's list are filled up with rows it does list, switched off: a row that is NaN and
