@@ -271,6 +271,17 @@ def test_blockmask_row_order_is_a_permutation_that_groups_similar_rows():
     assert lib.fa_blocksparse_row_order(None, 4, 4, None) == -1
 
 
+@pytest.mark.parametrize("rows, cols, crc", [(256, 16, 501783833), (37, 5, 137879411), (1, 1, 558161692), (100, 64, 4146698765), (130, 70, 3019294916)])
+def test_blockmask_row_order_stays_what_it_was(rows, cols, crc):
+    """The order of a layout, which results follow in their last bits, is the one that recomputing every group's lists at every exchange gives (checksums
+    of its orders): whole and partial groups, one row, one word of key blocks and two"""
+    import zlib
+    from flash_attn import flash_attn_gfx950 as be
+    r, c = torch.arange(rows)[:, None], torch.arange(cols)[None]
+    layout = ((r * 7 + c * 13) * (r + 3 * c + 1) + r * r // 5) % 11 < 4
+    assert zlib.crc32(be.blockmask_row_order(layout).numpy().tobytes()) == crc
+
+
 # ---------------------------------------------------------------- host helpers
 def _layouts_to_order(n):
     """0 / 1 layouts whose row orders are not the plain one and differ"""
