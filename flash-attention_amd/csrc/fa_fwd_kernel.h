@@ -247,7 +247,8 @@ FA_DEVICE void fa_fwd_body(const FwdParams& p) {
   // wave-uniform and kept in scalar registers: the activity bits of 64 consecutive key blocks (16384 keys) for the query tile and for
   // the wave's two row blocks, and the lanes whose row block attends the tile in hand.  The search sits in front of the next tile's loads
   // in every wave, a chain of dependent scalar instructions and branches, so it runs once per key block: within one the next tile is the
-  // next (d = 64, a quarter to a third of the 16 x 256 blocks, 1 x 8 heads x 4959 70.3 / 66.3 us, 2 x 16 x 5584 148 / 140).
+  // next (d = 64, a quarter to a third of the 16 x 256 blocks, 1 x 8 heads x 4959 70.3 / 66.3 us, 2 x 16 x 5584 148 / 140; the dQ kernel, with no register to
+  // spare, is 1 % slower for it and searches tile by tile).
   uint64_t tile_bits = 0, bits_a = 0, bits_b = 0;
   int bits_word = -1;
   const int qt_u = __builtin_amdgcn_readfirstlane(qt);
