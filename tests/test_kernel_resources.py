@@ -4,11 +4,11 @@ The d = 64 kernels are tuned to the register counts at which one more wave fits 
 One extra live register in a main loop silently costs a wave per SIMD or turns into scratch traffic, so the counts the
 compiler reports (-Rpass-analysis=kernel-resource-usage) are pinned here for the variants the headline workloads run.
 """
-import functools
 import os
 import re
 import subprocess
 import sys
+import threading
 from concurrent.futures import ThreadPoolExecutor
 
 import pytest
@@ -18,8 +18,20 @@ sys.path.insert(0, os.path.join(ROOT, "flash-attention_amd"))
 import build as fa_build  # noqa: E402
 
 
-@functools.lru_cache(maxsize=None)
+_UNITS = ["fa_%s_d%d.hip" % (w, d) for w in ("bwd", "fwd") for d in (128, 64, 32, 16)] + ["fa_bwd_fused.hip", "fa_decode.hip"]
+_pool, _compiled, _compiled_lock = ThreadPoolExecutor(8), {}, threading.Lock()
+
+
 def _resources(src):
+    """What the compiler reports of a unit's kernels.  Units take up to two minutes: the first call asks for all of them, unless other processes do, too."""
+    with _compiled_lock:
+        for unit in [src] + (_UNITS if "PYTEST_XDIST_WORKER" not in os.environ else []):
+            if unit not in _compiled:
+                _compiled[unit] = _pool.submit(_compile, unit)
+    return _compiled[src].result()
+
+
+def _compile(src):
     cmd = [fa_build.HIPCC] + fa_build.FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-c",
                                                os.path.join(fa_build.CSRC, src), "-o", os.devnull]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
